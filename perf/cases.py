@@ -205,6 +205,13 @@ def _device_state(case, seed):
     return s, g, proto, t
 
 
+def _step_state(case, seed):
+    """_device_state and a batch of images."""
+    s, g, proto, t = _device_state(case, seed)
+    s["x"], _ = _data(g, proto, case["batch"], case["inputs"], t)
+    return s
+
+
 def prepare(case, seed):
     kind = case["kind"]
     if kind in ("infer", "layer", "fit", "epoch"):
@@ -222,11 +229,10 @@ def prepare(case, seed):
         rng = np.random.default_rng(seed)
         return {**s, "perm": rng.permutation(case["samples"]), "hc_perm": rng.permutation(case["hyper"])}
     _capi.init()
-    s, g, proto, t = _device_state(case, seed)
     if kind == "rewire":
-        return s
+        return _device_state(case, seed)[0]
     n, hyper, mini, b = case["inputs"], case["hyper"], case["mini"], case["batch"]
-    s["x"], _ = _data(g, proto, b, n, t)
+    s, t = _step_state(case, seed), torch.float32 if case["dtype"] == "f32" else torch.float64
     s["act"] = torch.empty(b, hyper * mini, device="cuda", dtype=t)
     # a sparse layer of a shape the row-list kernel takes is run over its connected rows
     s["sparse"] = case["density"] <= 0.7 and mini % (4 if case["dtype"] == "f32" else 2) == 0 and mini <= 200
@@ -331,3 +337,54 @@ def tolerance(case):
     if case["dtype"] == "f32":
         return {"rel": 1e-4, "max": 6e-3, "differ": 1e-3}
     return {"rel": 2e-13, "max": 1.2e-11, "differ": 0.0}
+
+
+# -------------------------------------------------------------------------------------- results in 64 bits
+def _softmax_units(logits, mini):
+    return torch.softmax(logits.view(logits.shape[0], -1, mini), 2).view_as(logits)
+
+
+def _exact_step(s, x, tau, khalf, pmin, taubdt, mini):
+    """One training step on the state `s` (doubles, updated in place): activations, traces, bias, weights, mask."""
+    act = _softmax_units(x @ s["W"] + s["bias"], mini)
+    cthr = tau / 2
+    for name, batch_mean in (("Ci", x.mean(0)), ("Cj", act.mean(0))):
+        s[name] = (s[name] * (1 - tau) + tau * batch_mean).clamp_(min=0)
+    s["Cij"].mul_(1 - tau).add_(x.t() @ act, alpha=tau / x.shape[0]).clamp_(min=0)
+    p4 = pmin / 4
+    k = 1 + (khalf - 1) * p4 * p4 / (s["Cj"] - p4) ** 2
+    k[(s["Cj"] < p4) | (k < khalf)] = khalf
+    s["kbi"] = (1 - taubdt) * s["kbi"] + taubdt * k
+    s["bias"] = s["kbi"] * torch.where(s["Cj"] < cthr, 2 * cthr, s["Cj"]).log()
+    s["W"] = _weights(s["Ci"], s["Cj"], s["Cij"], cthr)
+    s["W"][:, s["Cj"] < cthr] = 0
+    s["W"].view(x.shape[1], -1, mini).mul_(s["wmask"][:, :, None])
+    return act
+
+
+def exact(case, seed):
+    """None: whole numbers (the class, the mask), weights of a step that rewires, and epochs, over which the
+    rounding of one step moves single samples of the next ones."""
+    kind, dtype = case["kind"], _np_type(case)
+    tau, khalf, pmin, taubdt = (float(dtype(v)) for v in (TAUPDT, KHALF, PMIN, TAUBDT))
+    if kind == "step":
+        s = {k: v.double() if isinstance(v, torch.Tensor) and v.is_floating_point() else v
+             for k, v in _step_state(case, seed).items()}
+        act = _exact_step(s, s["x"], tau, khalf, pmin, taubdt, case["mini"])
+        rewires = case["dtype"] == "f64"
+        return {"act": act, **{k: s[k] for k in ("bias", "Ci", "Cj", "Cij", "kbi")},
+                "W": None if rewires else s["W"], "wmask": None}
+    if kind == "layer" or (kind == "infer" and case["what"] == "forward"):
+        p = prepare(case, seed)
+        states = [{"W" if k == "weights" else k: torch.from_numpy(np.array(v)).double().cuda()
+                   for k, v in _layer_state(layer).items()} for layer in p["layers"]]
+        if kind == "infer":
+            x = torch.from_numpy(p["x"]).double().cuda()
+            for layer, s in zip(p["layers"], states):
+                x = _softmax_units(x @ s["W"] + s["bias"], layer.minicolumns)
+            return x
+        s, tau = states[0], float(dtype(p["layers"][0].taupdt))
+        for x in p["x"]:
+            act = _exact_step(s, torch.from_numpy(x).double().cuda(), tau, khalf, pmin, taubdt, case["mini"])
+        return {"act": act, "weights": s["W"], **{k: s[k] for k in ("bias", "Ci", "Cj", "Cij", "kbi")}, "wmask": None}
+    return None
