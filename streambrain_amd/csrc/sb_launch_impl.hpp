@@ -578,8 +578,9 @@ int launch_gather_rows_blocked(hipStream_t st, T *dst, T *plain, const T *src, c
   SB_REQUIRE(dst && src, "null pointer");
   SB_REQUIRE(rows > 0 && cols > 0 && cdiv(rows, 16) < (1L << 31), "bad shape");
   ProfScope prof_(st, K_GATHER);
-  hipLaunchKernelGGL((k_gather_rows_blocked<T>), dim3((unsigned)cdiv(rows, 16)), dim3(256), 0, st, dst, plain,
-                     src, idx, rows, cols);
+  const long col_groups = cdiv(cols, 256) < 65535 ? cdiv(cols, 256) : 65535;
+  hipLaunchKernelGGL((k_gather_rows_blocked<T>), dim3((unsigned)cdiv(rows, 16), (unsigned)col_groups), dim3(256), 0,
+                     st, dst, plain, src, idx, rows, cols);
   SB_LAUNCH_CHECK();
   return 0;
 }
