@@ -1,72 +1,29 @@
-// Register-resident variant of the greedy swap loop of the mask rewiring (omp.cc:289-315, where
-// "omp.cc" = BCPNN/backend/_kernels/kernels_openmp_internal.cc of the reference) for layers with at
-// most NT*R input rows: one workgroup of NT threads, thread t owns rows t, t+NT, ...; score
-// nominators, connection counts, mask bits and scores stay in registers over all iterations.  Per
-// iteration: a DPP / shuffle reduction inside each wavefront, one partial result per wavefront through
-// LDS, a second reduction that leaves the decision in every lane -- one barrier.  Same decisions as
-// k_mask_swap (which keeps its state in global memory and serves larger layers).
+// The greedy swap loop of the mask rewiring (omp.cc:289-315, where "omp.cc" =
+// BCPNN/backend/_kernels/kernels_openmp_internal.cc of the reference), on the scores that k_mask_scores has left in
+// memory.  One workgroup.
+//
+// An iteration changes nothing but the two rows it swaps, so over at most 16 iterations only the 16 best silent rows
+// and the 16 worst active rows of the state they start from (plus rows that changed sides on the way) can ever be
+// picked.  The kernel therefore works in rounds of 16 iterations:
+//   phase A (whole workgroup): the 16 best rows of either side in the strict order (score, row index), which is the
+//     order the picks take them in, equal scores included.  The rows are dealt into 64 bins by their index modulo
+//     64; the 16th largest of the 64 bins' best is a bound that at least 16 rows reach and few others do (about 3
+//     more where the order knows nothing of the index), the rows that reach it go to a list in LDS, and a
+//     row's place is the number of listed rows ahead of it;
+//   phase B (one wavefront, one candidate per lane and side): the iterations themselves, with the same picks, tie
+//     rule, break conditions and score expression as a full scan.
+// A round reads the N scores and sides twice (the second time from L2) and has six barriers; its time is latency.
+// What a round does not cover -- a side whose first candidate row has a NaN score or may come to have one, or a
+// list that overflows -- is left to a full scan per iteration (swap_by_scans).
+// 27648 rows, floats: 25 us; 318 us with the state in registers and a radix select on 2048-bin histograms, whose
+// counters all threads hit together (scores share their leading bits), and a scan per iteration once any score is
+// NaN, as the scores of inputs that are always on are (1 - Ci = 0).
 #pragma once
 #include "sb_kernels.hpp"
 
 namespace sb {
 
-template <typename T>
-__device__ __forceinline__ T mask_score(T nom, int csum) {
-  // nominator / (1.0 + (REAL)csum): formed in double and narrowed, as the reference's expression
-  return (T)((double)nom / (1.0 + (double)(T)csum));
-}
-
-// candidate row: score and row index (-1: none)
-template <typename T>
-struct RowCand {
-  T val;
-  int idx;
-};
-template <typename T>
-__device__ __forceinline__ RowCand<T> shfl_xor_cand(RowCand<T> c, int o) {
-  return RowCand<T>{__shfl_xor(c.val, o), __shfl_xor(c.idx, o)};
-}
-template <int CTRL, typename T>
-__device__ __forceinline__ RowCand<T> dpp_cand(RowCand<T> c) {
-  return RowCand<T>{dpp_move<CTRL>(c.val), dpp_move<CTRL>(c.idx)};
-}
-// reduce over the 16 lanes of each row with `pick`; every lane of the row ends with the result
-#define SB_ROW_REDUCE(pick, c)                        \
-  do {                                                \
-    c = pick(c, dpp_cand<kDppSwap1, T>(c));           \
-    c = pick(c, dpp_cand<kDppSwap2, T>(c));           \
-    c = pick(c, dpp_cand<kDppHalfMirror, T>(c));      \
-    c = pick(c, dpp_cand<kDppMirror, T>(c));          \
-  } while (0)
-// ascending scan with ">=" keeps the later of two equal maxima; with "<=" the later of two equal minima
-template <typename T>
-__device__ __forceinline__ RowCand<T> pick_max(RowCand<T> a, RowCand<T> b) {
-  const bool take = b.idx >= 0 && (a.idx < 0 || b.val > a.val || (b.val == a.val && b.idx > a.idx));
-  return take ? b : a;
-}
-template <typename T>
-__device__ __forceinline__ RowCand<T> pick_min(RowCand<T> a, RowCand<T> b) {
-  const bool take = b.idx >= 0 && (a.idx < 0 || b.val < a.val || (b.val == a.val && b.idx > a.idx));
-  return take ? b : a;
-}
-template <typename T>
-__device__ __forceinline__ RowCand<T> pick_first(RowCand<T> a, RowCand<T> b) {
-  const bool take = b.idx >= 0 && (a.idx < 0 || b.idx < a.idx);
-  return take ? b : a;
-}
-
-// ---------------------------------------------------------------------------------------------------
-// Fast path of the swap loop.  Over at most 16 iterations only the 16 best silent rows and the 16 worst
-// active rows of the INITIAL state (plus rows that changed sides on the way) can ever be picked, because
-// an iteration changes nothing but the two rows it swaps.  So:
-//   phase A (whole workgroup): a radix select on monotone integer keys of the scores finds a threshold
-//     per group such that the rows beyond it are a small superset of those 16; a large group of exactly
-//     equal scores at the threshold (rows of dead inputs all score 0) is cut down to its highest indices,
-//     which is the order the tie rule would take them in;
-//   phase B (one wavefront, one candidate per lane and group): the iterations themselves, with the same
-//     picks, tie rule, break conditions and score expression as the full scan.
-// Anything the fast path does not cover (NaN scores, more iterations, too many near-equal candidates)
-// returns false and the caller runs the full scan.
+// Monotone integer keys of the scores.
 template <typename T>
 struct ScoreKey;
 template <>
@@ -156,247 +113,247 @@ __device__ __forceinline__ KeyIdx<uint32_t> wave_pick(KeyIdx<uint32_t> c) {
   return KeyIdx<uint32_t>{(uint32_t)(m >> 32), (int)(uint32_t)m - 1};
 }
 
-// Scatter inside a wavefront: v of every lane with `on` lands in lane `to`.  The targets must be distinct and
-// must be lanes that push themselves (a permutation among the pushing lanes); the other lanes keep 0.
-__device__ __forceinline__ uint32_t push_to_lane(uint32_t v, int to, bool on) {
-  const int lane = (int)(threadIdx.x & 63);
-  return (uint32_t)__builtin_amdgcn_ds_permute((on ? to : lane) * 4, on ? (int)v : 0);
-}
-__device__ __forceinline__ uint64_t push_to_lane(uint64_t v, int to, bool on) {
-  return ((uint64_t)push_to_lane((uint32_t)(v >> 32), to, on) << 32) | push_to_lane((uint32_t)v, to, on);
-}
-
-__device__ __forceinline__ void note_changed(int *changed, int *nchanged, int row) {
+__device__ __forceinline__ void note_changed(int *changed, int *nchanged, long row) {
   const int at = atomicAdd(nchanged, 1);
-  if (at < kMaxChangedRows) changed[at] = row;
+  if (at < kMaxChangedRows) changed[at] = (int)row;
 }
 
-template <typename T, int NT, int R>
-struct MaskSwapFast {
+// reduction over a wavefront of an integer; the result is in every lane
+template <typename Op>
+__device__ __forceinline__ int wave_reduce(int v, Op op) {
+  v = row16_reduce(v, op);
+  return op(op(__builtin_amdgcn_readlane(v, 0), __builtin_amdgcn_readlane(v, 16)),
+            op(__builtin_amdgcn_readlane(v, 32), __builtin_amdgcn_readlane(v, 48)));
+}
+
+template <typename T>
+struct MaskSwap {
   using SK = ScoreKey<T>;
   using K = typename SK::K;
-  static constexpr int TOPK = 16, CAP = 48, DIG = 11, BINS = 1 << DIG, PER = BINS / NT, NWV = NT / 64;
-  // index bins of the tie cut: (row index) >> ISH, the smallest shift that fits NT * R rows into BINS bins
-  static constexpr int ish_for(int rows) { return rows <= BINS ? 0 : 1 + ish_for((rows + 1) / 2); }
-  static constexpr int ISH = ish_for(NT * R);
-  static_assert(((NT * R - 1) >> ISH) < BINS && BINS % NT == 0, "row indices must fit the index histogram");
+  static constexpr int NT = 1024, NWV = NT / 64, TOP = 16, LIST = 1024, U = 8;
   struct Shared {
-    unsigned hist[2][BINS];
-    int cand[2][64], cand_cs[2][64];  // candidate rows, their connection counts ...
-    T cand_nom[2][64];                // ... and score nominators
-    int ncand[2], sel_bin[2], sel_above[2], wtot[2][NWV];
-    K eq_min[2], eq_max[2];
+    K bin_key[2][NWV][64];  // per side and wavefront: the best row of each bin ...
+    int bin_idx[2][NWV][64];
+    K list_key[2][LIST];  // ... and the rows at or beyond the bound
+    int list_idx[2][LIST];
+    K bound_key[2];
+    int bound_idx[2], nlist[2], top[2][TOP];
+    int nan_first[2], ahead[2];  // lowest row with a NaN score; rows with a score below it
+    int swaps;
   };
 
-  // Largest bin b with (rows in bins >= b) >= need, per group; sel_bin stays -1 when the histogram holds
-  // fewer than `need` rows.  Two barriers inside.
-  static __device__ void crossing(Shared &sh, const int (&need)[2], const bool (&active)[2]) {
+  // This thread's rows i0 + tid, i0 + tid + NT, ..: scores and sides (2: no candidate, or no row), loads in flight
+  // together.
+  struct Rows {
+    T s[U];
+    int m[U];
+  };
+  static __device__ __forceinline__ void load_rows(const MaskArgs<T> &a, Rows &v, int i0) {
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const long i = (long)i0 + (int)threadIdx.x + NT * u;
+      v.s[u] = a.score[i < a.N ? i : 0];
+      v.m[u] = i < a.N ? a.side[i] : 2;
+    }
+  }
+  // Calls f(row, side, score) for all of this thread's rows, which lie in bin tid % 64, in ascending order.
+  // `first`: the first NT * U rows, already loaded.  (No guards around the calls: what they hold is a few selects.)
+  template <typename F>
+  static __device__ __forceinline__ void for_rows(const MaskArgs<T> &a, const Rows &first, F &&f) {
+    const int tid = threadIdx.x;
+#pragma unroll
+    for (int u = 0; u < U; u++) f(tid + NT * u, first.m[u], first.s[u]);
+    for (long i0 = NT * U; i0 < a.N; i0 += NT * U) {
+      Rows v;
+      load_rows(a, v, (int)i0);
+#pragma unroll
+      for (int u = 0; u < U; u++) f((int)i0 + tid + NT * u, v.m[u], v.s[u]);
+    }
+  }
+  // in both groups the wanted rows are those with the LARGEST keys
+  static __device__ __forceinline__ K key_of(int side, T s) {
+    const K u = SK::of(s);
+    return side == 0 ? u : (K)~u;
+  }
+
+  // One round of at most TOP iterations.  Returns the number of swaps, or -1: nothing was changed, and the
+  // round has to be left to the full scan.  (uniform)
+  static __device__ int round(const MaskArgs<T> &a, Shared &sh, int iterations, int *changed, int *nchanged) {
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-    int c[2], incl[2];
-#pragma unroll
-    for (int g = 0; g < 2; g++) {
-      c[g] = 0;
-#pragma unroll
-      for (int b = 0; b < PER; b++) c[g] += (int)sh.hist[g][PER * tid + b];
-      int s = c[g];
-#pragma unroll
-      for (int o = 1; o < 64; o <<= 1) {  // inclusive suffix sum inside the wavefront
-        const int v = __shfl_down(s, o);
-        if (lane + o < 64) s += v;
-      }
-      incl[g] = s;
-      if (lane == 0) sh.wtot[g][wv] = s;
-    }
+    constexpr int kNone = 0x7fffffff;
+    if (tid < 2) sh.nlist[tid] = 0, sh.nan_first[tid] = kNone, sh.ahead[tid] = 0;
     __syncthreads();
-#pragma unroll
-    for (int g = 0; g < 2; g++) {
-      // (all totals requested at once; the ones of the wavefronts behind this one are added)
-#pragma unroll
-      for (int w2 = 0; w2 < NWV; w2++) {
-        const int v = sh.wtot[g][w2];
-        incl[g] += w2 > wv ? v : 0;
-      }
-      const int after = incl[g] - c[g];
-      if (active[g] && after < need[g] && need[g] <= incl[g]) {  // exactly one thread per group
-        int acc = after;
-        for (int b = PER - 1; b >= 0; b--) {
-          const int hb = (int)sh.hist[g][PER * tid + b];
-          if (acc + hb >= need[g]) {
-            sh.sel_bin[g] = PER * tid + b;
-            sh.sel_above[g] = acc;
-            break;
-          }
-          acc += hb;
-        }
-      }
-    }
-    __syncthreads();
-  }
-
-  static __device__ void clear(Shared &sh) {
-    for (int i = threadIdx.x; i < 2 * BINS; i += NT) (&sh.hist[0][0])[i] = 0u;
-    if (threadIdx.x < 2) sh.sel_bin[threadIdx.x] = -1;
-  }
-
-  // true: the swaps are done and written back; false: nothing was changed, run the full scan
-  // changed / nchanged (LDS): the rows that end on the other side are appended there
-  static __device__ bool run(const MaskArgs<T> &a, Shared &sh, const T (&score)[R], const int (&m)[R],
-                             const T (&nom)[R], const int (&cs)[R], int *changed, int *nchanged) {
-    const int tid = threadIdx.x, lane = tid & 63;
-    K key[R];
-#pragma unroll
-    for (int k = 0; k < R; k++) {
-      const K u = SK::of(score[k]);
-      key[k] = m[k] == 0 ? u : (K)~u;  // in both groups the wanted rows are those with the LARGEST keys
-    }
-    K prefix[2] = {0, 0};
-    int need[2] = {TOPK, TOPK};
-    bool all[2] = {false, false};  // the whole group is wanted (it has fewer than TOPK rows)
-    // ---- phase A: threshold on the leading DIG * PASSES key bits
-#pragma unroll
-    for (int p = 0; p < SK::PASSES; p++) {
-      const int shift = SK::BITS - DIG * (p + 1);
-      clear(sh);
-      __syncthreads();
-#pragma unroll
-      for (int k = 0; k < R; k++) {
-        const int g = m[k];
-        if (g < 2 && !all[g] && (p == 0 || (key[k] >> (shift + DIG)) == prefix[g]))
-          atomicAdd(&sh.hist[g][(unsigned)(key[k] >> shift) & (BINS - 1)], 1u);
-      }
-      __syncthreads();
-      const bool active[2] = {!all[0], !all[1]};
-      crossing(sh, need, active);
+    // ---- phase A
+    Rows first;
+    load_rows(a, first, 0);
+    KeyIdx<K> best[2] = {{0, -1}, {0, -1}};
+    int nan_first[2] = {kNone, kNone};
+    for_rows(a, first, [&](int i, int side, T s) {
+      const bool num = s == s;
+      const K key = key_of(side, s);  // (at least 1 for a number)
 #pragma unroll
       for (int g = 0; g < 2; g++) {
-        if (all[g]) continue;
-        if (sh.sel_bin[g] < 0) {
-          all[g] = true;
-        } else {
-          prefix[g] = (prefix[g] << DIG) | (K)sh.sel_bin[g];
-          need[g] -= sh.sel_above[g];
-        }
+        const bool take = num && side == g && key >= best[g].key;
+        best[g].key = take ? key : best[g].key;
+        best[g].idx = take ? i : best[g].idx;
       }
-      __syncthreads();  // everybody has read the selection before the next pass clears it
-    }
-    constexpr int TAIL = SK::BITS - DIG * SK::PASSES;  // key bits below the threshold's resolution
-    // ---- candidates: rows at or beyond the threshold
-    if (tid < 2) {
-      sh.ncand[tid] = 0;
-      sh.eq_min[tid] = ~(K)0;
-      sh.eq_max[tid] = 0;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int k = 0; k < R; k++) {
-      const int g = m[k];
-      if (g >= 2) continue;
-      const K top = key[k] >> TAIL;
-      if (all[g] || top >= prefix[g]) {
-        const int pos = atomicAdd(&sh.ncand[g], 1);
-        if (pos < 64) sh.cand[g][pos] = tid + NT * k, sh.cand_cs[g][pos] = cs[k], sh.cand_nom[g][pos] = nom[k];
+      if (!num) {
+        if (side == 0) nan_first[0] = i < nan_first[0] ? i : nan_first[0];
+        else if (side == 1) nan_first[1] = i < nan_first[1] ? i : nan_first[1];
       }
-      if (!all[g] && top == prefix[g]) {
-        atomicMin(&sh.eq_min[g], key[k]);
-        atomicMax(&sh.eq_max[g], key[k]);
-      }
-    }
-    __syncthreads();
-    // ---- too many candidates: a block of exactly equal scores at the threshold is cut down to its
-    // `need` highest row indices (the tie rule takes equal scores from the highest index down)
-    bool cut[2];
-    bool any_cut = false;
+    });
 #pragma unroll
     for (int g = 0; g < 2; g++) {
-      cut[g] = sh.ncand[g] > CAP;
-      if (cut[g] && sh.eq_min[g] != sh.eq_max[g]) return false;  // uniform: read from LDS by everybody
-      any_cut |= cut[g];
-    }
-    if (any_cut) {
-      __syncthreads();
-      clear(sh);
-      if (tid < 2 && cut[tid]) sh.ncand[tid] = 0;
-      __syncthreads();
-#pragma unroll
-      for (int k = 0; k < R; k++) {
-        const int g = m[k];
-        if (g < 2 && cut[g] && (key[k] >> TAIL) == prefix[g]) atomicAdd(&sh.hist[g][(tid + NT * k) >> ISH], 1u);
+      sh.bin_key[g][wv][lane] = best[g].key;
+      sh.bin_idx[g][wv][lane] = best[g].idx;
+      if (__ballot(nan_first[g] != kNone)) {  // one atomic per wavefront: they all hit one address
+        const int lowest = wave_reduce(nan_first[g], [](int x, int y) { return y < x ? y : x; });
+        if (lane == 0) atomicMin(&sh.nan_first[g], lowest);
       }
-      __syncthreads();
-      crossing(sh, need, cut);
+    }
+    __syncthreads();
+    if (wv < 2) {  // wavefront g finds side g's bound
+      const int g = wv;
+      KeyIdx<K> b{0, -1};
 #pragma unroll
-      for (int k = 0; k < R; k++) {
-        const int g = m[k];
-        if (g >= 2 || !cut[g]) continue;
-        const K top = key[k] >> TAIL;
-        const int i = tid + NT * k;
-        if (top > prefix[g] || (top == prefix[g] && (i >> ISH) >= sh.sel_bin[g])) {
-          const int pos = atomicAdd(&sh.ncand[g], 1);
-          if (pos < 64) sh.cand[g][pos] = i, sh.cand_cs[g][pos] = cs[k], sh.cand_nom[g][pos] = nom[k];
+      for (int w = 0; w < NWV; w++) b = pick_key<K>(b, KeyIdx<K>{sh.bin_key[g][w][lane], sh.bin_idx[g][w][lane]});
+      int rank = 0;
+#pragma unroll
+      for (int m = 0; m < 64; m++) {
+        const K km = readlane_k(b.key, m);
+        const int im = __builtin_amdgcn_readlane(b.idx, m);
+        rank += (im >= 0 && (km > b.key || (km == b.key && im > b.idx))) ? 1 : 0;
+      }
+      const bool enough = __popcll(__ballot(b.idx >= 0)) >= TOP;  // else the side's rows are all listed
+      if (enough ? (b.idx >= 0 && rank == TOP - 1) : lane == 0) {
+        sh.bound_key[g] = enough ? b.key : 0;
+        sh.bound_idx[g] = enough ? b.idx : -1;
+      }
+    }
+    __syncthreads();
+    {
+      const K bk[2] = {sh.bound_key[0], sh.bound_key[1]};
+      const int bi[2] = {sh.bound_idx[0], sh.bound_idx[1]}, nf[2] = {sh.nan_first[0], sh.nan_first[1]};
+      int ahead[2] = {0, 0};
+      const bool nans = nf[0] != kNone || nf[1] != kNone;  // (uniform)
+      for_rows(a, first, [&](int i, int side, T s) {
+        const K key = key_of(side, s), bks = side == 0 ? bk[0] : bk[1];
+        const bool num = side < 2 && s == s;
+        if (num && key >= bks && (key > bks || i >= (side == 0 ? bi[0] : bi[1]))) {
+          const int pos = atomicAdd(&sh.nlist[side], 1);
+          if (pos < LIST) sh.list_key[side][pos] = key, sh.list_idx[side][pos] = i;
         }
-      }
-      __syncthreads();
-      if (sh.ncand[0] > CAP || sh.ncand[1] > CAP) return false;
+        if (nans) {
+#pragma unroll
+          for (int g = 0; g < 2; g++) ahead[g] += (num && side == g && i < nf[g]) ? 1 : 0;
+        }
+      });
+#pragma unroll
+      for (int g = 0; g < 2; g++)
+        if (nf[g] != kNone) {  // (uniform)
+          const int sum = wave_reduce(ahead[g], [](int x, int y) { return x + y; });
+          if (lane == 0) atomicAdd(&sh.ahead[g], sum);
+        }
     }
-    if (tid >= 64) return true;  // phase B is the first wavefront's
+    __syncthreads();
+    int ntop[2];
+#pragma unroll
+    for (int g = 0; g < 2; g++) {
+      if (sh.nlist[g] > LIST) return -1;
+      ntop[g] = sh.nlist[g] < TOP ? sh.nlist[g] : TOP;
+    }
+    {
+      const int g = tid >> 9, n = sh.nlist[g];
+      for (int e = tid & 511; e < n; e += 512) {
+        const K key = sh.list_key[g][e];
+        const int idx = sh.list_idx[g][e];
+        int rank = 0;
+        constexpr int V = 8;  // entries whose LDS reads are in flight together
+        for (int o0 = 0; o0 < n; o0 += V) {
+          K ko[V];
+          int io[V];
+#pragma unroll
+          for (int v = 0; v < V; v++) {  // (past the list: an entry that is not ahead of any)
+            const int o = o0 + v < n ? o0 + v : e;
+            ko[v] = sh.list_key[g][o], io[v] = sh.list_idx[g][o];
+          }
+#pragma unroll
+          for (int v = 0; v < V; v++) rank += (ko[v] > key || (ko[v] == key && io[v] > idx)) ? 1 : 0;
+        }
+        if (rank < TOP) sh.top[g][rank] = idx;
+      }
+    }
+    __syncthreads();
+    // A NaN score counts only on a side's first candidate row.  While one of the scored rows ahead of the side's first
+    // NaN is not among the rows that can be picked, that row (or one that joined the side ahead of it) is the first.
+#pragma unroll
+    for (int g = 0; g < 2; g++) {
+      if (sh.nan_first[g] == kNone) continue;
+      int pickable = 0;
+      for (int k = 0; k < ntop[g]; k++) pickable += sh.top[g][k] < sh.nan_first[g] ? 1 : 0;
+      if (sh.ahead[g] <= pickable) return -1;
+    }
+    if (wv == 0) {
+      const int n = swaps_of_top(a, sh, iterations, ntop[0], ntop[1], changed, nchanged);
+      if (lane == 0) sh.swaps = n;
+    }
+    __syncthreads();
+    return sh.swaps;
+  }
 
-    // ---- phase B: lane l holds silent candidate l and active candidate l.  A pick is the maximum of
-    // (key, row index) pairs -- the key orders the scores, the index settles equal scores in favour of
-    // the later row, as the sequential >= / <= scans do.  A row that changes sides takes the score of
-    // its other side along (csum +- 1), computed once up front, so the loop holds no division.
-    int nS = sh.ncand[0], nA = sh.ncand[1];
+  // a row that has changed sides, as the next round and the caller find it
+  static __device__ __forceinline__ void put_row(const MaskArgs<T> &a, int i, int side, int cs, T nom, int *changed,
+                                                 int *nchanged) {
+    a.wmask[(long)i * a.H + a.h] = (uint8_t)side;
+    a.csum[i] = cs;
+    a.side[i] = side;
+    a.score[i] = mask_score<T>(nom, cs);
+    note_changed(changed, nchanged, i);
+  }
+
+  // Phase B, by one wavefront: lane l holds the rank-l silent and the rank-l active candidate.  A pick is the maximum
+  // of (key, row index) pairs -- the key orders the scores, the index settles equal scores in favour of the later
+  // row, as the sequential >= / <= scans do.  A row that changes sides takes the score of its other side along
+  // (csum +- 1), computed once up front, so the loop holds no division.
+  static __device__ int swaps_of_top(const MaskArgs<T> &a, const Shared &sh, int iterations, int nS, int nA,
+                                     int *changed, int *nchanged) {
+    const int lane = threadIdx.x & 63;
     const int nS0 = nS, nA0 = nA;  // rows that change sides are appended from these slots on
     bool vS = lane < nS, vA = lane < nA;
-    int iS = vS ? sh.cand[0][lane] : 0, iA = vA ? sh.cand[1][lane] : 0;
-    int csS = vS ? sh.cand_cs[0][lane] : 0, csA = vA ? sh.cand_cs[1][lane] : 0;
-    const T nomS = vS ? sh.cand_nom[0][lane] : T(0), nomA = vA ? sh.cand_nom[1][lane] : T(0);
+    int iS = vS ? sh.top[0][lane] : 0, iA = vA ? sh.top[1][lane] : 0;
+    int csS = vS ? a.csum[iS] : 0, csA = vA ? a.csum[iA] : 0;
+    T nomS = vS ? a.nom[iS] : T(0), nomA = vA ? a.nom[iA] : T(0);
     // keys as seen from the silent side (largest score wins) and from the active side (smallest wins)
     K kS = SK::of(mask_score<T>(nomS, csS)), kS_other = (K)~SK::of(mask_score<T>(nomS, csS + 1));
     K kA = (K)~SK::of(mask_score<T>(nomA, csA)), kA_other = SK::of(mask_score<T>(nomA, csA - 1));
-    // ---- All swaps at once, when that provably equals the loop below.  Rank the candidates of each side
-    // by (key, row index), the order the picks take them in; iteration k of the loop then picks the
-    // rank-k candidates of both sides and swaps them unless the silent one scores lower, so the number of
+    // ---- All swaps at once, when that provably equals the loop below.  Iteration k of the loop picks the rank-k
+    // candidates of both sides and swaps them unless the silent one scores lower, so the number of
     // swaps n is the length of the run of such pairs from rank 0 -- provided no row that changed sides
     // is ever picked again.  That holds when every new active row scores strictly above, and every new
     // silent row strictly below, the last pair the loop would look at; otherwise (blocks of equal scores,
     // dead inputs) the loop runs.  Both sides must also hold a candidate for every iteration that happens.
     {
-      const int kmax = (int)(a.iterations < (nS < nA ? nS : nA) ? a.iterations : (nS < nA ? nS : nA));
-      int rS = 0, rA = 0;
-      const int widest = nS > nA ? nS : nA;
-      for (int m = 0; m < widest; m++) {  // uniform
-        const K kSm = readlane_k(kS, m), kAm = readlane_k(kA, m);
-        const int iSm = __builtin_amdgcn_readlane(iS, m), iAm = __builtin_amdgcn_readlane(iA, m);
-        rS += (m < nS && (kSm > kS || (kSm == kS && iSm > iS))) ? 1 : 0;
-        rA += (m < nA && (kAm > kA || (kAm == kA && iAm > iA))) ? 1 : 0;
-      }
-      // lane k: the score keys of the rank-k silent and rank-k active candidates
-      const K sortedS = push_to_lane(kS, rS, vS), sortedA = (K)~push_to_lane(kA, rA, vA);
-      const unsigned long long keep_going = __ballot(lane < kmax && !(sortedS < sortedA));
+      const int pairs = nS < nA ? nS : nA, kmax = iterations < pairs ? iterations : pairs;
+      const K activeK = (K)~kA;  // (the key of the active candidate's score as the silent side has it)
+      const unsigned long long keep_going = __ballot(lane < kmax && !(kS < activeK));
       const int n = __builtin_ctzll(~keep_going);  // (kmax <= 16: bit kmax is clear)
-      const bool complete = n < kmax || kmax == (int)a.iterations;
-      if (n == 0 && complete) return true;  // nothing to swap
-      if (complete) {
+      if (n < kmax || kmax == iterations) {
+        if (n == 0) return 0;  // nothing to swap
         const int last = n < kmax ? n : kmax - 1;  // the last pair the loop looks at
-        const K lastS = readlane_k(sortedS, last), lastA = readlane_k(sortedA, last);
-        const bool toA = vS && rS < n, toS = vA && rA < n;
-        const bool again = (toA && !((K)~kS_other > lastA)) || (toS && !(kA_other < lastS));
+        const K lastS = readlane_k(kS, last), lastA = readlane_k(activeK, last);
+        const bool swapped = lane < n;
+        const bool again = swapped && (!((K)~kS_other > lastA) || !(kA_other < lastS));
         if (__ballot(again) == 0) {
-          if (toA) {
-            a.wmask[(long)iS * a.H + a.h] = 1;
-            a.csum[iS] = csS + 1;
-            note_changed(changed, nchanged, iS);
+          if (swapped) {
+            put_row(a, iS, 1, csS + 1, nomS, changed, nchanged);
+            put_row(a, iA, 0, csA - 1, nomA, changed, nchanged);
           }
-          if (toS) {
-            a.wmask[(long)iA * a.H + a.h] = 0;
-            a.csum[iA] = csA - 1;
-            note_changed(changed, nchanged, iA);
-          }
-          return true;
+          return n;
         }
       }
     }
-    for (long it = 0; it < a.iterations; it++) {
+    int it = 0;
+    for (; it < iterations; it++) {
       KeyIdx<K> cmax{kS, vS ? iS : -1}, cmin{kA, vA ? iA : -1};
       cmax = wave_pick(cmax);
       cmin = wave_pick(cmin);
@@ -407,31 +364,121 @@ struct MaskSwapFast {
       const K wOther = readlane_k(kS_other, lS), wThis = cmax.key;  // winner: its active-side key, ...
       const K lOther = readlane_k(kA_other, lA), lThis = cmin.key;
       const int csW = __builtin_amdgcn_readlane(csS, lS), csL = __builtin_amdgcn_readlane(csA, lA);
+      const T nomW = readlane_t(nomS, lS), nomL = readlane_t(nomA, lA);
       if (lane == lS) vS = false;
       if (lane == lA) vA = false;
       if (lane == nA) {  // the best silent row becomes active
-        vA = true, iA = cmax.idx, csA = csW + 1;
+        vA = true, iA = cmax.idx, csA = csW + 1, nomA = nomW;
         kA = wOther, kA_other = wThis;
       }
       if (lane == nS) {  // the worst active row becomes silent
-        vS = true, iS = cmin.idx, csS = csL - 1;
+        vS = true, iS = cmin.idx, csS = csL - 1, nomS = nomL;
         kS = lOther, kS_other = lThis;
       }
       nA++, nS++;
     }
-    if (vS) {
-      a.wmask[(long)iS * a.H + a.h] = 0;
-      a.csum[iS] = csS;
-      if (lane >= nS0) note_changed(changed, nchanged, iS);
-    }
-    if (vA) {
-      a.wmask[(long)iA * a.H + a.h] = 1;
-      a.csum[iA] = csA;
-      if (lane >= nA0) note_changed(changed, nchanged, iA);
-    }
-    return true;
+    if (vS && lane >= nS0) put_row(a, iS, 0, csS, nomS, changed, nchanged);
+    if (vA && lane >= nA0) put_row(a, iA, 1, csA, nomA, changed, nchanged);
+    return it;
   }
 };
+
+// candidate row: score and row index (-1: none)
+template <typename T>
+struct Cand {
+  T val;
+  long idx;
+};
+// a sequential ascending scan with ">=" keeps the later of two equal maxima, with "<=" the later of two equal minima
+template <typename T>
+__device__ __forceinline__ Cand<T> better_max(Cand<T> a, Cand<T> b) {
+  if (a.idx < 0) return b;
+  if (b.idx < 0) return a;
+  if (b.val > a.val || (b.val == a.val && b.idx > a.idx)) return b;
+  return a;
+}
+template <typename T>
+__device__ __forceinline__ Cand<T> better_min(Cand<T> a, Cand<T> b) {
+  if (a.idx < 0) return b;
+  if (b.idx < 0) return a;
+  if (b.val < a.val || (b.val == a.val && b.idx > a.idx)) return b;
+  return a;
+}
+
+// The iterations one by one, each a scan over all rows: what MaskSwap::round does not cover.
+template <typename T>
+__device__ void swap_by_scans(const MaskArgs<T> &a, long iterations, int *changed, int *nchanged) {
+  __shared__ Cand<T> smax[16], smin[16];
+  __shared__ long sfirst0[16], sfirst1[16];
+  __shared__ int sstop;
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  for (long it = 0; it < iterations; it++) {
+    Cand<T> cmax{T(0), -1}, cmin{T(0), -1};
+    long first0 = a.N, first1 = a.N;  // first candidate rows (for the NaN rule)
+    for (long i = tid; i < a.N; i += 1024) {
+      const int m = a.side[i];
+      if (m > 1) continue;
+      const T s = a.score[i];
+      if (m == 0) {
+        first0 = i < first0 ? i : first0;
+        if (s == s) cmax = better_max<T>(cmax, Cand<T>{s, i});
+      } else {
+        first1 = i < first1 ? i : first1;
+        if (s == s) cmin = better_min<T>(cmin, Cand<T>{s, i});
+      }
+    }
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) {
+      Cand<T> o1{__shfl_xor(cmax.val, o), __shfl_xor(cmax.idx, o)};
+      cmax = better_max<T>(cmax, o1);
+      Cand<T> o2{__shfl_xor(cmin.val, o), __shfl_xor(cmin.idx, o)};
+      cmin = better_min<T>(cmin, o2);
+      const long f0 = __shfl_xor(first0, o), f1 = __shfl_xor(first1, o);
+      first0 = f0 < first0 ? f0 : first0;
+      first1 = f1 < first1 ? f1 : first1;
+    }
+    if (lane == 0) {
+      smax[wv] = cmax;
+      smin[wv] = cmin;
+      sfirst0[wv] = first0;
+      sfirst1[wv] = first1;
+    }
+    __syncthreads();
+    if (tid == 0) {
+      for (int k = 1; k < 16; k++) {
+        cmax = better_max<T>(cmax, smax[k]);
+        cmin = better_min<T>(cmin, smin[k]);
+        first0 = sfirst0[k] < first0 ? sfirst0[k] : first0;
+        first1 = sfirst1[k] < first1 ? sfirst1[k] : first1;
+      }
+      int stop = 0;
+      if (first0 >= a.N || first1 >= a.N) {
+        stop = 1;  // no silent or no active row
+      } else {
+        const T sf0 = a.score[first0], sf1 = a.score[first1];
+        long imax0 = cmax.idx, imin1 = cmin.idx;
+        T vmax0 = cmax.val, vmin1 = cmin.val;
+        if (sf0 != sf0 || imax0 < 0) { imax0 = first0; vmax0 = sf0; }
+        if (sf1 != sf1 || imin1 < 0) { imin1 = first1; vmin1 = sf1; }
+        if (vmax0 < vmin1) {
+          stop = 1;
+        } else {
+          const int cs1 = a.csum[imax0] + 1, cs0 = a.csum[imin1] - 1;
+          a.wmask[imax0 * a.H + a.h] = 1;
+          a.wmask[imin1 * a.H + a.h] = 0;
+          a.csum[imax0] = cs1, a.side[imax0] = 1, a.score[imax0] = mask_score<T>(a.nom[imax0], cs1);
+          a.csum[imin1] = cs0, a.side[imin1] = 0, a.score[imin1] = mask_score<T>(a.nom[imin1], cs0);
+          note_changed(changed, nchanged, imax0);
+          note_changed(changed, nchanged, imin1);
+        }
+      }
+      sstop = stop;
+    }
+    __syncthreads();
+    if (sstop) break;
+    __syncthreads();
+  }
+}
 
 // Steps 3 and 4 in the swap kernel's wake (a.W_fix != nullptr), by the whole workgroup: the weights of the
 // rows that changed sides -- every other row of the hypercolumn already holds what its unchanged mask byte
@@ -441,155 +488,56 @@ __device__ __forceinline__ void mask_swap_finish(const MaskArgs<T> &a, const int
   if (a.W_fix == nullptr) return;  // uniform
   __syncthreads();                 // mask bytes and the list of changed rows are written
   if (a.rows != nullptr) mask_rows_block<NT>(a.rows, a.row_cnt, a.wmask, a.N, a.H, a.cap, a.h);
-  const unsigned nc = *nchanged < kMaxChangedRows ? *nchanged : kMaxChangedRows, Mc = (unsigned)a.Mc;
-  for (unsigned e = threadIdx.x; e < nc * Mc; e += NT) {
-    const unsigned r = e / Mc, c = e - r * Mc;
-    const long i = changed[r], j = a.h * a.Mc + c;
-    T wgt = T(0);
-    if (a.wmask[i * a.H + a.h] != 0)
-      wgt = weight_from_traces<T>(a.Cij[i * a.M + j], trace_reciprocal<T>(a.Ci[i], a.cthr),
-                                  trace_reciprocal<T>(a.Cj[j], a.cthr), a.cthr4);
-    a.W_fix[i * a.M + j] = wgt;
+  // A thread owns a column (or every NT-th) and walks the rows, so that a reciprocal is formed once per row and once
+  // per thread; one CU does all of this, and in doubles its vector unit is what it waits for.
+  __shared__ T row_rci[kMaxChangedRows];
+  const int nc = *nchanged < kMaxChangedRows ? *nchanged : kMaxChangedRows, tid = threadIdx.x;
+  if (tid < nc) row_rci[tid] = trace_reciprocal<T>(a.Ci[changed[tid]], a.cthr);
+  __syncthreads();
+  const int cols = a.Mc < NT ? (int)a.Mc : NT, groups = NT / cols;
+  if (tid >= groups * cols) return;
+  constexpr int U = 8;  // rows whose loads are in flight together
+  for (long c = tid % cols; c < a.Mc; c += cols) {
+    const long j = a.h * a.Mc + c;
+    const T rcj = trace_reciprocal<T>(a.Cj[j], a.cthr);
+    for (int r0 = tid / cols; r0 < nc; r0 += groups * U) {
+      long i[U];
+      T cij[U];
+      uint8_t on[U];
+#pragma unroll
+      for (int u = 0; u < U; u++) {
+        i[u] = changed[r0 + groups * u < nc ? r0 + groups * u : r0];
+        cij[u] = a.Cij[i[u] * a.M + j], on[u] = a.wmask[i[u] * a.H + a.h];
+      }
+#pragma unroll
+      for (int u = 0; u < U; u++) {
+        const int r = r0 + groups * u;
+        if (r >= nc) break;
+        a.W_fix[i[u] * a.M + j] = on[u] != 0 ? weight_from_traces<T>(cij[u], row_rci[r], rcj, a.cthr4) : T(0);
+      }
+    }
   }
 }
 
-// NT threads (64 to 1024 in powers of two), thread t owns rows t, t+NT, ..., t+(R-1)*NT.  1024 threads
-// with few rows each measured faster than 256 with more (1568 rows: 19.8 against 21.8 us).
-template <typename T, int NT, int R>
-__global__ __launch_bounds__(NT) void k_mask_swap_reg(MaskArgs<T> a) {
-  constexpr int NWV = NT / 64;
-  static_assert(NWV == 1 || NWV == 2 || NWV == 4 || NWV == 8 || NWV == 16, "1 to 16 wavefronts");
-  __shared__ RowCand<T> part[2][4][NWV];  // [buffer][max0, min1, first0, first1][wavefront]
-  __shared__ int changed[kMaxChangedRows], nchanged;
-  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-  if (tid == 0) nchanged = 0;  // (published by the barrier below)
-
-  T nom[R], score[R];
-  int cs[R], m[R];  // m: 0 silent, 1 active, 2 not a candidate (row out of range or odd mask value)
-  bool dirty[R];
-  int has_nan = 0;
-#pragma unroll
-  for (int k = 0; k < R; k++) {
-    const long i = tid + (long)NT * k;
-    dirty[k] = false;
-    m[k] = 2;
-    nom[k] = T(0);
-    cs[k] = 0;
-    if (i < a.N) {
-      const uint8_t b = a.wmask[i * a.H + a.h];
-      m[k] = b > 1 ? 2 : b;
-      nom[k] = a.nom[i];
-      cs[k] = a.csum[i];
-    }
-    score[k] = mask_score<T>(nom[k], cs[k]);
-    has_nan |= (score[k] != score[k]) ? 1 : 0;
-  }
-  // NaN scores need the "first candidate" bookkeeping of the sequential scan; without any NaN (the
-  // normal case; a score is NaN iff its nominator is) that half of the reduction is skipped
-  const bool track_first = __syncthreads_or(has_nan) != 0;
-  if (!track_first && a.iterations <= MaskSwapFast<T, NT, R>::TOPK) {
-    __shared__ typename MaskSwapFast<T, NT, R>::Shared fast_lds;
-    if (MaskSwapFast<T, NT, R>::run(a, fast_lds, score, m, nom, cs, changed, &nchanged)) {
-      mask_swap_finish<T, NT>(a, changed, &nchanged);
-      return;
-    }
-    __syncthreads();
-  }
-
-  for (long it = 0; it < a.iterations; it++) {
-    const int buf = (int)(it & 1);
-    RowCand<T> cmax{T(0), -1}, cmin{T(0), -1}, f0{T(0), -1}, f1{T(0), -1};
-#pragma unroll
-    for (int k = 0; k < R; k++) {  // ascending row order within the thread
-      const int i = tid + NT * k;
-      const RowCand<T> me{score[k], i};
-      const bool num = score[k] == score[k];  // a NaN never wins a comparison
-      if (m[k] == 0) {
-        if (track_first) f0 = pick_first<T>(f0, me);
-        if (num) cmax = pick_max<T>(cmax, me);
-      } else if (m[k] == 1) {
-        if (track_first) f1 = pick_first<T>(f1, me);
-        if (num) cmin = pick_min<T>(cmin, me);
-      }
-    }
-    SB_ROW_REDUCE(pick_max<T>, cmax);
-    SB_ROW_REDUCE(pick_min<T>, cmin);
-    if (track_first) {
-      SB_ROW_REDUCE(pick_first<T>, f0);
-      SB_ROW_REDUCE(pick_first<T>, f1);
-    }
-#pragma unroll
-    for (int o = 16; o <= 32; o <<= 1) {  // across the four rows of the wavefront
-      cmax = pick_max<T>(cmax, shfl_xor_cand<T>(cmax, o));
-      cmin = pick_min<T>(cmin, shfl_xor_cand<T>(cmin, o));
-      if (track_first) {
-        f0 = pick_first<T>(f0, shfl_xor_cand<T>(f0, o));
-        f1 = pick_first<T>(f1, shfl_xor_cand<T>(f1, o));
-      }
-    }
-    if (NWV > 1) {
-      if (lane == 0) {
-        part[buf][0][wv] = cmax;
-        part[buf][1][wv] = cmin;
-        part[buf][2][wv] = f0;
-        part[buf][3][wv] = f1;
-      }
+template <typename T>
+__global__ __launch_bounds__(1024) void k_mask_swap(MaskArgs<T> a) {
+  using S = MaskSwap<T>;
+  __shared__ typename S::Shared sh;
+  __shared__ int changed[kMaxChangedRows], nchanged;  // rows that changed sides, see mask_swap_finish
+  if (threadIdx.x == 0) nchanged = 0;                 // (published by the barriers of the first round)
+  __syncthreads();
+  for (long left = a.iterations; left > 0;) {
+    const int n = (int)(left < S::TOP ? left : S::TOP);
+    const int done = a.N < (1L << 31) ? S::round(a, sh, n, changed, &nchanged) : -1;  // (row indices are 32-bit there)
+    if (done < 0) {
       __syncthreads();
-      // every group of NWV lanes reads the NWV partials and reduces them: all lanes get the result
-      cmax = part[buf][0][lane % NWV];
-      cmin = part[buf][1][lane % NWV];
-      f0 = part[buf][2][lane % NWV];
-      f1 = part[buf][3][lane % NWV];
-      cmax = pick_max<T>(cmax, dpp_cand<kDppSwap1, T>(cmax));
-      cmin = pick_min<T>(cmin, dpp_cand<kDppSwap1, T>(cmin));
-      f0 = pick_first<T>(f0, dpp_cand<kDppSwap1, T>(f0));
-      f1 = pick_first<T>(f1, dpp_cand<kDppSwap1, T>(f1));
-      if (NWV > 2) {
-        cmax = pick_max<T>(cmax, dpp_cand<kDppSwap2, T>(cmax));
-        cmin = pick_min<T>(cmin, dpp_cand<kDppSwap2, T>(cmin));
-        f0 = pick_first<T>(f0, dpp_cand<kDppSwap2, T>(f0));
-        f1 = pick_first<T>(f1, dpp_cand<kDppSwap2, T>(f1));
-      }
-      if (NWV > 4) {  // the lanes of a quad agree by now, so mirroring 8 (16) lanes pairs the quads
-        cmax = pick_max<T>(cmax, dpp_cand<kDppHalfMirror, T>(cmax));
-        cmin = pick_min<T>(cmin, dpp_cand<kDppHalfMirror, T>(cmin));
-        f0 = pick_first<T>(f0, dpp_cand<kDppHalfMirror, T>(f0));
-        f1 = pick_first<T>(f1, dpp_cand<kDppHalfMirror, T>(f1));
-      }
-      if (NWV > 8) {
-        cmax = pick_max<T>(cmax, dpp_cand<kDppMirror, T>(cmax));
-        cmin = pick_min<T>(cmin, dpp_cand<kDppMirror, T>(cmin));
-        f0 = pick_first<T>(f0, dpp_cand<kDppMirror, T>(f0));
-        f1 = pick_first<T>(f1, dpp_cand<kDppMirror, T>(f1));
-      }
+      swap_by_scans<T>(a, left, changed, &nchanged);
+      break;
     }
-    if (cmax.idx < 0 && f0.idx < 0) break;  // no silent row (uniform over the workgroup)
-    if (cmin.idx < 0 && f1.idx < 0) break;  // no active row
-    int imax0 = cmax.idx, imin1 = cmin.idx;
-    T vmax0 = cmax.val, vmin1 = cmin.val;
-    // a NaN score wins only when it belongs to the first candidate row (sequential >= / <= scan)
-    if (track_first) {
-      if (f0.val != f0.val || imax0 < 0) { imax0 = f0.idx; vmax0 = f0.val; }
-      if (f1.val != f1.val || imin1 < 0) { imin1 = f1.idx; vmin1 = f1.val; }
-    }
-    if (vmax0 < vmin1) break;
-#pragma unroll
-    for (int k = 0; k < R; k++) {
-      const int i = tid + NT * k;
-      if (i == imax0) { m[k] = 1; cs[k] += 1; dirty[k] = true; score[k] = mask_score<T>(nom[k], cs[k]); }
-      if (i == imin1) { m[k] = 0; cs[k] -= 1; dirty[k] = true; score[k] = mask_score<T>(nom[k], cs[k]); }
-    }
+    if (done < n) break;
+    left -= n;
   }
-#pragma unroll
-  for (int k = 0; k < R; k++) {
-    const long i = tid + (long)NT * k;
-    if (dirty[k]) {
-      a.wmask[i * a.H + a.h] = (uint8_t)m[k];
-      a.csum[i] = cs[k];
-      note_changed(changed, &nchanged, (int)i);
-    }
-  }
-  mask_swap_finish<T, NT>(a, changed, &nchanged);
+  mask_swap_finish<T, S::NT>(a, changed, &nchanged);
 }
 
 }  // namespace sb

@@ -201,14 +201,13 @@ __global__ __launch_bounds__(256) void k_count_unmasked(const T *W, const uint8_
 
 // =====================================================================================================
 // Structural-plasticity rewiring of one hypercolumn                      omp.cc:248-320
-// Step 1 (k_mask_scores): per input row, the score nominator over the Mc columns of hypercolumn h and
-//   the number of hypercolumns the row is connected to.  One wavefront per row.  When W is nullptr the
-//   (unmasked) weight is recomputed from the traces with the trace/weight kernel's own formula.
-// Step 2 (k_mask_swap): one workgroup repeats up to `iterations` times: best silent row (max score,
-//   highest index among equals), worst active row (min score, highest index among equals), swap unless
-//   vmax0 < vmin1.  The quotient nominator / (1 + csum) is formed in double and narrowed, as the
-//   reference's expression does.  A NaN score behaves as in a sequential scan with >= / <=: it is
-//   picked only when it belongs to the first candidate row.
+// Step 1 (k_mask_scores): per input row, the score nominator over the Mc columns of hypercolumn h, the number of
+//   hypercolumns the row is connected to, the score -- nominator / (1 + csum), formed in double and narrowed, as the
+//   reference's expression does -- and the side the row is on.  When W is nullptr the (unmasked) weight is
+//   recomputed from the traces with the weight pass's own formula.
+// Step 2 (k_mask_swap, sb_k_mask_swap.hpp): up to `iterations` times: best silent row (max score, highest index
+//   among equals), worst active row (min score, highest index among equals), swap unless vmax0 < vmin1.  A NaN
+//   score behaves as in a sequential scan with >= / <=: it is picked only when it belongs to the first candidate row.
 // Step 3 (k_mask_fix_weights): rewrites W[:, hypercolumn h] under the new mask (network path only,
 //   where W is kept masked).
 // Step 4: see mask_rows_block below.
@@ -220,9 +219,9 @@ struct MaskArgs {
   const T *Ci, *Cj, *Cij;
   T cthr, cthr4;
   long N, M, H, Mc, h, iterations;
-  T *nom;     // [N] scratch
-  int *csum;  // [N] scratch
-  // Network path (k_mask_swap_reg only): after the swaps the same workgroup rewrites W[i, columns of h] of
+  T *nom, *score;   // [N] scratch each
+  int *csum, *side;  // [N] scratch each; side: 0 silent, 1 active, 2 not a candidate (odd mask value)
+  // Network path: after the swaps the same workgroup rewrites W[i, columns of h] of
   // the rows that changed sides under the new mask (steps 3) and, with a row list, rebuilds the list of
   // hypercolumn h (step 4).  W_fix == nullptr: neither.
   T *W_fix;
@@ -231,166 +230,111 @@ struct MaskArgs {
 };
 constexpr int kMaxChangedRows = 64;  // rows that change sides in one merged launch: two per iteration
 
-// One wavefront per input row.  The score nominator is the reference's own expression, operation by operation
-// (omp.cc:257-277): every product, difference, quotient and sum rounded once, the logarithms accurate to the
-// last bit or so (evaluated in double and narrowed for floats), and the Mc terms of a row added in ascending
-// column order starting from zero -- so that two builds that start from the same traces pick the same rows.
-// The lanes evaluate 64 terms at a time; the sum then walks them in order (lane by lane through scalar
-// registers), which every lane does for itself.  Without a W array (the network path, where W is kept masked)
-// the weight is recomputed as the reference's weight pass forms it (omp.cc:192-199): log(max(Cij, cthr^4) /
+// The score nominator is the reference's own expression, operation by operation (omp.cc:257-277): every product,
+// difference, quotient and sum rounded once, the logarithms accurate to the last bit or so (evaluated in double and
+// narrowed for floats), and the Mc terms of a row added in ascending column order starting from zero -- so that two
+// builds that start from the same traces pick the same rows.  Without a W array (the network path, where W is kept
+// masked) the weight is recomputed as the reference's weight pass forms it (omp.cc:192-199): log(max(Cij, cthr^4) /
 // (Ci Cj)) with the product and the quotient rounded like there.
+// A workgroup takes ROWS rows: its threads evaluate the terms, dealt out as one run so that no lane idles
+// whatever Mc is, and put them down in LDS; then a lane per row adds up its row in order, all rows side by side.
+// (A wavefront per row that walks its terms through scalar registers spends as long on the ordered sums as on the
+// logarithms: 27648 rows x 200 columns, floats, 52 us against 28 with sixteen rows per workgroup.)  Sixteen rows
+// where that fills the chip; four below, where the terms a thread evaluates one after the other are what the launch
+// waits for (784 rows x 200, doubles: 16.1 us with sixteen rows, 7.3 with four).
 template <typename T>
 __device__ __forceinline__ T accurate_log(T x) {
-  if constexpr (sizeof(T) == 4) return (T)log((double)x);
+  if constexpr (sizeof(T) == 4) return (T)Real<double>::wlog((double)x);
   else return log(x);
 }
 template <typename T>
+__device__ __forceinline__ T mask_score(T nom, int csum) {
+  // nominator / (1.0 + (REAL)csum): formed in double and narrowed, as the reference's expression
+  return (T)((double)nom / (1.0 + (double)(T)csum));
+}
+constexpr int kScoreCols = 256;  // columns whose terms are in LDS at a time
+template <typename T, int ROWS>
 __global__ __launch_bounds__(256) void k_mask_scores(MaskArgs<T> a) {
   using R = Real<T>;
-  const int lane = threadIdx.x & 63;
-  const long i = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (i >= a.N) return;
-  const T pi = a.Ci[i];
+  // (an odd pitch: the lanes that add up the rows read one column of all of them at a time)
+  __shared__ T terms[ROWS][kScoreCols + 1];
+  __shared__ T row_pi[ROWS];
+  static_assert(ROWS % 4 == 0 && ROWS <= 16, "rows per workgroup");
+  constexpr int U = 4;
+  const int tid = threadIdx.x;
+  const long i0 = (long)blockIdx.x * ROWS;
+  // connections per row: sixteen threads each
+  if ((tid >> 4) < ROWS) {  // (whole wavefronts)
+    const long i = i0 + (tid >> 4);
+    int cs = 0;
+    if (i < a.N)
+      for (long g = tid & 15; g < a.H; g += 16) cs += a.wmask[i * a.H + g];
+    cs = row16_reduce(cs, [](int x, int y) { return x + y; });
+    if ((tid & 15) == 0) {
+      row_pi[tid >> 4] = i < a.N ? a.Ci[i] : T(0);
+      if (i < a.N) a.csum[i] = cs;
+    }
+  }
   T score = T(0);
-  if (pi >= a.cthr) {  // (uniform per wavefront)
-    const T omp = R::add(T(1), -pi);
-    for (long c0 = 0; c0 < a.Mc; c0 += 64) {
-      const long c = c0 + lane;
-      const long j = a.h * a.Mc + (c < a.Mc ? c : a.Mc - 1);
-      const T pj = a.Cj[j];
-      T term = T(0);
-      if (c < a.Mc && pj >= a.cthr) {
-        const T pij = a.Cij[i * a.M + j];
-        T wij;
-        if (a.W) {
-          wij = a.W[i * a.M + j];
-        } else {
-          const T num = pij > a.cthr4 ? pij : a.cthr4;  // cthr^4 as well when pij is NaN
-          wij = accurate_log<T>(R::div(num, R::mul(pi, pj)));
+  for (long c0 = 0; c0 < a.Mc; c0 += kScoreCols) {  // uniform
+    const unsigned cols = a.Mc - c0 < kScoreCols ? (unsigned)(a.Mc - c0) : (unsigned)kScoreCols;
+    __syncthreads();  // row_pi is there; the previous columns' terms have been added up
+    const unsigned dr = 256 / cols, dc = 256 % cols;  // 256 items further on: dr rows and dc columns
+    unsigned r = tid / cols, c = tid % cols;
+    const unsigned items = ROWS * cols;
+    for (unsigned e0 = tid; e0 < items; e0 += 256 * U) {
+      // the loads of U items are in flight before the first is used (no guards: out-of-range items read element 0
+      // of a row that is there)
+      T pj[U], pij[U], wgt[U];
+      unsigned ru[U], cu[U];
+#pragma unroll
+      for (int u = 0; u < U; u++) {
+        const bool on = e0 + 256 * u < items && i0 + r < a.N;
+        ru[u] = r, cu[u] = c;
+        const long j = a.h * a.Mc + c0 + (on ? c : 0), at = (on ? i0 + r : i0) * a.M + j;
+        pj[u] = a.Cj[j];
+        pij[u] = a.Cij[at];
+        wgt[u] = a.W ? a.W[at] : T(0);
+        r += dr, c += dc;
+        if (c >= cols) c -= cols, r++;
+      }
+#pragma unroll
+      for (int u = 0; u < U; u++) {
+        if (e0 + 256 * u >= items) break;
+        const T pi = row_pi[ru[u]];
+        T term = T(0);  // columns and rows below the threshold, and rows past the matrix, contribute an exact zero
+        if (i0 + ru[u] < a.N && pi >= a.cthr && pj[u] >= a.cthr) {
+          T wij = wgt[u];
+          if (!a.W) {
+            const T num = pij[u] > a.cthr4 ? pij[u] : a.cthr4;  // cthr^4 as well when pij is NaN
+            wij = accurate_log<T>(R::div(num, R::mul(pi, pj[u])));
+          }
+          const T d = R::add(pj[u], -pij[u]);
+          const T yy = R::div(d, R::mul(R::add(T(1), -pi), pj[u]));
+          term = R::add(R::mul(pij[u], wij), R::mul(d, accurate_log<T>(yy)));
         }
-        const T d = R::add(pj, -pij);
-        const T yy = R::div(d, R::mul(omp, pj));
-        term = R::add(R::mul(pij, wij), R::mul(d, accurate_log<T>(yy)));
+        terms[ru[u]][cu[u]] = term;
       }
-      // columns past the hypercolumn and columns below the threshold contribute an exact zero
-#pragma unroll
-      for (int k = 0; k < 64; k++) {
-        T tk;
-        if constexpr (sizeof(T) == 4) {
-          tk = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(term), k));
-        } else {
-          const long long b = __double_as_longlong(term);
-          const int lo = __builtin_amdgcn_readlane((int)(b & 0xffffffffLL), k);
-          const int hi = __builtin_amdgcn_readlane((int)(b >> 32), k);
-          tk = __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
-        }
-        score = R::add(score, tk);
-      }
-    }
-  }
-  int cs = 0;
-  for (long g = lane; g < a.H; g += 64) cs += a.wmask[i * a.H + g];
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) cs += __shfl_xor(cs, o);
-  if (lane == 0) {
-    a.nom[i] = score;
-    a.csum[i] = cs;
-  }
-}
-
-template <typename T>
-struct Cand {
-  T val;
-  long idx;  // -1: none
-};
-
-// a sequential ascending scan with ">=" keeps the later of two equal maxima
-template <typename T>
-__device__ __forceinline__ Cand<T> better_max(Cand<T> a, Cand<T> b) {
-  if (a.idx < 0) return b;
-  if (b.idx < 0) return a;
-  if (b.val > a.val || (b.val == a.val && b.idx > a.idx)) return b;
-  return a;
-}
-template <typename T>
-__device__ __forceinline__ Cand<T> better_min(Cand<T> a, Cand<T> b) {
-  if (a.idx < 0) return b;
-  if (b.idx < 0) return a;
-  if (b.val < a.val || (b.val == a.val && b.idx > a.idx)) return b;
-  return a;
-}
-
-template <typename T>
-__global__ __launch_bounds__(1024) void k_mask_swap(MaskArgs<T> a) {
-  __shared__ Cand<T> smax[16], smin[16];
-  __shared__ long sfirst0[16], sfirst1[16];
-  __shared__ int sstop;
-  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-  for (long it = 0; it < a.iterations; it++) {
-    Cand<T> cmax{T(0), -1}, cmin{T(0), -1};
-    long first0 = a.N, first1 = a.N;  // first candidate rows (for the NaN rule)
-    for (long i = tid; i < a.N; i += 1024) {
-      const uint8_t m = a.wmask[i * a.H + a.h];
-      if (m > 1) continue;
-      const T s = (T)((double)a.nom[i] / (1.0 + (double)(T)a.csum[i]));
-      if (m == 0) {
-        first0 = i < first0 ? i : first0;
-        if (s == s) cmax = better_max<T>(cmax, Cand<T>{s, i});
-      } else {
-        first1 = i < first1 ? i : first1;
-        if (s == s) cmin = better_min<T>(cmin, Cand<T>{s, i});
-      }
-    }
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) {
-      Cand<T> o1{__shfl_xor(cmax.val, o), __shfl_xor(cmax.idx, o)};
-      cmax = better_max<T>(cmax, o1);
-      Cand<T> o2{__shfl_xor(cmin.val, o), __shfl_xor(cmin.idx, o)};
-      cmin = better_min<T>(cmin, o2);
-      const long f0 = __shfl_xor(first0, o), f1 = __shfl_xor(first1, o);
-      first0 = f0 < first0 ? f0 : first0;
-      first1 = f1 < first1 ? f1 : first1;
-    }
-    if (lane == 0) {
-      smax[wv] = cmax;
-      smin[wv] = cmin;
-      sfirst0[wv] = first0;
-      sfirst1[wv] = first1;
     }
     __syncthreads();
-    if (tid == 0) {
-      for (int k = 1; k < 16; k++) {
-        cmax = better_max<T>(cmax, smax[k]);
-        cmin = better_min<T>(cmin, smin[k]);
-        first0 = sfirst0[k] < first0 ? sfirst0[k] : first0;
-        first1 = sfirst1[k] < first1 ? sfirst1[k] : first1;
+    if (tid < ROWS) {
+      unsigned k = 0;
+      for (; k + 8 <= cols; k += 8) {
+        T v[8];
+#pragma unroll
+        for (int u = 0; u < 8; u++) v[u] = terms[tid][k + u];
+#pragma unroll
+        for (int u = 0; u < 8; u++) score = R::add(score, v[u]);
       }
-      int stop = 0;
-      if (first0 >= a.N || first1 >= a.N) {
-        stop = 1;  // no silent or no active row
-      } else {
-        const T sf0 = (T)((double)a.nom[first0] / (1.0 + (double)(T)a.csum[first0]));
-        const T sf1 = (T)((double)a.nom[first1] / (1.0 + (double)(T)a.csum[first1]));
-        long imax0 = cmax.idx, imin1 = cmin.idx;
-        T vmax0 = cmax.val, vmin1 = cmin.val;
-        if (sf0 != sf0 || imax0 < 0) { imax0 = first0; vmax0 = sf0; }
-        if (sf1 != sf1 || imin1 < 0) { imin1 = first1; vmin1 = sf1; }
-        if (vmax0 < vmin1) {
-          stop = 1;
-        } else {
-          a.wmask[imax0 * a.H + a.h] = 1;
-          a.wmask[imin1 * a.H + a.h] = 0;
-          a.csum[imax0] += 1;
-          a.csum[imin1] -= 1;
-        }
-      }
-      sstop = stop;
-      __threadfence_block();
+      for (; k < cols; k++) score = R::add(score, terms[tid][k]);
     }
-    __syncthreads();
-    if (sstop) break;
-    __syncthreads();
   }
+  const long i = i0 + tid;
+  if (tid >= ROWS || i >= a.N) return;
+  const uint8_t m = a.wmask[i * a.H + a.h];
+  a.nom[i] = score;
+  a.score[i] = mask_score<T>(score, a.csum[i]);  // (csum: written by this workgroup, ahead of a barrier)
+  a.side[i] = m > 1 ? 2 : m;
 }
 
 // Step 4 (mask_rows_block / k_mask_rows): the list of connected rows of a hypercolumn, which the forward

@@ -115,7 +115,7 @@ int launch_update_bias(hipStream_t st, T *bias, const T *Cj, T cthr, long M);
 template <typename T>
 int launch_update_bias_regularized(hipStream_t st, T *bias, T *kbi, const T *Cj, T cthr, T khalf,
                                    T pmin, T taubdt, long M);
-// nom / csum: scratch of N elements each.  W == nullptr: weights recomputed from the traces.
+// nom / csum: scratch of 2 N elements each.  W == nullptr: weights recomputed from the traces.
 template <typename T>
 int launch_update_mask(hipStream_t st, uint8_t *wmask, const T *W, const T *Ci, const T *Cj,
                        const T *Cij, T cthr, long N, long H, long Mc, long h, long iterations, T *nom,

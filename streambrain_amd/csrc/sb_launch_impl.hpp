@@ -439,10 +439,11 @@ static int update_mask_impl(hipStream_t st, uint8_t *wmask, const T *W, const T 
   const TraceScalars<T> s = TraceScalars<T>::from(T(0), cthr);
   MaskArgs<T> a;
   a.wmask = wmask; a.W = W; a.Ci = Ci; a.Cj = Cj; a.Cij = Cij; a.cthr = cthr; a.cthr4 = s.cthr4;
-  a.N = N; a.M = H * Mc; a.H = H; a.Mc = Mc; a.h = h; a.iterations = iterations; a.nom = nom;
-  a.csum = csum;
-  // two rows change sides per iteration; the kernels for more than 65536 rows have no such tail
-  const bool merge = W_fix != nullptr && iterations > 0 && 2 * iterations <= kMaxChangedRows && N <= 65536 &&
+  a.N = N; a.M = H * Mc; a.H = H; a.Mc = Mc; a.h = h; a.iterations = iterations;
+  a.nom = nom; a.score = nom + N;
+  a.csum = csum; a.side = csum + N;
+  // two rows change sides per iteration; the rows that did are noted and rewritten with 32-bit indices
+  const bool merge = W_fix != nullptr && iterations > 0 && 2 * iterations <= kMaxChangedRows && N < (1L << 31) &&
                      N * Mc < (1L << 31);
   a.W_fix = merge ? W_fix : nullptr;
   a.rows = merge ? rows : nullptr;
@@ -451,21 +452,15 @@ static int update_mask_impl(hipStream_t st, uint8_t *wmask, const T *W, const T 
   if (merged) *merged = merge;
   {
     ProfScope prof_(st, K_MASK_SCORES);
-    hipLaunchKernelGGL((k_mask_scores<T>), dim3((unsigned)cdiv(N, 4)), dim3(256), 0, st, a);
+    if (N >= 16L * 2 * device_cu_count())  // two workgroups of sixteen rows for every CU
+      hipLaunchKernelGGL((k_mask_scores<T, 16>), dim3((unsigned)cdiv(N, 16)), dim3(256), 0, st, a);
+    else
+      hipLaunchKernelGGL((k_mask_scores<T, 4>), dim3((unsigned)cdiv(N, 4)), dim3(256), 0, st, a);
     SB_LAUNCH_CHECK();
   }
   if (iterations > 0) {
     ProfScope prof_(st, K_MASK_SWAP);
-    if (N <= 2048)
-      hipLaunchKernelGGL((k_mask_swap_reg<T, 1024, 2>), dim3(1), dim3(1024), 0, st, a);
-    else if (N <= 8192)
-      hipLaunchKernelGGL((k_mask_swap_reg<T, 1024, 8>), dim3(1), dim3(1024), 0, st, a);
-    else if (N <= 32768)
-      hipLaunchKernelGGL((k_mask_swap_reg<T, 1024, 32>), dim3(1), dim3(1024), 0, st, a);
-    else if (N <= 65536)
-      hipLaunchKernelGGL((k_mask_swap_reg<T, 1024, 64>), dim3(1), dim3(1024), 0, st, a);
-    else
-      hipLaunchKernelGGL((k_mask_swap<T>), dim3(1), dim3(1024), 0, st, a);
+    hipLaunchKernelGGL((k_mask_swap<T>), dim3(1), dim3(1024), 0, st, a);
     SB_LAUNCH_CHECK();
   }
   return 0;

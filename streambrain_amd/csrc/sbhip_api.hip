@@ -278,8 +278,8 @@ static int ensure_mask_scratch(long N) {
   g_ctx.mask_nom = nullptr;
   g_ctx.mask_csum = nullptr;
   g_ctx.mask_cap = 0;
-  SB_HIP(dev_malloc(&g_ctx.mask_nom, (size_t)N * sizeof(double)));
-  SB_HIP(dev_malloc((void **)&g_ctx.mask_csum, (size_t)N * sizeof(int)));
+  SB_HIP(dev_malloc(&g_ctx.mask_nom, 2 * (size_t)N * sizeof(double)));
+  SB_HIP(dev_malloc((void **)&g_ctx.mask_csum, 2 * (size_t)N * sizeof(int)));
   g_ctx.mask_cap = N;
   return 0;
 }
@@ -325,7 +325,7 @@ struct Layer {
   uint8_t *wmask = nullptr;
   void *act = nullptr;  // [act_rows, M]
   long act_rows = 0;
-  void *nom = nullptr;  // rewiring scratch [N]
+  void *nom = nullptr;  // rewiring scratch [2 N], csum too
   int *csum = nullptr;
   // Sparse layers (at most 70 % of wmask set): per-hypercolumn lists of the connected rows for the
   // forward pass, kept in step with wmask.  They are used while W is known to be zero wherever wmask
@@ -420,8 +420,8 @@ static int layer_alloc(Layer &L, T ci0, T cj0, T cij0) {
   if (L.plastic) {
     SB_HIP(dev_malloc(&L.kbi, L.M * sizeof(T)));
     SB_HIP(dev_malloc((void **)&L.wmask, (size_t)L.N * L.H));
-    SB_HIP(dev_malloc(&L.nom, L.N * sizeof(T)));
-    SB_HIP(dev_malloc((void **)&L.csum, L.N * sizeof(int)));
+    SB_HIP(dev_malloc(&L.nom, 2 * L.N * sizeof(T)));
+    SB_HIP(dev_malloc((void **)&L.csum, 2 * L.N * sizeof(int)));
     if ((rc = launch_fill<T>(st, (T *)L.kbi, T(1), L.M))) return rc;
     if ((rc = launch_fill_bytes(st, L.wmask, 1, (size_t)L.N * L.H))) return rc;
   }

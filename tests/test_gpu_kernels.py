@@ -429,6 +429,28 @@ def test_update_mask_nan_scores(k, oracle, dtype, N):
 
 
 @pytest.mark.parametrize("dtype", DT)
+@pytest.mark.parametrize("N", [1, 15, 17, 63, 64, 65, 1023, 1025, 4099, 27648])
+@pytest.mark.parametrize("iterations", [15, 17, 40])
+@pytest.mark.parametrize("kind", ["numbers", "nan_behind", "nan_between", "one_bin"])
+def test_update_mask_rounds(k, oracle, dtype, N, iterations, kind):
+    """More iterations than one round of the swap loop takes; NaN scores behind and among the rows that can be
+    picked; the best rows of a side all in one of the 64 bins of the preselection."""
+    rng = np.random.default_rng(N + iterations + len(kind))
+    H, Mc = 2, 5
+    wmask, W, Ci, Cj, Cij = _mask_problem(rng, N, H, Mc, dtype, density=0.4)
+    if kind.startswith("nan"):
+        bad = rng.choice(N, size=N // 8, replace=False)
+        bad = bad[bad >= (N // 2 if kind == "nan_behind" else 20)]
+        Ci[bad] = 1.0
+        Cij[bad, :] = Cj[None, :]
+    elif kind == "one_bin":
+        W[np.arange(N) % 64 == 5] += 3
+    ref = oracle.update_mask(wmask.copy(), W, Ci, Cj, Cij, 0.01, H, Mc, 1, iterations)
+    got = k.update_mask(wmask.copy(), W, Ci, Cj, Cij, 0.01, H, Mc, 1, iterations)
+    assert np.array_equal(got, ref), f"masks differ in {(got != ref).sum()} entries"
+
+
+@pytest.mark.parametrize("dtype", DT)
 @pytest.mark.parametrize("N,H,Mc", [(1, 1, 1), (13, 4, 5), (1568, 30, 100), (100, 7, 9), (37, 3, 260), (50, 40, 100)])
 def test_apply_mask(k, oracle, dtype, N, H, Mc):
     rng = np.random.default_rng(N)
