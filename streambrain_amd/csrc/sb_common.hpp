@@ -231,11 +231,12 @@ struct BufferWindow {
   // keeps the following instructions from overwriting them only for stores without a scalar offset
   // register (with one, the first vector instruction after the store clobbered the data of its last lanes
   // whenever the memory pipeline was busy -- seen on gfx950 as wrong elements 1 and 2 of stored vectors).
+  template <int AUX = kStoreAux>
   __device__ __forceinline__ void store_vec(const T (&in)[Real<T>::VW], unsigned at, unsigned uniform) const {
     typename Real<T>::vec_t v;
 #pragma unroll
     for (int e = 0; e < Real<T>::VW; e++) v[e] = in[e];
-    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, v), rsrc, (int)(at + uniform), 0, kStoreAux);
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, v), rsrc, (int)(at + uniform), 0, AUX);
   }
   // NE consecutive elements (4, 8, 12 or 16 bytes) as one access; element-aligned
   template <int NE>
@@ -258,7 +259,7 @@ struct BufferWindow {
     }
     __builtin_memcpy(out, raw, BYTES);
   }
-  template <bool VEC>
+  template <bool VEC, int AUX = kStoreAux>
   __device__ __forceinline__ void store(const T (&in)[Real<T>::VW], unsigned at, unsigned uniform, long col,
                                         long limit) const {
     constexpr int VW = Real<T>::VW;
@@ -267,22 +268,22 @@ struct BufferWindow {
 #pragma unroll
       for (int e = 0; e < VW; e++) v[e] = in[e];
       __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, v), rsrc,
-                                             (int)((col < limit ? at : kOutside) + uniform), 0, kStoreAux);
+                                             (int)((col < limit ? at : kOutside) + uniform), 0, AUX);
     } else if (col + VW <= limit) {
       // (rows that are no whole number of vectors: only the last vector of a row runs over its end, so
       // in all but the last tile column this branch is taken by every lane)
       typename Real<T>::vec_t v;
 #pragma unroll
       for (int e = 0; e < VW; e++) v[e] = in[e];
-      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, v), rsrc, (int)(at + uniform), 0, kStoreAux);
+      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, v), rsrc, (int)(at + uniform), 0, AUX);
     } else {
 #pragma unroll
       for (int e = 0; e < VW; e++) {
         const int o = (int)(col + e < limit ? at + e * (unsigned)sizeof(T) : kOutside);
         if constexpr (sizeof(T) == 4)
-          __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, in[e]), rsrc, o, (int)uniform, kStoreAux);
+          __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, in[e]), rsrc, o, (int)uniform, AUX);
         else
-          __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u2, in[e]), rsrc, o, (int)uniform, kStoreAux);
+          __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u2, in[e]), rsrc, o, (int)uniform, AUX);
       }
     }
   }

@@ -86,6 +86,87 @@ __device__ inline T trace_next(T cold, T sum, const TrainArgs<T> &a) {
   return c > T(0) ? c : T(0);
 }
 
+// The first workgroups of the grid (the launcher adds them when there is something to prefetch; a multiple
+// of 8, so that the tiles keep their XCDs) touch one element of every 128-byte line of the region, a lane per line,
+// and leave (true): the lines come from HBM into the memory-side cache while the tiles compute.  A cold line takes
+// microseconds to arrive, which is why no tile does this on the side -- its own loads, which return in issue order,
+// would queue behind.
+template <typename T>
+__device__ __forceinline__ bool prefetch_region(const TrainArgs<T> &a) {
+  if (blockIdx.x >= a.prefetch_groups) return false;  // uniform
+  const __amdgpu_buffer_rsrc_t pwin = __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(a.prefetch), 0,
+                                                                        (int)a.prefetch_bytes, 0x00020000);
+  uint32_t sum = 0;
+  for (unsigned line = blockIdx.x * 256 + threadIdx.x; line < a.prefetch_lines; line += a.prefetch_groups * 256)
+    sum += __builtin_amdgcn_raw_buffer_load_b32(pwin, (int)(line * 128u), 0, 0);
+  asm volatile("" ::"v"(sum));  // (the loads have a consumer)
+  return true;
+}
+
+// The workgroup's tile (returned: its number in the order below).  Workgroup ids are dealt round-robin to the 8
+// XCDs, each with its own L2.  Renumbered so that one XCD
+// gets a contiguous run of tiles.  The run walks the tile grid in panels of panel_cols tile columns,
+// row by row inside a panel, so the tiles in flight at any time share a few column slabs of y and a
+// limited set of row slabs of x.  One column per panel (column-major order) when the whole batch of x
+// fits an L2 anyway: a few hundred KB of y plus all of x per L2.  For big layers a column-major order
+// re-read x from HBM once per tile column (measured 460 GB per launch at 65536 x 100000, batch 1024).
+// The grid has one workgroup per tile; XCD x = blockIdx % 8 holds tiles_of(x) = ntiles / 8 (+1 for
+// x < ntiles % 8) consecutive tiles.
+template <typename T>
+__device__ __forceinline__ unsigned tile_of_workgroup(const TrainArgs<T> &a, unsigned &it, unsigned &jt) {
+  const unsigned ntiles = (unsigned)a.tiles_i * (unsigned)a.tiles_j;  // < 2^31, checked by the launcher
+  const unsigned wg = blockIdx.x - a.prefetch_groups;
+  const unsigned xcd = wg & 7, rem = ntiles & 7;
+  const unsigned tile = xcd * (ntiles >> 3) + (xcd < rem ? xcd : rem) + (wg >> 3);
+  if (a.panel_cols == 1) {  // uniform
+    jt = a.by_panel.div(tile);
+    it = tile - jt * (unsigned)a.tiles_i;
+  } else {
+    const unsigned panel = a.by_panel.div(tile);
+    const unsigned in_panel = tile - panel * ((unsigned)a.tiles_i * a.panel_cols);
+    const unsigned first = panel * a.panel_cols;
+    const unsigned width = (unsigned)a.tiles_j - first < a.panel_cols ? (unsigned)a.tiles_j - first : a.panel_cols;
+    it = width == a.panel_cols ? in_panel >> __builtin_ctz(a.panel_cols) : in_panel / width;
+    jt = first + (in_panel - it * width);
+  }
+  return tile;
+}
+
+// ---- a float as three bfloat16: x = h + m + l exactly (for |x| of at least 2^-110; below, up to the smallest
+// bfloat16).  h holds the leading 8 bits, cut off, so that it is never beyond x; m the next 8, rounded; l the rest, at
+// most 8 bits.  For |x| below kSplitLimit: products of larger numbers, infinities and NaN are not what the products of
+// their pieces add up to.
+constexpr float kSplitLimit = 0x1p60f;
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+struct Split8 {  // eight consecutive batch rows of one column
+  bf16x8 h, m, l;
+};
+__device__ __forceinline__ Split8 split_bf16(const float (&x)[8]) {
+  Split8 s;
+#pragma unroll
+  for (int k = 0; k < 8; k++) {
+    const unsigned bits = __float_as_uint(x[k]);
+    const float rest = x[k] - __uint_as_float(bits & 0xffff0000u);
+    s.h[k] = __builtin_bit_cast(__bf16, (unsigned short)(bits >> 16));
+    s.m[k] = (__bf16)rest;
+    s.l[k] = (__bf16)(rest - (float)s.m[k]);
+  }
+  return s;
+}
+// The batch x [B, N] (or y) split like that, in the operand layout of the 16x16x32 bfloat16 MFMA: a lane takes
+// eight consecutive batch rows of one column as one 16-byte vector.  Vector ((b / 8) * 3 + piece) * width + slot(c)
+// holds rows 8 (b / 8) .. + 7 of column c; pieces in the order h, m, l; width is the number of columns padded to
+// whole tiles (what lies in the padding is never looked at).  Rows past the batch are zero, up to a whole number of
+// kSumRows.  slot(c) = c for x; for y the 64 columns of a tile are stored as four runs of 16, c % 4 first, which
+// makes a lane's results of a row four consecutive columns.
+// x_odd, y_odd: per 64 columns, whether one of their values is out of the range of the split.
+struct SplitBatch {
+  const bf16x8 *x, *y;
+  const int *x_odd, *y_odd;
+  unsigned x_width, y_width;
+};
+__device__ __forceinline__ unsigned y_slot(unsigned c) { return (c & ~63u) + (c & 3u) * 16 + ((c & 63u) >> 2); }
+
 // The new traces Ci_next, Cj_next (and the regularized bias) on their own: what every tile of k_train_fused
 // otherwise repeats for its own 64 rows and 64 columns.  Launched ahead of k_train_fused<.., PRE = true> when a
 // layer has so many tiles that the repetition costs more than a launch.  A workgroup takes 64 columns of x or
@@ -94,9 +175,11 @@ __device__ inline T trace_next(T cold, T sum, const TrainArgs<T> &a) {
 // chain: all 256 threads load the next 64 batch rows (16 independent loads each) into registers while 64 of
 // them add up the previous 64 rows from LDS, where the block was put down ahead of a barrier.  (1568 x 10000
 // doubles, batch 512: 27 -> 12 us, which is the 47 MB of x and y at 4 TB/s; a second block in flight: slower.)
+// SPLIT (float): the other three wavefronts meanwhile split the block into bfloat16 (see SplitBatch).
 constexpr int kSumRows = 64;  // batch rows per block
-template <typename T>
-__global__ __launch_bounds__(256) void k_trace_sums(TrainArgs<T> a) {
+template <typename T, bool SPLIT = false>
+__global__ __launch_bounds__(256) void k_trace_sums(TrainArgs<T> a, SplitBatch sp) {
+  static_assert(!SPLIT || sizeof(T) == 4, "floats are split");
   using R = Real<T>;
   __shared__ T block[2][kSumRows][64];
   const int tid = threadIdx.x, col = tid & 63, sub = tid >> 6;  // thread (sub, col) loads rows sub, sub + 4, ..
@@ -124,6 +207,7 @@ __global__ __launch_bounds__(256) void k_trace_sums(TrainArgs<T> a) {
   };
   request(0);
   T sum = T(0);
+  bool odd = false;
   int buf = 0;
   for (long b0 = 0; b0 < a.B; b0 += kSumRows, buf ^= 1) {
 #pragma unroll
@@ -139,7 +223,26 @@ __global__ __launch_bounds__(256) void k_trace_sums(TrainArgs<T> a) {
 #pragma unroll
         for (int k = 0; k < U; k++) sum = R::add(sum, w[k]);  // (zeros past the batch change nothing)
       }
+    } else if constexpr (SPLIT) {
+      const unsigned c0 = (unsigned)(idx - col), row_len = is_i ? sp.x_width : sp.y_width;
+      bf16x8 *const out = const_cast<bf16x8 *>(is_i ? sp.x : sp.y) + (b0 / 8) * 3 * (long)row_len;
+      for (int e = tid - 64; e < kSumRows / 8 * 64; e += 192) {
+        const int o = e >> 6, c = e & 63;
+        float v8[8];
+#pragma unroll
+        for (int k = 0; k < 8; k++) {
+          v8[k] = block[buf][8 * o + k][c];
+          odd = odd || !(__builtin_fabsf(v8[k]) < kSplitLimit);
+        }
+        const Split8 s8 = split_bf16(v8);
+        bf16x8 *const at = out + (long)o * 3 * row_len + (is_i ? c0 + c : y_slot(c0 + c));
+        at[0] = s8.h, at[row_len] = s8.m, at[2 * (long)row_len] = s8.l;
+      }
     }
+  }
+  if constexpr (SPLIT) {
+    const bool any = __syncthreads_or(odd) != 0;
+    if (tid == 0) const_cast<int *>(is_i ? sp.x_odd : sp.y_odd)[(idx - col) / 64] = any;
   }
   if (sub != 0 || idx >= width) return;
   const T cnew = trace_next<T>((is_i ? a.Ci : a.Cj)[idx], sum, a);
@@ -197,45 +300,9 @@ void k_train_fused(TrainArgs<T> a) {
   __shared__ int slow_s[2];
 
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, p = lane & 15, q = lane >> 4;
-  // Workgroup ids are dealt round-robin to the 8 XCDs, each with its own L2.  Renumbered so that one XCD
-  // gets a contiguous run of tiles.  The run walks the tile grid in panels of panel_cols tile columns,
-  // row by row inside a panel, so the tiles in flight at any time share a few column slabs of y and a
-  // limited set of row slabs of x.  One column per panel (column-major order) when the whole batch of x
-  // fits an L2 anyway: a few hundred KB of y plus all of x per L2.  For big layers a column-major order
-  // re-read x from HBM once per tile column (measured 460 GB per launch at 65536 x 100000, batch 1024).
-  // The grid has one workgroup per tile; XCD x = blockIdx % 8 holds tiles_of(x) = ntiles / 8 (+1 for
-  // x < ntiles % 8) consecutive tiles.
-  const unsigned ntiles = (unsigned)a.tiles_i * (unsigned)a.tiles_j;  // < 2^31, checked by the launcher
-  // The first workgroups of the grid (the launcher adds them when there is something to prefetch; a multiple
-  // of 8, so that the tiles keep their XCDs) touch one element
-  // of every 128-byte line of the region, a lane per line, and leave: the lines come from HBM into the
-  // memory-side cache while the tiles compute.  A cold line takes microseconds to arrive, which is why no
-  // tile does this on the side -- its own loads, which return in issue order, would queue behind.
-  if (blockIdx.x < a.prefetch_groups) {  // uniform
-    const __amdgpu_buffer_rsrc_t pwin = __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(a.prefetch), 0,
-                                                                          (int)a.prefetch_bytes, 0x00020000);
-    const unsigned first = blockIdx.x * 256 + tid;
-    uint32_t sum = 0;
-    for (unsigned line = first; line < a.prefetch_lines; line += a.prefetch_groups * 256)
-      sum += __builtin_amdgcn_raw_buffer_load_b32(pwin, (int)(line * 128u), 0, 0);
-    asm volatile("" ::"v"(sum));  // (the loads have a consumer)
-    return;
-  }
-  const unsigned wg = blockIdx.x - a.prefetch_groups;
-  const unsigned xcd = wg & 7, rem = ntiles & 7;
-  const unsigned tile = xcd * (ntiles >> 3) + (xcd < rem ? xcd : rem) + (wg >> 3);
+  if (prefetch_region(a)) return;
   unsigned it, jt;
-  if (a.panel_cols == 1) {  // uniform
-    jt = a.by_panel.div(tile);
-    it = tile - jt * (unsigned)a.tiles_i;
-  } else {
-    const unsigned panel = a.by_panel.div(tile);
-    const unsigned in_panel = tile - panel * ((unsigned)a.tiles_i * a.panel_cols);
-    const unsigned first = panel * a.panel_cols;
-    const unsigned width = (unsigned)a.tiles_j - first < a.panel_cols ? (unsigned)a.tiles_j - first : a.panel_cols;
-    it = width == a.panel_cols ? in_panel >> __builtin_ctz(a.panel_cols) : in_panel / width;
-    jt = first + (in_panel - it * width);
-  }
+  const unsigned tile = tile_of_workgroup(a, it, jt);
   // every index below fits 32 bits: N, M < 2^31 and 64 rows of x, y, Cij or W stay below 2 GiB (launcher)
   const unsigned N = (unsigned)a.N, M = (unsigned)a.M;
   const unsigned i0 = it * TS, j0 = jt * TS;
@@ -636,6 +703,207 @@ void k_train_fused(TrainArgs<T> a) {
       }
       wwin.template store<VEC>(wv, tat[g], v * vstep, ecol[g], a.M);
     }
+}
+
+// The fused pass for big float layers: Cij and W as k_train_fused writes them, with x^T y on the bfloat16 matrix
+// cores, which multiply sixteen times as fast as the float ones.  Both operands are split exactly into three bfloat16
+// (SplitBatch, written by k_trace_sums<float, true>, which also leaves the new traces), and the six products down to
+// 2^-16 are accumulated in float: h h + h m + m h + h l + l h + m m.  What is left out is below 2^-24 of a product
+// on either side of zero, less than the rounding of a float product, and an accumulator is rounded six times per 32
+// batch rows instead of 32.
+// Bound: Cij read and written once, W written once, against 6 x 2 B N M flops on the matrix cores; with the float
+// instructions those were 2 B N M at a sixteenth of the rate, which is what k_train_fused waits for here.
+// A workgroup (4 wavefronts) owns a tile of 128 x 64, a wavefront 32 rows of it: 2 x 4 blocks of 16 x 16, so
+// that 18 operand vectors from LDS feed 48 MFMAs.  32 batch rows at a time go from memory straight to LDS (36 KiB,
+// one buffer: the workgroups that share the CU fill each other's waits).  The Cij tile is requested ahead of the last
+// products.  A tile with a value out of the split's range takes the float instructions.
+// VEC, MB: as for k_train_fused.
+// Stores are non-temporal.  Rows that are no whole number of 128-byte lines (3000 columns) leave the ends of their
+// tiles' row pieces to be merged with the neighbouring tile's, and the write-through policy of k_train_fused, which
+// suits matrices that stay in the memory-side cache, pays for that once they do not (sums included, batch 128: 12288 x
+// 3000 87 us non-temporal, 192 us written through, 123 us with the default policy; 12288 x 3200 91 / 119 / 116 us).
+constexpr int kSplitTileI = 128, kSplitTileJ = 64, kSplitRows = 32;
+template <bool VEC, int MB>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4)))
+void k_train_split(TrainArgs<float> a, SplitBatch sp) {
+  using R = Real<float>;
+  constexpr unsigned ES = 4, kOutside = BufferWindow<float>::kOutside;
+  constexpr int TI = kSplitTileI, TJ = kSplitTileJ, OCT = kSplitRows / 8, kNonTemporal = 2;
+  __shared__ __attribute__((aligned(16))) bf16x8 xs[OCT * 3 * TI], ys[OCT * 3 * TJ];
+  __shared__ __attribute__((aligned(16))) float rci_s[TI], rcj_s[TJ];
+  const int tid = threadIdx.x, lane = tid & 63, p = lane & 15, q = lane >> 4;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  if (prefetch_region(a)) return;
+  unsigned it, jt;
+  tile_of_workgroup(a, it, jt);
+  const unsigned N = (unsigned)a.N, M = (unsigned)a.M;
+  const unsigned i0 = it * TI, j0 = jt * TJ;
+
+  // 32 batch rows into LDS: wavefront w brings octet w of either slab, 1 KiB per load
+  using lds_t = __attribute__((address_space(3))) void;
+  auto stage = [&](long chunk) {
+    const __amdgpu_buffer_rsrc_t xwin = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<bf16x8 *>(uniform_pointer(sp.x + chunk * OCT * 3 * sp.x_width)), 0, (int)(OCT * 3 * sp.x_width * 16), 0x00020000);
+    const __amdgpu_buffer_rsrc_t ywin = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<bf16x8 *>(uniform_pointer(sp.y + chunk * OCT * 3 * sp.y_width)), 0, (int)(OCT * 3 * sp.y_width * 16), 0x00020000);
+#pragma unroll
+    for (int piece = 0; piece < 3; piece++) {
+#pragma unroll
+      for (int half = 0; half < 2; half++)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(xwin, (lds_t *)&xs[(w * 3 + piece) * TI + 64 * half], 16,
+                                                 (int)((i0 + 64 * half + lane) * 16), (int)((w * 3 + piece) * sp.x_width * 16), 0, 0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(ywin, (lds_t *)&ys[(w * 3 + piece) * TJ], 16, (int)((j0 + lane) * 16),
+                                               (int)((w * 3 + piece) * sp.y_width * 16), 0, 0);
+    }
+  };
+  stage(0);
+
+  // reciprocals of the new traces, and whether the tile can take the short form of the weight (see k_train_fused)
+  bool odd = false;
+  if (tid < TI + TJ) {
+    const bool is_i = tid < TI;
+    const unsigned idx = is_i ? i0 + tid : j0 + (tid - TI);
+    const bool inside = idx < (is_i ? N : M);
+    const float c = inside ? (is_i ? a.Ci_next : a.Cj_next)[idx] : 1.0f;
+    odd = inside && (!(c >= a.cthr) || !(c <= a.lim));
+    (is_i ? rci_s[tid] : rcj_s[tid - TI]) = trace_reciprocal<float>(c, a.cthr);
+  }
+  const bool slow = __syncthreads_or(odd) != 0;
+
+  f32x4 acc[2][4];
+#pragma unroll
+  for (int r = 0; r < 2; r++)
+#pragma unroll
+    for (int c = 0; c < 4; c++) acc[r][c] = f32x4{0, 0, 0, 0};
+  auto multiply = [&]() {
+    bf16x8 xa[2][3];
+#pragma unroll
+    for (int r = 0; r < 2; r++)
+#pragma unroll
+      for (int k = 0; k < 3; k++) xa[r][k] = xs[(q * 3 + k) * TI + 32 * w + 16 * r + p];
+#pragma unroll
+    for (int c = 0; c < 4; c++) {
+      bf16x8 yb[3];
+#pragma unroll
+      for (int k = 0; k < 3; k++) yb[k] = ys[(q * 3 + k) * TJ + 16 * c + p];
+      // the smallest products first
+      constexpr int pair[6][2] = {{2, 0}, {0, 2}, {1, 1}, {1, 0}, {0, 1}, {0, 0}};
+#pragma unroll
+      for (int k = 0; k < 6; k++)
+#pragma unroll
+        for (int r = 0; r < 2; r++)
+          acc[r][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xa[r][pair[k][0]], yb[pair[k][1]], acc[r][c], 0, 0, 0);
+    }
+  };
+
+  // this lane's share of the tile: rows r0 + 16 r + v, columns 4 p .. 4 p + 3
+  const unsigned r0 = 32 * w + 4 * q, ecol = j0 + 4 * p;
+  const long tile_rows = (long)N - i0 < TI ? (long)N - i0 : TI;
+  const unsigned tile_bytes = (unsigned)tile_rows * M * ES;  // at most 2 GiB (launcher)
+  const BufferWindow<float> cwin(uniform_pointer(a.Cij + (long)i0 * a.M), BufferWindow<float>::Bytes{tile_bytes}),
+      wwin(uniform_pointer(a.W + (long)i0 * a.M), BufferWindow<float>::Bytes{a.W ? tile_bytes : 0u});
+  const bool col_ok = ecol < M, masked = a.wmask != nullptr;
+  auto at = [&](int r, int v) { return col_ok ? ((r0 + 16 * r + v) * M + ecol) * ES : kOutside; };
+  float cpre[2][4][4];
+  uint32_t mb[2][4][MB];
+  auto request_tile = [&]() {
+    const ByteWindow mwin(masked ? a.wmask + (long)i0 * a.H : nullptr, tile_rows * a.H);
+    unsigned hc[MB];
+#pragma unroll
+    for (int e = 0; e < MB; e++) hc[e] = ecol + e < M ? a.by_Mc.div(ecol + e) : 0u;
+#pragma unroll
+    for (int r = 0; r < 2; r++)
+#pragma unroll
+      for (int v = 0; v < 4; v++) {
+        cwin.load_vec(cpre[r][v], at(r, v), 0);
+#pragma unroll
+        for (int e = 0; e < MB; e++) mb[r][v][e] = mwin.load((r0 + 16 * r + v) * (unsigned)a.H + hc[e], 0);
+      }
+  };
+
+  // the products in float, operands straight from memory, four batch rows at a time
+  auto multiply_float = [&]() {
+    const unsigned i = i0 + 32 * w + p;
+    for (long b0 = 0; b0 < a.B; b0 += 4) {
+      const unsigned rows = a.B - b0 < 4 ? (unsigned)(a.B - b0) : 4u;
+      const BufferWindow<float> xwin(uniform_pointer(a.x + b0 * a.N), BufferWindow<float>::Bytes{rows * N * ES}),
+          ywin(uniform_pointer(a.y + b0 * a.M), BufferWindow<float>::Bytes{rows * M * ES});
+      float xv[2][1], yv[4];
+#pragma unroll
+      for (int r = 0; r < 2; r++) xwin.load_n<1>(xv[r], i + 16 * r < N ? (q * N + i + 16 * r) * ES : kOutside);
+      ywin.load_vec(yv, col_ok ? (q * M + ecol) * ES : kOutside, 0);
+#pragma unroll
+      for (int c = 0; c < 4; c++)
+#pragma unroll
+        for (int r = 0; r < 2; r++) acc[r][c] = R::mfma(xv[r][0], yv[c], acc[r][c]);
+    }
+  };
+  const bool in_float = sp.x_odd[i0 / 64] | sp.x_odd[i0 + 64 < N ? i0 / 64 + 1 : i0 / 64] | sp.y_odd[j0 / 64];
+
+  const long chunks = (a.B + kSplitRows - 1) / kSplitRows;
+  // (what is outstanding at a wait below are this wavefront's loads to LDS)
+  constexpr int kNoLoadsLeft = 0x0f70;  // vmcnt(0)
+  if (in_float) {  // uniform
+    multiply_float();
+    request_tile();
+  } else {
+    for (long ch = 0; ch + 1 < chunks; ch++) {
+      __builtin_amdgcn_s_waitcnt(kNoLoadsLeft);
+      __syncthreads();  // the slab is there
+      multiply();
+      __syncthreads();  // everybody has read it
+      stage(ch + 1);
+    }
+    __builtin_amdgcn_s_waitcnt(kNoLoadsLeft);
+    __syncthreads();
+    request_tile();
+    multiply();
+  }
+
+  const float scale = a.invB * a.tau;
+#pragma unroll
+  for (int r = 0; r < 2; r++)
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+      float cv[4];
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        cpre[r][v][e] = cpre[r][v][e] * a.omt + acc[r][e][v] * scale;
+        cv[e] = fmax(cpre[r][v][e], 0.0f);  // 0 as well when it is NaN, like the reference's `cn > 0 ? cn : 0`
+      }
+      cwin.template store<VEC, kNonTemporal>(cv, at(r, v), 0, ecol, a.M);
+    }
+  if (a.W == nullptr) return;  // (uniform) traces only
+  const f32x4 rcj = *reinterpret_cast<const f32x4 *>(&rcj_s[4 * p]);
+#pragma unroll
+  for (int r = 0; r < 2; r++) {
+    const f32x4 rci = *reinterpret_cast<const f32x4 *>(&rci_s[r0 + 16 * r]);
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+      bool on[4], connected = false;
+#pragma unroll
+      for (int e = 0; e < 4; e++) on[e] = !masked || mb[r][v][MB == 1 ? 0 : e] != 0, connected = connected || on[e];
+      // (where the caller vouches that W is zero under the mask, such vectors are not stored)
+      if (a.w_masked && __builtin_amdgcn_ballot_w64(connected) == 0) continue;
+      float wv[4];
+      if (!slow) {  // uniform
+#pragma unroll
+        for (int e = 0; e < 4; e++) wv[e] = R::wlog_normal(R::max_floor(cpre[r][v][e], a.cthr4) * rci[v] * rcj[e]);
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          wv[e] = R::wlog(R::max_floor(cpre[r][v][e], a.cthr4) * rci[v] * rcj[e]);
+          if (rci[v] < 0.0f || rcj[e] < 0.0f) wv[e] = 0.0f;
+        }
+      }
+#pragma unroll
+      for (int e = 0; e < 4; e++) wv[e] = on[e] ? wv[e] : 0.0f;
+      if (VEC && MB == 1)
+        wwin.template store_vec<kNonTemporal>(wv, (a.w_masked && !connected) ? kOutside : at(r, v), 0);
+      else
+        wwin.template store<VEC, kNonTemporal>(wv, at(r, v), 0, ecol, a.M);
+    }
+  }
 }
 
 }  // namespace sb

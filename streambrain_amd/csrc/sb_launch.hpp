@@ -102,7 +102,12 @@ template <typename T>
 int launch_train_fused(hipStream_t st, const T *x, const T *y, T *Cij, T *W, const T *Ci, const T *Cj,
                        T *Ci_next, T *Cj_next, const uint8_t *wmask, int bias_mode, T *bias, T *kbi,
                        long B, long N, long H, long Mc, T taupdt, T cthr, T khalf, T pmin, T taubdt,
-                       bool w_masked, const void *prefetch = nullptr, size_t prefetch_bytes = 0);
+                       bool w_masked, const void *prefetch = nullptr, size_t prefetch_bytes = 0,
+                       void *split = nullptr);
+// Bytes of scratch (16-byte aligned) that launch_train_fused makes use of as `split` for a layer and batch of these
+// sizes; 0: none.  Without it (nullptr) the launch does without the kernel that needs it.
+template <typename T>
+size_t train_split_bytes(long B, long N, long H, long Mc);
 // W from the traces as they are, the fused kernel's expression; wmask != nullptr: zero under zero mask bytes
 // (w_masked: the caller vouches that W is zero there already, and such entries are left alone).
 template <typename T>

@@ -247,11 +247,32 @@ int launch_softmax(hipStream_t st, T *act, long B, long H, long Mc) {
 }
 
 // ------------------------------------------------------------------------------------- fused training
+// One round of workgroups: every one finds a slot at once (five per CU for floats of whole vectors, else four).
+template <typename T>
+static long train_tiles_of_one_round() { return (long)train_waves_per_simd<T, true, 1>() * device_cu_count(); }
+
+// Floats go through k_trace_sums<float, true> and k_train_split from one round of 64 x 64 tiles on, with small batches,
+// which leave the matrix cores little to do, from five.  Sums included, against k_train_fused on its own, 3000
+// columns: batch 128, 1568 rows (0.9 rounds) 24.3 / 18.8 us, 2048 rows 26.0 / 26.7, 4096 39.7 / 47.8, 16384 110 / 257; batch
+// 512, 2048 rows 53.6 / 75.0; batch 32, 2048 rows 19.2 / 16.1, 8192 (4.7 rounds) 54.6 / 53.5, 27648 255 / 369.
+// Its windows hold 128 rows of Cij and 32 split batch rows.
+template <typename T>
+size_t train_split_bytes(long B, long N, long H, long Mc) {
+  if constexpr (sizeof(T) != 4) return 0;
+  if (B <= 0 || N <= 0 || H <= 0 || Mc <= 0) return 0;
+  const long M = H * Mc;
+  if (M <= 32 || cdiv(N, 64) * cdiv(M, 64) <= (B > 32 ? 1 : 5) * train_tiles_of_one_round<T>()) return 0;
+  const long xw = cdiv(N, kSplitTileI) * kSplitTileI, yw = cdiv(M, kSplitTileJ) * kSplitTileJ;
+  const long wider = xw > yw ? xw : yw;
+  if (128 * M * 4 >= (1L << 31) || wider * (kSplitRows / 8) * 3 * 16 >= (1L << 31)) return 0;
+  return (size_t)(xw + yw) * 6 * (size_t)(cdiv(B, kSumRows) * kSumRows) + (size_t)(xw + yw) / 64 * sizeof(int);
+}
+
 template <typename T>
 int launch_train_fused(hipStream_t st, const T *x, const T *y, T *Cij, T *W, const T *Ci, const T *Cj,
                        T *Ci_next, T *Cj_next, const uint8_t *wmask, int bias_mode, T *bias, T *kbi,
                        long B, long N, long H, long Mc, T taupdt, T cthr, T khalf, T pmin, T taubdt,
-                       bool w_masked, const void *prefetch, size_t prefetch_bytes) {
+                       bool w_masked, const void *prefetch, size_t prefetch_bytes, void *split) {
   constexpr int VW = Real<T>::VW;
   SB_REQUIRE(x && y && Cij && Ci && Cj && Ci_next && Cj_next, "null pointer");  // W may be null: traces only
   SB_REQUIRE(Ci != Ci_next && Cj != Cj_next, "old and new traces must be distinct buffers");
@@ -325,25 +346,47 @@ int launch_train_fused(hipStream_t st, const T *x, const T *y, T *Cij, T *W, con
   const bool one_byte = Mc % VW == 0;  // every vector of VW columns lies inside one hypercolumn
   ProfScope prof_(st, K_TRAIN_FUSED, true);
   // one launch, or the sum launch and the tile launch, with the profile's events riding on them
-  auto launch = [&](auto kernel, dim3 g, bool first, bool last) {
+  auto launch = [&](auto kernel, dim3 g, bool first, bool last, auto... more) {
     if (prof_.carries())
       hipExtLaunchKernelGGL(kernel, g, dim3(256), 0, st, first ? prof_.start() : nullptr,
-                            last ? prof_.stop() : nullptr, 0, a);
+                            last ? prof_.stop() : nullptr, 0, a, more...);
     else
-      hipLaunchKernelGGL(kernel, g, dim3(256), 0, st, a);
+      hipLaunchKernelGGL(kernel, g, dim3(256), 0, st, a, more...);
   };
+  const dim3 sums((unsigned)(cdiv(N, 64) + cdiv(M, 64)));
+  if constexpr (sizeof(T) == 4) {
+    if (split && train_split_bytes<T>(B, N, H, Mc) > 0) {
+      SplitBatch sp;
+      sp.x_width = (unsigned)(cdiv(N, kSplitTileI) * kSplitTileI);
+      sp.y_width = (unsigned)(cdiv(M, kSplitTileJ) * kSplitTileJ);
+      sp.x = (const bf16x8 *)split;
+      const long octets = cdiv(B, kSumRows) * kSumRows / 8;
+      sp.y = sp.x + octets * 3 * sp.x_width;
+      sp.x_odd = (const int *)(sp.y + octets * 3 * sp.y_width);
+      sp.y_odd = sp.x_odd + sp.x_width / 64;
+      a.tiles_i = cdiv(N, kSplitTileI);
+      a.tiles_j = cdiv(M, kSplitTileJ);
+      a.by_panel = FastDiv::of(a.tiles_i * a.panel_cols);
+      launch(k_trace_sums<T, true>, sums, true, false, sp);
+      const dim3 tiles((unsigned)(a.tiles_i * a.tiles_j) + a.prefetch_groups);
+      if (vec && one_byte) launch(k_train_split<true, 1>, tiles, false, true, sp);
+      else if (vec) launch(k_train_split<true, VW>, tiles, false, true, sp);
+      else launch(k_train_split<false, VW>, tiles, false, true, sp);  // (one_byte implies vec)
+      SB_LAUNCH_CHECK();
+      return 0;
+    }
+  }
   // Every tile adds up the batch's x and y columns for its own rows and columns, which with many tile
   // rows and columns is most of the kernel's vector arithmetic (43 % at 65536 x 100000, batch 1024).
-  // From one and a half rounds of workgroups on (floats; doubles: two and a half), a small launch computes the
-  // new traces once and the tiles read them.  Timed, 4096 inputs, batch 128, floats, with / without that
+  // From one and a half rounds of workgroups on (floats with more than 32 rows; doubles: two and a half), a small launch
+  // computes the new traces once and the tiles read them (floats: only where k_train_split has no scratch).  Timed, 4096 inputs, batch 128, floats, with / without that
   // launch: 23.7 / 22.5 us at 1.05 rounds, 29.3 / 29.9 at 1.5, 34.6 / 35.6 at 2, 45.5 / 48.5 at 3, 67.1 / 69.2
   // at 5; doubles: 48.1 / 47.3 at 1.6 rounds, 55.8 / 54.3 at 2, 110.3 / 113.7 at 2.5.
   const long ntiles = a.tiles_i * a.tiles_j;
-  // one round: every workgroup finds a slot at once (five per CU for floats of whole vectors, else four)
-  const bool one_round = ntiles <= (long)train_waves_per_simd<T, true, 1>() * device_cu_count();
+  const bool one_round = ntiles <= train_tiles_of_one_round<T>();
   const long pre_from = sizeof(T) == 8 ? 5 * 4 : 3 * 5;  // in half workgroups per CU
-  if (vec && one_byte && 2 * ntiles >= pre_from * device_cu_count()) {
-    launch(k_trace_sums<T>, dim3((unsigned)(cdiv(N, 64) + cdiv(M, 64))), true, false);
+  if (vec && one_byte && 2 * ntiles >= pre_from * device_cu_count() && (sizeof(T) == 8 || B > 32)) {
+    launch(k_trace_sums<T>, sums, true, false, SplitBatch{});
     launch(k_train_fused<T, KCH, true, 1, true>, grid, false, true);
   } else if (vec && one_byte && one_round)
     launch(k_train_fused<T, KCH, true, 1, false, true>, grid, true, true);
@@ -625,7 +668,8 @@ int launch_copy_pair(hipStream_t st, T *dst1, const T *src1, size_t n1, T *dst2,
   template int launch_softmax<T>(hipStream_t, T *, long, long, long);                                 \
   template int launch_train_fused<T>(hipStream_t, const T *, const T *, T *, T *, const T *, const T *, \
                                      T *, T *, const uint8_t *, int, T *, T *, long, long, long, long, \
-                                     T, T, T, T, T, bool, const void *, size_t);                                             \
+                                     T, T, T, T, T, bool, const void *, size_t, void *);              \
+  template size_t train_split_bytes<T>(long, long, long, long);                                       \
   template int launch_update_bias<T>(hipStream_t, T *, const T *, T, long);                           \
   template int launch_weights_from_traces<T>(hipStream_t, T *, const T *, const T *, const T *,       \
                                              const uint8_t *, T, long, long, long, bool);             \

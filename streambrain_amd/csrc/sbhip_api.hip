@@ -54,6 +54,9 @@ struct Context {
   // scratch of the per-kernel training entry points: the "next" Ci / Cj of the fused kernel
   void *trace_next = nullptr;
   long trace_cap = 0;  // elements of 8 bytes
+  // scratch of the per-kernel training entry points: the split batch (train_split_bytes)
+  void *split = nullptr;
+  size_t split_cap = 0;
   // device address of `scratch` on this context's device
   void *noalloc_scratch = nullptr;
 };
@@ -295,6 +298,21 @@ static int ensure_trace_scratch(long elems) {
   return 0;
 }
 
+// The context's scratch for a split batch of `bytes`, or nullptr when none is asked for or the memory is not there (the
+// training pass then does without).
+static void *split_scratch(size_t bytes) {
+  if (bytes > g_ctx.split_cap) {
+    (void)hipStreamSynchronize(g_ctx.stream);
+    if (g_ctx.split) (void)hipFree(g_ctx.split);
+    g_ctx.split = nullptr;
+    g_ctx.split_cap = 0;
+    if (dev_malloc(&g_ctx.split, bytes) == hipSuccess) g_ctx.split_cap = bytes;
+    else g_ctx.split = nullptr;
+    (void)hipGetLastError();
+  }
+  return bytes ? g_ctx.split : nullptr;
+}
+
 // Per-kernel entry points keep the reference's in-place contract: the fused kernel writes the new
 // Ci / Cj into scratch, which is then copied over the caller's arrays.
 // `fixed_scratch`: room for N + M elements that the caller brings (no allocation here), or nullptr to
@@ -310,7 +328,8 @@ static int train_in_place(const T *x, const T *y, T *Cij, T *W, T *Ci, T *Cj, co
   if (rc) return rc;
   T *ci_next = fixed_scratch ? fixed_scratch : (T *)g_ctx.trace_next, *cj_next = ci_next + N;
   rc = launch_train_fused<T>(st, x, y, Cij, W, Ci, Cj, ci_next, cj_next, wmask, bias_mode, bias, kbi, B,
-                             N, H, Mc, taupdt, cthr, khalf, pmin, taubdt, false);
+                             N, H, Mc, taupdt, cthr, khalf, pmin, taubdt, false, nullptr, 0,
+                             fixed_scratch ? nullptr : split_scratch(train_split_bytes<T>(B, N, H, Mc)));
   if (rc) return rc;
   return launch_copy_pair<T>(st, Ci, ci_next, (size_t)N, Cj, cj_next, (size_t)M);
 }
@@ -365,6 +384,7 @@ struct sb_net {
     void *p = nullptr;
     size_t cap = 0;
   } ev_x, ev_xb, ev_y, ev_p;
+  Reusable split;  // a training batch split into bfloat16 (train_split_bytes)
 };
 
 namespace sb {
@@ -488,16 +508,22 @@ static int layer_forward(sb_net *net, Layer &L, const T *x, long B, const T *x_b
 // is re-scored from the traces and its W columns rewritten under the new mask.
 // next / next_bytes: what the step after this one reads first (its batch of inputs), or nullptr
 template <typename T>
-static int layer_train_step(Layer &L, const T *x, const T *y, long B, long h, const void *next = nullptr,
+static int layer_train_step(sb_net *net, Layer &L, const T *x, const T *y, long B, long h, const void *next = nullptr,
                             size_t next_bytes = 0) {
   hipStream_t st = g_ctx.stream;
   const T tau = (T)L.taupdt;
   const T cthr = (T)(L.taupdt / 2);
   int rc = 0;
+  const size_t split_bytes = train_split_bytes<T>(B, L.N, L.H, L.Mc);
+  if (reuse_dev(net->split, split_bytes)) {  // no memory for it: the training pass does without
+    (void)hipGetLastError();
+    net->split.p = nullptr;
+  }
   rc = launch_train_fused<T>(st, x, y, (T *)L.Cij, (T *)L.W, (const T *)L.Ci, (const T *)L.Cj,
                              (T *)L.Ci_alt, (T *)L.Cj_alt, L.plastic ? L.wmask : nullptr,
                              L.plastic ? 1 : 0, (T *)L.bias, (T *)L.kbi, B, L.N, L.H, L.Mc, tau, cthr,
-                             (T)L.khalf, (T)L.pmin, (T)L.taubdt, L.w_masked, next, next_bytes);
+                             (T)L.khalf, (T)L.pmin, (T)L.taubdt, L.w_masked, next, next_bytes,
+                             split_bytes ? net->split.p : nullptr);
   if (rc) return rc;
   std::swap(L.Ci, L.Ci_alt);
   std::swap(L.Cj, L.Cj_alt);
@@ -688,7 +714,7 @@ static int net_train_batches(sb_net *net, int layer, long maxB, const int64_t *h
     if (last) {
       // the reference also evaluates the last layer's activation here and drops it
       // (_cpu_base_backend.py:290-295, 304-306); it has no effect on any state
-      rc = layer_train_step<T>(target, x, (const T *)net->Yp + lo * net->NC, B, -1);
+      rc = layer_train_step<T>(net, target, x, (const T *)net->Yp + lo * net->NC, B, -1);
     } else {
       if ((rc = layer_forward<T>(net, target, x, B, layer == 0 ? xb : nullptr))) return rc;
       // The next step's images, when its forward pass is the dense one, which reads its input in step with W
@@ -699,7 +725,7 @@ static int net_train_batches(sb_net *net, int layer, long maxB, const int64_t *h
       const bool more = layer == 0 && i + 1 < nb && !(target.rows && target.w_masked);
       const long nB = more ? (nlo + maxB <= Ns ? maxB : Ns - nlo) : 0;
       const T *nx = xb ? xb + maxB * net->NF : (const T *)net->Xp + nlo * net->NF;
-      rc = layer_train_step<T>(target, x, (const T *)target.act, B, h, more ? nx : nullptr,
+      rc = layer_train_step<T>(net, target, x, (const T *)target.act, B, h, more ? nx : nullptr,
                                (size_t)nB * net->NF * sizeof(T));
     }
     if (rc) return rc;
@@ -833,7 +859,7 @@ static int net_layer_train_step(sb_net *net, int layer, const void *h_in, const 
   SB_HIP(dev_malloc(&bY.p, (size_t)rows * L.M * sizeof(T)));
   SB_HIP(hipMemcpy(bX.p, h_in, (size_t)rows * L.N * sizeof(T), hipMemcpyHostToDevice));
   SB_HIP(hipMemcpy(bY.p, h_out, (size_t)rows * L.M * sizeof(T), hipMemcpyHostToDevice));
-  rc = layer_train_step<T>(L, (const T *)bX.p, (const T *)bY.p, rows, h);
+  rc = layer_train_step<T>(net, L, (const T *)bX.p, (const T *)bY.p, rows, h);
   SB_HIP(hipStreamSynchronize(g_ctx.stream));  // the staging buffers go out of scope
   return rc;
 }
@@ -952,6 +978,7 @@ int sb_shutdown(void) {
   if (g_ctx.mask_nom) SB_HIP(hipFree(g_ctx.mask_nom));
   if (g_ctx.mask_csum) SB_HIP(hipFree(g_ctx.mask_csum));
   if (g_ctx.trace_next) SB_HIP(hipFree(g_ctx.trace_next));
+  if (g_ctx.split) SB_HIP(hipFree(g_ctx.split));
   stager_release();
   SB_HIP(hipStreamDestroy(g_ctx.stream));
   g_ctx = Context();
@@ -1186,6 +1213,7 @@ int sb_net_destroy(sb_net *net) {
   int rc = sb_net_training_done(net);
   for (auto &L : net->layers) rc |= layer_free(L);
   rc |= free_dev(net->ev_x.p); rc |= free_dev(net->ev_xb.p); rc |= free_dev(net->ev_y.p); rc |= free_dev(net->ev_p.p);
+  rc |= free_dev(net->split.p);
   if (net->d_correct) SB_HIP(hipFree(net->d_correct));
   if (net->d_unmasked) SB_HIP(hipFree(net->d_unmasked));
   if (net->perm_copied) SB_HIP(hipEventDestroy(net->perm_copied));

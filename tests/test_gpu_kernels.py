@@ -479,6 +479,46 @@ def test_plastic_train_step(k, oracle, dtype, B, N, H, Mc, h):
     _check_plastic_train_step(k, oracle, dtype, B, N, H, Mc, h, np.random.default_rng(B + N + H + Mc))
 
 
+# 64 x 64 tiles of these layers: more than 1280 with more than 32 rows, more than 6400 below, which is where the pass
+# goes over to bfloat16 pieces
+@pytest.mark.parametrize("B,N,H,Mc,masked", [
+    (1, 8200, 33, 100, True), (31, 8193, 50, 66, False), (32, 8257, 33, 101, True),
+    *[(B, *s) for B in (33, 63, 64, 65, 128, 257) for s in ((2689, 30, 100, True), (4096, 21, 64, True),
+                                                           (4097, 46, 66, True), (4159, 3, 676, False),
+                                                           (3001, 29, 101, True), (8001, 331, 4, True))]])
+def test_train_pass_of_big_float_layers(k, B, N, H, Mc, masked):
+    """Tile remainders on either side, batch remainders, values over 40 binary orders of magnitude, and values out of
+    the range of the bfloat16 pieces (1e30, infinity), which only the tiles that hold them treat differently."""
+    rng = np.random.default_rng(B + N)
+    M, f = H * Mc, np.float32
+    x = (rng.random((B, N)) * np.exp2(-40 * rng.random((1, N))) * (rng.random((B, N)) < 0.7)).astype(f)
+    y = np.exp2(-20 * rng.random((B, M)) ** 2).astype(f)
+    x[0, 5], x[B // 2, 200] = 1e30, np.inf
+    st = {"weights": np.ones((N, M), f), "bias": np.zeros(M, f), "kbi": np.ones(M, f), "Ci": rng.random(N).astype(f),
+          "Cj": rng.random(M).astype(f), "Cij": rng.random((N, M)).astype(f),
+          "wmask": (rng.random((N, H)) < (0.3 if masked else 2)).astype(np.uint8)}
+    tau = f(0.1)
+    got = k.plastic_train_step({n: v.copy() for n, v in st.items()}, x, y, H, Mc, tau, -139.0, 0.062, 0.022,
+                               hypercolumn=None)
+    t, x64, y64 = float(tau), x.astype(np.float64), y.astype(np.float64)
+    ci, cj = ((1 - t) * st[n] + t * a.mean(0) for n, a in (("Ci", x64), ("Cj", y64)))
+    cij = (1 - t) * st["Cij"] + t * (x64.T @ y64) / B
+    # an accumulator is rounded six times per 32 batch rows (a row of ones among them: four times per 4 rows in the
+    # tiles that stay in float), the decay, the scale and their sum four times
+    bound = 2.0 ** -24 * (4 + np.where((np.arange(N) // 128 < 2), B + 4, 6 * (B // 32 + 1)))[:, None]
+    fin = np.isfinite(cij)
+    assert np.array_equal(got["Cij"][~fin], cij[~fin].astype(f))
+    off = np.abs(got["Cij"][fin] - cij[fin]) / cij[fin]
+    assert np.all(off <= np.broadcast_to(bound, fin.shape)[fin]), f"Cij: {off.max():.2e}"
+    with np.errstate(invalid="ignore"):
+        w = np.where((ci < t / 2)[:, None] | (cj < t / 2)[None], 0, np.log(np.maximum(cij, (t / 2) ** 4) / (ci[:, None] * cj)))
+    w *= np.repeat(st["wmask"], Mc, axis=1)
+    rows = np.arange(N) != 200
+    assert_close(got["weights"][rows], w[rows], f, "W")
+    assert_close(got["Ci"][rows], ci[rows], f, "Ci", scale=10)
+    assert_close(got["Cj"], cj, f, "Cj")
+
+
 def _random_shapes(seed, count):
     """Shapes off every tiling's grid: mostly odd widths, batches around the 16- and 32-row boundaries."""
     rng = np.random.default_rng(seed)
