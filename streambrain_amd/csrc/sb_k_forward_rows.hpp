@@ -55,7 +55,9 @@ constexpr int forward_rows_waves_per_simd() {
 // SEG: list entries staged per segment, 2048 or, for lists of at most 256 entries, 256: every thread loads
 // and stores SEG / 256 entries per segment whatever the list's length, and at batch 128 the kernel is a
 // chain of latencies that starts with this staging (1568 -> 30x100, density 0.1, lists of 157: 6.31 -> 6.13 us).
-template <typename T, int NG, int NWAVES, int RB = 1, bool XT = false, int LW = Real<T>::VW, int SEG = 2048>
+// SPLIT: a split reduction (see ForwardArgs): a workgroup walks a.split_chunks chunks of its list.
+template <typename T, int NG, int NWAVES, int RB = 1, bool XT = false, int LW = Real<T>::VW, int SEG = 2048,
+          bool SPLIT = false>
 __global__ __launch_bounds__(64 * NWAVES)
 __attribute__((amdgpu_waves_per_eu(forward_rows_waves_per_simd<T, NG, RB>(),
                                    forward_rows_waves_per_simd<T, NG, RB>())))
@@ -106,8 +108,11 @@ void k_forward_rows(ForwardRowsArgs<T> ar) {
       sidx[tid + t * (64 * NWAVES)] = k < ar.cap ? mine[t] : -1;
     }
   };
-  request_segment(0);
-  const int cnt = ar.row_cnt[ct];
+  const long seg_first = SPLIT ? (long)blockIdx.y * a.split_chunks * KC : 0;
+  request_segment(seg_first);
+  // entries up to the end of this workgroup's part
+  const int in_list = ar.row_cnt[ct];
+  const int cnt = SPLIT && seg_first + a.split_chunks * KC < in_list ? (int)(seg_first + a.split_chunks * KC) : in_list;
 
   acc_t acc[RB][NG][VW];
 #pragma unroll
@@ -118,7 +123,12 @@ void k_forward_rows(ForwardRowsArgs<T> ar) {
       for (int c = 0; c < VW; c++) acc[r][g][c] = acc_t{0, 0, 0, 0};
 
   T bv[ForwardBias<T, NG, NWAVES>::PT];
-  ForwardBias<T, NG, NWAVES>::load(bv, a.bias, j0, ncol);
+  if constexpr (SPLIT) {
+#pragma unroll
+    for (int t = 0; t < ForwardBias<T, NG, NWAVES>::PT; t++) bv[t] = T(0);
+  } else {
+    ForwardBias<T, NG, NWAVES>::load(bv, a.bias, j0, ncol);
+  }
 
   // x through a bounds-checked window over this tile's batch rows: rows past the batch and padding
   // entries (offset kOutside) read zero.  Blocked copy: block b0/16 + r starts N*16 elements after the
@@ -179,16 +189,17 @@ void k_forward_rows(ForwardRowsArgs<T> ar) {
           }
   };
 
-  for (long seg0 = 0;;) {
+  for (long seg0 = seg_first;;) {
     publish_segment(seg0);
     __syncthreads();
     request(w, xr[0], wr[0]);  // this wavefront's first chunk of the segment
     // chunks w, w + NWAVES, ... of the segment that hold list entries: n of them (at least 1 in the
     // first segment, see above)
     const long left = (long)cnt - seg0;  // entries from the start of this segment
-    const long segc = left >= SEG ? SEGC : (left + KC - 1) / KC;
+    const long segc = left >= SEG ? SEGC : left > 0 ? (left + KC - 1) / KC : 0;
     long n = w < segc ? (segc - 1 - w) / NWAVES + 1 : 0;
-    if (seg0 == 0 && n == 0) n = 1;
+    // (past the end of a part: entries of the next part, or padding; a part that starts there multiplies nothing)
+    if (!SPLIT && seg0 == 0 && n == 0) n = 1;
     const bool more = left > SEG;
     if (more) request_segment(seg0 + SEG);  // uniform
     __builtin_amdgcn_sched_barrier(0);
@@ -212,7 +223,8 @@ void k_forward_rows(ForwardRowsArgs<T> ar) {
 #pragma unroll
   for (int r = 0; r < RB; r++) {
     if (r > 0) __syncthreads();  // the previous row block's sums have been read
-    forward_finish<T, NG, true, NWAVES, LW, false, NT>(acc[r], bv, red, a.act, a.B, a.M, b0 + 16 * r, j0, ncol);
+    forward_finish<T, NG, !SPLIT, NWAVES, LW, false, NT>(
+        acc[r], bv, red, SPLIT ? a.part + (long)blockIdx.y * a.B * a.M : a.act, a.B, a.M, b0 + 16 * r, j0, ncol);
   }
 }
 

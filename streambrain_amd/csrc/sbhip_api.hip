@@ -54,9 +54,6 @@ struct Context {
   // scratch of the per-kernel training entry points: the "next" Ci / Cj of the fused kernel
   void *trace_next = nullptr;
   long trace_cap = 0;  // elements of 8 bytes
-  // scratch of the per-kernel training entry points: the split batch (train_split_bytes)
-  void *split = nullptr;
-  size_t split_cap = 0;
   // device address of `scratch` on this context's device
   void *noalloc_scratch = nullptr;
 };
@@ -298,20 +295,33 @@ static int ensure_trace_scratch(long elems) {
   return 0;
 }
 
-// The context's scratch for a split batch of `bytes`, or nullptr when none is asked for or the memory is not there (the
-// training pass then does without).
-static void *split_scratch(size_t bytes) {
-  if (bytes > g_ctx.split_cap) {
-    (void)hipStreamSynchronize(g_ctx.stream);
-    if (g_ctx.split) (void)hipFree(g_ctx.split);
-    g_ctx.split = nullptr;
-    g_ctx.split_cap = 0;
-    if (dev_malloc(&g_ctx.split, bytes) == hipSuccess) g_ctx.split_cap = bytes;
-    else g_ctx.split = nullptr;
+// Scratch that a launch can do without: `bytes` of it in `b`, or nullptr when none is asked for, the memory is not there,
+// or the library's stream is being captured -- a graph would go on using a buffer that a later, larger call replaces.
+struct Reusable {
+  void *p = nullptr;
+  size_t cap = 0;
+};
+static void *optional_scratch(Reusable &b, size_t bytes) {
+  if (bytes == 0) return nullptr;
+  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(g_ctx.stream, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone) return nullptr;
+  if (bytes <= b.cap) return b.p;
+  (void)hipStreamSynchronize(g_ctx.stream);
+  if (b.p) (void)hipFree(b.p);
+  b = Reusable();
+  if (dev_malloc(&b.p, bytes) != hipSuccess) {
     (void)hipGetLastError();
+    b.p = nullptr;
+    return nullptr;
   }
-  return bytes ? g_ctx.split : nullptr;
+  b.cap = bytes;
+  return b.p;
 }
+// ... of the per-kernel entry points.  Whoever launches kernels that meet in it (or in the context's trace scratch) holds
+// the lock until all of them are in the stream, so that calls from several threads do not interleave.
+static Reusable g_work;
+static std::mutex g_work_mutex;
+static ForwardScratch forward_scratch(Reusable &b, size_t bytes) { return ForwardScratch{optional_scratch(b, bytes), bytes}; }
 
 // Per-kernel entry points keep the reference's in-place contract: the fused kernel writes the new
 // Ci / Cj into scratch, which is then copied over the caller's arrays.
@@ -324,12 +334,13 @@ static int train_in_place(const T *x, const T *y, T *Cij, T *W, T *Ci, T *Cj, co
   hipStream_t st = g_ctx.stream;
   const long M = H * Mc;
   SB_REQUIRE(N > 0 && M > 0, "sizes must be positive");
+  std::lock_guard<std::mutex> lock(g_work_mutex);
   int rc = fixed_scratch ? 0 : ensure_trace_scratch(N + M);
   if (rc) return rc;
   T *ci_next = fixed_scratch ? fixed_scratch : (T *)g_ctx.trace_next, *cj_next = ci_next + N;
   rc = launch_train_fused<T>(st, x, y, Cij, W, Ci, Cj, ci_next, cj_next, wmask, bias_mode, bias, kbi, B,
                              N, H, Mc, taupdt, cthr, khalf, pmin, taubdt, false, nullptr, 0,
-                             fixed_scratch ? nullptr : split_scratch(train_split_bytes<T>(B, N, H, Mc)));
+                             fixed_scratch ? nullptr : optional_scratch(g_work, train_split_bytes<T>(B, N, H, Mc)));
   if (rc) return rc;
   return launch_copy_pair<T>(st, Ci, ci_next, (size_t)N, Cj, cj_next, (size_t)M);
 }
@@ -380,11 +391,8 @@ struct sb_net {
   // evaluate / predict / forward: the device buffers of one chunk of the set (images, the same in blocks of 16
   // rows, labels, predictions), kept from call to call (an allocation and a release per buffer and call took a
   // fifth of an evaluate of 10000 images) and released with the network
-  struct Reusable {
-    void *p = nullptr;
-    size_t cap = 0;
-  } ev_x, ev_xb, ev_y, ev_p;
-  Reusable split;  // a training batch split into bfloat16 (train_split_bytes)
+  sb::Reusable ev_x, ev_xb, ev_y, ev_p;
+  sb::Reusable work;  // optional scratch of the launches (optional_scratch)
 };
 
 namespace sb {
@@ -409,7 +417,7 @@ static int free_dev(void *&p) {
 }
 
 // b holds at least `bytes` afterwards (contents undefined); nothing in flight may still use the old buffer
-static int reuse_dev(sb_net::Reusable &b, size_t bytes) {
+static int reuse_dev(Reusable &b, size_t bytes) {
   if (bytes <= b.cap) return 0;
   SB_HIP(hipStreamSynchronize(g_ctx.stream));
   int rc = free_dev(b.p);
@@ -498,9 +506,10 @@ static int layer_forward(sb_net *net, Layer &L, const T *x, long B, const T *x_b
   }
   if (L.rows && L.w_masked)
     return launch_forward_rows<T>(g_ctx.stream, (T *)L.act, x, (const T *)L.W, (const T *)L.bias, L.rows,
-                                  L.row_cnt, L.rows_cap, B, L.N, L.H, L.Mc, x_blocked);
+                                  L.row_cnt, L.rows_cap, B, L.N, L.H, L.Mc, x_blocked,
+                                  forward_scratch(net->work, forward_rows_part_bytes<T>(L.rows_cap, B, L.H, L.Mc)));
   return launch_forward<T>(g_ctx.stream, (T *)L.act, x, (const T *)L.W, (const T *)L.bias, B, L.N, L.H,
-                           L.Mc, true);
+                           L.Mc, true, forward_scratch(net->work, forward_part_bytes<T>(B, L.N, L.H, L.Mc, true)));
 }
 
 // One training step of `L` on input x (and on y = its own activation or the labels), in the order of
@@ -514,16 +523,11 @@ static int layer_train_step(sb_net *net, Layer &L, const T *x, const T *y, long 
   const T tau = (T)L.taupdt;
   const T cthr = (T)(L.taupdt / 2);
   int rc = 0;
-  const size_t split_bytes = train_split_bytes<T>(B, L.N, L.H, L.Mc);
-  if (reuse_dev(net->split, split_bytes)) {  // no memory for it: the training pass does without
-    (void)hipGetLastError();
-    net->split.p = nullptr;
-  }
   rc = launch_train_fused<T>(st, x, y, (T *)L.Cij, (T *)L.W, (const T *)L.Ci, (const T *)L.Cj,
                              (T *)L.Ci_alt, (T *)L.Cj_alt, L.plastic ? L.wmask : nullptr,
                              L.plastic ? 1 : 0, (T *)L.bias, (T *)L.kbi, B, L.N, L.H, L.Mc, tau, cthr,
                              (T)L.khalf, (T)L.pmin, (T)L.taubdt, L.w_masked, next, next_bytes,
-                             split_bytes ? net->split.p : nullptr);
+                             optional_scratch(net->work, train_split_bytes<T>(B, L.N, L.H, L.Mc)));
   if (rc) return rc;
   std::swap(L.Ci, L.Ci_alt);
   std::swap(L.Cj, L.Cj_alt);
@@ -805,7 +809,8 @@ static int net_forward_batches(sb_net *net, const void *h_images, const void *h_
           // output layer: activation and classification (first maximal unit, comparison with the labels)
           rc = launch_forward_classify<T>(st, (T *)L.act, x, (const T *)L.W, (const T *)L.bias, B, L.N, L.H,
                                           L.Mc, true, h_labels ? (const T *)dY + lo * NC : nullptr,
-                                          dP ? dP + lo : nullptr, net->d_correct);
+                                          dP ? dP + lo : nullptr, net->d_correct,
+                                          forward_scratch(net->work, forward_part_bytes<T>(B, L.N, L.H, L.Mc, true)));
         else
           rc = layer_forward<T>(net, L, x, B, l == 0 ? xb : nullptr);
         x = (const T *)L.act;
@@ -978,7 +983,8 @@ int sb_shutdown(void) {
   if (g_ctx.mask_nom) SB_HIP(hipFree(g_ctx.mask_nom));
   if (g_ctx.mask_csum) SB_HIP(hipFree(g_ctx.mask_csum));
   if (g_ctx.trace_next) SB_HIP(hipFree(g_ctx.trace_next));
-  if (g_ctx.split) SB_HIP(hipFree(g_ctx.split));
+  if (g_work.p) SB_HIP(hipFree(g_work.p));
+  g_work = Reusable();
   stager_release();
   SB_HIP(hipStreamDestroy(g_ctx.stream));
   g_ctx = Context();
@@ -1044,7 +1050,9 @@ int sb_fill_bytes(void *d_dst, int value, size_t bytes) {
 #define SB_DEFINE_KERNEL_API(SFX, T)                                                                   \
   int sb_update_state_##SFX(T *act, const T *x, const T *W, const T *bias, long B, long N, long M) {   \
     SB_READY();                                                                                        \
-    return launch_forward<T>(g_ctx.stream, act, x, W, bias, B, N, 1, M, false);                        \
+    std::lock_guard<std::mutex> lock(g_work_mutex);                                                    \
+    return launch_forward<T>(g_ctx.stream, act, x, W, bias, B, N, 1, M, false,                         \
+                             forward_scratch(g_work, forward_part_bytes<T>(B, N, 1, M, false)));       \
   }                                                                                                    \
   int sb_softmax_minicolumns_##SFX(T *act, long B, long H, long Mc) {                                  \
     SB_READY();                                                                                        \
@@ -1054,14 +1062,18 @@ int sb_fill_bytes(void *d_dst, int value, size_t bytes) {
                                   long H, long Mc) {                                                   \
     SB_READY();                                                                                        \
     SB_REQUIRE(B > 0 && N > 0 && H > 0 && Mc > 0, "sizes must be positive");                           \
-    return launch_forward<T>(g_ctx.stream, act, x, W, bias, B, N, H, Mc, true);                        \
+    std::lock_guard<std::mutex> lock(g_work_mutex);                                                    \
+    return launch_forward<T>(g_ctx.stream, act, x, W, bias, B, N, H, Mc, true,                         \
+                             forward_scratch(g_work, forward_part_bytes<T>(B, N, H, Mc, true)));       \
   }                                                                                                    \
   int sb_compute_activation_rows_##SFX(T *act, const T *x, const T *W, const T *bias, const int *rows, \
                                        const int *row_cnt, long cap, long B, long N, long H, long Mc,  \
                                        const T *x_blocked) {                                           \
     SB_READY();                                                                                        \
+    std::lock_guard<std::mutex> lock(g_work_mutex);                                                    \
     return launch_forward_rows<T>(g_ctx.stream, act, x, W, bias, rows, row_cnt, cap, B, N, H, Mc,      \
-                                  x_blocked);                                                          \
+                                  x_blocked,                                                           \
+                                  forward_scratch(g_work, forward_rows_part_bytes<T>(cap, B, H, Mc))); \
   }                                                                                                    \
   int sb_rows_in_blocks_##SFX(T *dst, const T *src, long rows, long cols) {                            \
     SB_READY();                                                                                        \
@@ -1213,7 +1225,7 @@ int sb_net_destroy(sb_net *net) {
   int rc = sb_net_training_done(net);
   for (auto &L : net->layers) rc |= layer_free(L);
   rc |= free_dev(net->ev_x.p); rc |= free_dev(net->ev_xb.p); rc |= free_dev(net->ev_y.p); rc |= free_dev(net->ev_p.p);
-  rc |= free_dev(net->split.p);
+  rc |= free_dev(net->work.p);
   if (net->d_correct) SB_HIP(hipFree(net->d_correct));
   if (net->d_unmasked) SB_HIP(hipFree(net->d_unmasked));
   if (net->perm_copied) SB_HIP(hipEventDestroy(net->perm_copied));
