@@ -468,6 +468,17 @@ static int layer_free(Layer &L) {
   return rc;
 }
 
+// Batch rows that one pass over the layers takes when nothing ties it to the caller's batch size (a sample's activations
+// do not depend on the others'): launches then have work for the whole chip and are few.  As many as keep the
+// widest activations within 64 MiB, a multiple of `unit`, at least one unit.
+constexpr size_t kPassBytes = (size_t)64 << 20;
+static long pass_rows(const sb_net *net, long unit) {
+  long widest = 1;
+  for (const auto &L : net->layers) widest = std::max(widest, L.M);
+  const long rows = (long)(kPassBytes / ((size_t)widest * net->esize)) / unit * unit;
+  return rows < unit ? unit : rows;
+}
+
 static int ensure_act(sb_net *net, long rows) {
   for (auto &L : net->layers) {
     if (L.act_rows >= rows) continue;
@@ -497,18 +508,19 @@ static int layer_check_masked(sb_net *net, Layer &L) {
   return 0;
 }
 
-// x_blocked: the same batch in blocks of 16 rows, or nullptr
+// x_blocked: the same batch in blocks of 16 rows, or nullptr; out: where the activations go (nullptr: L.act)
 template <typename T>
-static int layer_forward(sb_net *net, Layer &L, const T *x, long B, const T *x_blocked = nullptr) {
+static int layer_forward(sb_net *net, Layer &L, const T *x, long B, const T *x_blocked = nullptr, T *out = nullptr) {
+  T *const act = out ? out : (T *)L.act;
   if (L.w_unchecked) {
     int rc = layer_check_masked<T>(net, L);
     if (rc) return rc;
   }
   if (L.rows && L.w_masked)
-    return launch_forward_rows<T>(g_ctx.stream, (T *)L.act, x, (const T *)L.W, (const T *)L.bias, L.rows,
+    return launch_forward_rows<T>(g_ctx.stream, act, x, (const T *)L.W, (const T *)L.bias, L.rows,
                                   L.row_cnt, L.rows_cap, B, L.N, L.H, L.Mc, x_blocked,
                                   forward_scratch(net->work, forward_rows_part_bytes<T>(L.rows_cap, B, L.H, L.Mc)));
-  return launch_forward<T>(g_ctx.stream, (T *)L.act, x, (const T *)L.W, (const T *)L.bias, B, L.N, L.H,
+  return launch_forward<T>(g_ctx.stream, act, x, (const T *)L.W, (const T *)L.bias, B, L.N, L.H,
                            L.Mc, true, forward_scratch(net->work, forward_part_bytes<T>(B, L.N, L.H, L.Mc, true)));
 }
 
@@ -596,8 +608,8 @@ static int drop_frozen_cache(sb_net *net) {
   return rc;
 }
 
-// Activations of layer `upto` for all training samples in data-set order, in batches of maxB (the batch
-// size the training steps use, so the same kernel variants run).
+// Activations of layer `upto` for all training samples in data-set order, as many samples per pass as pass_rows says
+// (157 batches of 128 through 784 -> 15x200: 1.25 ms of launches of 8 us and a copy each, in passes of 5504 0.45 ms).
 template <typename T>
 static int build_frozen_cache(sb_net *net, int upto, long maxB) {
   const long Ns = net->Ns, Mo = net->layers[upto].M;
@@ -612,15 +624,16 @@ static int build_frozen_cache(sb_net *net, int upto, long maxB) {
     net->Hc = nullptr;
     return 0;
   }
-  for (long lo = 0; lo < Ns; lo += maxB) {
-    const long B = lo + maxB <= Ns ? maxB : Ns - lo;
+  const long pass = std::min(Ns, pass_rows(net, maxB));
+  if (upto > 0 && (rc = ensure_act(net, pass))) return rc;
+  for (long lo = 0; lo < Ns; lo += pass) {
+    const long B = lo + pass <= Ns ? pass : Ns - lo;
     const T *x = (const T *)net->X + lo * net->NF;
     for (int l = 0; l <= upto; l++) {
-      if ((rc = layer_forward<T>(net, net->layers[l], x, B))) return rc;
+      T *const out = l == upto ? (T *)net->Hc + lo * Mo : (T *)nullptr;
+      if ((rc = layer_forward<T>(net, net->layers[l], x, B, (const T *)nullptr, out))) return rc;
       x = (const T *)net->layers[l].act;
     }
-    SB_HIP(hipMemcpyAsync((T *)net->Hc + lo * Mo, x, (size_t)B * Mo * sizeof(T), hipMemcpyDeviceToDevice,
-                          g_ctx.stream));
   }
   net->Hc_layer = upto;
   return 0;
@@ -754,8 +767,7 @@ static int net_forward_batches(sb_net *net, const void *h_images, const void *h_
   Layer &out = net->layers[last_layer];
   SB_REQUIRE(!h_labels || NC == out.M, "label width does not match the last layer");
   if (n == 0) return 0;
-  int rc = ensure_act(net, maxB < n ? maxB : n);
-  if (rc) return rc;
+  int rc = 0;
   // stream the set through HBM in chunks of whole batches (<= ~256 MiB of images at a time)
   long chunk = (256L << 20) / (long)(NF * sizeof(T));
   chunk = chunk / maxB * maxB;
@@ -773,33 +785,30 @@ static int net_forward_batches(sb_net *net, const void *h_images, const void *h_
     unsigned long long zero = 0;
     SB_HIP(hipMemcpy(net->d_correct, &zero, sizeof(zero), hipMemcpyHostToDevice));
   }
-  // Inside a chunk the images go up in pieces of whole batches (about 16 MiB) on a copy stream of their own,
-  // through the pinned staging ring; the library's stream waits for a piece's event and works on its batches
-  // while the next piece is on its way.
+  // Inside a chunk the images go up in pieces of whole batches (about 8 MiB, or what a pass over the layers takes) on a
+  // copy stream of their own, through the pinned staging ring; the library's stream waits for a piece's event and takes
+  // the piece through the layers in one pass while the next piece is on its way.
   if ((rc = stager_init())) return rc;
   hipStream_t up = g_stager.copy_stream;
   long piece = ((long)HostStager::kChunkBytes / (long)(NF * sizeof(T))) / maxB * maxB;
   if (piece < maxB) piece = maxB;
+  piece = std::min(piece, pass_rows(net, maxB));
+  if ((rc = ensure_act(net, std::min(piece, n)))) return rc;
   for (long c0 = 0; c0 < n && !rc; c0 += chunk) {
     const long rows = (c0 + chunk <= n) ? chunk : n - c0;
     if (h_labels) {
       if ((rc = staged_upload(dY, (const T *)h_labels + c0 * NC, (size_t)rows * NC * sizeof(T), up))) break;
     }
-    for (long lo = 0; lo < rows && !rc; lo += maxB) {
-      if (lo % piece == 0) {  // the piece that starts here
-        const long prows = lo + piece <= rows ? piece : rows - lo;
-        if ((rc = staged_upload((T *)dX + lo * NF, (const T *)h_images + (c0 + lo) * NF,
-                                (size_t)prows * NF * sizeof(T), up)))
-          break;
-        SB_HIP(hipEventRecord(g_stager.uploaded, up));
-        SB_HIP(hipStreamWaitEvent(st, g_stager.uploaded, 0));
-        // (pieces start on multiples of the batch size, which is a multiple of 16 where blocks are used)
-        if (blocked)
-          rc = launch_gather_rows_blocked<T>(st, (T *)dXB + lo * NF, (T *)nullptr, (const T *)dX + lo * NF, nullptr,
-                                             prows, NF);
-        if (rc) break;
-      }
-      const long B = (lo + maxB <= rows) ? maxB : rows - lo;
+    for (long lo = 0; lo < rows && !rc; lo += piece) {
+      const long B = lo + piece <= rows ? piece : rows - lo;
+      if ((rc = staged_upload((T *)dX + lo * NF, (const T *)h_images + (c0 + lo) * NF, (size_t)B * NF * sizeof(T), up)))
+        break;
+      SB_HIP(hipEventRecord(g_stager.uploaded, up));
+      SB_HIP(hipStreamWaitEvent(st, g_stager.uploaded, 0));
+      // (pieces start on multiples of the batch size, which is a multiple of 16 where blocks are used)
+      if (blocked)
+        rc = launch_gather_rows_blocked<T>(st, (T *)dXB + lo * NF, (T *)nullptr, (const T *)dX + lo * NF, nullptr, B, NF);
+      if (rc) break;
       const T *x = (const T *)dX + lo * NF;
       const T *xb = blocked ? (const T *)dXB + lo * NF : nullptr;
       const bool classify = h_labels || h_pred;
