@@ -214,11 +214,11 @@ bool forward_rows_supported(const T *W, long N, long H, long Mc) {
 }
 
 // The split of long lists where the hypercolumns and blocks of 16 batch rows are few (see split_chunks_of): chunks
-// of 4 VW entries; parts of at least 512 entries.
+// of 4 VW entries; parts of at least 1024 entries (below, the second launch takes most of the gain).
 template <typename T>
 static long forward_rows_split_chunks(long cap, long B, long H) {
   const long kc = 4 * Real<T>::VW;
-  return split_chunks_of(H * cdiv(B, 16), cdiv(cap, kc), device_cu_count(), 512 / kc);
+  return split_chunks_of(H * cdiv(B, 16), cdiv(cap, kc), device_cu_count(), 1024 / kc);
 }
 template <typename T>
 size_t forward_rows_part_bytes(long cap, long B, long H, long Mc) {
@@ -334,17 +334,19 @@ int launch_softmax(hipStream_t st, T *act, long B, long H, long Mc) {
 template <typename T>
 static long train_tiles_of_one_round() { return (long)train_waves_per_simd<T, true, 1>() * device_cu_count(); }
 
-// Floats go through k_trace_sums<float, true> and k_train_split from one round of 64 x 64 tiles on, with small batches,
-// which leave the matrix cores little to do, from five.  Sums included, against k_train_fused on its own, 3000
-// columns: batch 128, 1568 rows (0.9 rounds) 24.3 / 18.8 us, 2048 rows 26.0 / 26.7, 4096 39.7 / 47.8, 16384 110 / 257; batch
-// 512, 2048 rows 53.6 / 75.0; batch 32, 2048 rows 19.2 / 16.1, 8192 (4.7 rounds) 54.6 / 53.5, 27648 255 / 369.
+// Floats go through k_trace_sums<float, true> and k_train_split from two and a half rounds of 64 x 64 tiles on, with
+// small batches, which leave the matrix cores little to do, from five.  Sums included, against k_train_fused on its
+// own, 3000 columns: batch 128, 2048 rows (1.2 rounds) 26.0 / 26.7 us, 4096 (2.4) 39.7 / 47.8, 8192 (4.7) 66 / 94, 16384
+// 110 / 257; batch 512, 8192 rows 141 / 239; batch 32, 8192 rows 54.6 / 53.5, 27648 255 / 369.  Between one round and the
+// line there are 15 % to gain, and the small layers below it, which train for epochs in moments, keep the rounding of
+// their trajectories (after a few dozen steps those tell one order of sums from another).
 // Its windows hold 128 rows of Cij and 32 split batch rows.
 template <typename T>
 size_t train_split_bytes(long B, long N, long H, long Mc) {
   if constexpr (sizeof(T) != 4) return 0;
   if (B <= 0 || N <= 0 || H <= 0 || Mc <= 0) return 0;
   const long M = H * Mc;
-  if (M <= 32 || cdiv(N, 64) * cdiv(M, 64) <= (B > 32 ? 1 : 5) * train_tiles_of_one_round<T>()) return 0;
+  if (M <= 32 || 2 * cdiv(N, 64) * cdiv(M, 64) < (B > 32 ? 5 : 10) * train_tiles_of_one_round<T>()) return 0;
   const long xw = cdiv(N, kSplitTileI) * kSplitTileI, yw = cdiv(M, kSplitTileJ) * kSplitTileJ;
   const long wider = xw > yw ? xw : yw;
   if (128 * M * 4 >= (1L << 31) || wider * (kSplitRows / 8) * 3 * 16 >= (1L << 31)) return 0;

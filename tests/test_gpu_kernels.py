@@ -479,13 +479,13 @@ def test_plastic_train_step(k, oracle, dtype, B, N, H, Mc, h):
     _check_plastic_train_step(k, oracle, dtype, B, N, H, Mc, h, np.random.default_rng(B + N + H + Mc))
 
 
-# 64 x 64 tiles of these layers: more than 1280 with more than 32 rows, more than 6400 below, which is where the pass
+# 64 x 64 tiles of these layers: 3200 and more with more than 32 rows, 6400 and more below, which is where the pass
 # goes over to bfloat16 pieces
 @pytest.mark.parametrize("B,N,H,Mc,masked", [
     (1, 8200, 33, 100, True), (31, 8193, 50, 66, False), (32, 8257, 33, 101, True),
-    *[(B, *s) for B in (33, 63, 64, 65, 128, 257) for s in ((2689, 30, 100, True), (4096, 21, 64, True),
-                                                           (4097, 46, 66, True), (4159, 3, 676, False),
-                                                           (3001, 29, 101, True), (8001, 331, 4, True))]])
+    *[(B, *s) for B in (33, 64, 65, 257) for s in ((4353, 30, 100, True), (6464, 32, 64, False), (4160, 48, 66, True),
+                                                   (4737, 29, 101, True), (9985, 331, 4, True))],
+    (63, 4353, 30, 100, True), (128, 4737, 29, 101, False)])
 def test_train_pass_of_big_float_layers(k, B, N, H, Mc, masked):
     """Tile remainders on either side, batch remainders, values over 40 binary orders of magnitude, and values out of
     the range of the bfloat16 pieces (1e30, infinity), which only the tiles that hold them treat differently."""
