@@ -272,13 +272,15 @@ constexpr int train_waves_per_simd() { return sizeof(T) == 8 ? 4 : (VEC && MB ==
 // inside one hypercolumn), VW otherwise.
 // PRE: Ci_next and Cj_next already hold the new traces (k_trace_sums): no column sums here.
 // LATE1: the second chunk of the batch is requested only once the first has been staged (see the kernel).
-template <typename T, int KCH, bool VEC, int MB, bool PRE = false, bool LATE1 = false>
+// NT: non-temporal stores, for matrices that do not stay in the memory-side cache (see k_train_split).
+template <typename T, int KCH, bool VEC, int MB, bool PRE = false, bool LATE1 = false, bool NT = false>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(train_waves_per_simd<T, VEC, MB>())))
 void k_train_fused(TrainArgs<T> a) {
   using R = Real<T>;
   using acc_t = typename R::acc_t;
   using vec_t = typename R::vec_t;
   constexpr int VW = R::VW;             // elements per 16-byte vector
+  constexpr int AUX = NT ? 2 : BufferWindow<T>::kStoreAux;
   constexpr int TS = 64;                // tile side
   constexpr int G = TS / VW;            // 16-byte groups per slab row
   constexpr int RPP = 256 / G;          // slab rows the workgroup stages per pass
@@ -645,8 +647,8 @@ void k_train_fused(TrainArgs<T> a) {
         cn[v][g][e] = cpre[v][g][e] * a.omt + acc[g * VW + e][v] * scale;
         cv[e] = fmax(cn[v][g][e], T(0));  // 0 as well when cn is NaN, like the reference's `cn > 0 ? cn : 0`
       }
-      if (VEC) cwin.store_vec(cv, tat[g], v * vstep);
-      else cwin.template store<false>(cv, tat[g], v * vstep, ecol[g], a.M);
+      if (VEC) cwin.template store_vec<AUX>(cv, tat[g], v * vstep);
+      else cwin.template store<false, AUX>(cv, tat[g], v * vstep, ecol[g], a.M);
     }
   if (a.W == nullptr) return;  // (uniform) traces only
 
@@ -678,7 +680,7 @@ void k_train_fused(TrainArgs<T> a) {
 #pragma unroll
           for (int e = 0; e < VW; e++) wv[e] = connected ? wv[e] : T(0);
         }
-        wwin.store_vec(wv, (a.w_masked && !connected) ? kOutside : tat[g], v * vstep);
+        wwin.template store_vec<AUX>(wv, (a.w_masked && !connected) ? kOutside : tat[g], v * vstep);
       }
     return;
   }
@@ -701,7 +703,7 @@ void k_train_fused(TrainArgs<T> a) {
         const bool keep = row_live && !(rcj[g][e] < T(0)) && (MB == 1 || !masked || mb[v][g][e] != 0);
         wv[e] = keep ? wgt : T(0);
       }
-      wwin.template store<VEC>(wv, tat[g], v * vstep, ecol[g], a.M);
+      wwin.template store<VEC, AUX>(wv, tat[g], v * vstep, ecol[g], a.M);
     }
 }
 

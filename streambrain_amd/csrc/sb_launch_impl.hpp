@@ -470,6 +470,21 @@ int launch_train_fused(hipStream_t st, const T *x, const T *y, T *Cij, T *W, con
   const long ntiles = a.tiles_i * a.tiles_j;
   const bool one_round = ntiles <= train_tiles_of_one_round<T>();
   const long pre_from = sizeof(T) == 8 ? 5 * 4 : 3 * 5;  // in half workgroups per CU
+  if constexpr (sizeof(T) == 8) {
+    // Cij and W together beyond what the 256 MB memory-side cache keeps: non-temporal stores (batch 128, rows of 3000
+    // doubles, whole steps: 8000 rows, 384 MB, 366 us written through, 218 us non-temporal; 20000 rows 1364 / 626;
+    // rows of whole cache lines, 1568 x 10000, 414 / 411; odd rows, 5000 x 9999, batch 77, 806 / 643)
+    if (2 * N * M * (long)sizeof(T) > (192L << 20) && (!vec || one_byte)) {
+      if (vec) {
+        launch(k_trace_sums<T>, sums, true, false, SplitBatch{});
+        launch(k_train_fused<T, KCH, true, 1, true, false, true>, grid, false, true);
+      } else {
+        launch(k_train_fused<T, KCH, false, VW, false, false, true>, grid, true, true);
+      }
+      SB_LAUNCH_CHECK();
+      return 0;
+    }
+  }
   if (vec && one_byte && 2 * ntiles >= pre_from * device_cu_count() && (sizeof(T) == 8 || B > 32)) {
     launch(k_trace_sums<T>, sums, true, false, SplitBatch{});
     launch(k_train_fused<T, KCH, true, 1, true>, grid, false, true);
