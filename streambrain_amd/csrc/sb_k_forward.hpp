@@ -29,10 +29,6 @@ struct ForwardArgs {
   long B, N, M, Mc;
   long col_tiles, batch_tiles;
   FastDiv by_batch_tiles;  // division by batch_tiles (set by the launcher along with it)
-  // Split reductions (part != nullptr, grid y = splits): workgroup y multiplies the reduction's chunks y * split_chunks
-  // .. + split_chunks - 1 only and leaves its sums, without bias, in part[y][B][M]; k_forward_reduce does the rest.
-  T *part;
-  long split_chunks;
 };
 
 // Column layout of a tile, shared by the kernels below: NG groups of 16 lanes-columns, group g holding
@@ -346,28 +342,18 @@ void k_forward(ForwardArgs<T> a) {
   // the epilogue's bias values are requested before the K loop, so their latency is not added to it
   const long ncol = jend - j0;
   T bv[ForwardBias<T, NG, NWAVES>::PT];
-  const bool split = !FUSE && a.part != nullptr;  // (uniform)
-  if (split) {
-#pragma unroll
-    for (int t = 0; t < ForwardBias<T, NG, NWAVES>::PT; t++) bv[t] = T(0);
-  } else {
-    ForwardBias<T, NG, NWAVES>::load(bv, a.bias, j0, ncol);
-  }
-  // chunks first .. nfull - 1, with all KC reduction indices inside the matrix, and perhaps a partial one behind them
-  const long first = split ? (long)blockIdx.y * a.split_chunks : 0;
-  const bool to_end = !split || blockIdx.y + 1 == gridDim.y;
-  const long nfull = to_end ? a.N / KC : first + a.split_chunks;
+  ForwardBias<T, NG, NWAVES>::load(bv, a.bias, j0, ncol);
+  const long nfull = a.N / KC;  // chunks with all KC reduction indices inside the matrix
   {
-    // Chunk `first + w` first; every later chunk of this wavefront is NWAVES chunks further on.  x and W are
+    // Chunk `w` first; every later chunk of this wavefront is NWAVES chunks further on.  x and W are
     // reached through bounds-checked buffer windows that start at the chunk (a scalar base address,
     // advanced with scalar instructions), so the per-lane offsets never change and the loop body is
     // loads and MFMAs only.  Batch rows past the end and columns past the tile read zero.
     constexpr unsigned ES = sizeof(T);
-    const long k0 = (first + w) * KC;
-    const T *xbase = a.x + b0 * a.N + k0;      // uniform
-    const T *wbase = a.W + k0 * a.M + j0;      // uniform
-    long xleft = (a.B - b0) * a.N - k0;        // elements from xbase to the end of x
-    long wleft = (a.N - k0) * a.M - j0;        // ... of W
+    const T *xbase = a.x + b0 * a.N + (long)w * KC;             // uniform
+    const T *wbase = a.W + (long)w * KC * a.M + j0;             // uniform
+    long xleft = (a.B - b0) * a.N - (long)w * KC;               // elements from xbase to the end of x
+    long wleft = (a.N - (long)w * KC) * a.M - j0;               // ... of W
     unsigned xat[RB];
 #pragma unroll
     for (int r = 0; r < RB; r++) xat[r] = (unsigned)(((long)(16 * r + p) * a.N + VW * q) * ES);
@@ -383,10 +369,10 @@ void k_forward(ForwardArgs<T> a) {
     for (int s = 0; s < VW; s++) tat[s] = (unsigned)(((long)(VW * q + s) * a.M + tail_col0 + (p & 3)) * ES);
     const long xstep = (long)NWAVES * KC;
     const long wstep = (long)NWAVES * KC * a.M;
-    // Chunks first + w, first + w + NWAVES, ... < nfull: n of them for this wavefront.  The loop is branch-free: a load
+    // Chunks w, w + NWAVES, ... < nfull: n of them for this wavefront.  The loop is branch-free: a load
     // past the last chunk reads whatever lies there (or zeros past the arrays) and is never used, so
     // the compiler can keep exact wait counts and D-1 chunks really are in flight.
-    const long n = first + w < nfull ? (nfull - 1 - first - w) / NWAVES + 1 : 0;
+    const long n = w < nfull ? (nfull - 1 - w) / NWAVES + 1 : 0;
     auto load_next = [&](T(&xo)[RB][VW], T(&wo)[VW][NG][VW], T(&to)[VW]) {
       const BufferWindow<T> xwin(xbase, xleft), wwin(wbase, wleft);
 #pragma unroll
@@ -434,7 +420,7 @@ void k_forward(ForwardArgs<T> a) {
         if (i + u < n) compute(xr[u], wr[u], wt[u]);
     }
     // partial last chunk (N % KC != 0): one wavefront takes it through the guarded path
-    if (to_end && nfull * KC < a.N && w == (int)(nfull % NWAVES)) {
+    if (nfull * KC < a.N && w == (int)(nfull % NWAVES)) {
       load_guarded(nfull, xr[0], wr[0], wt[0]);
       compute(xr[0], wr[0], wt[0]);
     }
@@ -442,72 +428,46 @@ void k_forward(ForwardArgs<T> a) {
 #pragma unroll
   for (int r = 0; r < RB; r++) {
     if (r > 0) __syncthreads();  // the previous row block's sums have been read
-    T *const out = split ? a.part + (long)blockIdx.y * a.B * a.M : a.act;
-    forward_finish<T, NG, FUSE, NWAVES, LW, TAIL>(acc[r], bv, red, out, a.B, a.M, b0 + 16 * r, j0, ncol, tacc[r]);
+    forward_finish<T, NG, FUSE, NWAVES, LW, TAIL>(acc[r], bv, red, a.act, a.B, a.M, b0 + 16 * r, j0, ncol, tacc[r]);
   }
 }
 
-// The end of a split reduction: the splits' sums added up in order, the bias, and (softmax) the softmax over the
-// minicolumns of each hypercolumn (kernels_numpy.py:13-25).  One wavefront per (row, hypercolumn); up to 64 PL units
-// stay in registers, the rest goes through act.
-template <typename T>
-__global__ __launch_bounds__(256) void k_forward_reduce(T *act, const T *part, const T *bias, int splits, long B, long M,
-                                                        long H, long Mc, int softmax) {
-  constexpr int PL = 4;
-  const int lane = threadIdx.x & 63;
-  const long g = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (g >= B * H) return;
-  const long b = g / H, j0 = (g - b * H) * Mc, plane = B * M;
-  const T *const src = part + b * M + j0;
-  T *const out = act + b * M + j0;
-  T v[PL];
+// The softmax of forward_finish on stored logits (kernels_numpy.py:13-25), in place, with the same arithmetic in the same
+// order, so that a pass whose hypercolumns are computed by several workgroups gives the bits of one that is
+// fused: TPR threads per (row, hypercolumn), thread lr has units lr + TPR t, at most 16 of them.
+template <typename T, int TPR>
+__global__ __launch_bounds__(256) void k_softmax_as_fused(T *act, long groups, long Mc) {
+  constexpr int PT = 16;
+  static_assert(TPR == 16 || TPR == 32, "rows of 16 lanes");
+  const long g = (long)blockIdx.x * (256 / TPR) + threadIdx.x / TPR;
+  const int lr = threadIdx.x % TPR;
+  T *const v = act + (g < groups ? g : groups - 1) * Mc;  // (lanes past the end take part in the exchanges)
+  T vals[PT], mx = -INFINITY;
 #pragma unroll
-  for (int t = 0; t < PL; t++) v[t] = T(0);
-  T mx = -INFINITY;
-  auto unit = [&](long c) {
-    T s = src[c];
-    for (int k = 1; k < splits; k++) s += src[k * plane + c];
-    return s + bias[j0 + c];
-  };
-#pragma unroll
-  for (int t = 0; t < PL; t++) {
-    const long c = lane + 64 * t;
-    if (c < Mc) {
-      v[t] = unit(c);
-      mx = v[t] > mx ? v[t] : mx;
-    }
+  for (int t = 0; t < PT; t++) {
+    const long col = lr + TPR * t;
+    vals[t] = v[col < Mc ? col : 0];
+    mx = (col < Mc && vals[t] > mx) ? vals[t] : mx;
   }
-  for (long c = lane + 64 * PL; c < Mc; c += 64) {
-    const T s = unit(c);
-    out[c] = s;
-    mx = s > mx ? s : mx;
+  mx = row16_reduce(mx, [](T x, T y) { return y > x ? y : x; });
+  if constexpr (TPR == 32) {
+    const T other = __shfl_xor(mx, 16);
+    mx = other > mx ? other : mx;
   }
-  T sum = T(1);
-  if (softmax) {  // (uniform)
+  T sum = T(0);
 #pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) {
-      const T other = __shfl_xor(mx, o);
-      mx = other > mx ? other : mx;
+  for (int t = 0; t < PT; t++)
+    if (lr + TPR * t < Mc) {
+      vals[t] = Real<T>::exp_nonpos(vals[t] - mx);
+      sum += vals[t];
     }
-    sum = T(0);
+  sum = row16_reduce(sum, [](T x, T y) { return x + y; });
+  if constexpr (TPR == 32) sum += __shfl_xor(sum, 16);
+  const T r = T(1) / sum;
+  if (g >= groups) return;
 #pragma unroll
-    for (int t = 0; t < PL; t++)
-      if (lane + 64 * t < Mc) {
-        v[t] = Real<T>::exp_(v[t] - mx);
-        sum += v[t];
-      }
-    for (long c = lane + 64 * PL; c < Mc; c += 64) {
-      const T e = Real<T>::exp_(out[c] - mx);
-      out[c] = e;
-      sum += e;
-    }
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) sum += __shfl_xor(sum, o);
-    for (long c = lane + 64 * PL; c < Mc; c += 64) out[c] = out[c] / sum;
-  }
-#pragma unroll
-  for (int t = 0; t < PL; t++)
-    if (lane + 64 * t < Mc) out[lane + 64 * t] = softmax ? v[t] / sum : v[t];
+  for (int t = 0; t < PT; t++)
+    if (lr + TPR * t < Mc) v[lr + TPR * t] = sizeof(T) == 4 ? vals[t] * r : vals[t] / sum;
 }
 
 }  // namespace sb

@@ -55,7 +55,8 @@ constexpr int forward_rows_waves_per_simd() {
 // SEG: list entries staged per segment, 2048 or, for lists of at most 256 entries, 256: every thread loads
 // and stores SEG / 256 entries per segment whatever the list's length, and at batch 128 the kernel is a
 // chain of latencies that starts with this staging (1568 -> 30x100, density 0.1, lists of 157: 6.31 -> 6.13 us).
-// SPLIT: a split reduction (see ForwardArgs): a workgroup walks a.split_chunks chunks of its list.
+// SPLIT: a workgroup computes column group blockIdx.y (NG groups wide) of its hypercolumn only and stores the logits;
+// every sum is formed as without (same wavefronts, same chunks), k_softmax_as_fused does the rest.
 template <typename T, int NG, int NWAVES, int RB = 1, bool XT = false, int LW = Real<T>::VW, int SEG = 2048,
           bool SPLIT = false>
 __global__ __launch_bounds__(64 * NWAVES)
@@ -87,8 +88,9 @@ void k_forward_rows(ForwardRowsArgs<T> ar) {
   const int tid = threadIdx.x, lane = tid & 63, p = lane & 15, q = lane >> 4;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const long b0 = bt * (16 * RB);
-  const long j0 = ct * a.Mc;
-  const long ncol = a.Mc;
+  const long jg = SPLIT ? (long)blockIdx.y * (NG * 16 * VW) : 0;  // first column inside the hypercolumn
+  const long j0 = ct * a.Mc + jg;
+  const long ncol = SPLIT && a.Mc - jg > NG * 16 * VW ? NG * 16 * VW : a.Mc - jg;
   const int *list = ar.rows + ct * ar.cap;
 
   // first segment of the list on its way before anything else
@@ -108,11 +110,8 @@ void k_forward_rows(ForwardRowsArgs<T> ar) {
       sidx[tid + t * (64 * NWAVES)] = k < ar.cap ? mine[t] : -1;
     }
   };
-  const long seg_first = SPLIT ? (long)blockIdx.y * a.split_chunks * KC : 0;
-  request_segment(seg_first);
-  // entries up to the end of this workgroup's part
-  const int in_list = ar.row_cnt[ct];
-  const int cnt = SPLIT && seg_first + a.split_chunks * KC < in_list ? (int)(seg_first + a.split_chunks * KC) : in_list;
+  request_segment(0);
+  const int cnt = ar.row_cnt[ct];
 
   acc_t acc[RB][NG][VW];
 #pragma unroll
@@ -123,12 +122,7 @@ void k_forward_rows(ForwardRowsArgs<T> ar) {
       for (int c = 0; c < VW; c++) acc[r][g][c] = acc_t{0, 0, 0, 0};
 
   T bv[ForwardBias<T, NG, NWAVES>::PT];
-  if constexpr (SPLIT) {
-#pragma unroll
-    for (int t = 0; t < ForwardBias<T, NG, NWAVES>::PT; t++) bv[t] = T(0);
-  } else {
-    ForwardBias<T, NG, NWAVES>::load(bv, a.bias, j0, ncol);
-  }
+  ForwardBias<T, NG, NWAVES>::load(bv, a.bias, j0, ncol);
 
   // x through a bounds-checked window over this tile's batch rows: rows past the batch and padding
   // entries (offset kOutside) read zero.  Blocked copy: block b0/16 + r starts N*16 elements after the
@@ -189,17 +183,16 @@ void k_forward_rows(ForwardRowsArgs<T> ar) {
           }
   };
 
-  for (long seg0 = seg_first;;) {
+  for (long seg0 = 0;;) {
     publish_segment(seg0);
     __syncthreads();
     request(w, xr[0], wr[0]);  // this wavefront's first chunk of the segment
     // chunks w, w + NWAVES, ... of the segment that hold list entries: n of them (at least 1 in the
     // first segment, see above)
     const long left = (long)cnt - seg0;  // entries from the start of this segment
-    const long segc = left >= SEG ? SEGC : left > 0 ? (left + KC - 1) / KC : 0;
+    const long segc = left >= SEG ? SEGC : (left + KC - 1) / KC;
     long n = w < segc ? (segc - 1 - w) / NWAVES + 1 : 0;
-    // (past the end of a part: entries of the next part, or padding; a part that starts there multiplies nothing)
-    if (!SPLIT && seg0 == 0 && n == 0) n = 1;
+    if (seg0 == 0 && n == 0) n = 1;
     const bool more = left > SEG;
     if (more) request_segment(seg0 + SEG);  // uniform
     __builtin_amdgcn_sched_barrier(0);
@@ -223,8 +216,7 @@ void k_forward_rows(ForwardRowsArgs<T> ar) {
 #pragma unroll
   for (int r = 0; r < RB; r++) {
     if (r > 0) __syncthreads();  // the previous row block's sums have been read
-    forward_finish<T, NG, !SPLIT, NWAVES, LW, false, NT>(
-        acc[r], bv, red, SPLIT ? a.part + (long)blockIdx.y * a.B * a.M : a.act, a.B, a.M, b0 + 16 * r, j0, ncol);
+    forward_finish<T, NG, !SPLIT, NWAVES, LW, false, NT>(acc[r], bv, red, a.act, a.B, a.M, b0 + 16 * r, j0, ncol);
   }
 }
 

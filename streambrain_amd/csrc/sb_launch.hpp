@@ -68,26 +68,15 @@ int hip_fail(hipError_t e, const char *what, const char *file, int line);
     }                                                 \
   } while (0)
 
-// Scratch of the forward launchers: room for the sums of a split reduction, `bytes` of it at `p` (16-byte aligned).  They
-// make use of up to forward_part_bytes / forward_rows_part_bytes (0: the shape is not split); without it they do
-// without.
-struct ForwardScratch {
-  void *p = nullptr;
-  size_t bytes = 0;
-};
-template <typename T>
-size_t forward_part_bytes(long B, long N, long H, long Mc, bool softmax);
-template <typename T>
-size_t forward_rows_part_bytes(long cap, long B, long H, long Mc);
 template <typename T>
 int launch_forward(hipStream_t st, T *act, const T *x, const T *W, const T *bias, long B, long N,
-                   long H, long Mc, bool softmax, ForwardScratch part = ForwardScratch());
+                   long H, long Mc, bool softmax);
 // The same followed by launch_argmax_rows on the result (pred and / or labels + correct given); layers of
 // at most 32 units do both in one launch.
 template <typename T>
 int launch_forward_classify(hipStream_t st, T *act, const T *x, const T *W, const T *bias, long B, long N,
                             long H, long Mc, bool softmax, const T *labels, int32_t *pred,
-                            unsigned long long *correct, ForwardScratch part = ForwardScratch());
+                            unsigned long long *correct);
 // The same result for a layer whose W is zero wherever wmask is 0, from the per-hypercolumn lists of
 // connected rows that launch_mask_rows builds (rows: [H, cap] ascending indices, the rest -1; cap a
 // multiple of 16; row_cnt: [H]); forward_rows_supported says whether the kernel takes the shape.
@@ -97,8 +86,7 @@ template <typename T>
 bool forward_rows_supported(const T *W, long N, long H, long Mc);
 template <typename T>
 int launch_forward_rows(hipStream_t st, T *act, const T *x, const T *W, const T *bias, const int *rows,
-                        const int *row_cnt, long cap, long B, long N, long H, long Mc, const T *x_blocked,
-                        ForwardScratch part = ForwardScratch());
+                        const int *row_cnt, long cap, long B, long N, long H, long Mc, const T *x_blocked);
 // Lists of hypercolumns h0 .. h0 + count - 1 rebuilt from wmask.
 int launch_mask_rows(hipStream_t st, int *rows, int *row_cnt, const uint8_t *wmask, long N, long H,
                      long cap, long h0, long count);

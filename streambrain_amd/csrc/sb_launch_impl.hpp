@@ -37,71 +37,40 @@ static int forward_variant(hipStream_t st, ForwardArgs<T> a, bool vec) {
   a.by_batch_tiles = FastDiv::of(a.batch_tiles);
   // 8 workgroup ids per round of XCDs; ids beyond the last tile exit at once
   const long ntiles = a.col_tiles * a.batch_tiles;
-  const long tiles8 = 8 * cdiv(ntiles, 8);
-  if (tiles8 >= (1L << 31)) {
+  const long grid = 8 * cdiv(ntiles, 8);
+  if (grid >= (1L << 31)) {
     set_error("launch_forward: too many tiles for one launch");
     return -1;
   }
-  const dim3 grid((unsigned)tiles8, a.part ? (unsigned)cdiv(cdiv(a.N, 4 * Real<T>::VW), a.split_chunks) : 1u);
   if (vec)
-    hipLaunchKernelGGL((k_forward<T, NG, FUSE, true, 8>), grid, dim3(512), 0, st, a);
+    hipLaunchKernelGGL((k_forward<T, NG, FUSE, true, 8>), dim3((unsigned)grid), dim3(512), 0, st, a);
   else
-    hipLaunchKernelGGL((k_forward<T, NG, FUSE, false, 8>), grid, dim3(512), 0, st, a);
+    hipLaunchKernelGGL((k_forward<T, NG, FUSE, false, 8>), dim3((unsigned)grid), dim3(512), 0, st, a);
   SB_LAUNCH_CHECK();
   return 0;
 }
 
-template <typename T>
-static int launch_forward_reduce(hipStream_t st, const ForwardArgs<T> &a, long splits, long H, bool softmax) {
-  SB_REQUIRE(cdiv(a.B * H, 4) < (1L << 31), "too many groups");
-  hipLaunchKernelGGL((k_forward_reduce<T>), dim3((unsigned)cdiv(a.B * H, 4)), dim3(256), 0, st, a.act, a.part, a.bias,
-                     (int)splits, a.B, a.M, H, a.Mc, softmax ? 1 : 0);
+// The softmax behind a pass whose hypercolumns are spread over workgroups (TPR: as of the fused kernel it stands in for).
+template <typename T, int TPR>
+static int launch_softmax_as_fused(hipStream_t st, T *act, long B, long H, long Mc) {
+  SB_REQUIRE(Mc <= 16 * TPR, "hypercolumn too wide");
+  const long groups = B * H, blocks = cdiv(groups, 256 / TPR);
+  SB_REQUIRE(blocks < (1L << 31), "too many groups");
+  hipLaunchKernelGGL((k_softmax_as_fused<T, TPR>), dim3((unsigned)blocks), dim3(256), 0, st, act, groups, Mc);
   SB_LAUNCH_CHECK();
   return 0;
-}
-
-// A split reduction of `chunks` chunks for `tiles` workgroups of which `resident` find a place at once: enough parts
-// for two rounds of workgroups, none below `least` chunks, at most 32.  Returns the chunks per part, or 0 where
-// the tiles fill three fifths of the CUs by themselves or the parts would be too short to pay for the second launch.
-// (27648 -> 15 x 200 over row lists of 15800, batch 128, 120 tiles: 286 us in one piece, 168 + 7 us in eight; 32 batch
-// rows per workgroup instead of 16: 180 + 11 us.)
-static inline long split_chunks_of(long tiles, long chunks, long resident, long least) {
-  if (5 * tiles > 3L * device_cu_count()) return 0;
-  long splits = 2 * resident / tiles;
-  if (splits > 32) splits = 32;
-  if (splits > chunks / least) splits = chunks / least;
-  return splits < 2 ? 0 : cdiv(chunks, splits);
-}
-
-// The dense forward pass: split where its fused tiles (16 batch rows of a hypercolumn), or else the tiles of two column
-// groups, are that few; parts of at least 64 chunks, eight per wavefront.
-template <typename T>
-static long forward_split_chunks(long B, long N, long H, long Mc, bool softmax) {
-  constexpr long VW = Real<T>::VW, GW = 16 * VW;
-  const long M = H * Mc;
-  if (M <= (sizeof(T) == 4 ? 32 : 16)) return 0;
-  const long tiles = cdiv(M, 2 * GW) * cdiv(B, 16);
-  const bool fused = softmax && cdiv(Mc, GW) <= (sizeof(T) == 4 ? 4 : 7);
-  if (fused && 5 * H * cdiv(B, 16) > 3L * device_cu_count()) return 0;
-  return split_chunks_of(tiles, cdiv(N, 4 * VW), device_cu_count(), 8 * 8);
-}
-template <typename T>
-size_t forward_part_bytes(long B, long N, long H, long Mc, bool softmax) {
-  if (B <= 0 || N <= 0 || H <= 0 || Mc <= 0) return 0;
-  const long per = forward_split_chunks<T>(B, N, H, Mc, softmax);
-  return per ? (size_t)cdiv(cdiv(N, 4 * Real<T>::VW), per) * B * H * Mc * sizeof(T) : 0;
 }
 
 template <typename T>
 int launch_forward(hipStream_t st, T *act, const T *x, const T *W, const T *bias, long B, long N,
-                   long H, long Mc, bool softmax, ForwardScratch part) {
-  return launch_forward_classify<T>(st, act, x, W, bias, B, N, H, Mc, softmax, nullptr, nullptr, nullptr, part);
+                   long H, long Mc, bool softmax) {
+  return launch_forward_classify<T>(st, act, x, W, bias, B, N, H, Mc, softmax, nullptr, nullptr, nullptr);
 }
 
 template <typename T>
 int launch_forward_classify(hipStream_t st, T *act, const T *x, const T *W, const T *bias, long B, long N,
                             long H, long Mc, bool softmax, const T *labels, int32_t *pred,
-                            unsigned long long *correct, ForwardScratch part) {
+                            unsigned long long *correct) {
   constexpr int VW = Real<T>::VW;
   constexpr int GW = 16 * VW;
   SB_REQUIRE(act && x && W && bias, "null pointer");
@@ -121,25 +90,14 @@ int launch_forward_classify(hipStream_t st, T *act, const T *x, const T *W, cons
     return 0;
   }
   if (labels || pred) {  // wider layers: the forward pass, then the classification kernel
-    int rc = launch_forward<T>(st, act, x, W, bias, B, N, H, Mc, softmax, part);
+    int rc = launch_forward<T>(st, act, x, W, bias, B, N, H, Mc, softmax);
     if (rc) return rc;
     return launch_argmax_rows<T>(st, act, labels, B, M, pred, correct);
   }
   // per-lane byte offsets inside one chunk of 16 rows of x or W are 32-bit
   SB_REQUIRE(16 * (N > M ? N : M) * (long)sizeof(T) < (1L << 31), "layer too wide for the forward kernel");
-  ForwardArgs<T> a{act, x, W, bias, B, N, M, Mc, 0, cdiv(B, 16), {}, nullptr, 0};
+  ForwardArgs<T> a{act, x, W, bias, B, N, M, Mc, 0, cdiv(B, 16), {}};
   const bool base_vec = (N % VW == 0) && (M % VW == 0) && aligned16(x) && aligned16(W);
-  if (part.p) {
-    const size_t bytes = forward_part_bytes<T>(B, N, H, Mc, softmax);
-    if (bytes > 0 && bytes <= part.bytes) {
-      a.part = (T *)part.p;
-      a.split_chunks = forward_split_chunks<T>(B, N, H, Mc, softmax);
-      a.col_tiles = cdiv(M, 2 * GW);
-      int rc = forward_variant<T, 2, false>(st, a, base_vec);
-      if (rc) return rc;
-      return launch_forward_reduce<T>(st, a, cdiv(cdiv(N, 4 * VW), a.split_chunks), H, softmax);
-    }
-  }
   const long need = cdiv(Mc, GW);
   const long max_fused = sizeof(T) == 4 ? 4 : 7;
   // The fused kernel runs one workgroup per hypercolumn and 16 batch rows, one workgroup per CU.  For wide
@@ -150,6 +108,17 @@ int launch_forward_classify(hipStream_t st, T *act, const T *x, const T *W, cons
   const bool enough_tiles = need <= 2 || 20 * fused_tiles >= 17 * cdiv(fused_tiles, cus_) * cus_;
   if (softmax && need <= max_fused && enough_tiles) {
     const bool vec = base_vec && (Mc % VW == 0);
+    // Hypercolumns of two column groups whose tiles leave half the CUs idle and that have a long reduction: a
+    // workgroup per group, then the softmax.  Every sum as in the fused kernel, except in the four columns that
+    // it takes as 4x4 products, so not those (whole steps:
+    // 10000 -> 20 x 101, batch 32, 179 us fused, 156 us this way; doubles 20000 -> 3 x 100, batch 77, 386 / 254).
+    const bool tail4 = sizeof(T) == 4 && vec && Mc == 100;
+    if (need == 2 && 2 * fused_tiles <= cus_ && N >= 2048 && !tail4) {
+      a.col_tiles = cdiv(M, GW);
+      int rc = forward_variant<T, 1, false>(st, a, base_vec);
+      if (rc) return rc;
+      return launch_softmax_as_fused<T, 32>(st, act, B, H, Mc);
+    }
     a.col_tiles = H;
     // Hypercolumns that need 7 column blocks of 16 (97..112 columns, e.g. 100): the last group runs
     // with 3 (float) or 1 (double) blocks instead of VW, provided none of its vectors straddles the
@@ -197,8 +166,10 @@ int launch_forward_classify(hipStream_t st, T *act, const T *x, const T *W, cons
     if (need <= 4) return forward_variant<T, 4, true>(st, a, vec);
     if constexpr (sizeof(T) == 8) return forward_variant<T, 7, true>(st, a, vec);
   }
-  a.col_tiles = cdiv(M, 2 * GW);
-  int rc = forward_variant<T, 2, false>(st, a, base_vec);
+  // tiles of two column groups, of one where the former leave half the CUs idle
+  const bool narrow = 2 * cdiv(M, 2 * GW) * cdiv(B, 16) <= cus_;
+  a.col_tiles = cdiv(M, narrow ? GW : 2 * GW);
+  int rc = narrow ? forward_variant<T, 1, false>(st, a, base_vec) : forward_variant<T, 2, false>(st, a, base_vec);
   if (rc) return rc;
   if (softmax) return launch_softmax<T>(st, act, B, H, Mc);
   return 0;
@@ -213,33 +184,9 @@ bool forward_rows_supported(const T *W, long N, long H, long Mc) {
          cdiv(Mc, 16 * VW) <= (sizeof(T) == 4 ? 4 : 7) && 16 * N * (long)sizeof(T) < (1L << 31);
 }
 
-// The split of long lists where the hypercolumns and blocks of 16 batch rows are few (see split_chunks_of): chunks
-// of 4 VW entries; parts of at least 1024 entries (below, the second launch takes most of the gain).
-template <typename T>
-static long forward_rows_split_chunks(long cap, long B, long H) {
-  const long kc = 4 * Real<T>::VW;
-  return split_chunks_of(H * cdiv(B, 16), cdiv(cap, kc), device_cu_count(), 1024 / kc);
-}
-template <typename T>
-size_t forward_rows_part_bytes(long cap, long B, long H, long Mc) {
-  if (B <= 0 || cap <= 0 || H <= 0 || Mc <= 0) return 0;
-  const long per = forward_rows_split_chunks<T>(cap, B, H);
-  return per ? (size_t)cdiv(cdiv(cap, 4 * Real<T>::VW), per) * B * H * Mc * sizeof(T) : 0;
-}
-
 template <typename T, int NG, int LW = Real<T>::VW>
 static int forward_rows_variant(hipStream_t st, ForwardRowsArgs<T> a) {
   ProfScope prof_(st, K_FORWARD);
-  if (a.f.part) {
-    constexpr int NW = 4;
-    a.f.by_batch_tiles = FastDiv::of(a.f.batch_tiles);
-    const long splits = cdiv(cdiv(a.cap, 4 * Real<T>::VW), a.f.split_chunks);
-    const dim3 g((unsigned)(8 * cdiv(a.f.col_tiles * a.f.batch_tiles, 8)), (unsigned)splits), blk(64 * NW);
-    if (a.xt) hipLaunchKernelGGL((k_forward_rows<T, NG, NW, 1, true, LW, 2048, true>), g, blk, 0, st, a);
-    else hipLaunchKernelGGL((k_forward_rows<T, NG, NW, 1, false, LW, 2048, true>), g, blk, 0, st, a);
-    SB_LAUNCH_CHECK();
-    return launch_forward_reduce<T>(st, a.f, splits, a.f.col_tiles, true);
-  }
   // four wavefronts measured best (8: 8.8 us, 4: 8.2 us, 2: 9.9 us, 16: 10.7 us at 1568 -> 30x100, density 0.1)
   constexpr int NW = 4;
   // large batches: 64 or 32 rows per workgroup while there are tiles for eight rounds / three quarters
@@ -286,18 +233,25 @@ static int forward_rows_variant(hipStream_t st, ForwardRowsArgs<T> a) {
 
 template <typename T>
 int launch_forward_rows(hipStream_t st, T *act, const T *x, const T *W, const T *bias, const int *rows,
-                        const int *row_cnt, long cap, long B, long N, long H, long Mc, const T *x_blocked,
-                        ForwardScratch part) {
+                        const int *row_cnt, long cap, long B, long N, long H, long Mc, const T *x_blocked) {
   SB_REQUIRE(act && x && W && bias && rows && row_cnt, "null pointer");
   SB_REQUIRE(B > 0 && N > 0 && H > 0 && Mc > 0, "sizes must be positive");
   SB_REQUIRE(H * Mc < (1L << 31) && N < (1L << 31), "dimension too large");
   SB_REQUIRE(cap > 0 && cap % 16 == 0, "row lists must be padded to a multiple of 16");
   SB_REQUIRE(forward_rows_supported<T>(W, N, H, Mc), "shape not supported by the row-list forward kernel");
-  ForwardRowsArgs<T> a{{act, x, W, bias, B, N, H * Mc, Mc, H, cdiv(B, 16), {}, nullptr, 0}, rows, row_cnt, cap, x_blocked};
-  const size_t bytes = part.p ? forward_rows_part_bytes<T>(cap, B, H, Mc) : 0;
-  if (bytes > 0 && bytes <= part.bytes) {
-    a.f.part = (T *)part.p;
-    a.f.split_chunks = forward_rows_split_chunks<T>(cap, B, H);
+  ForwardRowsArgs<T> a{{act, x, W, bias, B, N, H * Mc, Mc, H, cdiv(B, 16), {}}, rows, row_cnt, cap, x_blocked};
+  // Wide hypercolumns, few of them and long lists: a workgroup per column group, then the softmax, every sum as in
+  // the fused kernel (27648 -> 15 x 200, lists of 15800, batch 128, 120 tiles: 286 us fused, 240 us this way, whole steps 577 and 480 us).
+  constexpr int GW1 = 16 * Real<T>::VW;
+  if (Mc > GW1 && 5 * H * cdiv(B, 16) <= 3L * device_cu_count() && cap >= 1024) {
+    ProfScope prof_(st, K_FORWARD);
+    a.f.by_batch_tiles = FastDiv::of(a.f.batch_tiles);
+    const dim3 g((unsigned)(8 * cdiv(H * a.f.batch_tiles, 8)), (unsigned)cdiv(Mc, GW1)), blk(256);
+    constexpr int VWc = Real<T>::VW;
+    if (x_blocked) hipLaunchKernelGGL((k_forward_rows<T, 1, 4, 1, true, VWc, 2048, true>), g, blk, 0, st, a);
+    else hipLaunchKernelGGL((k_forward_rows<T, 1, 4, 1, false, VWc, 2048, true>), g, blk, 0, st, a);
+    SB_LAUNCH_CHECK();
+    return launch_softmax_as_fused<T, 16>(st, act, B, H, Mc);
   }
   const long need = cdiv(Mc, 16 * Real<T>::VW);
   // hypercolumns of 7 column blocks of 16 (97..112 columns): the last group runs with 3 (float) or 1
@@ -756,16 +710,13 @@ int launch_copy_pair(hipStream_t st, T *dst1, const T *src1, size_t n1, T *dst2,
 
 #define SB_INSTANTIATE_LAUNCHERS(T)                                                                   \
   template int launch_forward<T>(hipStream_t, T *, const T *, const T *, const T *, long, long, long, \
-                                 long, bool, ForwardScratch);                                         \
+                                 long, bool);                                                         \
   template int launch_forward_classify<T>(hipStream_t, T *, const T *, const T *, const T *, long,    \
                                           long, long, long, bool, const T *, int32_t *,               \
-                                          unsigned long long *, ForwardScratch);                      \
-  template size_t forward_part_bytes<T>(long, long, long, long, bool);                                \
-  template size_t forward_rows_part_bytes<T>(long, long, long, long);                                 \
+                                          unsigned long long *);                                      \
   template bool forward_rows_supported<T>(const T *, long, long, long);                               \
   template int launch_forward_rows<T>(hipStream_t, T *, const T *, const T *, const T *, const int *, \
-                                      const int *, long, long, long, long, long, const T *,           \
-                                      ForwardScratch);                                                \
+                                      const int *, long, long, long, long, long, const T *);          \
   template int launch_gather_rows_blocked<T>(hipStream_t, T *, T *, const T *, const int64_t *, long, \
                                              long);                                                  \
   template int launch_softmax<T>(hipStream_t, T *, long, long, long);                                 \

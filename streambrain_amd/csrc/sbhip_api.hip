@@ -369,7 +369,6 @@ static void *optional_scratch(Reusable &b, size_t bytes) {
 // the lock until all of them are in the stream, so that calls from several threads do not interleave.
 static Reusable g_work;
 static std::mutex g_work_mutex;
-static ForwardScratch forward_scratch(Reusable &b, size_t bytes) { return ForwardScratch{optional_scratch(b, bytes), bytes}; }
 
 // Per-kernel entry points keep the reference's in-place contract: the fused kernel writes the new
 // Ci / Cj into scratch, which is then copied over the caller's arrays.
@@ -555,10 +554,9 @@ static int layer_forward(sb_net *net, Layer &L, const T *x, long B, const T *x_b
   }
   if (L.rows && L.w_masked)
     return launch_forward_rows<T>(g_ctx.stream, act, x, (const T *)L.W, (const T *)L.bias, L.rows,
-                                  L.row_cnt, L.rows_cap, B, L.N, L.H, L.Mc, x_blocked,
-                                  forward_scratch(net->work, forward_rows_part_bytes<T>(L.rows_cap, B, L.H, L.Mc)));
+                                  L.row_cnt, L.rows_cap, B, L.N, L.H, L.Mc, x_blocked);
   return launch_forward<T>(g_ctx.stream, act, x, (const T *)L.W, (const T *)L.bias, B, L.N, L.H,
-                           L.Mc, true, forward_scratch(net->work, forward_part_bytes<T>(B, L.N, L.H, L.Mc, true)));
+                           L.Mc, true);
 }
 
 // One training step of `L` on input x (and on y = its own activation or the labels), in the order of
@@ -861,8 +859,7 @@ static int net_forward_batches(sb_net *net, const void *h_images, const void *h_
           // output layer: activation and classification (first maximal unit, comparison with the labels)
           rc = launch_forward_classify<T>(st, (T *)L.act, x, (const T *)L.W, (const T *)L.bias, B, L.N, L.H,
                                           L.Mc, true, h_labels ? (const T *)dY + lo * NC : nullptr,
-                                          dP ? dP + lo : nullptr, net->d_correct,
-                                          forward_scratch(net->work, forward_part_bytes<T>(B, L.N, L.H, L.Mc, true)));
+                                          dP ? dP + lo : nullptr, net->d_correct);
         else
           rc = layer_forward<T>(net, L, x, B, l == 0 ? xb : nullptr);
         x = (const T *)L.act;
@@ -1094,9 +1091,7 @@ int sb_fill_bytes(void *d_dst, int value, size_t bytes) {
 #define SB_DEFINE_KERNEL_API(SFX, T)                                                                   \
   int sb_update_state_##SFX(T *act, const T *x, const T *W, const T *bias, long B, long N, long M) {   \
     SB_READY();                                                                                        \
-    std::lock_guard<std::mutex> lock(g_work_mutex);                                                    \
-    return launch_forward<T>(g_ctx.stream, act, x, W, bias, B, N, 1, M, false,                         \
-                             forward_scratch(g_work, forward_part_bytes<T>(B, N, 1, M, false)));       \
+    return launch_forward<T>(g_ctx.stream, act, x, W, bias, B, N, 1, M, false);                        \
   }                                                                                                    \
   int sb_softmax_minicolumns_##SFX(T *act, long B, long H, long Mc) {                                  \
     SB_READY();                                                                                        \
@@ -1106,18 +1101,14 @@ int sb_fill_bytes(void *d_dst, int value, size_t bytes) {
                                   long H, long Mc) {                                                   \
     SB_READY();                                                                                        \
     SB_REQUIRE(B > 0 && N > 0 && H > 0 && Mc > 0, "sizes must be positive");                           \
-    std::lock_guard<std::mutex> lock(g_work_mutex);                                                    \
-    return launch_forward<T>(g_ctx.stream, act, x, W, bias, B, N, H, Mc, true,                         \
-                             forward_scratch(g_work, forward_part_bytes<T>(B, N, H, Mc, true)));       \
+    return launch_forward<T>(g_ctx.stream, act, x, W, bias, B, N, H, Mc, true);                        \
   }                                                                                                    \
   int sb_compute_activation_rows_##SFX(T *act, const T *x, const T *W, const T *bias, const int *rows, \
                                        const int *row_cnt, long cap, long B, long N, long H, long Mc,  \
                                        const T *x_blocked) {                                           \
     SB_READY();                                                                                        \
-    std::lock_guard<std::mutex> lock(g_work_mutex);                                                    \
     return launch_forward_rows<T>(g_ctx.stream, act, x, W, bias, rows, row_cnt, cap, B, N, H, Mc,      \
-                                  x_blocked,                                                           \
-                                  forward_scratch(g_work, forward_rows_part_bytes<T>(cap, B, H, Mc))); \
+                                  x_blocked);                                                          \
   }                                                                                                    \
   int sb_rows_in_blocks_##SFX(T *dst, const T *src, long rows, long cols) {                            \
     SB_READY();                                                                                        \
