@@ -241,7 +241,7 @@ int launch_forward_rows(hipStream_t st, T *act, const T *x, const T *W, const T 
   SB_REQUIRE(forward_rows_supported<T>(W, N, H, Mc), "shape not supported by the row-list forward kernel");
   ForwardRowsArgs<T> a{{act, x, W, bias, B, N, H * Mc, Mc, H, cdiv(B, 16), {}}, rows, row_cnt, cap, x_blocked};
   // Wide hypercolumns, few of them and long lists: a workgroup per column group, then the softmax, every sum as in
-  // the fused kernel (27648 -> 15 x 200, lists of 15800, batch 128, 120 tiles: 286 us fused, 240 us this way, whole steps 577 and 480 us).
+  // the fused kernel (27648 -> 15 x 200, lists of 15800, batch 128, 120 tiles: 286 us fused, 249 + 5 us this way, whole steps 516 and 480 us).
   constexpr int GW1 = 16 * Real<T>::VW;
   if (Mc > GW1 && 5 * H * cdiv(B, 16) <= 3L * device_cu_count() && cap >= 1024) {
     ProfScope prof_(st, K_FORWARD);
