@@ -12,10 +12,10 @@
 //     row's place is the number of listed rows ahead of it;
 //   phase B (one wavefront, one candidate per lane and side): the iterations themselves, with the same picks, tie
 //     rule, break conditions and score expression as a full scan.
-// A round reads the N scores and sides twice (the second time from L2) and has six barriers; its time is latency.
+// A round reads the N scores and sides twice (the second time from L2) and has seven barriers; its time is latency.
 // What a round does not cover -- a side whose first candidate row has a NaN score or may come to have one, or a
 // list that overflows -- is left to a full scan per iteration (swap_by_scans).
-// 27648 rows, floats: 25 us; 318 us with the state in registers and a radix select on 2048-bin histograms, whose
+// 27648 rows, floats: 22 us; 318 us with the state in registers and a radix select on 2048-bin histograms, whose
 // counters all threads hit together (scores share their leading bits), and a scan per iteration once any score is
 // NaN, as the scores of inputs that are always on are (1 - Ci = 0).
 #pragma once
@@ -138,6 +138,7 @@ struct MaskSwap {
     int list_idx[2][LIST];
     K bound_key[2];
     int bound_idx[2], nlist[2], top[2][TOP];
+    int rank[2][64];  // bins whose best row is ahead of this one's
     int nan_first[2], ahead[2];  // lowest row with a NaN score; rows with a score below it
     int swaps;
   };
@@ -182,6 +183,7 @@ struct MaskSwap {
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     constexpr int kNone = 0x7fffffff;
     if (tid < 2) sh.nlist[tid] = 0, sh.nan_first[tid] = kNone, sh.ahead[tid] = 0;
+    if (tid < 128) sh.rank[tid >> 6][tid & 63] = 0;
     __syncthreads();
     // ---- phase A
     Rows first;
@@ -212,22 +214,30 @@ struct MaskSwap {
       }
     }
     __syncthreads();
-    if (wv < 2) {  // wavefront g finds side g's bound
-      const int g = wv;
-      KeyIdx<K> b{0, -1};
+    // eight wavefronts per side: each has the side's 64 best rows, a lane each, and compares them with eight (one
+    // wavefront with all 64: 3.5 us)
+    const int g_of = wv / (NWV / 2);
+    KeyIdx<K> b{0, -1};
 #pragma unroll
-      for (int w = 0; w < NWV; w++) b = pick_key<K>(b, KeyIdx<K>{sh.bin_key[g][w][lane], sh.bin_idx[g][w][lane]});
+    for (int w = 0; w < NWV; w++) b = pick_key<K>(b, KeyIdx<K>{sh.bin_key[g_of][w][lane], sh.bin_idx[g_of][w][lane]});
+    {
+      constexpr int PER = 64 / (NWV / 2);
+      const int m0 = (wv % (NWV / 2)) * PER;
       int rank = 0;
 #pragma unroll
-      for (int m = 0; m < 64; m++) {
-        const K km = readlane_k(b.key, m);
-        const int im = __builtin_amdgcn_readlane(b.idx, m);
+      for (int m = 0; m < PER; m++) {
+        const K km = readlane_k(b.key, m0 + m);
+        const int im = __builtin_amdgcn_readlane(b.idx, m0 + m);
         rank += (im >= 0 && (km > b.key || (km == b.key && im > b.idx))) ? 1 : 0;
       }
+      if (rank) atomicAdd(&sh.rank[g_of][lane], rank);
+    }
+    __syncthreads();
+    if (wv % (NWV / 2) == 0) {
       const bool enough = __popcll(__ballot(b.idx >= 0)) >= TOP;  // else the side's rows are all listed
-      if (enough ? (b.idx >= 0 && rank == TOP - 1) : lane == 0) {
-        sh.bound_key[g] = enough ? b.key : 0;
-        sh.bound_idx[g] = enough ? b.idx : -1;
+      if (enough ? (b.idx >= 0 && sh.rank[g_of][lane] == TOP - 1) : lane == 0) {
+        sh.bound_key[g_of] = enough ? b.key : 0;
+        sh.bound_idx[g_of] = enough ? b.idx : -1;
       }
     }
     __syncthreads();
