@@ -133,9 +133,9 @@ __device__ __forceinline__ unsigned tile_of_workgroup(const TrainArgs<T> &a, uns
 }
 
 // ---- a float as three bfloat16: x = h + m + l exactly (for |x| of at least 2^-110; below, up to the smallest
-// bfloat16).  h holds the leading 8 bits, cut off, so that it is never beyond x; m the next 8, rounded; l the rest, at
-// most 8 bits.  For |x| below kSplitLimit: products of larger numbers, infinities and NaN are not what the products of
-// their pieces add up to.
+// bfloat16).  h holds the leading 8 bits, rounded to nearest, so that m, the next 8 bits, is at most 2^-8 of x's leading
+// bit, and l, the rest, at most 2^-17 of it.  (Rounding h cannot overflow: for |x| below kSplitLimit; products of larger
+// numbers, infinities and NaN are not what the products of their pieces add up to.)
 constexpr float kSplitLimit = 0x1p60f;
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 struct Split8 {  // eight consecutive batch rows of one column
@@ -145,9 +145,8 @@ __device__ __forceinline__ Split8 split_bf16(const float (&x)[8]) {
   Split8 s;
 #pragma unroll
   for (int k = 0; k < 8; k++) {
-    const unsigned bits = __float_as_uint(x[k]);
-    const float rest = x[k] - __uint_as_float(bits & 0xffff0000u);
-    s.h[k] = __builtin_bit_cast(__bf16, (unsigned short)(bits >> 16));
+    s.h[k] = (__bf16)x[k];
+    const float rest = x[k] - (float)s.h[k];
     s.m[k] = (__bf16)rest;
     s.l[k] = (__bf16)(rest - (float)s.m[k]);
   }
@@ -710,9 +709,12 @@ void k_train_fused(TrainArgs<T> a) {
 // The fused pass for big float layers: Cij and W as k_train_fused writes them, with x^T y on the bfloat16 matrix
 // cores, which multiply sixteen times as fast as the float ones.  Both operands are split exactly into three bfloat16
 // (SplitBatch, written by k_trace_sums<float, true>, which also leaves the new traces), and the six products down to
-// 2^-16 are accumulated in float: h h + h m + m h + h l + l h + m m.  What is left out is below 2^-24 of a product
-// on either side of zero, less than the rounding of a float product, and an accumulator is rounded six times per 32
-// batch rows instead of 32.
+// 2^-17 are accumulated in float: h h + h m + m h + h l + l h + m m.  What is left out, m l + l m + l l, is at most 2^-24
+// of a product, and an accumulator is rounded (cut off, rather) six times per 32 batch rows instead of 32.  Off the exact sums, measured
+// in units of 2^-24 (at worst / rms; in brackets the float instructions): 32 rows, equal ones 2.0 / 0.5 (8.5 / 3.4),
+// random ones 1.4 / 0.6 (7.3 / 1.5), values over 30 binary orders 7.7 / 1.2 (10.9 / 1.3); 128 rows 23 / 3.3 (32 / 13.7),
+// 9.8 / 1.9 (15.8 / 2.9), 14.6 / 2.0 (19.5 / 2.6).  Over many orders the float instructions are ahead below 32
+// rows (16: 6.9 / 1.18 against 8.7 / 1.00, 8: 7.2 / 1.19 against 5.8 / 0.78), so smaller batches stay with k_train_fused.
 // Bound: Cij read and written once, W written once, against 6 x 2 B N M flops on the matrix cores; with the float
 // instructions those were 2 B N M at a sixteenth of the rate, which is what k_train_fused waits for here.
 // A workgroup (4 wavefronts) owns a tile of 128 x 64, a wavefront 32 rows of it: 2 x 4 blocks of 16 x 16, so
@@ -725,6 +727,7 @@ void k_train_fused(TrainArgs<T> a) {
 // suits matrices that stay in the memory-side cache, pays for that once they do not (sums included, batch 128: 12288 x
 // 3000 87 us non-temporal, 192 us written through, 123 us with the default policy; 12288 x 3200 91 / 119 / 116 us).
 constexpr int kSplitTileI = 128, kSplitTileJ = 64, kSplitRows = 32;
+constexpr long kSplitBatch = 32;  // rows of the smallest batch that is split
 template <bool VEC, int MB>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4)))
 void k_train_split(TrainArgs<float> a, SplitBatch sp) {

@@ -289,16 +289,17 @@ template <typename T>
 static long train_tiles_of_one_round() { return (long)train_waves_per_simd<T, true, 1>() * device_cu_count(); }
 
 // Floats go through k_trace_sums<float, true> and k_train_split from two and a half rounds of 64 x 64 tiles on, with
-// small batches, which leave the matrix cores little to do, from five.  Sums included, against k_train_fused on its
+// batches of 32 rows, which leave the matrix cores little to do, from five.  Sums included, against k_train_fused on its
 // own, 3000 columns: batch 128, 2048 rows (1.2 rounds) 26.0 / 26.7 us, 4096 (2.4) 39.7 / 47.8, 8192 (4.7) 66 / 94, 16384
 // 110 / 257; batch 512, 8192 rows 141 / 239; batch 32, 8192 rows 54.6 / 53.5, 27648 255 / 369.  Between one round and the
 // line there are 15 % to gain, and the small layers below it, which train for epochs in moments, keep the rounding of
 // their trajectories (after a few dozen steps those tell one order of sums from another).
-// Its windows hold 128 rows of Cij and 32 split batch rows.
+// Batches of fewer than kSplitBatch rows stay with the float instructions, whose sums can be closer there (see
+// k_train_split).  Its windows hold 128 rows of Cij and 32 split batch rows.
 template <typename T>
 size_t train_split_bytes(long B, long N, long H, long Mc) {
   if constexpr (sizeof(T) != 4) return 0;
-  if (B <= 0 || N <= 0 || H <= 0 || Mc <= 0) return 0;
+  if (B < kSplitBatch || N <= 0 || H <= 0 || Mc <= 0) return 0;
   const long M = H * Mc;
   if (M <= 32 || 2 * cdiv(N, 64) * cdiv(M, 64) < (B > 32 ? 5 : 10) * train_tiles_of_one_round<T>()) return 0;
   const long xw = cdiv(N, kSplitTileI) * kSplitTileI, yw = cdiv(M, kSplitTileJ) * kSplitTileJ;

@@ -519,6 +519,31 @@ def test_train_pass_of_big_float_layers(k, B, N, H, Mc, masked):
     assert_close(got["Cj"], cj, f, "Cj")
 
 
+@pytest.mark.parametrize("B", [1, 2, 16, 32, 64])
+@pytest.mark.parametrize("equal_rows", [True, False])
+def test_products_of_big_float_layers_are_as_exact_as_floats(k, B, equal_rows):
+    """x^T y alone (traces of zero, taupdt 1, a batch that is a power of two: no other rounding), with the values whose
+    last bits the pieces of a float lose most of, in batches that do not average that out."""
+    N, H, Mc, f = 8192, 50, 64, np.float32  # 6400 tiles of 64 x 64
+    M, rng = H * Mc, np.random.default_rng(B)
+    values = np.array([1 + 2 ** -7 - 2 ** -16, 1.0038986, 1 + 2 ** -8 - 2 ** -17, 1 + 2 ** -9 + 2 ** -23], f)
+    x, y = (1 + rng.random((1 if equal_rows else B, n), dtype=f) for n in (N, M))
+    if equal_rows:
+        x[:, :N // 2], y[:, :M // 2] = np.resize(values, N // 2), np.repeat(values, M // 8)
+        x, y = np.repeat(x, B, 0), np.repeat(y, B, 0)
+    st = {"weights": np.zeros((N, M), f), "bias": np.zeros(M, f), "kbi": np.ones(M, f), "Ci": np.ones(N, f),
+          "Cj": np.ones(M, f), "Cij": np.zeros((N, M), f), "wmask": np.ones((N, H), np.uint8)}
+    got = k.plastic_train_step(st, x, y, H, Mc, 1.0, -139.0, 0.062, 0.022, hypercolumn=None)["Cij"]
+    want = (x.T.astype(np.float64) @ y) / B
+    # Below 32 rows one rounding, 2^-24, per batch row.  From there on the products that are left out, 2^-24 at most, and
+    # six additions of 32 products each per 32 rows, which the bfloat16 cores cut off rather than round, 2^-23 each (64
+    # equal rows are up to 10.9 2^-24 off, more than eight roundings to nearest come to); in the first 32 rows all but
+    # the last addition are of sums that are still small.
+    bound = 2.0 ** -24 * (B if B < 32 else 1 + 2 * (1 + 6 * (B // 32 - 1)))
+    off = np.max(np.abs(got - want) / want)
+    assert off <= bound * 1.001, f"{off * 2 ** 24:.2f} 2^-24"
+
+
 @pytest.mark.parametrize("dtype", DT)
 @pytest.mark.parametrize("B", [1, 16, 33])
 @pytest.mark.parametrize("N", [2048, 4113])
