@@ -132,11 +132,13 @@ __device__ __forceinline__ unsigned tile_of_workgroup(const TrainArgs<T> &a, uns
   return tile;
 }
 
-// ---- a float as three bfloat16: x = h + m + l exactly (for |x| of at least 2^-110; below, up to the smallest
-// bfloat16).  h holds the leading 8 bits, rounded to nearest, so that m, the next 8 bits, is at most 2^-8 of x's leading
-// bit, and l, the rest, at most 2^-17 of it.  (Rounding h cannot overflow: for |x| below kSplitLimit; products of larger
-// numbers, infinities and NaN are not what the products of their pieces add up to.)
-constexpr float kSplitLimit = 0x1p60f;
+// ---- a float as three bfloat16: kSplitScale x = h + m + l exactly.  h holds the leading 8 bits, rounded to nearest, so
+// that m, the next 8 bits, is at most 2^-8 of x's leading bit, and l, the rest, at most 2^-17 of it.  The scale keeps
+// every bit of the smallest float, 2^-149, inside the normal bfloat16 (from 2^-126; without it, l of numbers below 2^-110
+// was lost: at 2^-122, 2^-14 of the product); it is taken off the finished sums again.  For |x| below kSplitLimit, so
+// that neither h nor the sums overflow (2^108 each product): products of larger numbers, infinities and NaN are not
+// what the products of their pieces add up to.
+constexpr float kSplitScale = 0x1p24f, kSplitLimit = 0x1p30f;
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 struct Split8 {  // eight consecutive batch rows of one column
   bf16x8 h, m, l;
@@ -145,8 +147,9 @@ __device__ __forceinline__ Split8 split_bf16(const float (&x)[8]) {
   Split8 s;
 #pragma unroll
   for (int k = 0; k < 8; k++) {
-    s.h[k] = (__bf16)x[k];
-    const float rest = x[k] - (float)s.h[k];
+    const float v = x[k] * kSplitScale;
+    s.h[k] = (__bf16)v;
+    const float rest = v - (float)s.h[k];
     s.m[k] = (__bf16)rest;
     s.l[k] = (__bf16)(rest - (float)s.m[k]);
   }
@@ -863,6 +866,10 @@ void k_train_split(TrainArgs<float> a, SplitBatch sp) {
     __syncthreads();
     request_tile();
     multiply();
+#pragma unroll
+    for (int r = 0; r < 2; r++)
+#pragma unroll
+      for (int c = 0; c < 4; c++) acc[r][c] *= 1.0f / (kSplitScale * kSplitScale);
   }
 
   const float scale = a.invB * a.tau;

@@ -544,6 +544,25 @@ def test_products_of_big_float_layers_are_as_exact_as_floats(k, B, equal_rows):
     assert off <= bound * 1.001, f"{off * 2 ** 24:.2f} 2^-24"
 
 
+@pytest.mark.parametrize("magnitudes", [(2.0 ** -123, 1), (1, 2.0 ** -123), (2.0 ** -149, 2.0 ** 29), (2.0 ** -95, 2.0 ** -28),
+                                        (2.0 ** 29, 2.0 ** 29), (2.0 ** 31, 2.0 ** -90)])
+def test_products_of_big_float_layers_keep_the_bits_of_small_numbers(k, magnitudes):
+    """x^T y alone, with x and y anywhere in the range of floats: down to the smallest one, and up to where the pieces'
+    range ends and beyond."""
+    B, N, H, Mc, f = 32, 8192, 50, 64, np.float32
+    M, rng = H * Mc, np.random.default_rng(7)
+    x, y = (((1 + rng.random((B, n))) * m).astype(f) for n, m in zip((N, M), magnitudes))
+    st = {"weights": np.zeros((N, M), f), "bias": np.zeros(M, f), "kbi": np.ones(M, f), "Ci": np.ones(N, f),
+          "Cj": np.ones(M, f), "Cij": np.zeros((N, M), f), "wmask": np.ones((N, H), np.uint8)}
+    got = k.plastic_train_step(st, x, y, H, Mc, 1.0, -139.0, 0.062, 0.022, hypercolumn=None)["Cij"]
+    want = (x.T.astype(np.float64) @ y) / B
+    # (as above, twice the two roundings: the smallest products here are just above the subnormal range; 32 roundings where
+    # the tile stays with the float instructions, the last pair)
+    bound = 2.0 ** -24 * (32 if max(magnitudes) > 2 ** 30 else 5)
+    off = np.max(np.abs(got - want) / want)
+    assert off <= bound, f"{off * 2 ** 24:.2f} 2^-24"
+
+
 @pytest.mark.parametrize("dtype", DT)
 @pytest.mark.parametrize("B", [1, 16, 33])
 @pytest.mark.parametrize("N", [2048, 4113])
