@@ -374,6 +374,8 @@ static std::mutex g_work_mutex;
 // Ci / Cj into scratch, which is then copied over the caller's arrays.
 // `fixed_scratch`: room for N + M elements that the caller brings (no allocation here), or nullptr to
 // use the context's growable buffer.
+// Calls without a mask (sb_update_weights, sb_update_counters) do without the optional scratch at sizes that
+// sb_update_weights_noalloc_f32 takes, which has none and promises the same results.
 template <typename T>
 static int train_in_place(const T *x, const T *y, T *Cij, T *W, T *Ci, T *Cj, const uint8_t *wmask,
                           int bias_mode, T *bias, T *kbi, long B, long N, long H, long Mc, T taupdt,
@@ -385,9 +387,10 @@ static int train_in_place(const T *x, const T *y, T *Cij, T *W, T *Ci, T *Cj, co
   int rc = fixed_scratch ? 0 : ensure_trace_scratch(N + M);
   if (rc) return rc;
   T *ci_next = fixed_scratch ? fixed_scratch : (T *)g_ctx.trace_next, *cj_next = ci_next + N;
+  const bool as_noalloc = !wmask && N + M <= (long)SB_NOALLOC_MAX_UNITS;
   rc = launch_train_fused<T>(st, x, y, Cij, W, Ci, Cj, ci_next, cj_next, wmask, bias_mode, bias, kbi, B,
                              N, H, Mc, taupdt, cthr, khalf, pmin, taubdt, false, nullptr, 0,
-                             fixed_scratch ? nullptr : optional_scratch(g_work, train_split_bytes<T>(B, N, H, Mc)));
+                             as_noalloc ? nullptr : optional_scratch(g_work, train_split_bytes<T>(B, N, H, Mc)));
   if (rc) return rc;
   return launch_copy_pair<T>(st, Ci, ci_next, (size_t)N, Cj, cj_next, (size_t)M);
 }

@@ -59,6 +59,20 @@ def test_noalloc_update_weights_matches_the_allocating_entry_point(oracle):
         assert np.max(np.abs(got[3] - o[3]) / np.maximum(np.abs(o[3]), 1)) <= 1e-5
 
 
+@pytest.mark.parametrize("B,N,M", [(64, 4353, 3000), (33, 6464, 2049)])
+def test_noalloc_update_weights_matches_the_allocating_entry_point_for_big_layers(B, N, M):
+    """Layers of 3200 and more tiles of 64 x 64, for which the library has a second kernel that wants scratch."""
+    from streambrain_amd import _capi
+    _capi.init()
+    lib = _capi.lib()
+    p = _problem(np.random.default_rng(B), B, N, M)
+    got, allocated = _run(lib.sb_update_weights_noalloc_f32, *p, 0.01, 0.005)
+    assert allocated == 0
+    ref, _ = _run(lib.sb_update_weights_f32, *p, 0.01, 0.005)
+    for name, g, r in zip(("Ci", "Cj", "Cij", "W"), got, ref):
+        assert np.array_equal(g, r), name
+
+
 def test_noalloc_update_weights_rejects_sizes_beyond_its_array():
     from streambrain_amd import _capi
     _capi.init()
