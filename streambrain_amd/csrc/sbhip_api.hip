@@ -1316,6 +1316,7 @@ int sb_net_set_layer_state(sb_net *net, int layer, const char *name, const void 
   SB_REQUIRE(h_src, "null pointer");
   SB_REQUIRE(bytes == s.bytes, "size mismatch");
   rc = staged_upload(s.ptr, h_src, bytes, g_ctx.stream);
+  SB_HIP(hipStreamSynchronize(g_ctx.stream));  // (the call is synchronous: the last pieces may still be on their way)
   if (rc) return rc;
   if ((rc = drop_frozen_cache(net))) return rc;  // (whatever layer: the cache is cheap to rebuild)
   Layer &L = net->layers[layer];

@@ -526,6 +526,31 @@ def test_evaluate_of_many_batches_equals_single_batches(hb, dtype):
     assert int(correct[0]) == int((pred == np.argmax(Y, axis=1)).sum())
 
 
+def test_state_written_is_on_the_device_when_the_call_returns():
+    """sb_net_set_layer_state is synchronous: nothing of it is left in the library's stream, so that the caller may go
+    on with a stream of its own."""
+    import ctypes
+    from streambrain_amd import _capi
+    _capi.init()
+    lib, net = _capi.lib(), ctypes.c_void_p()
+    hip = ctypes.CDLL(_capi.LIB_PATH)  # (symbols of the runtime that the library is linked with)
+    hip.hipStreamQuery.argtypes, hip.hipStreamQuery.restype = [ctypes.c_void_p], ctypes.c_int
+    lib.sb_stream.restype = ctypes.c_void_p
+    _capi.check(lib.sb_net_create(ctypes.byref(net), 0))
+    try:
+        N, M = 16384, 2048  # 128 MiB of weights: many pieces of the staging ring
+        assert lib.sb_net_add_dense_layer(net, N, 1, M, 0.01, 1.0, 1.0 / M, 1.0 / M) == 0
+        W, back = np.random.default_rng(0).random((N, M), dtype=np.float32), np.zeros((N, M), np.float32)
+        _capi.check(lib.sb_sync())
+        _capi.check(lib.sb_net_set_layer_state(net, 0, b"weights", W.ctypes.data, W.nbytes))
+        left = hip.hipStreamQuery(lib.sb_stream())
+        assert left == 0, f"hipStreamQuery: {left}"
+        _capi.check(lib.sb_net_get_layer_state(net, 0, b"weights", back.ctypes.data, back.nbytes))
+        assert np.array_equal(W, back)
+    finally:
+        _capi.check(lib.sb_net_destroy(net))
+
+
 def test_errors_are_python_exceptions(hb):
     net = hb.Network(np.float32)
     with pytest.raises(Exception):
