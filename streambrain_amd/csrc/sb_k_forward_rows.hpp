@@ -25,15 +25,15 @@ struct ForwardRowsArgs {
 // Wavefronts per SIMD the kernel's registers are budgeted for: three or two (as many workgroups of four
 // wavefronts per CU, one computing while another waits for its gathers) where the operand ring, the
 // accumulators and the x operands leave room for that, one for the big tiles.
-template <typename T, int NG>
-constexpr int forward_rows_regs(int rb) {  // registers of the three, in 32-bit units
+template <typename T>
+constexpr int forward_rows_regs(int NG, int rb) {  // registers of the three, in 32-bit units
   constexpr int VW = Real<T>::VW, D = sizeof(T) / 4;
   return (2 * VW * NG * VW + rb * NG * VW * 4 + 2 * rb * VW) * D;
 }
 constexpr int kRowsRegsTwoWaves = 150, kRowsRegsThreeWaves = 104;  // measured: no spills up to these
 template <typename T, int NG, int RB>
 constexpr int forward_rows_waves_per_simd() {
-  constexpr int regs = forward_rows_regs<T, NG>(RB);
+  constexpr int regs = forward_rows_regs<T>(NG, RB);
   return regs <= kRowsRegsThreeWaves ? 3 : regs <= kRowsRegsTwoWaves ? 2 : 1;
 }
 
@@ -55,6 +55,7 @@ constexpr int forward_rows_waves_per_simd() {
 // SEG: list entries staged per segment, 2048 or, for lists of at most 256 entries, 256: every thread loads
 // and stores SEG / 256 entries per segment whatever the list's length, and at batch 128 the kernel is a
 // chain of latencies that starts with this staging (1568 -> 30x100, density 0.1, lists of 157: 6.31 -> 6.13 us).
+// It also decides in which order the wavefronts' partial sums are added (NT).
 // SPLIT: a workgroup computes column group blockIdx.y (NG groups wide) of its hypercolumn only and stores the logits;
 // every sum is formed as without (same wavefronts, same chunks), k_softmax_as_fused does the rest.
 template <typename T, int NG, int NWAVES, int RB = 1, bool XT = false, int LW = Real<T>::VW, int SEG = 2048,

@@ -68,15 +68,22 @@ int hip_fail(hipError_t e, const char *what, const char *file, int line);
     }                                                 \
   } while (0)
 
+// The kernels are chosen by the batch size, and not all of them add and exponentiate in the same way.  `like` (forward
+// launches; 0: B itself): rows get the bits that a batch of so many rows gives them, so that a caller may put many
+// batches into one launch.
 template <typename T>
 int launch_forward(hipStream_t st, T *act, const T *x, const T *W, const T *bias, long B, long N,
-                   long H, long Mc, bool softmax);
+                   long H, long Mc, bool softmax, long like = 0);
+// Batches of B1 and of B2 rows give a row the same bits (softmax included; cap: as of launch_forward_rows, 0 for the
+// dense pass).
+template <typename T>
+bool forward_bits_equal(long B1, long B2, long N, long H, long Mc, long cap);
 // The same followed by launch_argmax_rows on the result (pred and / or labels + correct given); layers of
 // at most 32 units do both in one launch.
 template <typename T>
 int launch_forward_classify(hipStream_t st, T *act, const T *x, const T *W, const T *bias, long B, long N,
                             long H, long Mc, bool softmax, const T *labels, int32_t *pred,
-                            unsigned long long *correct);
+                            unsigned long long *correct, long like = 0);
 // The same result for a layer whose W is zero wherever wmask is 0, from the per-hypercolumn lists of
 // connected rows that launch_mask_rows builds (rows: [H, cap] ascending indices, the rest -1; cap a
 // multiple of 16; row_cnt: [H]); forward_rows_supported says whether the kernel takes the shape.
@@ -86,7 +93,8 @@ template <typename T>
 bool forward_rows_supported(const T *W, long N, long H, long Mc);
 template <typename T>
 int launch_forward_rows(hipStream_t st, T *act, const T *x, const T *W, const T *bias, const int *rows,
-                        const int *row_cnt, long cap, long B, long N, long H, long Mc, const T *x_blocked);
+                        const int *row_cnt, long cap, long B, long N, long H, long Mc, const T *x_blocked,
+                        long like = 0);
 // Lists of hypercolumns h0 .. h0 + count - 1 rebuilt from wmask.
 int launch_mask_rows(hipStream_t st, int *rows, int *row_cnt, const uint8_t *wmask, long N, long H,
                      long cap, long h0, long count);

@@ -10,6 +10,7 @@
 #include <algorithm>
 #include <hip/hip_ext.h>
 #include <cstdlib>
+#include <type_traits>
 
 namespace sb {
 
@@ -63,14 +64,26 @@ static int launch_softmax_as_fused(hipStream_t st, T *act, long B, long H, long 
 
 template <typename T>
 int launch_forward(hipStream_t st, T *act, const T *x, const T *W, const T *bias, long B, long N,
-                   long H, long Mc, bool softmax) {
-  return launch_forward_classify<T>(st, act, x, W, bias, B, N, H, Mc, softmax, nullptr, nullptr, nullptr);
+                   long H, long Mc, bool softmax, long like) {
+  return launch_forward_classify<T>(st, act, x, W, bias, B, N, H, Mc, softmax, nullptr, nullptr, nullptr, like);
+}
+
+// The fused kernel runs one workgroup per hypercolumn and 16 batch rows, one workgroup per CU.  For wide
+// hypercolumns (more than two column groups) whose tiles fill their last round of workgroups badly,
+// tiles of two column groups plus a separate softmax pass are faster (1568 -> Hx200, batch 128, fused
+// against separate: H = 16: 31.7 / 23.4 us, H = 30: 33.9 / 40.0, H = 48: 63.4 / 57.1, H = 64: 66.1 / 74.5).
+// (The separate pass, k_softmax, has the library's exponential and divides: other bits.)
+template <typename T>
+static bool forward_fuses(long B, long H, long Mc) {
+  const long need = cdiv(Mc, 16 * Real<T>::VW), max_fused = sizeof(T) == 4 ? 4 : 7;
+  const long tiles = H * cdiv(B, 16), cus = device_cu_count();
+  return need <= max_fused && (need <= 2 || 20 * tiles >= 17 * cdiv(tiles, cus) * cus);
 }
 
 template <typename T>
 int launch_forward_classify(hipStream_t st, T *act, const T *x, const T *W, const T *bias, long B, long N,
                             long H, long Mc, bool softmax, const T *labels, int32_t *pred,
-                            unsigned long long *correct) {
+                            unsigned long long *correct, long like) {
   constexpr int VW = Real<T>::VW;
   constexpr int GW = 16 * VW;
   SB_REQUIRE(act && x && W && bias, "null pointer");
@@ -90,7 +103,7 @@ int launch_forward_classify(hipStream_t st, T *act, const T *x, const T *W, cons
     return 0;
   }
   if (labels || pred) {  // wider layers: the forward pass, then the classification kernel
-    int rc = launch_forward<T>(st, act, x, W, bias, B, N, H, Mc, softmax);
+    int rc = launch_forward<T>(st, act, x, W, bias, B, N, H, Mc, softmax, like);
     if (rc) return rc;
     return launch_argmax_rows<T>(st, act, labels, B, M, pred, correct);
   }
@@ -99,14 +112,8 @@ int launch_forward_classify(hipStream_t st, T *act, const T *x, const T *W, cons
   ForwardArgs<T> a{act, x, W, bias, B, N, M, Mc, 0, cdiv(B, 16), {}};
   const bool base_vec = (N % VW == 0) && (M % VW == 0) && aligned16(x) && aligned16(W);
   const long need = cdiv(Mc, GW);
-  const long max_fused = sizeof(T) == 4 ? 4 : 7;
-  // The fused kernel runs one workgroup per hypercolumn and 16 batch rows, one workgroup per CU.  For wide
-  // hypercolumns (more than two column groups) whose tiles fill their last round of workgroups badly,
-  // tiles of two column groups plus a separate softmax pass are faster (1568 -> Hx200, batch 128, fused
-  // against separate: H = 16: 31.7 / 23.4 us, H = 30: 33.9 / 40.0, H = 48: 63.4 / 57.1, H = 64: 66.1 / 74.5).
   const long fused_tiles = H * cdiv(B, 16), cus_ = device_cu_count();
-  const bool enough_tiles = need <= 2 || 20 * fused_tiles >= 17 * cdiv(fused_tiles, cus_) * cus_;
-  if (softmax && need <= max_fused && enough_tiles) {
+  if (softmax && forward_fuses<T>(like > 0 ? like : B, H, Mc)) {
     const bool vec = base_vec && (Mc % VW == 0);
     // Hypercolumns of two column groups whose tiles leave half the CUs idle and that have a long reduction: a
     // workgroup per group, then the softmax.  Every sum as in the fused kernel, except in the four columns that
@@ -184,56 +191,91 @@ bool forward_rows_supported(const T *W, long N, long H, long Mc) {
          cdiv(Mc, 16 * VW) <= (sizeof(T) == 4 ? 4 : 7) && 16 * N * (long)sizeof(T) < (1L << 31);
 }
 
+// Column groups of a hypercolumn in k_forward_rows, and column blocks of the last one (LW; 0: whole groups).
+struct RowsGroups {
+  int n, last;
+};
+template <typename T>
+static RowsGroups forward_rows_groups(long Mc) {
+  constexpr int VW = Real<T>::VW, GW = 16 * VW, NGL = 8 / VW, LWL = 7 - (NGL - 1) * VW;
+  // hypercolumns of 7 column blocks of 16 (97..112 columns): the last group runs with 3 (float) or 1
+  // (double) blocks, provided none of its vectors straddles the end of the hypercolumn (as in launch_forward)
+  if (cdiv(Mc, 16) == 7 && (Mc - (NGL - 1) * GW) % LWL == 0) return {NGL, LWL};
+  // and of 13 column blocks (193..208 columns, 200 among them): one block in the last group
+  // (float: 4 groups, 12 + 1 blocks; double: 7, 12 + 1)
+  if (cdiv(Mc, 16) == 13) return {VW == 2 ? 7 : 4, 1};
+  const long need = cdiv(Mc, GW);
+  return {need <= 1 ? 1 : need <= 2 ? 2 : need <= 4 ? 4 : 7, 0};
+}
+// Row blocks per workgroup.  Large batches: 64 or 32 rows while there are tiles for eight rounds / three quarters
+// of a round of workgroups (much as in launch_forward), as long as the kernel then still fits two wavefronts per SIMD:
+// two workgroups per CU with fewer rows each beat one with more (204 against 240 us at 1568 -> 30x100,
+// batch 8192; 70 against 83 us at 1568 -> 100x100 in double, batch 512)
+template <typename T>
+static int forward_rows_blocks(int groups, long B, long N, long H) {
+  const long cus = device_cu_count();
+  const bool fits4 = forward_rows_regs<T>(groups, 4) <= kRowsRegsTwoWaves;
+  int rb = fits4 && H * cdiv(B, 64) >= 8 * cus ? 4 : (4 * H * cdiv(B, 32) >= 3 * cus ? 2 : 1);
+  while (rb > 1 && forward_rows_regs<T>(groups, rb) > kRowsRegsTwoWaves) rb /= 2;
+  // (32-bit byte offsets inside the tile's rows)
+  while (rb > 1 && 16 * rb * N * (long)sizeof(T) >= (1L << 31)) rb /= 2;
+  return rb;
+}
+// Short lists, few rows: a segment of 256 list entries and partial sums that meet in one step (see the kernel).
+template <typename T>
+static bool forward_rows_short(long B, long N, long H, long Mc, long cap) {
+  return cap <= 256 && forward_rows_blocks<T>(forward_rows_groups<T>(Mc).n, B, N, H) == 1;
+}
+
+template <typename T>
+bool forward_bits_equal(long B1, long B2, long N, long H, long Mc, long cap) {
+  if (cap > 0) return forward_rows_short<T>(B1, N, H, Mc, cap) == forward_rows_short<T>(B2, N, H, Mc, cap);
+  return H * Mc <= (sizeof(T) == 4 ? 32 : 16) || forward_fuses<T>(B1, H, Mc) == forward_fuses<T>(B2, H, Mc);
+}
+
+// `like`: batch size whose order of sums is taken
 template <typename T, int NG, int LW = Real<T>::VW>
-static int forward_rows_variant(hipStream_t st, ForwardRowsArgs<T> a) {
+static int forward_rows_variant(hipStream_t st, ForwardRowsArgs<T> a, long like) {
   ProfScope prof_(st, K_FORWARD);
   // four wavefronts measured best (8: 8.8 us, 4: 8.2 us, 2: 9.9 us, 16: 10.7 us at 1568 -> 30x100, density 0.1)
   constexpr int NW = 4;
-  // large batches: 64 or 32 rows per workgroup while there are tiles for eight rounds / three quarters
-  // of a round of workgroups (much as in launch_forward), as long as the kernel then still fits two wavefronts per SIMD:
-  // two workgroups per CU with fewer rows each beat one with more (204 against 240 us at 1568 -> 30x100,
-  // batch 8192; 70 against 83 us at 1568 -> 100x100 in double, batch 512)
-  const long cus = device_cu_count(), H = a.f.col_tiles, B = a.f.B;
-  constexpr bool fits4 = forward_rows_regs<T, NG>(4) <= kRowsRegsTwoWaves;
-  long rb = fits4 && H * cdiv(B, 64) >= 8 * cus ? 4 : (4 * H * cdiv(B, 32) >= 3 * cus ? 2 : 1);
-  while (rb > 1 && forward_rows_regs<T, NG>((int)rb) > kRowsRegsTwoWaves) rb /= 2;
-  // (32-bit byte offsets inside the tile's rows)
-  while (rb > 1 && 16 * rb * a.f.N * (long)sizeof(T) >= (1L << 31)) rb /= 2;
+  const long H = a.f.col_tiles, B = a.f.B;
+  constexpr bool fits4 = forward_rows_regs<T>(NG, 4) <= kRowsRegsTwoWaves;
+  const int rb = forward_rows_blocks<T>(NG, B, a.f.N, H);
   a.f.batch_tiles = cdiv(B, 16 * rb);
   a.f.by_batch_tiles = FastDiv::of(a.f.batch_tiles);
   const long grid = 8 * cdiv(a.f.col_tiles * a.f.batch_tiles, 8);
   SB_REQUIRE(grid < (1L << 31), "too many tiles for one launch");
   const dim3 g((unsigned)grid), blk(64 * NW);
-  if (a.xt) {  // the batch is also at hand in blocks of 16 rows
+  const bool is_short = forward_rows_short<T>(like, a.f.N, H, a.f.Mc, a.cap);
+  auto launch = [&](auto blocked) {  // (with the batch at hand in blocks of 16 rows, or without)
+    constexpr bool XT = decltype(blocked)::value;
     if constexpr (fits4) {
-      if (rb == 4) hipLaunchKernelGGL((k_forward_rows<T, NG, NW, 4, true, LW>), g, blk, 0, st, a);
+      if (rb == 4) {
+        if (is_short) hipLaunchKernelGGL((k_forward_rows<T, NG, NW, 4, XT, LW, 256>), g, blk, 0, st, a);
+        else hipLaunchKernelGGL((k_forward_rows<T, NG, NW, 4, XT, LW>), g, blk, 0, st, a);
+        return;
+      }
     }
-    if (rb == 4) {
-    } else if (rb == 2)
-      hipLaunchKernelGGL((k_forward_rows<T, NG, NW, 2, true, LW>), g, blk, 0, st, a);
-    else if (a.cap <= 256)  // short lists: a segment of 256 entries (see the kernel)
-      hipLaunchKernelGGL((k_forward_rows<T, NG, NW, 1, true, LW, 256>), g, blk, 0, st, a);
-    else
-      hipLaunchKernelGGL((k_forward_rows<T, NG, NW, 1, true, LW>), g, blk, 0, st, a);
-  } else {
-    if constexpr (fits4) {
-      if (rb == 4) hipLaunchKernelGGL((k_forward_rows<T, NG, NW, 4, false, LW>), g, blk, 0, st, a);
+    if constexpr (forward_rows_regs<T>(NG, 2) <= kRowsRegsTwoWaves) {
+      if (rb == 2) {
+        if (is_short) hipLaunchKernelGGL((k_forward_rows<T, NG, NW, 2, XT, LW, 256>), g, blk, 0, st, a);
+        else hipLaunchKernelGGL((k_forward_rows<T, NG, NW, 2, XT, LW>), g, blk, 0, st, a);
+        return;
+      }
     }
-    if (rb == 4) {
-    } else if (rb == 2)
-      hipLaunchKernelGGL((k_forward_rows<T, NG, NW, 2, false, LW>), g, blk, 0, st, a);
-    else if (a.cap <= 256)
-      hipLaunchKernelGGL((k_forward_rows<T, NG, NW, 1, false, LW, 256>), g, blk, 0, st, a);
-    else
-      hipLaunchKernelGGL((k_forward_rows<T, NG, NW, 1, false, LW>), g, blk, 0, st, a);
-  }
+    if (is_short) hipLaunchKernelGGL((k_forward_rows<T, NG, NW, 1, XT, LW, 256>), g, blk, 0, st, a);
+    else hipLaunchKernelGGL((k_forward_rows<T, NG, NW, 1, XT, LW>), g, blk, 0, st, a);
+  };
+  if (a.xt) launch(std::true_type{});
+  else launch(std::false_type{});
   SB_LAUNCH_CHECK();
   return 0;
 }
 
 template <typename T>
 int launch_forward_rows(hipStream_t st, T *act, const T *x, const T *W, const T *bias, const int *rows,
-                        const int *row_cnt, long cap, long B, long N, long H, long Mc, const T *x_blocked) {
+                        const int *row_cnt, long cap, long B, long N, long H, long Mc, const T *x_blocked, long like) {
   SB_REQUIRE(act && x && W && bias && rows && row_cnt, "null pointer");
   SB_REQUIRE(B > 0 && N > 0 && H > 0 && Mc > 0, "sizes must be positive");
   SB_REQUIRE(H * Mc < (1L << 31) && N < (1L << 31), "dimension too large");
@@ -253,20 +295,15 @@ int launch_forward_rows(hipStream_t st, T *act, const T *x, const T *W, const T 
     SB_LAUNCH_CHECK();
     return launch_softmax_as_fused<T, 16>(st, act, B, H, Mc);
   }
-  const long need = cdiv(Mc, 16 * Real<T>::VW);
-  // hypercolumns of 7 column blocks of 16 (97..112 columns): the last group runs with 3 (float) or 1
-  // (double) blocks, provided none of its vectors straddles the end of the hypercolumn (as in launch_forward)
-  {
-    constexpr int VW = Real<T>::VW, GW = 16 * VW, NGL = 8 / VW, LWL = 7 - (NGL - 1) * VW;
-    if (cdiv(Mc, 16) == 7 && (Mc - (NGL - 1) * GW) % LWL == 0) return forward_rows_variant<T, NGL, LWL>(st, a);
-    // and of 13 column blocks (193..208 columns, 200 among them): one block in the last group
-    constexpr int NGM = 16 / VW - (VW == 2 ? 1 : 0);  // float: 4 groups (12 + 1 blocks); double: 7 (12 + 1)
-    if (cdiv(Mc, 16) == 13) return forward_rows_variant<T, NGM, 1>(st, a);
-  }
-  if (need <= 1) return forward_rows_variant<T, 1>(st, a);
-  if (need <= 2) return forward_rows_variant<T, 2>(st, a);
-  if (need <= 4) return forward_rows_variant<T, 4>(st, a);
-  if constexpr (sizeof(T) == 8) return forward_rows_variant<T, 7>(st, a);
+  if (like <= 0) like = B;
+  constexpr int VW = Real<T>::VW, NGL = 8 / VW, LWL = 7 - (NGL - 1) * VW, NGM = VW == 2 ? 7 : 4;
+  const RowsGroups groups = forward_rows_groups<T>(Mc);
+  if (groups.last > 0 && cdiv(Mc, 16) == 7) return forward_rows_variant<T, NGL, LWL>(st, a, like);
+  if (groups.last > 0) return forward_rows_variant<T, NGM, 1>(st, a, like);
+  if (groups.n == 1) return forward_rows_variant<T, 1>(st, a, like);
+  if (groups.n == 2) return forward_rows_variant<T, 2>(st, a, like);
+  if (groups.n == 4) return forward_rows_variant<T, 4>(st, a, like);
+  if constexpr (sizeof(T) == 8) return forward_rows_variant<T, 7>(st, a, like);
   return -1;
 }
 
@@ -711,13 +748,14 @@ int launch_copy_pair(hipStream_t st, T *dst1, const T *src1, size_t n1, T *dst2,
 
 #define SB_INSTANTIATE_LAUNCHERS(T)                                                                   \
   template int launch_forward<T>(hipStream_t, T *, const T *, const T *, const T *, long, long, long, \
-                                 long, bool);                                                         \
+                                 long, bool, long);                                                   \
   template int launch_forward_classify<T>(hipStream_t, T *, const T *, const T *, const T *, long,    \
                                           long, long, long, bool, const T *, int32_t *,               \
-                                          unsigned long long *);                                      \
+                                          unsigned long long *, long);                                \
+  template bool forward_bits_equal<T>(long, long, long, long, long, long);                            \
   template bool forward_rows_supported<T>(const T *, long, long, long);                               \
   template int launch_forward_rows<T>(hipStream_t, T *, const T *, const T *, const T *, const int *, \
-                                      const int *, long, long, long, long, long, const T *);          \
+                                      const int *, long, long, long, long, long, const T *, long);    \
   template int launch_gather_rows_blocked<T>(hipStream_t, T *, T *, const T *, const int64_t *, long, \
                                              long);                                                  \
   template int launch_softmax<T>(hipStream_t, T *, long, long, long);                                 \

@@ -547,9 +547,11 @@ static int layer_check_masked(sb_net *net, Layer &L) {
   return 0;
 }
 
-// x_blocked: the same batch in blocks of 16 rows, or nullptr; out: where the activations go (nullptr: L.act)
+// x_blocked: the same batch in blocks of 16 rows, or nullptr; out: where the activations go (nullptr: L.act); like: batch
+// size whose bits the rows get (0: B)
 template <typename T>
-static int layer_forward(sb_net *net, Layer &L, const T *x, long B, const T *x_blocked = nullptr, T *out = nullptr) {
+static int layer_forward(sb_net *net, Layer &L, const T *x, long B, const T *x_blocked = nullptr, T *out = nullptr,
+                         long like = 0) {
   T *const act = out ? out : (T *)L.act;
   if (L.w_unchecked) {
     int rc = layer_check_masked<T>(net, L);
@@ -557,9 +559,22 @@ static int layer_forward(sb_net *net, Layer &L, const T *x, long B, const T *x_b
   }
   if (L.rows && L.w_masked)
     return launch_forward_rows<T>(g_ctx.stream, act, x, (const T *)L.W, (const T *)L.bias, L.rows,
-                                  L.row_cnt, L.rows_cap, B, L.N, L.H, L.Mc, x_blocked);
+                                  L.row_cnt, L.rows_cap, B, L.N, L.H, L.Mc, x_blocked, like);
   return launch_forward<T>(g_ctx.stream, act, x, (const T *)L.W, (const T *)L.bias, B, L.N, L.H,
-                           L.Mc, true);
+                           L.Mc, true, like);
+}
+
+// Batches of B1 and of B2 rows give a row the same bits in all layers up to `last` (*equal).
+template <typename T>
+static int net_bits_equal(sb_net *net, int last, long B1, long B2, bool *equal) {
+  *equal = true;
+  for (int l = 0; l <= last; l++) {
+    Layer &L = net->layers[l];
+    int rc = L.w_unchecked ? layer_check_masked<T>(net, L) : 0;
+    if (rc) return rc;
+    if (!forward_bits_equal<T>(B1, B2, L.N, L.H, L.Mc, L.rows && L.w_masked ? L.rows_cap : 0)) *equal = false;
+  }
+  return 0;
 }
 
 // One training step of `L` on input x (and on y = its own activation or the labels), in the order of
@@ -834,6 +849,11 @@ static int net_forward_batches(sb_net *net, const void *h_images, const void *h_
   if (piece < maxB) piece = maxB;
   piece = std::min(piece, pass_rows(net, maxB));
   if ((rc = ensure_act(net, std::min(piece, n)))) return rc;
+  // Every row gets the bits of its batch: passes run like batches of maxB rows, and what is left of the set behind the
+  // last whole batch runs on its own where a batch of that size takes other kernels.
+  const long tail = n > maxB ? n % maxB : 0;
+  bool tail_alike = true;
+  if (tail && (rc = net_bits_equal<T>(net, last_layer, maxB, tail, &tail_alike))) return rc;
   // (a set of one piece has nothing to overlap: it goes up on the library's stream)
   const hipStream_t up = n > piece ? g_stager.copy_stream : st;
   for (long c0 = 0; c0 < n && !rc; c0 += chunk) {
@@ -841,8 +861,13 @@ static int net_forward_batches(sb_net *net, const void *h_images, const void *h_
     if (h_labels) {
       if ((rc = staged_upload(dY, (const T *)h_labels + c0 * NC, (size_t)rows * NC * sizeof(T), up))) break;
     }
-    for (long lo = 0; lo < rows && !rc; lo += piece) {
-      const long B = lo + piece <= rows ? piece : rows - lo;
+    for (long lo = 0, B = 0; lo < rows && !rc; lo += B) {
+      long like = std::min(maxB, n);
+      B = lo + piece <= rows ? piece : rows - lo;
+      if (!tail_alike && c0 + lo + B == n) {
+        if (B > tail) B -= tail;
+        else like = tail;
+      }
       if ((rc = staged_upload((T *)dX + lo * NF, (const T *)h_images + (c0 + lo) * NF, (size_t)B * NF * sizeof(T), up)))
         break;
       if (up != st) {
@@ -862,9 +887,9 @@ static int net_forward_batches(sb_net *net, const void *h_images, const void *h_
           // output layer: activation and classification (first maximal unit, comparison with the labels)
           rc = launch_forward_classify<T>(st, (T *)L.act, x, (const T *)L.W, (const T *)L.bias, B, L.N, L.H,
                                           L.Mc, true, h_labels ? (const T *)dY + lo * NC : nullptr,
-                                          dP ? dP + lo : nullptr, net->d_correct);
+                                          dP ? dP + lo : nullptr, net->d_correct, like);
         else
-          rc = layer_forward<T>(net, L, x, B, l == 0 ? xb : nullptr);
+          rc = layer_forward<T>(net, L, x, B, l == 0 ? xb : nullptr, (T *)nullptr, like);
         x = (const T *)L.act;
       }
       if (rc) break;

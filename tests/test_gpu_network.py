@@ -526,6 +526,24 @@ def test_evaluate_of_many_batches_equals_single_batches(hb, dtype):
     assert int(correct[0]) == int((pred == np.argmax(Y, axis=1)).sum())
 
 
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("n_pix,H,Mc,density", [(784, 30, 100, 0.1), (392, 15, 200, 1.0), (300, 70, 60, 0.3)])
+@pytest.mark.parametrize("B", [128, 256])
+def test_inference_passes_keep_the_bits_of_single_batches(hb, dtype, n_pix, H, Mc, density, B):
+    """Layers whose kernels add up or exponentiate differently in batches of few and of many rows: a set that goes
+    through the layers in passes of many batches gives what its batches give one at a time, the ragged last one too."""
+    rng = np.random.default_rng(13)
+    n = 3000
+    X, Y = synthetic_images(rng, n, n_pix), one_hot_labels(rng, n, 10)
+    net = build_two_layer(hb, 2 * n_pix, H, Mc, 10, MNIST_HP, dtype, seed=5, density=density)
+    net.fit(X[:512], Y[:512], B, [(0, 1), (1, 1)])
+    whole, hidden, pred = net.forward(X, B), net.forward(X, B, 0), net.predict(X, B)
+    for lo in range(0, n, B):
+        assert np.array_equal(whole[lo:lo + B], net.forward(X[lo:lo + B], B)), lo
+        assert np.array_equal(hidden[lo:lo + B], net.forward(X[lo:lo + B], B, 0)), lo
+    assert np.array_equal(pred, np.argmax(whole, axis=1))
+
+
 def test_state_written_is_on_the_device_when_the_call_returns():
     """sb_net_set_layer_state is synchronous: nothing of it is left in the library's stream, so that the caller may go
     on with a stream of its own."""
