@@ -663,8 +663,9 @@ static int drop_frozen_cache(sb_net *net) {
 
 // Activations of layer `upto` for all training samples in data-set order, as many samples per pass as pass_rows says
 // (157 batches of 128 through 784 -> 15x200: 1.25 ms of launches of 8 us and a copy each, in passes of 5504 0.45 ms).
+// like: the batch size whose bits they get, as the steps that do without the cache ask for it.
 template <typename T>
-static int build_frozen_cache(sb_net *net, int upto, long maxB) {
+static int build_frozen_cache(sb_net *net, int upto, long maxB, long like) {
   const long Ns = net->Ns, Mo = net->layers[upto].M;
   int rc = drop_frozen_cache(net);
   if (rc) return rc;
@@ -684,7 +685,7 @@ static int build_frozen_cache(sb_net *net, int upto, long maxB) {
     const T *x = (const T *)net->X + lo * net->NF;
     for (int l = 0; l <= upto; l++) {
       T *const out = l == upto ? (T *)net->Hc + lo * Mo : (T *)nullptr;
-      if ((rc = layer_forward<T>(net, net->layers[l], x, B, (const T *)nullptr, out))) return rc;
+      if ((rc = layer_forward<T>(net, net->layers[l], x, B, (const T *)nullptr, out, like))) return rc;
       x = (const T *)net->layers[l].act;
     }
   }
@@ -710,6 +711,9 @@ static int net_train_batches(sb_net *net, int layer, long maxB, const int64_t *h
   SB_REQUIRE(first_batch >= 0 && n_batches >= 0 && first_batch + n_batches <= nb, "batch range");
   int rc = ensure_act(net, maxB < Ns ? maxB : Ns);
   if (rc) return rc;
+  // The frozen layers give a sample the same activations with and without their cache, and in whichever batch it is:
+  // those of a whole batch.
+  const long like = std::min(maxB, Ns);
   const bool permute = first_batch == 0;  // a later range continues the epoch already laid out
   SB_REQUIRE(permute || net->Xp, "the epoch's first batches have not been run");
   // a training step of a layer below the last changes what the cache was computed from
@@ -748,7 +752,7 @@ static int net_train_batches(sb_net *net, int layer, long maxB, const int64_t *h
       if ((rc = launch_gather_rows<T>(st, (T *)net->Yp, (const T *)net->Y, net->d_perm, Ns, net->NC)))
         return rc;
     if (cache_fits) {
-      if (net->Hc_layer != layer - 1 && (rc = build_frozen_cache<T>(net, layer - 1, maxB))) return rc;
+      if (net->Hc_layer != layer - 1 && (rc = build_frozen_cache<T>(net, layer - 1, maxB, like))) return rc;
       if (net->Hc_layer == layer - 1 &&
           (rc = launch_gather_rows<T>(st, (T *)net->Hcp, (const T *)net->Hc, net->d_perm, Ns, Mprev)))
         return rc;
@@ -768,7 +772,7 @@ static int net_train_batches(sb_net *net, int layer, long maxB, const int64_t *h
       x = (const T *)net->Hcp + lo * Mprev;
     } else {
       for (int l = 0; l < layer; l++) {
-        if ((rc = layer_forward<T>(net, net->layers[l], x, B, l == 0 ? xb : nullptr))) return rc;
+        if ((rc = layer_forward<T>(net, net->layers[l], x, B, l == 0 ? xb : nullptr, (T *)nullptr, like))) return rc;
         x = (const T *)net->layers[l].act;
       }
     }

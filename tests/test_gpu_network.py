@@ -206,6 +206,53 @@ def test_classifier_epochs_without_the_activation_cache_are_bit_identical(hb, dt
             assert np.array_equal(value, other[name]), name
 
 
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("n_pix,H,Mc,density,Ns,B", [(784, 30, 100, 0.1, 6000, 128), (100, 15, 200, 1.0, 6100, 256),
+                                                   (300, 70, 60, 0.3, 4500, 64)])
+def test_classifier_epochs_of_several_cache_passes_are_bit_identical(hb, dtype, n_pix, H, Mc, density, Ns, B):
+    """The same with more samples than the cache is computed of in one go (64 MiB of activations), with layers whose
+    kernels add up or exponentiate differently in such passes, in whole batches and in the ragged last one."""
+    assert Ns * H * Mc * np.dtype(dtype).itemsize > 64 << 20
+    rng = np.random.default_rng(79)
+    X, Y = synthetic_images(rng, Ns, n_pix), one_hot_labels(rng, Ns, 10)
+    states = []
+    for limit in (None, 0):
+        net = build_two_layer(hb, 2 * n_pix, H, Mc, 10, MNIST_HP, dtype, seed=5, density=density)
+        if limit == 0:
+            net.net.set_frozen_cache_limit(0)
+        np.random.seed(11)
+        net.fit(X[:1000], Y[:1000], B, [(0, 1)])
+        net.fit(X, Y, B, [(1, 2)])
+        states.append({name: np.array(getattr(net._layers[1], name)) for name in ("Ci", "Cj", "Cij", "weights", "bias")})
+    for name, value in states[0].items():
+        assert np.array_equal(value, states[1][name]), name
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+def test_classifier_above_two_frozen_layers_is_bit_identical_without_the_cache(hb, dtype):
+    """The cache of a network of three layers is computed through both layers below the classifier, pass by pass."""
+    rng = np.random.default_rng(80)
+    Ns, B, H, Mc = 4500, 100, 24, 100
+    X, Y = synthetic_images(rng, Ns, 30), one_hot_labels(rng, Ns, 10)
+    assert 2 * Ns * H * Mc * 4 > 64 << 20  # (of the wider one of the two, 4800 units)
+    states = []
+    for limit in (None, 0):
+        np.random.seed(5)
+        net = hb.Network(dtype)
+        layer = lambda n, h, m: hb.StructuralPlasticityLayer(n, h, m, 0.007, -139.0, 0.062, 0.022, 0.2, 16, (1, 1 / m, 1 / m))
+        net.add_layer(layer(60, 2 * H, Mc))
+        net.add_layer(layer(2 * H * Mc, H, Mc))
+        net.add_layer(hb.DenseLayer(H * Mc, 1, 10, 0.001, (1 / Mc, 1 / 10, 1 / Mc / 10)))
+        if limit == 0:
+            net.net.set_frozen_cache_limit(0)
+        np.random.seed(11)
+        net.fit(X[:300], Y[:300], B, [(0, 1), (1, 1)])
+        net.fit(X, Y, B, [(2, 2)])
+        states.append({name: np.array(getattr(net._layers[2], name)) for name in ("Ci", "Cj", "Cij", "weights", "bias")})
+    for name, value in states[0].items():
+        assert np.array_equal(value, states[1][name]), name
+
+
 def test_small_network_one_epoch_f32(hb):
     # float32, one epoch per layer (13 batches, short last one).  Stated drift bound after one epoch:
     # 1e-5 relative (rounding differences of ~1e-7 per step, amplified by the log of small traces).
