@@ -36,7 +36,12 @@ static long g_allocation_calls = 0;
 template <typename P>
 static hipError_t dev_malloc(P **p, size_t bytes) {
   g_allocation_calls++;
-  return hipMalloc((void **)p, bytes);
+  const hipError_t e = hipMalloc((void **)p, bytes);
+  if (e != hipSuccess) {
+    *p = nullptr;
+    (void)hipGetLastError();  // reported by the return value; the check behind the next launch must not find it
+  }
+  return e;
 }
 static hipError_t event_create(hipEvent_t *e) {
   g_allocation_calls++;
@@ -357,11 +362,7 @@ static void *optional_scratch(Reusable &b, size_t bytes) {
   (void)hipStreamSynchronize(g_ctx.stream);
   if (b.p) (void)hipFree(b.p);
   b = Reusable();
-  if (dev_malloc(&b.p, bytes) != hipSuccess) {
-    (void)hipGetLastError();
-    b.p = nullptr;
-    return nullptr;
-  }
+  if (dev_malloc(&b.p, bytes) != hipSuccess) return nullptr;
   b.cap = bytes;
   return b.p;
 }
@@ -523,6 +524,7 @@ static int ensure_act(sb_net *net, long rows) {
     if (L.act_rows >= rows) continue;
     SB_HIP(hipStreamSynchronize(g_ctx.stream));
     int rc = free_dev(L.act);
+    L.act_rows = 0;
     if (rc) return rc;
     SB_HIP(dev_malloc(&L.act, (size_t)rows * L.M * net->esize));
     L.act_rows = rows;
@@ -672,8 +674,6 @@ static int build_frozen_cache(sb_net *net, int upto, long maxB, long like) {
   // without the memory for both copies the caller goes on uncached (Hc_layer stays -1): not an error
   if (dev_malloc(&net->Hc, (size_t)Ns * Mo * sizeof(T)) != hipSuccess ||
       dev_malloc(&net->Hcp, (size_t)Ns * Mo * sizeof(T)) != hipSuccess) {
-    (void)hipGetLastError();
-    net->Hcp = nullptr;
     if (net->Hc) (void)hipFree(net->Hc);
     net->Hc = nullptr;
     return 0;

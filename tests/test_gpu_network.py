@@ -616,6 +616,28 @@ def test_state_written_is_on_the_device_when_the_call_returns():
         _capi.check(lib.sb_net_destroy(net))
 
 
+def test_a_layer_goes_on_after_an_allocation_that_failed():
+    """A batch whose activations (2 TiB) do not fit fails with a status; the next one of a size that did fit succeeds."""
+    import ctypes
+    from streambrain_amd import _capi
+    _capi.init()
+    lib, net = _capi.lib(), ctypes.c_void_p()
+    _capi.check(lib.sb_net_create(ctypes.byref(net), 0))
+    try:
+        H = Mc = 1024
+        assert lib.sb_net_add_dense_layer(net, 1, H, Mc, 0.01, 1.0, 1.0 / Mc, 1.0 / Mc) == 0
+        x, act = np.zeros(1 << 19, np.float32), np.zeros((4, H * Mc), np.float32)
+        _capi.check(lib.sb_net_layer_activation(net, 0, x.ctypes.data, 4, act.ctypes.data))
+        assert np.all(act == 1 / Mc)
+        # (nothing is written: the call ends at the allocation)
+        assert lib.sb_net_layer_activation(net, 0, x.ctypes.data, 1 << 19, act.ctypes.data) == -2, "SB_ERR_HIP"
+        act[:] = 0
+        _capi.check(lib.sb_net_layer_activation(net, 0, x.ctypes.data, 4, act.ctypes.data))
+        assert np.all(act == 1 / Mc)
+    finally:
+        _capi.check(lib.sb_net_destroy(net))
+
+
 def test_errors_are_python_exceptions(hb):
     net = hb.Network(np.float32)
     with pytest.raises(Exception):
