@@ -510,12 +510,13 @@ static int layer_free(Layer &L) {
 
 // Batch rows that one pass over the layers takes when nothing ties it to the caller's batch size (a sample's activations
 // do not depend on the others'): launches then have work for the whole chip and are few.  As many as keep the
-// widest activations within 64 MiB, a multiple of `unit`, at least one unit.
-constexpr size_t kPassBytes = (size_t)64 << 20;
+// widest activations within 64 MiB, a multiple of `unit`, at least one unit.  (And no more than the 2^32 threads of a
+// launch take: the kernels of narrow layers have 256 per row.)
+constexpr size_t kPassBytes = (size_t)64 << 20, kPassRows = (size_t)1 << 20;
 static long pass_rows(const sb_net *net, long unit) {
   long widest = 1;
   for (const auto &L : net->layers) widest = std::max(widest, L.M);
-  const long rows = (long)(kPassBytes / ((size_t)widest * net->esize)) / unit * unit;
+  const long rows = (long)std::min(kPassBytes / ((size_t)widest * net->esize), kPassRows) / unit * unit;
   return rows < unit ? unit : rows;
 }
 
@@ -530,6 +531,15 @@ static int ensure_act(sb_net *net, long rows) {
     L.act_rows = rows;
   }
   return 0;
+}
+
+// Activations for passes of `rows` rows, or, where the memory for those is not there, of `batch`, which the caller needs at
+// least.  Returns a negative status or 0; *got: which of the two.
+static int ensure_pass_act(sb_net *net, long rows, long batch, long *got) {
+  *got = rows;
+  if (ensure_act(net, rows) == 0) return 0;
+  *got = batch;
+  return ensure_act(net, batch);
 }
 
 // After W or wmask of a layer with row lists has been written from outside (a restored checkpoint, say),
@@ -678,8 +688,8 @@ static int build_frozen_cache(sb_net *net, int upto, long maxB, long like) {
     net->Hc = nullptr;
     return 0;
   }
-  const long pass = std::min(Ns, pass_rows(net, maxB));
-  if (upto > 0 && (rc = ensure_act(net, pass))) return rc;
+  long pass = std::min(Ns, pass_rows(net, maxB));
+  if (upto > 0 && (rc = ensure_pass_act(net, pass, std::min(Ns, maxB), &pass))) return rc;
   for (long lo = 0; lo < Ns; lo += pass) {
     const long B = lo + pass <= Ns ? pass : Ns - lo;
     const T *x = (const T *)net->X + lo * net->NF;
@@ -852,7 +862,7 @@ static int net_forward_batches(sb_net *net, const void *h_images, const void *h_
   long piece = ((long)HostStager::kChunkBytes / (long)(NF * sizeof(T))) / maxB * maxB;
   if (piece < maxB) piece = maxB;
   piece = std::min(piece, pass_rows(net, maxB));
-  if ((rc = ensure_act(net, std::min(piece, n)))) return rc;
+  if ((rc = ensure_pass_act(net, std::min(piece, n), std::min(maxB, n), &piece))) return rc;
   // Every row gets the bits of its batch: passes run like batches of maxB rows, and what is left of the set behind the
   // last whole batch runs on its own where a batch of that size takes other kernels.
   const long tail = n > maxB ? n % maxB : 0;
