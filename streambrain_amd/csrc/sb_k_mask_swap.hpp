@@ -6,10 +6,12 @@
 // and the 16 worst active rows of the state they start from (plus rows that changed sides on the way) can ever be
 // picked.  The kernel therefore works in rounds of 16 iterations:
 //   phase A (whole workgroup): the 16 best rows of either side in the strict order (score, row index), which is the
-//     order the picks take them in, equal scores included.  The rows are dealt into 64 bins by their index modulo
-//     64; the 16th largest of the 64 bins' best is a bound that at least 16 rows reach and few others do (about 3
-//     more where the order knows nothing of the index), the rows that reach it go to a list in LDS, and a
-//     row's place is the number of listed rows ahead of it;
+//     order the picks take them in, equal scores included.  The rows are dealt into 64 bins, a lane each; the 16th
+//     largest of the 64 bins' best is a bound that at least 16 rows reach and few others do (about 3
+//     more where the order knows nothing of the bins), the rows that reach it go to a list in LDS, and a
+//     row's place is the number of listed rows ahead of it.  The wavefronts deal their rows in orders of their own
+//     (row_at): by the index modulo 64 alone, images 64 pixels wide have whole columns in a bin, whose scores
+//     resemble each other, and the list overflows (24576 rows, floats: 57 us instead of 18);
 //   phase B (one wavefront, one candidate per lane and side): the iterations themselves, with the same picks, tie
 //     rule, break conditions and score expression as a full scan.
 // A round reads the N scores and sides twice (the second time from L2) and has seven barriers; its time is latency.
@@ -29,7 +31,6 @@ struct ScoreKey;
 template <>
 struct ScoreKey<float> {
   using K = uint32_t;
-  static constexpr int BITS = 32, PASSES = 2;
   static __device__ __forceinline__ K of(float s) {
     const uint32_t b = __float_as_uint(s + 0.0f);  // -0 and +0 compare equal, so they share a key
     return b ^ ((b >> 31) ? 0xffffffffu : 0x80000000u);
@@ -38,7 +39,6 @@ struct ScoreKey<float> {
 template <>
 struct ScoreKey<double> {
   using K = uint64_t;
-  static constexpr int BITS = 64, PASSES = 3;
   static __device__ __forceinline__ K of(double s) {
     const uint64_t b = (uint64_t)__double_as_longlong(s + 0.0);
     return b ^ ((b >> 63) ? ~0ull : (1ull << 63));
@@ -143,16 +143,23 @@ struct MaskSwap {
     int swaps;
   };
 
-  // This thread's rows i0 + tid, i0 + tid + NT, ..: scores and sides (2: no candidate, or no row), loads in flight
+  // This thread's first row among the NT * U from i0 on; the others follow NT apart.
+  static __device__ __forceinline__ int row_at(long i0) {
+    const unsigned tid = threadIdx.x;
+    return (int)(tid ^ ((4 * (tid >> 6) + 11 * (unsigned)(i0 >> 13)) & 63));
+  }
+  static_assert(NT * U == 1 << 13, "the shift above");
+  // This thread's rows among the NT * U from i0 on: scores and sides (2: no candidate, or no row), loads in flight
   // together.
   struct Rows {
     T s[U];
     int m[U];
   };
-  static __device__ __forceinline__ void load_rows(const MaskArgs<T> &a, Rows &v, int i0) {
+  static __device__ __forceinline__ void load_rows(const MaskArgs<T> &a, Rows &v, long i0) {
+    const int first = row_at(i0);
 #pragma unroll
     for (int u = 0; u < U; u++) {
-      const long i = (long)i0 + (int)threadIdx.x + NT * u;
+      const long i = i0 + first + NT * u;
       v.s[u] = a.score[i < a.N ? i : 0];
       v.m[u] = i < a.N ? a.side[i] : 2;
     }
@@ -161,14 +168,15 @@ struct MaskSwap {
   // `first`: the first NT * U rows, already loaded.  (No guards around the calls: what they hold is a few selects.)
   template <typename F>
   static __device__ __forceinline__ void for_rows(const MaskArgs<T> &a, const Rows &first, F &&f) {
-    const int tid = threadIdx.x;
+    const int r = row_at(0);
 #pragma unroll
-    for (int u = 0; u < U; u++) f(tid + NT * u, first.m[u], first.s[u]);
+    for (int u = 0; u < U; u++) f(r + NT * u, first.m[u], first.s[u]);
     for (long i0 = NT * U; i0 < a.N; i0 += NT * U) {
       Rows v;
-      load_rows(a, v, (int)i0);
+      load_rows(a, v, i0);
+      const int r = (int)i0 + row_at(i0);
 #pragma unroll
-      for (int u = 0; u < U; u++) f((int)i0 + tid + NT * u, v.m[u], v.s[u]);
+      for (int u = 0; u < U; u++) f(r + NT * u, v.m[u], v.s[u]);
     }
   }
   // in both groups the wanted rows are those with the LARGEST keys

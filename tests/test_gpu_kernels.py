@@ -3,6 +3,8 @@
 Tolerance (floating point): |gpu - ref| <= tol * max(|ref|, 1) with tol = 1e-5 (float32) and 1e-12
 (float64); masks, class labels and everything integer are compared bit for bit.
 """
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -448,6 +450,59 @@ def test_update_mask_rounds(k, oracle, dtype, N, iterations, kind):
     ref = oracle.update_mask(wmask.copy(), W, Ci, Cj, Cij, 0.01, H, Mc, 1, iterations)
     got = k.update_mask(wmask.copy(), W, Ci, Cj, Cij, 0.01, H, Mc, 1, iterations)
     assert np.array_equal(got, ref), f"masks differ in {(got != ref).sum()} entries"
+
+
+def _swap_bins(N):
+    """The bin that the preselection of the swap loop deals every row into."""
+    i = np.arange(N)
+    return (i & 63) ^ ((4 * (i >> 6 & 15) + 11 * (i >> 13)) & 63)
+
+
+@pytest.mark.parametrize("dtype", DT)
+@pytest.mark.parametrize("N", [24576, 27648])
+@pytest.mark.parametrize("iterations", [16, 20])
+@pytest.mark.parametrize("side", [1, -1])
+def test_update_mask_more_rows_beyond_the_bound_than_are_listed(k, oracle, dtype, N, iterations, side):
+    """The best (worst) rows all in eight of the 64 bins: 1500 and more of the side reach the bound, the list holds 1024,
+    and the iterations are left to full scans."""
+    rng = np.random.default_rng(N + iterations)
+    H, Mc = 2, 5
+    wmask, W, Ci, Cj, Cij = _mask_problem(rng, N, H, Mc, dtype, density=0.5)
+    W[_swap_bins(N) < 8] += 3 * side
+    ref = oracle.update_mask(wmask.copy(), W, Ci, Cj, Cij, 0.01, H, Mc, 1, iterations)
+    got = k.update_mask(wmask.copy(), W, Ci, Cj, Cij, 0.01, H, Mc, 1, iterations)
+    assert np.array_equal(got, ref), f"masks differ in {(got != ref).sum()} entries"
+
+
+@pytest.mark.parametrize("dtype", DT)
+@pytest.mark.parametrize("width", [32, 64, 96, 128])
+def test_update_mask_takes_no_longer_for_the_columns_of_an_image(k, oracle, dtype, width):
+    """Scores that go with the column of a pixel (the middle eighth of images 32 .. 128 pixels wide is the best): the
+    swap kernel takes as long as for the same rows in random order.  Measured by the library's own event brackets."""
+    from streambrain_amd import _capi
+    lib, N, H, Mc = _capi.lib(), 24576, 2, 5
+    rng = np.random.default_rng(width)
+    problem = _mask_problem(rng, N, H, Mc, dtype, density=0.5)
+    middle = np.abs(np.arange(N) % width - width // 2 + 0.5) < width / 16
+    problem[1][middle] += 3
+    order = rng.permutation(N)
+    swap = [n for n in range(lib.sb_profile_kernels()) if lib.sb_profile_kernel_name(n) == b"mask_swap"][0]
+    best = []
+    for rows in (np.arange(N), order):
+        wmask, W, Ci, Cj, Cij = (a if a is problem[3] else np.ascontiguousarray(a[rows]) for a in problem)
+        ref = oracle.update_mask(wmask.copy(), W, Ci, Cj, Cij, 0.01, H, Mc, 1, 16)
+        times = []
+        for _ in range(5):
+            ms, launches = ctypes.c_double(), ctypes.c_long()
+            _capi.check(lib.sb_profile_start())
+            got = k.update_mask(wmask.copy(), W, Ci, Cj, Cij, 0.01, H, Mc, 1, 16)
+            _capi.check(lib.sb_profile_stop())
+            _capi.check(lib.sb_profile_get(swap, ctypes.byref(ms), ctypes.byref(launches)))
+            assert launches.value == 1 and np.array_equal(got, ref)
+            times.append(ms.value)
+        best.append(min(times))
+    print(f"image {best[0] * 1e3:.1f} us, random order {best[1] * 1e3:.1f} us")
+    assert best[0] < 2 * best[1]  # (a scan per iteration takes ten times as long)
 
 
 @pytest.mark.parametrize("dtype", DT)
