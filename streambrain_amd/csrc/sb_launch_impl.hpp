@@ -325,20 +325,29 @@ int launch_softmax(hipStream_t st, T *act, long B, long H, long Mc) {
 template <typename T>
 static long train_tiles_of_one_round() { return (long)train_waves_per_simd<T, true, 1>() * device_cu_count(); }
 
-// Floats go through k_trace_sums<float, true> and k_train_split from two and a half rounds of 64 x 64 tiles on, with
-// batches of 32 rows, which leave the matrix cores little to do, from five.  Sums included, against k_train_fused on its
-// own, 3000 columns: batch 128, 2048 rows (1.2 rounds) 26.0 / 26.7 us, 4096 (2.4) 39.7 / 47.8, 8192 (4.7) 66 / 94, 16384
-// 110 / 257; batch 512, 8192 rows 141 / 239; batch 32, 8192 rows 54.6 / 53.5, 27648 255 / 369.  Between one round and the
-// line there are 15 % to gain, and the small layers below it, which train for epochs in moments, keep the rounding of
-// their trajectories (after a few dozen steps those tell one order of sums from another).
-// Batches of fewer than kSplitBatch rows stay with the float instructions, whose sums can be closer there (see
-// k_train_split).  Its windows hold 128 rows of Cij and 32 split batch rows.
+// Floats go through k_trace_sums<float, true> and k_train_split in layers of 2.5 rounds of 64 x 64 tiles and more where
+// that is faster, sums included (k_train_fused / k_train_split, whole steps, 1.0 and more in all 400 sizes tried
+// but for those named here):
+//   Cij and W beyond the memory-side cache: any batch (from 32 rows, see k_train_split: 12670 x 3000 1.7, 9306 x 4000 1.2,
+//   3800 x 10000 1.7; 64 rows 2.2, 1.2, 1.7; 300 rows 2.0, 1.6, 1.7).  In it the matrix instructions have to
+//   gain what the split costs: rows that are no whole number of 128-byte lines from 65 rows (77 rows, 4600 to 8700 x
+//   3000 0.99 to 1.06, 2929 columns 1.10 to 1.15; 64 rows 0.98 to 0.99 and 1.0), others from 97 (100 rows, 3440 to 6550 x
+//   4000 1.03 to 1.10, 128 rows 1.05 to 1.10; 77 rows 0.97 to 1.00, 33 rows 0.89 to 0.92);
+//   not for few columns, between which the split of x cannot be shared out: from 192 columns (200: 1.0 to 2.0, below 100
+//   MB or beyond 200 rows down to 0.95; 100 columns: 0.7 to 1.2), or from 640 where rows are whole lines (640: 0.94 at 700
+//   MB to 1.4; 320: 0.8 to 1.15), which k_train_fused writes at full rate.
+// The layers below the 2.5 rounds, which train for epochs in moments, keep the rounding of their trajectories (after a
+// few dozen steps those tell one order of sums from another); there are up to 15 % to gain there.
+// Its windows hold 128 rows of Cij and 32 split batch rows.
 template <typename T>
 size_t train_split_bytes(long B, long N, long H, long Mc) {
   if constexpr (sizeof(T) != 4) return 0;
   if (B < kSplitBatch || N <= 0 || H <= 0 || Mc <= 0) return 0;
   const long M = H * Mc;
-  if (M <= 32 || 2 * cdiv(N, 64) * cdiv(M, 64) < (B > 32 ? 5 : 10) * train_tiles_of_one_round<T>()) return 0;
+  const bool whole_lines = M % 32 == 0;
+  if (M < (whole_lines ? 640 : 192) || 2 * cdiv(N, 64) * cdiv(M, 64) < 5 * train_tiles_of_one_round<T>()) return 0;
+  const bool cached = 2 * N * M * (long)sizeof(T) <= (256L << 20);
+  if (cached && B <= (whole_lines ? 96 : 64)) return 0;
   const long xw = cdiv(N, kSplitTileI) * kSplitTileI, yw = cdiv(M, kSplitTileJ) * kSplitTileJ;
   const long wider = xw > yw ? xw : yw;
   if (128 * M * 4 >= (1L << 31) || wider * (kSplitRows / 8) * 3 * 16 >= (1L << 31)) return 0;
@@ -443,6 +452,9 @@ int launch_train_fused(hipStream_t st, const T *x, const T *y, T *Cij, T *W, con
       sp.y_odd = sp.x_odd + sp.x_width / 64;
       a.tiles_i = cdiv(N, kSplitTileI);
       a.tiles_j = cdiv(M, kSplitTileJ);
+      // (always in panels: column by column the split batch of x, six bytes a value, does not stay in an L2: 5570 x 4000,
+      // batch 100, 1.25 times the time)
+      a.panel_cols = wide_panels ? 16u : 8u;
       a.by_panel = FastDiv::of(a.tiles_i * a.panel_cols);
       launch(k_trace_sums<T, true>, sums, true, false, sp);
       const dim3 tiles((unsigned)(a.tiles_i * a.tiles_j) + a.prefetch_groups);
@@ -456,17 +468,19 @@ int launch_train_fused(hipStream_t st, const T *x, const T *y, T *Cij, T *W, con
   // Every tile adds up the batch's x and y columns for its own rows and columns, which with many tile
   // rows and columns is most of the kernel's vector arithmetic (43 % at 65536 x 100000, batch 1024).
   // From one and a half rounds of workgroups on (floats with more than 32 rows; doubles: two and a half), a small launch
-  // computes the new traces once and the tiles read them (floats: only where k_train_split has no scratch).  Timed, 4096 inputs, batch 128, floats, with / without that
+  // computes the new traces once and the tiles read them (floats: where k_train_split does not run).  Timed, 4096 inputs, batch 128, floats, with / without that
   // launch: 23.7 / 22.5 us at 1.05 rounds, 29.3 / 29.9 at 1.5, 34.6 / 35.6 at 2, 45.5 / 48.5 at 3, 67.1 / 69.2
   // at 5; doubles: 48.1 / 47.3 at 1.6 rounds, 55.8 / 54.3 at 2, 110.3 / 113.7 at 2.5.
   const long ntiles = a.tiles_i * a.tiles_j;
   const bool one_round = ntiles <= train_tiles_of_one_round<T>();
   const long pre_from = sizeof(T) == 8 ? 5 * 4 : 3 * 5;  // in half workgroups per CU
   if constexpr (sizeof(T) == 8) {
-    // Cij and W together beyond what the 256 MB memory-side cache keeps: non-temporal stores (batch 128, rows of 3000
-    // doubles, whole steps: 8000 rows, 384 MB, 366 us written through, 218 us non-temporal; 20000 rows 1364 / 626;
-    // rows of whole cache lines, 1568 x 10000, 414 / 411; odd rows, 5000 x 9999, batch 77, 806 / 643)
-    if (2 * N * M * (long)sizeof(T) > (192L << 20) && (!vec || one_byte)) {
+    // Cij and W together beyond what the memory-side cache keeps: non-temporal stores (whole steps, batch 128, written
+    // through / non-temporal: 7208 x 3000, 330 MiB, 190 / 141 us, 9174 x 3000, 420 MiB, 238 / 180, 20000 rows
+    // 1364 / 626; rows of whole cache lines, 10000 columns, batch 512, 239 MiB 412 / 407, batch 128, 420 MiB 190 / 177;
+    // time written through over time non-temporal between batches of 16 and 300: at 220 MiB 0.9 to 1.1, at 235
+    // 0.95 to 1.4, at 265 1.0 to 1.6)
+    if (2 * N * M * (long)sizeof(T) > (230L << 20) && (!vec || one_byte)) {
       if (vec) {
         launch(k_trace_sums<T>, sums, true, false, SplitBatch{});
         launch(k_train_fused<T, KCH, true, 1, true, false, true>, grid, false, true);

@@ -534,13 +534,15 @@ def test_plastic_train_step(k, oracle, dtype, B, N, H, Mc, h):
     _check_plastic_train_step(k, oracle, dtype, B, N, H, Mc, h, np.random.default_rng(B + N + H + Mc))
 
 
-# 64 x 64 tiles of these layers: 3200 and more with more than 32 rows, 6400 and more below, which is where the pass
-# goes over to bfloat16 pieces
+# Layers of 3200 and more tiles of 64 x 64 go over to bfloat16 pieces with more than 64 or 96 batch rows (rows of Cij that
+# are no whole number of 128-byte lines, or are), beyond 256 MiB of Cij and W from 32 rows on.
 @pytest.mark.parametrize("B,N,H,Mc,masked", [
     (1, 8200, 33, 100, True), (31, 8193, 50, 66, False), (32, 8257, 33, 101, True),
     *[(B, *s) for B in (33, 64, 65, 257) for s in ((4353, 30, 100, True), (6464, 32, 64, False), (4160, 48, 66, True),
                                                    (4737, 29, 101, True), (9985, 331, 4, True))],
-    (63, 4353, 30, 100, True), (128, 4737, 29, 101, False)])
+    (63, 4353, 30, 100, True), (128, 4737, 29, 101, False), (96, 6464, 32, 64, False), (97, 6465, 32, 64, True),
+    (66, 65601, 3, 67, False), (97, 20481, 10, 64, True),
+    (32, 11585, 29, 101, True), (33, 11200, 30, 100, True), (63, 8257, 65, 64, False), (64, 16577, 10, 203, True)])
 def test_train_pass_of_big_float_layers(k, B, N, H, Mc, masked):
     """Tile remainders on either side, batch remainders, values over 40 binary orders of magnitude, and values out of
     the range of the bfloat16 pieces (1e30, infinity), which only the tiles that hold them treat differently."""
@@ -579,7 +581,7 @@ def test_train_pass_of_big_float_layers(k, B, N, H, Mc, masked):
 def test_products_of_big_float_layers_are_as_exact_as_floats(k, B, equal_rows):
     """x^T y alone (traces of zero, taupdt 1, a batch that is a power of two: no other rounding), with the values whose
     last bits the pieces of a float lose most of, in batches that do not average that out."""
-    N, H, Mc, f = 8192, 50, 64, np.float32  # 6400 tiles of 64 x 64
+    N, H, Mc, f = 8192, 65, 64, np.float32  # 260 MiB of Cij and W
     M, rng = H * Mc, np.random.default_rng(B)
     values = np.array([1 + 2 ** -7 - 2 ** -16, 1.0038986, 1 + 2 ** -8 - 2 ** -17, 1 + 2 ** -9 + 2 ** -23], f)
     x, y = (1 + rng.random((1 if equal_rows else B, n), dtype=f) for n in (N, M))
@@ -604,7 +606,7 @@ def test_products_of_big_float_layers_are_as_exact_as_floats(k, B, equal_rows):
 def test_products_of_big_float_layers_keep_the_bits_of_small_numbers(k, magnitudes):
     """x^T y alone, with x and y anywhere in the range of floats: down to the smallest one, and up to where the pieces'
     range ends and beyond."""
-    B, N, H, Mc, f = 32, 8192, 50, 64, np.float32
+    B, N, H, Mc, f = 32, 8192, 65, 64, np.float32
     M, rng = H * Mc, np.random.default_rng(7)
     x, y = (((1 + rng.random((B, n))) * m).astype(f) for n, m in zip((N, M), magnitudes))
     st = {"weights": np.zeros((N, M), f), "bias": np.zeros(M, f), "kbi": np.ones(M, f), "Ci": np.ones(N, f),

@@ -59,7 +59,7 @@ def test_noalloc_update_weights_matches_the_allocating_entry_point(oracle):
         assert np.max(np.abs(got[3] - o[3]) / np.maximum(np.abs(o[3]), 1)) <= 1e-5
 
 
-@pytest.mark.parametrize("B,N,M", [(64, 4353, 3000), (33, 6464, 2049)])
+@pytest.mark.parametrize("B,N,M", [(128, 4353, 3000), (100, 6464, 2049)])
 def test_noalloc_update_weights_matches_the_allocating_entry_point_for_big_layers(B, N, M):
     """Layers of 3200 and more tiles of 64 x 64, for which the library has a second kernel that wants scratch."""
     from streambrain_amd import _capi
