@@ -620,6 +620,80 @@ def test_products_of_big_float_layers_keep_the_bits_of_small_numbers(k, magnitud
     assert off <= bound, f"{off * 2 ** 24:.2f} 2^-24"
 
 
+@pytest.mark.parametrize("B,N,H,Mc", [(33, 1600, 33, 303), (16, 5209, 30, 101), (20, 160001, 1, 101)])
+def test_train_pass_of_big_double_layers_with_odd_rows(k, B, N, H, Mc):
+    """Cij and W beyond what the memory-side cache keeps, rows that are no whole number of vectors: the pass with
+    non-temporal stores, element by element at the ends of the rows."""
+    M, rng = H * Mc, np.random.default_rng(B)
+    assert 2 * N * M * 8 > 230 << 20
+    x, y = rng.random((B, N)) * (rng.random((B, N)) < 0.7), rng.random((B, M))
+    st = {"weights": np.ones((N, M)), "bias": np.zeros(M), "kbi": np.ones(M), "Ci": rng.random(N), "Cj": rng.random(M),
+          "Cij": rng.random((N, M)), "wmask": (rng.random((N, H)) < 0.5).astype(np.uint8)}
+    t = 0.1
+    got = k.plastic_train_step(st, x, y, H, Mc, t, -139.0, 0.062, 0.022, hypercolumn=None)
+    ci, cj = (1 - t) * st["Ci"] + t * x.mean(0), (1 - t) * st["Cj"] + t * y.mean(0)
+    cij = (1 - t) * st["Cij"] + t * (x.T @ y) / B
+    assert_close(got["Ci"], ci, np.float64, "Ci")
+    assert_close(got["Cj"], cj, np.float64, "Cj")
+    assert_close(got["Cij"], cij, np.float64, "Cij")
+    w = np.where((ci < t / 2)[:, None] | (cj < t / 2)[None], 0, np.log(np.maximum(cij, (t / 2) ** 4) / (ci[:, None] * cj)))
+    assert_close(got["weights"], w * np.repeat(st["wmask"], Mc, axis=1), np.float64, "W")
+
+
+def test_captured_train_step_does_without_the_scratch_that_later_calls_replace(k):
+    """A big float step recorded into a graph takes the kernels that need no optional scratch: it allocates nothing, and
+    its replays give the eager result, also after an eager call has grown, and so moved, the scratch."""
+    from streambrain_amd import _capi
+    from streambrain_amd._capi import DeviceArray, check
+    lib, f = _capi.lib(), np.float32
+    hip = ctypes.CDLL(_capi.LIB_PATH)  # (symbols of the runtime that the library is linked with)
+    P, I = ctypes.c_void_p, ctypes.c_int
+    for name, args in (("hipStreamBeginCapture", [P, I]), ("hipStreamEndCapture", [P, ctypes.POINTER(P)]),
+                       ("hipGraphInstantiate", [ctypes.POINTER(P), P, P, P, ctypes.c_size_t]), ("hipGraphLaunch", [P, P]),
+                       ("hipGraphExecDestroy", [P]), ("hipGraphDestroy", [P])):
+        getattr(hip, name).argtypes, getattr(hip, name).restype = args, I
+    N, H, Mc, big = 4353, 30, 100, 256
+    M, rng = H * Mc, np.random.default_rng(3)
+    names = ("weights", "bias", "Ci", "Cj", "Cij", "kbi", "wmask")
+    st = {"weights": np.zeros((N, M), f), "bias": np.zeros(M, f), "kbi": np.ones(M, f), "Ci": rng.random(N).astype(f),
+          "Cj": rng.random(M).astype(f), "Cij": rng.random((N, M)).astype(f),
+          "wmask": (rng.random((N, H)) < 0.5).astype(np.uint8)}
+    dev = {n: DeviceArray.from_numpy(st[n]) for n in names}
+    x, y = (DeviceArray.from_numpy(rng.random((big, n)).astype(f)) for n in (N, M))
+
+    def step(B):
+        check(lib.sb_plastic_train_step_f32(*(dev[n].ptr for n in names), x.ptr, y.ptr, B, N, H, Mc, 0.1, -139.0, 0.062,
+                                            0.022, -1))
+
+    def reset():
+        for n in names:
+            check(lib.sb_memcpy_h2d(dev[n].ptr, st[n].ctypes.data, st[n].nbytes))
+
+    step(128)
+    check(lib.sb_sync())
+    eager = {n: dev[n].numpy() for n in names}
+    stream, graph, run = lib.sb_stream(), P(), P()
+    reset()
+    before = lib.sb_allocation_calls()
+    assert hip.hipStreamBeginCapture(stream, 1) == 0  # (thread-local mode)
+    step(128)
+    assert hip.hipStreamEndCapture(stream, ctypes.byref(graph)) == 0
+    assert lib.sb_allocation_calls() == before
+    assert hip.hipGraphInstantiate(ctypes.byref(run), graph, None, None, 0) == 0
+    replays = []
+    for k_ in range(3):
+        reset()
+        assert hip.hipGraphLaunch(run, stream) == 0
+        check(lib.sb_sync())
+        replays.append({n: dev[n].numpy() for n in names})
+        for n in names:
+            assert_close(replays[-1][n], eager[n], f, n)
+            assert np.array_equal(replays[-1][n], replays[0][n]), n
+        step(128 if k_ else big)  # the scratch grows to twice its size
+        check(lib.sb_sync())
+    assert hip.hipGraphExecDestroy(run) == 0 and hip.hipGraphDestroy(graph) == 0
+
+
 @pytest.mark.parametrize("dtype", DT)
 @pytest.mark.parametrize("B", [1, 16, 33])
 @pytest.mark.parametrize("N", [2048, 4113])

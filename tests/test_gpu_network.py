@@ -638,6 +638,36 @@ def test_a_layer_goes_on_after_an_allocation_that_failed():
         _capi.check(lib.sb_net_destroy(net))
 
 
+def test_state_of_two_networks_from_two_threads():
+    """The pinned ring that state goes through is one for all networks: small arrays (moved by a kernel) and big ones (by
+    the copy engine, in pieces) of two networks, written and read back by a thread each, keep apart."""
+    import ctypes
+    import threading
+    from streambrain_amd import _capi
+    _capi.init()
+    lib, results = _capi.lib(), []
+
+    def work(seed):
+        rng, net = np.random.default_rng(seed), ctypes.c_void_p()
+        _capi.check(lib.sb_net_create(ctypes.byref(net), 0))
+        N, M = 2048 + 100 * seed, 1500
+        assert lib.sb_net_add_dense_layer(net, N, 1, M, 0.01, 1.0, 1.0 / M, 1.0 / M) == 0
+        for _ in range(8):
+            for name, shape in ((b"bias", M), (b"weights", (N, M)), (b"Ci", N), (b"Cij", (N, M))):
+                a, back = rng.random(shape, dtype=np.float32), np.zeros(shape, np.float32)
+                _capi.check(lib.sb_net_set_layer_state(net, 0, name, a.ctypes.data, a.nbytes))
+                _capi.check(lib.sb_net_get_layer_state(net, 0, name, back.ctypes.data, back.nbytes))
+                results.append((seed, name, np.array_equal(a, back)))
+        _capi.check(lib.sb_net_destroy(net))
+
+    threads = [threading.Thread(target=work, args=(seed,)) for seed in (1, 2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert len(results) == 2 * 8 * 4 and all(same for _, _, same in results), results
+
+
 def test_errors_are_python_exceptions(hb):
     net = hb.Network(np.float32)
     with pytest.raises(Exception):
