@@ -47,7 +47,7 @@ N_PIXELS, H, MC, N_OUT, BATCH, N_SAMPLES = 784, 30, 100, 10, 128, 60000
 HP = dict(l1_taupdt=0.006908854922437549, l1_pmin=0.06195283356566607, l1_khalf=-139.02586632856327,
           l1_taubdt=0.02218100432360414, l1_density=0.1, l2_taupdt=0.0007449780036161324)
 HBM_PEAK_GBS = 8000.0
-MFMA_PEAK_TFLOPS = {"f32": 157.3, "f64": 78.6}
+MFMA_PEAK_TFLOPS = {"f32": 157.3, "f64": 78.6, "bf16": 2500.0}
 PMC_PROFILE = os.path.join(ROOT, "profiles", "k_train_fused_mnist_f32_b128_pmc.txt")
 KERNEL_SOURCES = ("sb_k_train.hpp", "sb_common.hpp")
 
@@ -520,6 +520,15 @@ def large_cpu_baseline(name, x, wmask):
                         rewire_period=0, warm=not big)
 
 
+def splits_floats(dname, n, m, batch):
+    """Whether the training pass of such a layer runs on the bfloat16 matrix cores (k_train_split): the launcher's rule
+    (train_split_bytes in sb_launch_impl.hpp), for the 256 compute units of the card."""
+    whole_lines = m % 32 == 0
+    if dname != "f32" or batch < 32 or m < (640 if whole_lines else 192) or 2 * -(-n // 64) * -(-m // 64) < 5 * 1280:
+        return False
+    return 8 * n * m > 256 << 20 or batch > (96 if whole_lines else 64)
+
+
 def large_workload(name, steps, warmup, with_cpu=True):
     """Training steps of one structural-plasticity layer of a LARGE shape; returns the result line."""
     from streambrain_amd import _capi
@@ -581,21 +590,24 @@ def large_workload(name, steps, warmup, with_cpu=True):
     gemm = 2.0 * batch * n * m  # the Cij trace GEMM of a full batch
     fwd_flops = 2.0 * batch * connected * mc if cfg["density"] <= 0.5 else gemm
     stream_bytes = 3 * es * n * m
-    # which roof bounds the fused kernel: its GEMM at the MFMA peak against its 3 s N M stream at the HBM peak
-    # (against the peak of the element type's own instructions; big float layers do it on the bfloat16 cores)
-    mfma_bound = gemm / (peak * 1e12) >= stream_bytes / (HBM_PEAK_GBS * 1e9)
-    split = dname == "f32" and 2 * -(-n // 64) * -(-m // 64) >= 5 * 1280  # (batches of more than 32 rows)
-    train_kernel = "k_train_split" if split else "k_train_fused"
+    # which roof bounds the training kernel: its GEMM at the peak of the instructions that do it (big float layers: six
+    # bfloat16 products for every float one) against its 3 s N M stream at the HBM peak
+    split = splits_floats(dname, n, m, batch)
+    train_kernel, train_type = ("k_train_split", "bf16") if split else ("k_train_fused", dname)
+    train_flops, train_peak = (6 * gemm if split else gemm), MFMA_PEAK_TFLOPS[train_type]
+    mfma_bound = train_flops / (train_peak * 1e12) >= stream_bytes / (HBM_PEAK_GBS * 1e9)
     if mfma_bound:
-        roofline = {"bound": "mfma", "kernel": train_kernel, "achieved": gemm / tw / 1e12, "peak": peak,
-                    "unit": "TFLOP/s", "frac": gemm / tw / 1e12 / peak, "traffic": None,
-                    "algorithmic_flops_per_launch": gemm, "avg_launch_us": tw * 1e6,
+        roofline = {"bound": "mfma", "kernel": train_kernel, "achieved": train_flops / tw / 1e12, "peak": train_peak,
+                    "unit": "TFLOP/s", "frac": train_flops / tw / 1e12 / train_peak, "traffic": None,
+                    "instructions": train_type, "flops_per_launch": train_flops, "algorithmic_flops_per_launch": gemm,
+                    "avg_launch_us": tw * 1e6,
                     "bytes_3sNM_per_launch": stream_bytes, "achieved_GBps_on_3sNM": stream_bytes / tw / 1e9}
     else:
         roofline = {"bound": "hbm", "kernel": train_kernel, "achieved": stream_bytes / tw / 1e9,
                     "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": stream_bytes / tw / 1e9 / HBM_PEAK_GBS,
                     "traffic": None, "algorithmic_bytes_per_launch": stream_bytes, "avg_launch_us": tw * 1e6,
-                    "trace_gemm_tflops": gemm / tw / 1e12, "trace_gemm_frac_of_mfma_peak": gemm / tw / 1e12 / peak}
+                    "instructions": train_type, "trace_gemm_tflops": gemm / tw / 1e12,
+                    "trace_gemm_frac_of_mfma_peak": train_flops / tw / 1e12 / train_peak}
     return {
         "metric": "train samples/sec on 1 MI355X; % HBM / MFMA peak",
         "value": samples / dt_s, "unit": "samples/s", "n_gpus": 1, "steps": steps, "warmup": warmup,

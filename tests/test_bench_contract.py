@@ -82,3 +82,15 @@ def test_bracket_calibration_leaves_carried_events_alone():
     # a profiler that slows the bracketed pass down: no more than an empty bracket is taken off
     us = bench.calibrate_brackets(kernels, raw_ms + 1.0, 100, 100 * 22.5e-6, upper_us=4.4)
     assert us == 4.4 and abs(kernels["forward"]["avg_us"] - 4.6) < 1e-9
+
+
+def test_kernel_named_for_the_big_layers_follows_the_launcher():
+    """bench.py's restatement of the rule by which the launcher takes the split pass, at both sides of its lines."""
+    import bench
+    assert bench.splits_floats("f32", 55296, 20000, 256) and bench.splits_floats("f32", 65536, 100000, 1024)
+    assert not bench.splits_floats("f32", 1568, 3000, 128) and not bench.splits_floats("f64", 55296, 20000, 256)
+    assert not bench.splits_floats("f32", 55296, 20000, 31)
+    for m, line in ((3000, 64), (3008, 96)):  # (in the memory-side cache)
+        assert bench.splits_floats("f32", 5000, m, line + 1) and not bench.splits_floats("f32", 5000, m, line)
+        assert bench.splits_floats("f32", 27648, m, 32)
+    assert bench.splits_floats("f32", 200000, 200, 128) and not bench.splits_floats("f32", 200000, 320, 128)
