@@ -117,8 +117,9 @@ int launch_forward_classify(hipStream_t st, T *act, const T *x, const T *W, cons
     const bool vec = base_vec && (Mc % VW == 0);
     // Hypercolumns of two column groups whose tiles leave half the CUs idle and that have a long reduction: a
     // workgroup per group, then the softmax.  Every sum as in the fused kernel, except in the four columns that
-    // it takes as 4x4 products, so not those (whole steps:
-    // 10000 -> 20 x 101, batch 32, 179 us fused, 156 us this way; doubles 20000 -> 3 x 100, batch 77, 386 / 254).
+    // it takes as 4x4 products, so not those.  (Time fused over time this way, 120 tiles: 101 columns, 512 inputs
+    // 0.93, 1024 1.13, 2048 1.34, 4096 1.40; doubles, 50 columns 0.92, 1.07, 1.18, 1.27.  2048 inputs, 160 tiles 1.29 and
+    // 1.17, 240 tiles, where a CU gets two of these workgroups, 0.76 and 0.68.  The second launch costs 1 to 2 us.)
     const bool tail4 = sizeof(T) == 4 && vec && Mc == 100;
     if (need == 2 && 2 * fused_tiles <= cus_ && N >= 2048 && !tail4) {
       a.col_tiles = cdiv(M, GW);
@@ -173,7 +174,8 @@ int launch_forward_classify(hipStream_t st, T *act, const T *x, const T *W, cons
     if (need <= 4) return forward_variant<T, 4, true>(st, a, vec);
     if constexpr (sizeof(T) == 8) return forward_variant<T, 7, true>(st, a, vec);
   }
-  // tiles of two column groups, of one where the former leave half the CUs idle
+  // Tiles of two column groups, of one where the former leave half the CUs idle (time of two over time of one, 5 to 128
+  // tiles: 64 inputs 1.0 to 1.1, 200 1.3, 300 1.4, 1000 1.55; doubles 1.0, 1.25, 1.3, 1.5; at 192 tiles 0.75 to 0.9 for all)
   const bool narrow = 2 * cdiv(M, 2 * GW) * cdiv(B, 16) <= cus_;
   a.col_tiles = cdiv(M, narrow ? GW : 2 * GW);
   int rc = narrow ? forward_variant<T, 1, false>(st, a, base_vec) : forward_variant<T, 2, false>(st, a, base_vec);
@@ -283,7 +285,10 @@ int launch_forward_rows(hipStream_t st, T *act, const T *x, const T *W, const T 
   SB_REQUIRE(forward_rows_supported<T>(W, N, H, Mc), "shape not supported by the row-list forward kernel");
   ForwardRowsArgs<T> a{{act, x, W, bias, B, N, H * Mc, Mc, H, cdiv(B, 16), {}}, rows, row_cnt, cap, x_blocked};
   // Wide hypercolumns, few of them and long lists: a workgroup per column group, then the softmax, every sum as in
-  // the fused kernel (27648 -> 15 x 200, lists of 15800, batch 128, 120 tiles: 286 us fused, 249 + 5 us this way, whole steps 516 and 480 us).
+  // the fused kernel (27648 -> 15 x 200, lists of 15800, batch 128, 120 tiles: 286 us fused, 249 + 5 us this way).
+  // Time fused over time this way, at 2 / 120 / 160 tiles: 100 columns, lists of 512 0.96 / 0.94 / 0.71, of 1024 1.07 /
+  // 1.08 / 0.72, of 8192 1.40 / 1.38 / 0.76; 200 columns 1.45 / 1.05 / 0.78, 1.75 / 1.12 / 0.80, 2.28 / 1.28 / 0.80; doubles,
+  // 48 columns, lists of 512 0.94 / 0.91 / 0.80, of 1024 1.09 / 1.07 / 0.87, 200 columns, of 2048 2.8 / 1.2 / 1.07 (240: 0.79).
   constexpr int GW1 = 16 * Real<T>::VW;
   if (Mc > GW1 && 5 * H * cdiv(B, 16) <= 3L * device_cu_count() && cap >= 1024) {
     ProfScope prof_(st, K_FORWARD);
