@@ -366,10 +366,12 @@ static void *optional_scratch(Reusable &b, size_t bytes) {
   b.cap = bytes;
   return b.p;
 }
-// ... of the per-kernel entry points.  Whoever launches kernels that meet in it (or in the context's trace scratch) holds
+// ... of the per-kernel entry points, kept until sb_shutdown, so of a bounded size: calls that ask for more do without
+// (a batch of 1024 for 65536 x 100000 synapses takes 0.95 GiB).  Whoever launches kernels that meet in it (or in the context's trace scratch) holds
 // the lock until all of them are in the stream, so that calls from several threads do not interleave.
 static Reusable g_work;
 static std::mutex g_work_mutex;
+constexpr size_t kWorkLimit = (size_t)1 << 30;
 
 // Per-kernel entry points keep the reference's in-place contract: the fused kernel writes the new
 // Ci / Cj into scratch, which is then copied over the caller's arrays.
@@ -389,9 +391,10 @@ static int train_in_place(const T *x, const T *y, T *Cij, T *W, T *Ci, T *Cj, co
   if (rc) return rc;
   T *ci_next = fixed_scratch ? fixed_scratch : (T *)g_ctx.trace_next, *cj_next = ci_next + N;
   const bool as_noalloc = !wmask && N + M <= (long)SB_NOALLOC_MAX_UNITS;
+  const size_t split = train_split_bytes<T>(B, N, H, Mc);
   rc = launch_train_fused<T>(st, x, y, Cij, W, Ci, Cj, ci_next, cj_next, wmask, bias_mode, bias, kbi, B,
                              N, H, Mc, taupdt, cthr, khalf, pmin, taubdt, false, nullptr, 0,
-                             as_noalloc ? nullptr : optional_scratch(g_work, train_split_bytes<T>(B, N, H, Mc)));
+                             as_noalloc || split > kWorkLimit ? nullptr : optional_scratch(g_work, split));
   if (rc) return rc;
   return launch_copy_pair<T>(st, Ci, ci_next, (size_t)N, Cj, cj_next, (size_t)M);
 }

@@ -620,6 +620,33 @@ def test_products_of_big_float_layers_keep_the_bits_of_small_numbers(k, magnitud
     assert off <= bound, f"{off * 2 ** 24:.2f} 2^-24"
 
 
+def test_scratch_kept_for_the_entry_points_is_bounded(k):
+    """A batch that would keep more than 1 GiB of scratch until sb_shutdown goes by the kernels that need none: nothing is
+    allocated, and the traces are those of a batch of ones and halves."""
+    from streambrain_amd import _capi
+    from streambrain_amd._capi import DeviceArray, check
+    lib, f = _capi.lib(), np.float32
+    B, N, M = 2560, 102400, 201
+    dev = {n: DeviceArray(s, f) for n, s in dict(W=(N, M), b=(M,), Ci=(N,), Cj=(M,), Cij=(N, M), kbi=(M,), x=(B, N),
+                                                y=(B, M)).items()}
+    mask = DeviceArray((N, 1), np.uint8)
+    for d in (*dev.values(), mask):
+        check(lib.sb_fill_bytes(d.ptr, 0, d.nbytes))
+    ones, halves = np.ones((B, N), f), np.full((B, M), 0.5, f)
+    check(lib.sb_memcpy_h2d(dev["x"].ptr, ones.ctypes.data, ones.nbytes))
+    check(lib.sb_memcpy_h2d(dev["y"].ptr, halves.ctypes.data, halves.nbytes))
+
+    def step(B):
+        check(lib.sb_plastic_train_step_f32(dev["W"].ptr, dev["b"].ptr, dev["Ci"].ptr, dev["Cj"].ptr, dev["Cij"].ptr,
+                                            dev["kbi"].ptr, mask.ptr, dev["x"].ptr, dev["y"].ptr, B, N, 1, M, 1.0, -139.0,
+                                            0.062, 0.022, -1))
+    step(16)  # (the new traces have their scratch)
+    before = lib.sb_allocation_calls()
+    step(B)
+    assert lib.sb_allocation_calls() == before
+    assert np.all(dev["Ci"].numpy() == 1) and np.all(dev["Cj"].numpy() == 0.5) and np.all(dev["Cij"].numpy() == 0.5)
+
+
 @pytest.mark.parametrize("B,N,H,Mc", [(33, 1600, 33, 303), (16, 5209, 30, 101), (20, 160001, 1, 101)])
 def test_train_pass_of_big_double_layers_with_odd_rows(k, B, N, H, Mc):
     """Cij and W beyond what the memory-side cache keeps, rows that are no whole number of vectors: the pass with
