@@ -134,11 +134,11 @@ __device__ __forceinline__ unsigned tile_of_workgroup(const TrainArgs<T> &a, uns
 
 // ---- a float as three bfloat16: kSplitScale x = h + m + l exactly.  h holds the leading 8 bits, rounded to nearest, so
 // that m, the next 8 bits, is at most 2^-8 of x's leading bit, and l, the rest, at most 2^-17 of it.  The scale keeps
-// every bit of the smallest float, 2^-149, inside the normal bfloat16 (from 2^-126; without it, l of numbers below 2^-110
-// was lost: at 2^-122, 2^-14 of the product); it is taken off the finished sums again.  For |x| below kSplitLimit, so
-// that neither h nor the sums overflow (2^108 each product): products of larger numbers, infinities and NaN are not
-// what the products of their pieces add up to.
-constexpr float kSplitScale = 0x1p24f, kSplitLimit = 0x1p30f;
+// every bit of the smallest float, 2^-149, inside the normal bfloat16 (from 2^-126; without it, l of numbers below
+// 2^-110 was lost: at 2^-122, 2^-14 of the product); the factor of the finished sums, tau / B, takes it off again.  For
+// |x| below kSplitLimit, so that neither h nor the sums overflow (2^108 each product): products of larger numbers,
+// infinities and NaN are not what the products of their pieces add up to.
+constexpr float kSplitScale = 0x1p24f, kSplitLimit = 0x1p30f, kSplitUnscale = 1.0f / (kSplitScale * kSplitScale);
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 struct Split8 {  // eight consecutive batch rows of one column
   bf16x8 h, m, l;
@@ -712,12 +712,13 @@ void k_train_fused(TrainArgs<T> a) {
 // The fused pass for big float layers: Cij and W as k_train_fused writes them, with x^T y on the bfloat16 matrix
 // cores, which multiply sixteen times as fast as the float ones.  Both operands are split exactly into three bfloat16
 // (SplitBatch, written by k_trace_sums<float, true>, which also leaves the new traces), and the six products down to
-// 2^-17 are accumulated in float: h h + h m + m h + h l + l h + m m.  What is left out, m l + l m + l l, is at most 2^-24
-// of a product, and an accumulator is rounded (cut off, rather) six times per 32 batch rows instead of 32.  Off the exact sums, measured
-// in units of 2^-24 (at worst / rms; in brackets the float instructions): 32 rows, equal ones 2.0 / 0.5 (8.5 / 3.4),
-// random ones 1.4 / 0.6 (7.3 / 1.5), values over 30 binary orders 7.7 / 1.2 (10.9 / 1.3); 128 rows 23 / 3.3 (32 / 13.7),
-// 9.8 / 1.9 (15.8 / 2.9), 14.6 / 2.0 (19.5 / 2.6).  Over many orders the float instructions are ahead below 32
-// rows (16: 6.9 / 1.18 against 8.7 / 1.00, 8: 7.2 / 1.19 against 5.8 / 0.78), so smaller batches stay with k_train_fused.
+// 2^-17 are accumulated in float: h h + h m + m h + h l + l h + m m.  What is left out, m l + l m + l l, is at most
+// 2^-24 of a product, and an accumulator is rounded (cut off, rather) six times per 32 batch rows instead of 32.
+// Off the exact sums, measured in units of 2^-24 (at worst / rms; in brackets the float instructions): 32 rows, equal
+// ones 2.0 / 0.5 (8.5 / 3.4), random ones 1.4 / 0.6 (7.3 / 1.5), values over 30 binary orders 7.7 / 1.2 (10.9 / 1.3); 128
+// rows 23 / 3.3 (32 / 13.7), 9.8 / 1.9 (15.8 / 2.9), 14.6 / 2.0 (19.5 / 2.6).  Over many orders the float instructions are
+// ahead below 32 rows (16: 6.9 / 1.18 against 8.7 / 1.00, 8: 7.2 / 1.19 against 5.8 / 0.78), so smaller batches stay with
+// k_train_fused.
 // Bound: Cij read and written once, W written once, against 6 x 2 B N M flops on the matrix cores; with the float
 // instructions those were 2 B N M at a sixteenth of the rate, which is what k_train_fused waits for here.
 // A workgroup (4 wavefronts) owns a tile of 128 x 64, a wavefront 32 rows of it: 2 x 4 blocks of 16 x 16, so
@@ -866,13 +867,10 @@ void k_train_split(TrainArgs<float> a, SplitBatch sp) {
     __syncthreads();
     request_tile();
     multiply();
-#pragma unroll
-    for (int r = 0; r < 2; r++)
-#pragma unroll
-      for (int c = 0; c < 4; c++) acc[r][c] *= 1.0f / (kSplitScale * kSplitScale);
   }
 
-  const float scale = a.invB * a.tau;
+  // (a power of two from the pieces' scale: the sums keep their bits)
+  const float scale = a.invB * a.tau * (in_float ? 1.0f : kSplitUnscale);
 #pragma unroll
   for (int r = 0; r < 2; r++)
 #pragma unroll

@@ -446,7 +446,8 @@ int launch_train_fused(hipStream_t st, const T *x, const T *y, T *Cij, T *W, con
   };
   const dim3 sums((unsigned)(cdiv(N, 64) + cdiv(M, 64)));
   if constexpr (sizeof(T) == 4) {
-    if (split && train_split_bytes<T>(B, N, H, Mc) > 0) {
+    // (the factor of the sums stays normal with the pieces' scale in it)
+    if (split && train_split_bytes<T>(B, N, H, Mc) > 0 && a.invB * a.tau * kSplitUnscale >= 0x1p-126f) {
       SplitBatch sp;
       sp.x_width = (unsigned)(cdiv(N, kSplitTileI) * kSplitTileI);
       sp.y_width = (unsigned)(cdiv(M, kSplitTileJ) * kSplitTileJ);
