@@ -724,9 +724,9 @@ static int net_train_batches(sb_net *net, int layer, long maxB, const int64_t *h
   SB_REQUIRE(first_batch >= 0 && n_batches >= 0 && first_batch + n_batches <= nb, "batch range");
   int rc = ensure_act(net, maxB < Ns ? maxB : Ns);
   if (rc) return rc;
-  // The frozen layers give a sample the same activations with and without their cache, and in whichever batch it is:
-  // those of a whole batch.
-  const long like = std::min(maxB, Ns);
+  // While the last layer trains, the frozen ones give a sample the same activations with and without their cache, and
+  // in whichever batch it is: those of a whole batch.
+  const long like = last ? std::min(maxB, Ns) : 0;
   const bool permute = first_batch == 0;  // a later range continues the epoch already laid out
   SB_REQUIRE(permute || net->Xp, "the epoch's first batches have not been run");
   // a training step of a layer below the last changes what the cache was computed from
