@@ -70,7 +70,10 @@ static std::mutex g_ctx_mutex;
 // asynchronous copy while the threads fill the next one; on the way down the other way round (where the threads also
 // share the page faults of a fresh array: reading back a layer of two 18.8 MB matrices behind an epoch of 11.3 ms
 // took 1.9 ms in synchronous copies, 0.6 ms this way).  What fits kSmallCopy is moved by a kernel that reads or writes
-// the pinned chunk itself, which starts sooner than the copy engine (two of these per inference of one image: 59 -> 35 us).  (One synchronous copy straight from pageable memory
+// the pinned chunk itself, which starts sooner than the copy engine (straight copies / copy engine / kernel: one image
+// forward 59 / - / 35 us; compute_activation, 78 KiB up and 180 KiB down, 48 / 52 / 34; 392 up and 750 down 82 / 86 / 69;
+// weights of 614 KiB read back 34 / 40 / 36; beyond 1 MiB, where several host threads share a piece, no difference to the
+// copy engine and less than straight copies).  (One synchronous copy straight from pageable memory
 // runs at about 21 GB/s here; the reference's loader keeps pinned double buffers for the same reason,
 // full_cuda_backend/dataloader.h:36-212.)  The pinned chunks are allocated on first use and kept until
 // sb_shutdown.
@@ -149,7 +152,7 @@ struct HostStager {
   static constexpr int kChunks = 4;
   static constexpr size_t kChunkBytes = (size_t)8 << 20;
   static constexpr size_t kDownBytes = (size_t)2 << 20;  // piece of a chunk used on the way down
-  static constexpr size_t kSmallCopy = (size_t)64 << 10;
+  static constexpr size_t kSmallCopy = (size_t)1 << 20;  // (fits kDownBytes)
   void *pinned[kChunks] = {nullptr, nullptr, nullptr, nullptr};
   hipEvent_t sent[kChunks] = {nullptr, nullptr, nullptr, nullptr};  // the chunk's copy to the device has finished
   CopyPool *pool = nullptr;

@@ -638,6 +638,27 @@ def test_a_layer_goes_on_after_an_allocation_that_failed():
         _capi.check(lib.sb_net_destroy(net))
 
 
+@pytest.mark.parametrize("units", [1, 3, 255, 256, 257, 4095, 4096, 4097, 7000, 12345, 30000])
+def test_state_round_trip_around_the_sizes_that_change_the_way_of_the_copy(units):
+    """Arrays of 64 floats a row up to 7.5 MB and masks of eight bytes a row: by a kernel, in one piece and in several by the
+    copy engine, up and down."""
+    import ctypes
+    from streambrain_amd import _capi
+    _capi.init()
+    lib, net, rng = _capi.lib(), ctypes.c_void_p(), np.random.default_rng(units)
+    _capi.check(lib.sb_net_create(ctypes.byref(net), 0))
+    try:
+        assert lib.sb_net_add_plastic_layer(net, units, 8, 8, 0.01, 0.1, -100.0, 0.1, 1.0, 1.0, 1.0) == 0
+        for name, a in ((b"Cij", rng.random((units, 64), dtype=np.float32)), (b"Ci", rng.random(units, dtype=np.float32)),
+                        (b"wmask", rng.integers(0, 2, (units, 8), dtype=np.uint8))):
+            for back in (np.zeros_like(a), np.ones_like(a)):
+                _capi.check(lib.sb_net_set_layer_state(net, 0, name, a.ctypes.data, a.nbytes))
+                _capi.check(lib.sb_net_get_layer_state(net, 0, name, back.ctypes.data, back.nbytes))
+                assert np.array_equal(a, back), name
+    finally:
+        _capi.check(lib.sb_net_destroy(net))
+
+
 def test_state_of_two_networks_from_two_threads():
     """The pinned ring that state goes through is one for all networks: small arrays (moved by a kernel) and big ones (by
     the copy engine, in pieces) of two networks, written and read back by a thread each, keep apart."""
