@@ -6,12 +6,12 @@
 // and the 16 worst active rows of the state they start from (plus rows that changed sides on the way) can ever be
 // picked.  The kernel therefore works in rounds of 16 iterations:
 //   phase A (whole workgroup): the 16 best rows of either side in the strict order (score, row index), which is the
-//     order the picks take them in, equal scores included.  The rows are dealt into 64 bins, a lane each; the 16th
+//     order the picks take them in, equal scores included.  The rows are dealt into 64 bins; the 16th
 //     largest of the 64 bins' best is a bound that at least 16 rows reach and few others do (about 3
 //     more where the order knows nothing of the bins), the rows that reach it go to a list in LDS, and a
-//     row's place is the number of listed rows ahead of it.  The wavefronts deal their rows in orders of their own
-//     (row_at): by the index modulo 64 alone, images 64 pixels wide have whole columns in a bin, whose scores
-//     resemble each other, and the list overflows (24576 rows, floats: 57 us instead of 18);
+//     row's place is the number of listed rows ahead of it.  A lane's rows go into another bin in every wavefront: by
+//     the index modulo 64 alone, images 64 pixels wide have whole columns in a bin, whose scores resemble each
+//     other, and the list overflows (24576 rows, floats: 57 us instead of 18);
 //   phase B (one wavefront, one candidate per lane and side): the iterations themselves, with the same picks, tie
 //     rule, break conditions and score expression as a full scan.
 // A round reads the N scores and sides twice (the second time from L2) and has seven barriers; its time is latency.
@@ -143,40 +143,32 @@ struct MaskSwap {
     int swaps;
   };
 
-  // This thread's first row among the NT * U from i0 on; the others follow NT apart.
-  static __device__ __forceinline__ int row_at(long i0) {
-    const unsigned tid = threadIdx.x;
-    return (int)(tid ^ ((4 * (tid >> 6) + 11 * (unsigned)(i0 >> 13)) & 63));
-  }
-  static_assert(NT * U == 1 << 13, "the shift above");
-  // This thread's rows among the NT * U from i0 on: scores and sides (2: no candidate, or no row), loads in flight
+  // This thread's rows i0 + tid, i0 + tid + NT, ..: scores and sides (2: no candidate, or no row), loads in flight
   // together.
   struct Rows {
     T s[U];
     int m[U];
   };
-  static __device__ __forceinline__ void load_rows(const MaskArgs<T> &a, Rows &v, long i0) {
-    const int first = row_at(i0);
+  static __device__ __forceinline__ void load_rows(const MaskArgs<T> &a, Rows &v, int i0) {
 #pragma unroll
     for (int u = 0; u < U; u++) {
-      const long i = i0 + first + NT * u;
+      const long i = (long)i0 + (int)threadIdx.x + NT * u;
       v.s[u] = a.score[i < a.N ? i : 0];
       v.m[u] = i < a.N ? a.side[i] : 2;
     }
   }
-  // Calls f(row, side, score) for all of this thread's rows, which lie in bin tid % 64, in ascending order.
+  // Calls f(row, side, score) for all of this thread's rows in ascending order.
   // `first`: the first NT * U rows, already loaded.  (No guards around the calls: what they hold is a few selects.)
   template <typename F>
   static __device__ __forceinline__ void for_rows(const MaskArgs<T> &a, const Rows &first, F &&f) {
-    const int r = row_at(0);
+    const int tid = threadIdx.x;
 #pragma unroll
-    for (int u = 0; u < U; u++) f(r + NT * u, first.m[u], first.s[u]);
+    for (int u = 0; u < U; u++) f(tid + NT * u, first.m[u], first.s[u]);
     for (long i0 = NT * U; i0 < a.N; i0 += NT * U) {
       Rows v;
-      load_rows(a, v, i0);
-      const int r = (int)i0 + row_at(i0);
+      load_rows(a, v, (int)i0);
 #pragma unroll
-      for (int u = 0; u < U; u++) f(r + NT * u, v.m[u], v.s[u]);
+      for (int u = 0; u < U; u++) f((int)i0 + tid + NT * u, v.m[u], v.s[u]);
     }
   }
   // in both groups the wanted rows are those with the LARGEST keys
@@ -188,7 +180,7 @@ struct MaskSwap {
   // One round of at most TOP iterations.  Returns the number of swaps, or -1: nothing was changed, and the
   // round has to be left to the full scan.  (uniform)
   static __device__ int round(const MaskArgs<T> &a, Shared &sh, int iterations, int *changed, int *nchanged) {
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     constexpr int kNone = 0x7fffffff;
     if (tid < 2) sh.nlist[tid] = 0, sh.nan_first[tid] = kNone, sh.ahead[tid] = 0;
     if (tid < 128) sh.rank[tid >> 6][tid & 63] = 0;
@@ -214,8 +206,9 @@ struct MaskSwap {
     });
 #pragma unroll
     for (int g = 0; g < 2; g++) {
-      sh.bin_key[g][wv][lane] = best[g].key;
-      sh.bin_idx[g][wv][lane] = best[g].idx;
+      const int bin = lane ^ (4 * wv);
+      sh.bin_key[g][wv][bin] = best[g].key;
+      sh.bin_idx[g][wv][bin] = best[g].idx;
       if (__ballot(nan_first[g] != kNone)) {  // one atomic per wavefront: they all hit one address
         const int lowest = wave_reduce(nan_first[g], [](int x, int y) { return y < x ? y : x; });
         if (lane == 0) atomicMin(&sh.nan_first[g], lowest);
