@@ -331,10 +331,10 @@ template <typename T>
 static long train_tiles_of_one_round() { return (long)train_waves_per_simd<T, true, 1>() * device_cu_count(); }
 
 // Floats go through k_trace_sums<float, true> and k_train_split in layers of 2.5 rounds of 64 x 64 tiles and more where
-// that is faster, sums included (k_train_fused / k_train_split, whole steps, 1.0 and more in all 400 sizes tried
-// but for those named here):
-//   Cij and W beyond the memory-side cache: any batch (from 32 rows, see k_train_split: 12670 x 3000 1.7, 9306 x 4000 1.2,
-//   3800 x 10000 1.7; 64 rows 2.2, 1.2, 1.7; 300 rows 2.0, 1.6, 1.7).  In it the matrix instructions have to
+// that is faster, sums included (the numbers: time of whole steps with k_train_fused over that with k_train_split, at
+// 96 to 20000 columns, 100 to 700 MiB of Cij and W, 32 to 600 batch rows):
+//   Cij and W beyond the memory-side cache: any batch (from 32 rows, see k_train_split: 12670 x 3000 1.7, 9500 x 4000
+//   1.3, 3800 x 10000 1.7; 64 rows 2.2, 1.2, 1.7; 300 rows 2.0, 1.6, 1.7).  In it the matrix instructions have to
 //   gain what the split costs: rows that are no whole number of 128-byte lines from 65 rows (77 rows, 4600 to 8700 x
 //   3000 0.99 to 1.06, 2929 columns 1.10 to 1.15; 64 rows 0.98 to 0.99 and 1.0), others from 97 (100 rows, 3440 to 6550 x
 //   4000 1.03 to 1.10, 128 rows 1.05 to 1.10; 77 rows 0.97 to 1.00, 33 rows 0.89 to 0.92);
@@ -474,10 +474,10 @@ int launch_train_fused(hipStream_t st, const T *x, const T *y, T *Cij, T *W, con
   // Every tile adds up the batch's x and y columns for its own rows and columns, which with many tile
   // rows and columns is most of the kernel's vector arithmetic (43 % at 65536 x 100000, batch 1024).
   // From one and a half rounds of workgroups on (floats with more than 32 rows; doubles: two and a half), a small launch
-  // computes the new traces once and the tiles read them (floats: where k_train_split does not run).  Timed, 4096 inputs, batch 128, floats, with / without that
-  // launch: 23.7 / 22.5 us at 1.05 rounds, 29.3 / 29.9 at 1.5, 34.6 / 35.6 at 2, 45.5 / 48.5 at 3, 67.1 / 69.2
-  // at 5; doubles: 48.1 / 47.3 at 1.6 rounds, 55.8 / 54.3 at 2, 110.3 / 113.7 at 2.5.
-  const long ntiles = a.tiles_i * a.tiles_j;
+  // computes the new traces once and the tiles read them (floats: where k_train_split does not run).  Timed, 4096
+  // inputs, batch 128, floats, with / without that launch: 23.7 / 22.5 us at 1.05 rounds, 29.3 / 29.9 at 1.5, 34.6 /
+  // 35.6 at 2, 45.5 / 48.5 at 3, 67.1 / 69.2 at 5; doubles: 48.1 / 47.3 at 1.6 rounds, 55.8 / 54.3 at 2, 110.3 /
+  // 113.7 at 2.5.
   const bool one_round = ntiles <= train_tiles_of_one_round<T>();
   const long pre_from = sizeof(T) == 8 ? 5 * 4 : 3 * 5;  // in half workgroups per CU
   if constexpr (sizeof(T) == 8) {
