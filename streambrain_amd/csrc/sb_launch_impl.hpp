@@ -478,6 +478,7 @@ int launch_train_fused(hipStream_t st, const T *x, const T *y, T *Cij, T *W, con
   // inputs, batch 128, floats, with / without that launch: 23.7 / 22.5 us at 1.05 rounds, 29.3 / 29.9 at 1.5, 34.6 /
   // 35.6 at 2, 45.5 / 48.5 at 3, 67.1 / 69.2 at 5; doubles: 48.1 / 47.3 at 1.6 rounds, 55.8 / 54.3 at 2, 110.3 /
   // 113.7 at 2.5.
+  const long ntiles = a.tiles_i * a.tiles_j;
   const bool one_round = ntiles <= train_tiles_of_one_round<T>();
   const long pre_from = sizeof(T) == 8 ? 5 * 4 : 3 * 5;  // in half workgroups per CU
   if constexpr (sizeof(T) == 8) {
