@@ -56,10 +56,7 @@ constexpr int forward_rows_waves_per_simd() {
 // and stores SEG / 256 entries per segment whatever the list's length, and at batch 128 the kernel is a
 // chain of latencies that starts with this staging (1568 -> 30x100, density 0.1, lists of 157: 6.31 -> 6.13 us).
 // It also decides in which order the wavefronts' partial sums are added (NT).
-// SPLIT: a workgroup computes column group blockIdx.y (NG groups wide) of its hypercolumn only and stores the logits;
-// every sum is formed as without (same wavefronts, same chunks), k_softmax_as_fused does the rest.
-template <typename T, int NG, int NWAVES, int RB = 1, bool XT = false, int LW = Real<T>::VW, int SEG = 2048,
-          bool SPLIT = false>
+template <typename T, int NG, int NWAVES, int RB = 1, bool XT = false, int LW = Real<T>::VW, int SEG = 2048>
 __global__ __launch_bounds__(64 * NWAVES)
 __attribute__((amdgpu_waves_per_eu(forward_rows_waves_per_simd<T, NG, RB>(),
                                    forward_rows_waves_per_simd<T, NG, RB>())))
@@ -89,9 +86,7 @@ void k_forward_rows(ForwardRowsArgs<T> ar) {
   const int tid = threadIdx.x, lane = tid & 63, p = lane & 15, q = lane >> 4;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const long b0 = bt * (16 * RB);
-  const long jg = SPLIT ? (long)blockIdx.y * (NG * 16 * VW) : 0;  // first column inside the hypercolumn
-  const long j0 = ct * a.Mc + jg;
-  const long ncol = SPLIT && a.Mc - jg > NG * 16 * VW ? NG * 16 * VW : a.Mc - jg;
+  const long j0 = ct * a.Mc, ncol = a.Mc;
   const int *list = ar.rows + ct * ar.cap;
 
   // first segment of the list on its way before anything else
@@ -217,7 +212,7 @@ void k_forward_rows(ForwardRowsArgs<T> ar) {
 #pragma unroll
   for (int r = 0; r < RB; r++) {
     if (r > 0) __syncthreads();  // the previous row block's sums have been read
-    forward_finish<T, NG, !SPLIT, NWAVES, LW, false, NT>(acc[r], bv, red, a.act, a.B, a.M, b0 + 16 * r, j0, ncol);
+    forward_finish<T, NG, true, NWAVES, LW, false, NT>(acc[r], bv, red, a.act, a.B, a.M, b0 + 16 * r, j0, ncol);
   }
 }
 

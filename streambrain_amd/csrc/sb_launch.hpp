@@ -94,7 +94,11 @@ bool forward_rows_supported(const T *W, long N, long H, long Mc);
 template <typename T>
 int launch_forward_rows(hipStream_t st, T *act, const T *x, const T *W, const T *bias, const int *rows,
                         const int *row_cnt, long cap, long B, long N, long H, long Mc, const T *x_blocked,
-                        long like = 0);
+                        long like = 0, void *scratch = nullptr);
+// Bytes of scratch with which that pass spreads few tiles over more CUs (0: nothing to gain); the same bits with and
+// without.
+template <typename T>
+size_t forward_rows_bytes(long B, long N, long H, long Mc, long cap, long like = 0);
 // Lists of hypercolumns h0 .. h0 + count - 1 rebuilt from wmask.
 int launch_mask_rows(hipStream_t st, int *rows, int *row_cnt, const uint8_t *wmask, long N, long H,
                      long cap, long h0, long count);

@@ -4,6 +4,7 @@
 #include "sb_kernels.hpp"
 #include "sb_k_train.hpp"
 #include "sb_k_forward_rows.hpp"
+#include "sb_k_forward_chains.hpp"
 #include "sb_k_skinny.hpp"
 #include "sb_launch.hpp"
 
@@ -275,30 +276,80 @@ static int forward_rows_variant(hipStream_t st, ForwardRowsArgs<T> a, long like)
   return 0;
 }
 
+// How k_forward_chains covers a pass; no workgroups: it does not run.
+template <typename T>
+struct ChainsPlan {
+  long workgroups = 0;
+  int waves = 4;
+  ForwardChainsArgs<T> args{};
+};
+// Pieces of a hypercolumn: as many (of one to four blocks of 16 columns) as workgroups of four wavefronts find a CU each;
+// where even the fewest do not, workgroups of eight, whose wavefronts share the CU's SIMDs evenly.
+template <typename T>
+static ChainsPlan<T> forward_chains_plan(long B, long N, long H, long Mc, long cap, long like) {
+  ChainsPlan<T> plan;
+  const long M = H * Mc, cus = device_cu_count(), rbs = cdiv(B, 16), tiles = H * rbs;
+  if (forward_rows_short<T>(like > 0 ? like : B, N, H, Mc, cap)) return plan;  // (another order of the four sums)
+  if (N * M * (long)sizeof(T) > (1L << 32)) return plan;
+  // Few tiles and lists that pay for the second launch.  Time of k_forward_rows over time this way, at 40 / 80 / 120 / 152
+  // tiles: 100 columns, lists of 600 1.00 / 0.90 / 0.81 / 0.64, of 1200 1.26 / 1.13 / 1.01 / 0.76, of 6000 2.0 / 1.65 /
+  // 1.42 / 1.00; 200 columns 1.15 / 0.87 / 0.83 / 0.60, 1.52 / 1.06 / 1.03 / 0.71, 2.6 / 1.6 / 1.6 / 0.91; 64 columns,
+  // lists of 1200 1.02 / 0.92 / 0.89 / 0.71, of 2400 1.34 / 1.15 / 1.13 / 0.87; 12 columns 1.1, 1.47 whatever the tiles (at
+  // 320 1.30, 1.47); doubles, 64 columns, lists of 600 0.96 / 0.86 / 0.82 / 0.64, of 1200 1.24 / 1.05 / 1.01 / 0.77; 200
+  // columns 1.29 / 0.96 / 0.94 / 0.71, 1.71 / 1.21 / 1.18 / 0.78; 12 columns 0.97, 1.3.
+  const long blocks = cdiv(Mc, 16), fewest = cdiv(blocks, 4);
+  const bool heavy = blocks * (long)sizeof(T) >= 28, few = 6 * tiles <= cus;
+  if (2 * tiles > (blocks == 1 ? 3 * cus : cus)) return plan;
+  if (cap < (heavy ? (few ? 640 : 1152) : (few || blocks == 1 ? 1280 : 2048))) return plan;
+  ForwardChainsArgs<T> &c = plan.args;
+  c.waves_rows = rbs >= 4 ? 4 : rbs >= 2 ? 2 : 1;
+  c.row_groups = (int)cdiv(rbs, c.waves_rows);
+  auto groups = [&](long pieces) { return cdiv(pieces, std::min<long>(4 / c.waves_rows, pieces)); };
+  const long around = H * c.row_groups * kChains;
+  long pieces = blocks;
+  while (pieces > fewest && around * groups(pieces) > cus) pieces--;
+  c.pieces = (int)pieces;
+  c.waves_cols = (int)std::min<long>(4 / c.waves_rows, pieces);
+  if (around * groups(pieces) > cus) {
+    plan.waves = 8;
+    if (2 * c.waves_cols <= c.pieces) c.waves_cols *= 2;
+    else c.waves_rows *= 2, c.row_groups = (int)cdiv(rbs, c.waves_rows);
+  }
+  c.col_groups = (int)cdiv(c.pieces, c.waves_cols);
+  plan.workgroups = H * kChains * c.row_groups * c.col_groups;
+  return plan;
+}
+template <typename T>
+size_t forward_rows_bytes(long B, long N, long H, long Mc, long cap, long like) {
+  if (B <= 0 || N <= 0 || H <= 0 || Mc <= 0 || H * Mc >= (1L << 31) || N >= (1L << 31)) return 0;
+  return forward_chains_plan<T>(B, N, H, Mc, cap, like).workgroups > 0 ? kChains * sizeof(T) * (size_t)B * (size_t)(H * Mc) : 0;
+}
+
 template <typename T>
 int launch_forward_rows(hipStream_t st, T *act, const T *x, const T *W, const T *bias, const int *rows,
-                        const int *row_cnt, long cap, long B, long N, long H, long Mc, const T *x_blocked, long like) {
+                        const int *row_cnt, long cap, long B, long N, long H, long Mc, const T *x_blocked, long like,
+                        void *scratch) {
   SB_REQUIRE(act && x && W && bias && rows && row_cnt, "null pointer");
   SB_REQUIRE(B > 0 && N > 0 && H > 0 && Mc > 0, "sizes must be positive");
   SB_REQUIRE(H * Mc < (1L << 31) && N < (1L << 31), "dimension too large");
   SB_REQUIRE(cap > 0 && cap % 16 == 0, "row lists must be padded to a multiple of 16");
   SB_REQUIRE(forward_rows_supported<T>(W, N, H, Mc), "shape not supported by the row-list forward kernel");
   ForwardRowsArgs<T> a{{act, x, W, bias, B, N, H * Mc, Mc, H, cdiv(B, 16), {}}, rows, row_cnt, cap, x_blocked};
-  // Wide hypercolumns, few of them and long lists: a workgroup per column group, then the softmax, every sum as in
-  // the fused kernel (27648 -> 15 x 200, lists of 15800, batch 128, 120 tiles: 286 us fused, 249 + 5 us this way).
-  // Time fused over time this way, at 2 / 120 / 160 tiles: 100 columns, lists of 512 0.96 / 0.94 / 0.71, of 1024 1.07 /
-  // 1.08 / 0.72, of 8192 1.40 / 1.38 / 0.76; 200 columns 1.45 / 1.05 / 0.78, 1.75 / 1.12 / 0.80, 2.28 / 1.28 / 0.80; doubles,
-  // 48 columns, lists of 512 0.94 / 0.91 / 0.80, of 1024 1.09 / 1.07 / 0.87, 200 columns, of 2048 2.8 / 1.2 / 1.07 (240: 0.79).
-  constexpr int GW1 = 16 * Real<T>::VW;
-  if (Mc > GW1 && 5 * H * cdiv(B, 16) <= 3L * device_cu_count() && cap >= 1024) {
-    ProfScope prof_(st, K_FORWARD);
-    a.f.by_batch_tiles = FastDiv::of(a.f.batch_tiles);
-    const dim3 g((unsigned)(8 * cdiv(H * a.f.batch_tiles, 8)), (unsigned)cdiv(Mc, GW1)), blk(256);
-    constexpr int VWc = Real<T>::VW;
-    if (x_blocked) hipLaunchKernelGGL((k_forward_rows<T, 1, 4, 1, true, VWc, 2048, true>), g, blk, 0, st, a);
-    else hipLaunchKernelGGL((k_forward_rows<T, 1, 4, 1, false, VWc, 2048, true>), g, blk, 0, st, a);
-    SB_LAUNCH_CHECK();
-    return launch_softmax_as_fused<T, 16>(st, act, B, H, Mc);
+  if (scratch) {
+    ChainsPlan<T> plan = forward_chains_plan<T>(B, N, H, Mc, cap, like);
+    if (plan.workgroups > 0) {
+      ProfScope prof_(st, K_FORWARD);
+      plan.args.r = a;
+      plan.args.part = (T *)scratch;
+      const dim3 g((unsigned)(8 * cdiv(plan.workgroups, 8))), blk(64 * plan.waves);
+      if (x_blocked) hipLaunchKernelGGL((k_forward_chains<T, true>), g, blk, 0, st, plan.args);
+      else hipLaunchKernelGGL((k_forward_chains<T, false>), g, blk, 0, st, plan.args);
+      SB_LAUNCH_CHECK();
+      hipLaunchKernelGGL((k_softmax_of_chains<T>), dim3((unsigned)cdiv(B * H, 8)), dim3(128), 0, st, act,
+                         (const T *)plan.args.part, bias, B, H, Mc);
+      SB_LAUNCH_CHECK();
+      return 0;
+    }
   }
   if (like <= 0) like = B;
   constexpr int VW = Real<T>::VW, NGL = 8 / VW, LWL = 7 - (NGL - 1) * VW, NGM = VW == 2 ? 7 : 4;
@@ -776,7 +827,9 @@ int launch_copy_pair(hipStream_t st, T *dst1, const T *src1, size_t n1, T *dst2,
   template bool forward_bits_equal<T>(long, long, long, long, long, long);                            \
   template bool forward_rows_supported<T>(const T *, long, long, long);                               \
   template int launch_forward_rows<T>(hipStream_t, T *, const T *, const T *, const T *, const int *, \
-                                      const int *, long, long, long, long, long, const T *, long);    \
+                                      const int *, long, long, long, long, long, const T *, long,     \
+                                      void *);                                                        \
+  template size_t forward_rows_bytes<T>(long, long, long, long, long, long);                          \
   template int launch_gather_rows_blocked<T>(hipStream_t, T *, T *, const T *, const int64_t *, long, \
                                              long);                                                  \
   template int launch_softmax<T>(hipStream_t, T *, long, long, long);                                 \

@@ -577,7 +577,8 @@ static int layer_forward(sb_net *net, Layer &L, const T *x, long B, const T *x_b
   }
   if (L.rows && L.w_masked)
     return launch_forward_rows<T>(g_ctx.stream, act, x, (const T *)L.W, (const T *)L.bias, L.rows,
-                                  L.row_cnt, L.rows_cap, B, L.N, L.H, L.Mc, x_blocked, like);
+                                  L.row_cnt, L.rows_cap, B, L.N, L.H, L.Mc, x_blocked, like,
+                                  optional_scratch(net->work, forward_rows_bytes<T>(B, L.N, L.H, L.Mc, L.rows_cap, like)));
   return launch_forward<T>(g_ctx.stream, act, x, (const T *)L.W, (const T *)L.bias, B, L.N, L.H,
                            L.Mc, true, like);
 }
@@ -1155,8 +1156,9 @@ int sb_fill_bytes(void *d_dst, int value, size_t bytes) {
                                        const int *row_cnt, long cap, long B, long N, long H, long Mc,  \
                                        const T *x_blocked) {                                           \
     SB_READY();                                                                                        \
+    std::lock_guard<std::mutex> lock(g_work_mutex);                                                    \
     return launch_forward_rows<T>(g_ctx.stream, act, x, W, bias, rows, row_cnt, cap, B, N, H, Mc,      \
-                                  x_blocked);                                                          \
+                                  x_blocked, 0, optional_scratch(g_work, forward_rows_bytes<T>(B, N, H, Mc, cap))); \
   }                                                                                                    \
   int sb_rows_in_blocks_##SFX(T *dst, const T *src, long rows, long cols) {                            \
     SB_READY();                                                                                        \

@@ -747,6 +747,26 @@ def test_forward_with_few_tiles(k, dtype, B, N, H, Mc):
             assert np.array_equal(few, k.compute_activation_rows(W, bias, x, wmask, H, Mc, blocked)[:B])
 
 
+@pytest.mark.parametrize("dtype", DT)
+@pytest.mark.parametrize("B,N,H,Mc,more", [(100, 34000, 4, 12, 1552), (33, 3000, 5, 100, 448), (128, 2500, 9, 200, 272),
+                                           (7, 9000, 3, 64, 704), (16, 2100, 2, 36, 1040), (80, 2600, 3, 128, 704)])
+def test_chains_of_the_row_lists(k, dtype, B, N, H, Mc, more):
+    """The four sums of a tile on four CUs (few tiles, long lists): the bits that a larger batch, whose tiles form them
+    on one, gives the same rows.  Lists of more than one staged segment, of a few entries and of none; workgroups of four
+    and of eight wavefronts, some of them without batch rows or columns."""
+    rng = np.random.default_rng(N + B)
+    M = H * Mc
+    wmask = (rng.random((N, H)) < 0.51).astype(np.uint8)
+    wmask[:, 1] = 0
+    wmask[:37 if H > 2 else 0, 1] = rng.random(37 if H > 2 else 0) < 0.8
+    x = rng.random((more, N), dtype=dtype)
+    W = rng.standard_normal((N, M), dtype=dtype) * np.repeat(wmask, Mc, axis=1).astype(dtype) * dtype(4 / np.sqrt(N))
+    bias = rng.standard_normal(M).astype(dtype)
+    for blocked in (False, True):
+        few = k.compute_activation_rows(W, bias, x[:B], wmask, H, Mc, blocked)
+        assert np.array_equal(few, k.compute_activation_rows(W, bias, x, wmask, H, Mc, blocked)[:B])
+
+
 def _random_shapes(seed, count):
     """Shapes off every tiling's grid: mostly odd widths, batches around the 16- and 32-row boundaries."""
     rng = np.random.default_rng(seed)
