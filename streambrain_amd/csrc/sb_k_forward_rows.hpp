@@ -8,6 +8,8 @@
 // wmask) and gathers those rows of W and those columns of x.  Same tiling, accumulator layout and
 // epilogue as k_forward.
 #pragma once
+#include <type_traits>
+
 #include "sb_k_forward.hpp"
 #include "sb_kernels.hpp"
 
@@ -56,7 +58,15 @@ constexpr int forward_rows_waves_per_simd() {
 // and stores SEG / 256 entries per segment whatever the list's length, and at batch 128 the kernel is a
 // chain of latencies that starts with this staging (1568 -> 30x100, density 0.1, lists of 157: 6.31 -> 6.13 us).
 // It also decides in which order the wavefronts' partial sums are added (NT).
-template <typename T, int NG, int NWAVES, int RB = 1, bool XT = false, int LW = Real<T>::VW, int SEG = 2048>
+// The list is staged as byte offsets, so that an operand costs one addition of 32 bits: beside the matrix instructions, which
+// a wavefront's own vector instructions delay by five cycles each, the index times the row length in 64 bits took a fifth
+// of the time (54000 -> 190 x 100, density 0.05, batch 256: 315 -> 263 us; 3000 -> 100 x 64, density 0.1: 21.4 -> 19.1;
+// doubles 256 rows of 3000 -> 30 x 64, density 0.3: 25.5 -> 23.1).
+// WIDE: W beyond the 4 GiB that such an offset reaches.  Offsets then count from the segment's first row; a segment that
+// spans more than 4 GiB is walked with 64-bit addresses (55296 -> 200 x 100, density 0.05, batch 256: 362 -> 314 us, all
+// addresses in 64 bits 420).
+template <typename T, int NG, int NWAVES, int RB = 1, bool XT = false, int LW = Real<T>::VW, int SEG = 2048,
+          bool WIDE = false>
 __global__ __launch_bounds__(64 * NWAVES)
 __attribute__((amdgpu_waves_per_eu(forward_rows_waves_per_simd<T, NG, RB>(),
                                    forward_rows_waves_per_simd<T, NG, RB>())))
@@ -69,12 +79,12 @@ void k_forward_rows(ForwardRowsArgs<T> ar) {
   static_assert(SEGC >= NWAVES && SEG % (64 * NWAVES) == 0, "segment size");
   using acc_t = typename Real<T>::acc_t;
   using vec_t = typename Real<T>::vec_t;
-  typedef int ivec_t __attribute__((ext_vector_type(VW)));
+  typedef unsigned off_t __attribute__((ext_vector_type(VW)));
   // (the short-list variant is the one whose time is a chain of latencies: its partial sums meet in LDS in one
   // step instead of two, 6.14 -> 6.06 us at 1568 -> 30x100, batch 128)
   constexpr int NT = SEG == 256 ? NWAVES : NWAVES / 2;
   __shared__ __attribute__((aligned(16))) T red[NT][16][TC::CP];
-  __shared__ __attribute__((aligned(16))) int sidx[SEG];
+  __shared__ __attribute__((aligned(16))) unsigned woff[SEG], xoff[SEG];
 
   // XCD-aware renumbering, as in k_forward
   const long ntiles = a.col_tiles * a.batch_tiles;
@@ -89,6 +99,9 @@ void k_forward_rows(ForwardRowsArgs<T> ar) {
   const long j0 = ct * a.Mc, ncol = a.Mc;
   const int *list = ar.rows + ct * ar.cap;
 
+  constexpr unsigned XSTEP = (XT ? 16u : 1u) * (unsigned)sizeof(T);  // bytes between input columns
+  const unsigned wrow = (unsigned)(a.M * sizeof(T));  // bytes of a row of W (launcher: 16 rows are below 2 GiB)
+
   // first segment of the list on its way before anything else
   constexpr int PT = SEG / (64 * NWAVES);  // entries per thread and segment
   int mine[PT];
@@ -99,12 +112,25 @@ void k_forward_rows(ForwardRowsArgs<T> ar) {
       mine[t] = list[k < ar.cap ? k : 0];  // entries past the list are replaced by padding below
     }
   };
+  // Row whose start the staged offsets into W count from: 0, or with WIDE the segment's first.  Returns whether all of the
+  // thread's entries are in reach of 32 bits.
+  long wbase = 0;
   auto publish_segment = [&](long seg0) {
+    if constexpr (WIDE) {
+      const int r = list[seg0 < ar.cap ? seg0 : 0];  // (uniform)
+      wbase = r < 0 ? 0 : r;
+    }
+    bool reach = true;
 #pragma unroll
     for (int t = 0; t < PT; t++) {
       const long k = seg0 + tid + t * (64 * NWAVES);
-      sidx[tid + t * (64 * NWAVES)] = k < ar.cap ? mine[t] : -1;
+      const int r = k < ar.cap ? mine[t] : -1, e = tid + t * (64 * NWAVES);
+      const long rel = r < 0 ? 0 : r - wbase;
+      if constexpr (WIDE) reach = reach && rel >= 0 && (rel + 1) * (long)wrow <= (1L << 32);
+      woff[e] = (unsigned)rel * wrow;
+      xoff[e] = r < 0 ? BufferWindow<T>::kOutside : (unsigned)r * XSTEP;
     }
+    return reach;
   };
   request_segment(0);
   const int cnt = ar.row_cnt[ct];
@@ -130,36 +156,40 @@ void k_forward_rows(ForwardRowsArgs<T> ar) {
   for (int r = 0; r < RB; r++)
     xat[r] = XT ? (unsigned)(((long)r * a.N * 16 + p) * sizeof(T))
                 : (unsigned)((long)(16 * r + p) * a.N * sizeof(T));
-  constexpr unsigned XSTEP = (XT ? 16u : 1u) * (unsigned)sizeof(T);  // bytes between input columns
   // W: this lane's columns of group g, or the tile's first columns where the group hangs over the end
   // of the hypercolumn (those accumulator columns are never stored)
-  const T *wcol[NG];
+  unsigned wcol[NG];  // bytes
 #pragma unroll
-  for (int g = 0; g < NG; g++) wcol[g] = a.W + j0 + (TC::gcol(g, p) < ncol ? TC::gcol(g, p) : 0);
+  for (int g = 0; g < NG; g++) wcol[g] = (unsigned)((j0 + (TC::gcol(g, p) < ncol ? TC::gcol(g, p) : 0)) * sizeof(T));
 
   T xr[2][RB][VW];
   T wr[2][VW][NG][VW];
   // operands of chunk c of the staged segment (c past the segment: its last chunk again, never used)
-  auto request = [&](int c, T(&xo)[RB][VW], T(&wo)[VW][NG][VW]) {
-    const ivec_t idx = *reinterpret_cast<const ivec_t *>(&sidx[(c < SEGC ? c : SEGC - 1) * KC + VW * q]);
+  // FAR: of a segment whose rows are not in reach of 32-bit offsets.
+  auto request = [&](auto far, int c, T(&xo)[RB][VW], T(&wo)[VW][NG][VW]) {
+    constexpr bool FAR = decltype(far)::value;
+    const char *const wfrom = reinterpret_cast<const char *>(WIDE && !FAR ? a.W + wbase * a.M : a.W);
+    const int at = (c < SEGC ? c : SEGC - 1) * KC + VW * q;
+    const off_t wv = *reinterpret_cast<const off_t *>(&woff[at]), xv = *reinterpret_cast<const off_t *>(&xoff[at]);
 #pragma unroll
     for (int s = 0; s < VW; s++) {
-      const int r = idx[s];
 #pragma unroll
       for (int rb = 0; rb < RB; rb++) {
         T one[1];
-        xwin.template load_n<1>(one, r < 0 ? BufferWindow<T>::kOutside : xat[rb] + (unsigned)r * XSTEP);
+        xwin.template load_n<1>(one, xat[rb] + xv[s]);
         xo[rb][s] = one[0];
       }
-      const long roff = (long)(r < 0 ? 0 : r) * a.M;
 #pragma unroll
       for (int g = 0; g < NG; g++) {
+        const char *from = wfrom + (wcol[g] + wv[s]);
+        if constexpr (FAR)
+          from = wfrom + (wcol[g] + (unsigned long)(xv[s] == BufferWindow<T>::kOutside ? 0u : xv[s] / XSTEP) * wrow);
         if (TC::gwidth(g) == VW) {
-          const vec_t v = *reinterpret_cast<const vec_t *>(wcol[g] + roff);
+          const vec_t v = *reinterpret_cast<const vec_t *>(from);
 #pragma unroll
           for (int c2 = 0; c2 < VW; c2++) wo[s][g][c2] = v[c2];
         } else {
-          const PackedCols<T, LW> v = *reinterpret_cast<const PackedCols<T, LW> *>(wcol[g] + roff);
+          const PackedCols<T, LW> v = *reinterpret_cast<const PackedCols<T, LW> *>(from);
 #pragma unroll
           for (int c2 = 0; c2 < LW; c2++) wo[s][g][c2] = v.v[c2];
         }
@@ -180,9 +210,8 @@ void k_forward_rows(ForwardRowsArgs<T> ar) {
   };
 
   for (long seg0 = 0;;) {
-    publish_segment(seg0);
-    __syncthreads();
-    request(w, xr[0], wr[0]);  // this wavefront's first chunk of the segment
+    const bool reach = publish_segment(seg0);
+    const bool is_far = WIDE ? __syncthreads_or(!reach) != 0 : (__syncthreads(), false);
     // chunks w, w + NWAVES, ... of the segment that hold list entries: n of them (at least 1 in the
     // first segment, see above)
     const long left = (long)cnt - seg0;  // entries from the start of this segment
@@ -190,21 +219,31 @@ void k_forward_rows(ForwardRowsArgs<T> ar) {
     long n = w < segc ? (segc - 1 - w) / NWAVES + 1 : 0;
     if (seg0 == 0 && n == 0) n = 1;
     const bool more = left > SEG;
-    if (more) request_segment(seg0 + SEG);  // uniform
-    __builtin_amdgcn_sched_barrier(0);
-    long i = 0;
-    for (; i + 2 <= n; i += 2) {
-      // the scheduling fences keep the requests where they are written, ahead of the MFMAs
-      request(w + (int)(i + 1) * NWAVES, xr[1], wr[1]);
+    constexpr std::false_type near{};
+    if (WIDE && is_far) {  // (uniform, and rare: one chunk after the other)
+      if (more) request_segment(seg0 + SEG);
+      for (long i = 0; i < n; i++) {
+        request(std::true_type{}, w + (int)i * NWAVES, xr[0], wr[0]);
+        compute(xr[0], wr[0]);
+      }
+    } else {
+      request(near, w, xr[0], wr[0]);  // this wavefront's first chunk of the segment
+      if (more) request_segment(seg0 + SEG);  // uniform
       __builtin_amdgcn_sched_barrier(0);
-      compute(xr[0], wr[0]);
-      __builtin_amdgcn_sched_barrier(0);
-      request(w + (int)(i + 2) * NWAVES, xr[0], wr[0]);
-      __builtin_amdgcn_sched_barrier(0);
-      compute(xr[1], wr[1]);
-      __builtin_amdgcn_sched_barrier(0);
+      long i = 0;
+      for (; i + 2 <= n; i += 2) {
+        // the scheduling fences keep the requests where they are written, ahead of the MFMAs
+        request(near, w + (int)(i + 1) * NWAVES, xr[1], wr[1]);
+        __builtin_amdgcn_sched_barrier(0);
+        compute(xr[0], wr[0]);
+        __builtin_amdgcn_sched_barrier(0);
+        request(near, w + (int)(i + 2) * NWAVES, xr[0], wr[0]);
+        __builtin_amdgcn_sched_barrier(0);
+        compute(xr[1], wr[1]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      if (i < n) compute(xr[0], wr[0]);
     }
-    if (i < n) compute(xr[0], wr[0]);
     if (!more) break;
     seg0 += SEG;
     __syncthreads();  // everyone is done with the staged segment

@@ -251,24 +251,23 @@ static int forward_rows_variant(hipStream_t st, ForwardRowsArgs<T> a, long like)
   SB_REQUIRE(grid < (1L << 31), "too many tiles for one launch");
   const dim3 g((unsigned)grid), blk(64 * NW);
   const bool is_short = forward_rows_short<T>(like, a.f.N, H, a.f.Mc, a.cap);
-  auto launch = [&](auto blocked) {  // (with the batch at hand in blocks of 16 rows, or without)
+  const bool wide = a.f.N * a.f.M * (long)sizeof(T) > (1L << 32);
+  auto launch_rb = [&](auto blocked, auto row_blocks) {  // (with the batch at hand in blocks of 16 rows, or without)
     constexpr bool XT = decltype(blocked)::value;
+    constexpr int RB = decltype(row_blocks)::value;
+    if (wide && is_short) hipLaunchKernelGGL((k_forward_rows<T, NG, NW, RB, XT, LW, 256, true>), g, blk, 0, st, a);
+    else if (wide) hipLaunchKernelGGL((k_forward_rows<T, NG, NW, RB, XT, LW, 2048, true>), g, blk, 0, st, a);
+    else if (is_short) hipLaunchKernelGGL((k_forward_rows<T, NG, NW, RB, XT, LW, 256>), g, blk, 0, st, a);
+    else hipLaunchKernelGGL((k_forward_rows<T, NG, NW, RB, XT, LW>), g, blk, 0, st, a);
+  };
+  auto launch = [&](auto blocked) {
     if constexpr (fits4) {
-      if (rb == 4) {
-        if (is_short) hipLaunchKernelGGL((k_forward_rows<T, NG, NW, 4, XT, LW, 256>), g, blk, 0, st, a);
-        else hipLaunchKernelGGL((k_forward_rows<T, NG, NW, 4, XT, LW>), g, blk, 0, st, a);
-        return;
-      }
+      if (rb == 4) return launch_rb(blocked, std::integral_constant<int, 4>{});
     }
     if constexpr (forward_rows_regs<T>(NG, 2) <= kRowsRegsTwoWaves) {
-      if (rb == 2) {
-        if (is_short) hipLaunchKernelGGL((k_forward_rows<T, NG, NW, 2, XT, LW, 256>), g, blk, 0, st, a);
-        else hipLaunchKernelGGL((k_forward_rows<T, NG, NW, 2, XT, LW>), g, blk, 0, st, a);
-        return;
-      }
+      if (rb == 2) return launch_rb(blocked, std::integral_constant<int, 2>{});
     }
-    if (is_short) hipLaunchKernelGGL((k_forward_rows<T, NG, NW, 1, XT, LW, 256>), g, blk, 0, st, a);
-    else hipLaunchKernelGGL((k_forward_rows<T, NG, NW, 1, XT, LW>), g, blk, 0, st, a);
+    launch_rb(blocked, std::integral_constant<int, 1>{});
   };
   if (a.xt) launch(std::true_type{});
   else launch(std::false_type{});

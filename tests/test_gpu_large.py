@@ -166,3 +166,40 @@ def test_stl10_shaped_layer_f32_full_size():
 def test_largest_layer_f32_full_size():
     """65536 inputs, 1000 hypercolumns of 100, batch 1024, float32, dense mask (26 GB per matrix)."""
     _check_layer_at_size(np.float32, 1024, 65536, 1000, 100, 1.0, 14)
+
+
+@pytest.mark.parametrize("B,entries", [(20, 300), (20, 40), (256, 3000)])
+def test_row_lists_whose_rows_lie_more_than_4_gib_apart_f32(B, entries):
+    """The row-list forward pass on a W beyond 4 GiB whose lists span all of it in one segment (and in two): the bits of
+    the same rows packed into a small matrix."""
+    from streambrain_amd import _capi
+    from streambrain_amd._capi import DeviceArray
+    _capi.init(0)
+    lib = _capi.lib()
+    N, H, Mc = 55296, 200, 100
+    M, rng = H * Mc, np.random.default_rng(entries)
+    at = np.unique(np.concatenate([[0, N - 1], rng.choice(N, entries - 2, replace=False)])).astype(np.int64)
+    n = len(at)
+    w = rng.standard_normal((n, M), dtype=np.float32) * np.float32(4 / np.sqrt(n))
+    x = rng.random((B, n), dtype=np.float32)
+    wide = np.zeros((B, N), np.float32)
+    wide[:, at] = x
+    d_bias = DeviceArray.from_numpy(rng.standard_normal(M).astype(np.float32))
+    cap = (n + 15) // 16 * 16
+    lists = np.full((H, cap), -1, np.int32)
+    lists[:, :n] = at
+    packed = np.full((H, cap), -1, np.int32)
+    packed[:, :n] = np.arange(n)
+    d_cnt = DeviceArray.from_numpy(np.full(H, n, np.int32))
+    d_w = DeviceArray((N, M), np.float32)
+    _capi.check(lib.sb_fill_bytes(d_w.ptr, 0, N * M * 4))
+    for k, i in enumerate(at):
+        row = np.ascontiguousarray(w[k])
+        _capi.check(lib.sb_memcpy_h2d(ctypes.c_void_p(int(d_w.ptr) + int(i) * M * 4), row.ctypes.data, row.nbytes))
+    acts = []
+    for (W, inputs, rows, cols) in ((d_w, wide, lists, N), (DeviceArray.from_numpy(w), x, packed, n)):
+        d_act, d_x, d_rows = DeviceArray((B, M), np.float32), DeviceArray.from_numpy(inputs), DeviceArray.from_numpy(rows)
+        _capi.check(lib.sb_compute_activation_rows_f32(d_act.ptr, d_x.ptr, W.ptr, d_bias.ptr, d_rows.ptr, d_cnt.ptr, cap, B,
+                                                       cols, H, Mc, None))
+        acts.append(d_act.numpy())
+    assert np.array_equal(acts[0], acts[1])
