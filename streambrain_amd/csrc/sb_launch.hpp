@@ -120,6 +120,14 @@ int launch_train_fused(hipStream_t st, const T *x, const T *y, T *Cij, T *W, con
 // sizes; 0: none.  Without it (nullptr) the launch does without the kernel that needs it.
 template <typename T>
 size_t train_split_bytes(long B, long N, long H, long Mc);
+// launch_train_fused for `rows` rows in batches of B, one after the other, of a layer without mask and regularised bias of a
+// few units (train_skinny_epoch_supported).  Batch row b is x[order[b]] (order: device memory) and y[b].
+template <typename T>
+bool train_skinny_epoch_supported(long M);
+template <typename T>
+int launch_train_skinny_epoch(hipStream_t st, const T *x, const int64_t *order, const T *y, T *Cij, T *W, const T *Ci,
+                              const T *Cj, T *Ci_next, T *Cj_next, long B, long rows, long N, long H, long Mc, T taupdt,
+                              T cthr);
 // W from the traces as they are, the fused kernel's expression; wmask != nullptr: zero under zero mask bytes
 // (w_masked: the caller vouches that W is zero there already, and such entries are left alone).
 template <typename T>

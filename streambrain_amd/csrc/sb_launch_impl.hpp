@@ -566,6 +566,43 @@ int launch_train_fused(hipStream_t st, const T *x, const T *y, T *Cij, T *W, con
 }
 
 template <typename T>
+bool train_skinny_epoch_supported(long M) { return M <= 32; }
+
+template <typename T>
+int launch_train_skinny_epoch(hipStream_t st, const T *x, const int64_t *order, const T *y, T *Cij, T *W, const T *Ci,
+                              const T *Cj, T *Ci_next, T *Cj_next, long B, long rows, long N, long H, long Mc, T taupdt,
+                              T cthr) {
+  SB_REQUIRE(x && order && y && Cij && W && Ci && Cj && Ci_next && Cj_next, "null pointer");
+  SB_REQUIRE(Ci != Ci_next && Cj != Cj_next, "old and new traces must be distinct buffers");
+  SB_REQUIRE(B > 0 && rows > 0 && N > 0 && H > 0 && Mc > 0, "sizes must be positive");
+  const long M = H * Mc;
+  SB_REQUIRE(train_skinny_epoch_supported<T>(M), "too many units");
+  SB_REQUIRE(rows < (1L << 31), "too many rows");
+  const TraceScalars<T> s = TraceScalars<T>::from(taupdt, cthr);
+  SkinnyEpochArgs<T> e{};
+  TrainArgs<T> &a = e.a;
+  a.x = x; a.y = y; a.Cij = Cij; a.W = W; a.Ci = Ci; a.Cj = Cj; a.Ci_next = Ci_next; a.Cj_next = Cj_next;
+  a.B = B < rows ? B : rows; a.N = N; a.M = M; a.H = H; a.Mc = Mc;
+  a.tau = s.tau; a.omt = s.omt; a.fB = (T)a.B; a.invB = (T)1 / (T)a.B; a.cthr = s.cthr; a.cthr4 = s.cthr4;
+  e.order = order;
+  e.rows = rows;
+  const long last = rows - (cdiv(rows, a.B) - 1) * a.B;
+  e.fB_last = (T)last; e.invB_last = (T)1 / (T)last;
+  const long groups = cdiv(N, skinny_epoch_rows(M));
+  SB_REQUIRE(groups < (1L << 31) - 8, "too many rows for one launch");
+  ProfScope prof_(st, K_TRAIN_FUSED, true);
+  const dim3 g((unsigned)(8 * cdiv(groups, 8)));
+  auto launch = [&](auto kernel) {
+    if (prof_.carries()) hipExtLaunchKernelGGL(kernel, g, dim3(512), 0, st, prof_.start(), prof_.stop(), 0, e);
+    else hipLaunchKernelGGL(kernel, g, dim3(512), 0, st, e);
+  };
+  if (M <= 16) launch(k_train_skinny_epoch<T, 16>);
+  else launch(k_train_skinny_epoch<T, 32>);
+  SB_LAUNCH_CHECK();
+  return 0;
+}
+
+template <typename T>
 int launch_weights_from_traces(hipStream_t st, T *W, const T *Ci, const T *Cj, const T *Cij, const uint8_t *wmask,
                                T cthr, long N, long H, long Mc, bool w_masked) {
   SB_REQUIRE(W && Ci && Cj && Cij, "null pointer");
@@ -836,6 +873,10 @@ int launch_copy_pair(hipStream_t st, T *dst1, const T *src1, size_t n1, T *dst2,
                                      T *, T *, const uint8_t *, int, T *, T *, long, long, long, long, \
                                      T, T, T, T, T, bool, const void *, size_t, void *);              \
   template size_t train_split_bytes<T>(long, long, long, long);                                       \
+  template bool train_skinny_epoch_supported<T>(long);                                                \
+  template int launch_train_skinny_epoch<T>(hipStream_t, const T *, const int64_t *, const T *, T *,  \
+                                            T *, const T *, const T *, T *, T *, long, long, long,    \
+                                            long, long, T, T);                                        \
   template int launch_update_bias<T>(hipStream_t, T *, const T *, T, long);                           \
   template int launch_weights_from_traces<T>(hipStream_t, T *, const T *, const T *, const T *,       \
                                              const uint8_t *, T, long, long, long, bool);             \

@@ -432,6 +432,8 @@ struct sb_net {
   std::vector<sb::Layer> layers;
   // training set in HBM, its per-epoch permuted copy and the permutation
   void *X = nullptr, *Y = nullptr, *Xp = nullptr, *Yp = nullptr;
+  bool epoch_begun = false;  // d_perm holds the order of an epoch
+  bool images_laid = false;  // ... and Xp (XpB) its images
   long XpB_batch = 0;   // batch size XpB is valid for in the current epoch (0: not valid)
   void *XpB = nullptr;  // Xp in blocks of 16 rows (k_gather_rows_blocked), for the first layer's forward over row lists
   long Ns = 0, NF = 0, NC = 0;
@@ -439,7 +441,8 @@ struct sb_net {
   int64_t *h_perm = nullptr;  // pinned staging
   hipEvent_t perm_copied = nullptr;
   // While only the last layer trains, the layers below it are frozen: their output for every training
-  // sample is computed once (Hc, data-set order) and shuffled per epoch like the images (Hcp).
+  // sample is computed once (Hc, data-set order), and shuffled per epoch like the images (Hcp) where the steps do not
+  // read it in the epoch's order by themselves.
   void *Hc = nullptr, *Hcp = nullptr;
   int Hc_layer = -1;  // Hc holds the activations of this layer for the current training set (-1: none)
   size_t frozen_cache_limit = (size_t)16 << 30;  // bytes, both copies together (sb_net_set_frozen_cache_limit)
@@ -688,13 +691,8 @@ static int build_frozen_cache(sb_net *net, int upto, long maxB, long like) {
   const long Ns = net->Ns, Mo = net->layers[upto].M;
   int rc = drop_frozen_cache(net);
   if (rc) return rc;
-  // without the memory for both copies the caller goes on uncached (Hc_layer stays -1): not an error
-  if (dev_malloc(&net->Hc, (size_t)Ns * Mo * sizeof(T)) != hipSuccess ||
-      dev_malloc(&net->Hcp, (size_t)Ns * Mo * sizeof(T)) != hipSuccess) {
-    if (net->Hc) (void)hipFree(net->Hc);
-    net->Hc = nullptr;
-    return 0;
-  }
+  // without the memory the caller goes on uncached (Hc_layer stays -1): not an error
+  if (dev_malloc(&net->Hc, (size_t)Ns * Mo * sizeof(T)) != hipSuccess) return 0;
   long pass = std::min(Ns, pass_rows(net, maxB));
   if (upto > 0 && (rc = ensure_pass_act(net, pass, std::min(Ns, maxB), &pass))) return rc;
   for (long lo = 0; lo < Ns; lo += pass) {
@@ -732,52 +730,74 @@ static int net_train_batches(sb_net *net, int layer, long maxB, const int64_t *h
   // in whichever batch it is: those of a whole batch.
   const long like = last ? std::min(maxB, Ns) : 0;
   const bool permute = first_batch == 0;  // a later range continues the epoch already laid out
-  SB_REQUIRE(permute || net->Xp, "the epoch's first batches have not been run");
+  SB_REQUIRE(permute || (net->epoch_begun && (!last || net->Yp)), "the epoch's first batches have not been run");
   // a training step of a layer below the last changes what the cache was computed from
   if (!last && (rc = drop_frozen_cache(net))) return rc;
   const long Mprev = layer > 0 ? net->layers[layer - 1].M : 0;
   const bool cache_fits = last && layer > 0 &&
                           (net->Hc_layer == layer - 1 || frozen_cache_affordable(net, 2 * (size_t)Ns * Mprev * sizeof(T)));
+  // A dense output layer of a few units takes all of the call's batches in one launch, reading what it trains on in the
+  // epoch's order by itself: the data set, or the cached activations of the layers below.
+  const bool in_one = last && !target.plastic && train_skinny_epoch_supported<T>(target.M) && Ns < (1L << 31);
+  // images[idx, :]  (_cpu_base_backend.py:258-260)
+  auto lay_out_images = [&]() -> int {
+    if (!net->Xp) SB_HIP(dev_malloc(&net->Xp, (size_t)Ns * net->NF * net->esize));
+    net->images_laid = true;
+    // A first layer that walks row lists reads its input column by column: it gets the shuffled images a
+    // second time, in blocks of 16 rows (batches must then start on block boundaries); one kernel writes
+    // both copies from one read.
+    if (net->layers[0].rows && maxB % 16 == 0) {
+      if (!net->XpB) SB_HIP(dev_malloc(&net->XpB, (size_t)cdiv_l(Ns, 16) * 16 * net->NF * net->esize));
+      net->XpB_batch = maxB;
+      return launch_gather_rows_blocked<T>(st, (T *)net->XpB, (T *)net->Xp, (const T *)net->X, net->d_perm, Ns, net->NF);
+    }
+    net->XpB_batch = 0;
+    return launch_gather_rows<T>(st, (T *)net->Xp, (const T *)net->X, net->d_perm, Ns, net->NF);
+  };
   if (permute) {
     SB_REQUIRE(h_sample_perm, "sample order missing");
     for (long r = 0; r < Ns; r++)
       SB_REQUIRE(h_sample_perm[r] >= 0 && h_sample_perm[r] < Ns, "sample index out of range");
 
-    // images[idx, :] / labels[idx, :]  (_cpu_base_backend.py:258-260)
-    if (!net->Xp) SB_HIP(dev_malloc(&net->Xp, (size_t)Ns * net->NF * net->esize));
     if (last && !net->Yp) SB_HIP(dev_malloc(&net->Yp, (size_t)Ns * net->NC * net->esize));
     SB_HIP(hipEventSynchronize(net->perm_copied));  // staging buffer free again
     std::memcpy(net->h_perm, h_sample_perm, (size_t)Ns * sizeof(int64_t));
     SB_HIP(hipMemcpyAsync(net->d_perm, net->h_perm, (size_t)Ns * sizeof(int64_t), hipMemcpyHostToDevice,
                           st));
     SB_HIP(hipEventRecord(net->perm_copied, st));
-    // A first layer that walks row lists reads its input column by column: it gets the shuffled images a
-    // second time, in blocks of 16 rows (batches must then start on block boundaries); one kernel writes
-    // both copies from one read.
-    if (net->layers[0].rows && maxB % 16 == 0) {
-      if (!net->XpB) SB_HIP(dev_malloc(&net->XpB, (size_t)cdiv_l(Ns, 16) * 16 * net->NF * net->esize));
-      if ((rc = launch_gather_rows_blocked<T>(st, (T *)net->XpB, (T *)net->Xp, (const T *)net->X, net->d_perm, Ns,
-                                              net->NF)))
-        return rc;
-      net->XpB_batch = maxB;
-    } else {
-      if ((rc = launch_gather_rows<T>(st, (T *)net->Xp, (const T *)net->X, net->d_perm, Ns, net->NF)))
-        return rc;
-      net->XpB_batch = 0;
-    }
-    if (last)
+    net->epoch_begun = true;
+    net->images_laid = false;
+    if (last)  // labels[idx, :]
       if ((rc = launch_gather_rows<T>(st, (T *)net->Yp, (const T *)net->Y, net->d_perm, Ns, net->NC)))
         return rc;
     if (cache_fits) {
       if (net->Hc_layer != layer - 1 && (rc = build_frozen_cache<T>(net, layer - 1, maxB, like))) return rc;
-      if (net->Hc_layer == layer - 1 &&
-          (rc = launch_gather_rows<T>(st, (T *)net->Hcp, (const T *)net->Hc, net->d_perm, Ns, Mprev)))
-        return rc;
+      if (net->Hc_layer == layer - 1 && !in_one) {
+        if (!net->Hcp && dev_malloc(&net->Hcp, (size_t)Ns * Mprev * sizeof(T)) != hipSuccess) {
+          if ((rc = drop_frozen_cache(net))) return rc;
+        } else if ((rc = launch_gather_rows<T>(st, (T *)net->Hcp, (const T *)net->Hc, net->d_perm, Ns, Mprev))) {
+          return rc;
+        }
+      }
     } else if (last && (rc = drop_frozen_cache(net))) {
       return rc;
     }
   }
   const bool cached = cache_fits && net->Hc_layer == layer - 1;
+  if (in_one && (layer == 0 || cached)) {
+    const long lo = first_batch * maxB, rows = std::min(n_batches * maxB, Ns - lo);
+    if (rows > 0) {
+      rc = launch_train_skinny_epoch<T>(st, (const T *)(layer == 0 ? net->X : net->Hc), net->d_perm + lo,
+                                        (const T *)net->Yp + lo * net->NC, (T *)target.Cij, (T *)target.W,
+                                        (const T *)target.Ci, (const T *)target.Cj, (T *)target.Ci_alt, (T *)target.Cj_alt,
+                                        maxB, rows, target.N, target.H, target.Mc, (T)target.taupdt, (T)(target.taupdt / 2));
+      if (rc) return rc;
+      std::swap(target.Ci, target.Ci_alt);
+      std::swap(target.Cj, target.Cj_alt);
+    }
+    return finalize ? launch_update_bias<T>(st, (T *)target.bias, (const T *)target.Cj, (T)(target.taupdt / 2), target.M) : 0;
+  }
+  if (!cached && !net->images_laid && (rc = lay_out_images())) return rc;
 
   const long period = nb / (target.H + 1);  // _cpu_base_backend.py:297-299
   for (long i = first_batch; i < first_batch + n_batches; i++) {
@@ -1294,6 +1314,7 @@ int sb_net_training_done(sb_net *net) {
   rc |= free_dev(net->X); rc |= free_dev(net->Y); rc |= free_dev(net->Xp); rc |= free_dev(net->Yp);
   rc |= free_dev(net->XpB);
   net->XpB_batch = 0;
+  net->epoch_begun = net->images_laid = false;
   rc |= free_dev(net->Hc); rc |= free_dev(net->Hcp);
   net->Hc_layer = -1;
   rc |= free_dev(p);

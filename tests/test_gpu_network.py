@@ -174,6 +174,42 @@ def test_classifier_epochs_follow_changes_below_them_f64(hb):
 
 
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("N,H,Mc,Ns,B", [(3000, 1, 10, 700, 128), (1003, 1, 10, 350, 100), (37, 1, 2, 300, 32), (513, 4, 8, 300, 77),
+                                         (17, 1, 1, 5, 64), (16, 1, 17, 129, 64), (50, 1, 31, 200, 65), (200, 3, 4, 999, 500)])
+def test_classifier_epoch_in_one_launch_is_bit_identical(hb, dtype, N, H, Mc, Ns, B):
+    """All batches of a call in one launch: the bits of a launch per batch, batches that end inside and on the bounds of a
+    chunk, a short last one, columns and units that do not fill a workgroup, an epoch in two ranges."""
+    rng = np.random.default_rng(N + Mc)
+    X = (rng.random((Ns, N)) * (rng.random((Ns, N)) < 0.5)).astype(dtype)
+    Y = np.eye(H * Mc)[rng.integers(0, H * Mc, Ns)].astype(dtype)
+    cij = rng.random((N, H * Mc)).astype(dtype) * dtype(0.1)
+    orders = [rng.permutation(Ns) for _ in range(2)]
+
+    def network():
+        net = hb.Network(dtype)
+        layer = hb.DenseLayer(N, H, Mc, 0.01, (0.3, 0.1, 0.03), dtype)
+        net.add_layer(layer)
+        layer.Cij = cij
+        return net, layer
+
+    net, layer = network()
+    for order in orders:
+        for lo in range(0, Ns, B):
+            layer.train_step(X[order[lo:lo + B]], Y[order[lo:lo + B]])
+    other, whole = network()
+    other.net.initiate_training(X, Y)
+    other.net.train_epoch(0, B, orders[0], np.arange(H), 0)
+    batches = -(-Ns // B)
+    first = batches // 2
+    other.net.train_batches(0, B, orders[1], np.arange(H), 1, 0, first, False)
+    other.net.train_batches(0, B, orders[1], np.arange(H), 1, first, batches - first, True)
+    for name in ("Ci", "Cj", "Cij", "weights"):
+        assert np.array_equal(getattr(layer, name), getattr(whole, name)), name
+    layer.train_finalize()
+    assert np.array_equal(layer.bias, whole.bias)
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
 def test_classifier_epochs_without_the_activation_cache_are_bit_identical(hb, dtype):
     """The cache of the frozen layers' activations is an optimisation with a fallback: when it is not
     affordable (here: a limit of zero bytes, and a limit lowered while a cache is held) every step runs the
