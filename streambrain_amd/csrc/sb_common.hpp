@@ -214,9 +214,10 @@ struct BufferWindow {
       }
     }
   }
-  // one unconditional 16-byte access at byte offset `at` + `uniform` (kOutside as `at`: no access)
+  // one unconditional 16-byte access at byte offset `at` + `uniform` (kOutside as `at`: no access); AUX: cache policy
+  template <int AUX = 0>
   __device__ __forceinline__ void load_vec(T (&out)[Real<T>::VW], unsigned at, unsigned uniform) const {
-    const u4 raw = __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)at, (int)uniform, 0);
+    const u4 raw = __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)at, (int)uniform, AUX);
     const typename Real<T>::vec_t v = __builtin_bit_cast(typename Real<T>::vec_t, raw);
 #pragma unroll
     for (int e = 0; e < Real<T>::VW; e++) out[e] = v[e];

@@ -730,9 +730,14 @@ void k_train_fused(TrainArgs<T> a) {
 // tiles' row pieces to be merged with the neighbouring tile's, and the write-through policy of k_train_fused, which
 // suits matrices that stay in the memory-side cache, pays for that once they do not (sums included, batch 128: 12288 x
 // 3000 87 us non-temporal, 192 us written through, 123 us with the default policy; 12288 x 3200 91 / 119 / 116 us).
+// STREAM: Cij is read with non-temporal loads too, for matrices that nothing of is left in the memory-side cache from one
+// launch to the next: it then does not push the split batch out of the L2s (55296 x 20000, batch 256, all weights written:
+// 4.25 -> 3.45 ms; without the loads of the batch 2.94 ms, which is 4.5 TB/s, without the products 4.08 ms; tiles of 128
+// x 128, which ask for a third less of the batch: no difference).  A line that two tiles share is then fetched twice: rows
+// that are no whole number of lines lose by it (launch_train_fused has the rule).
 constexpr int kSplitTileI = 128, kSplitTileJ = 64, kSplitRows = 32;
 constexpr long kSplitBatch = 32;  // rows of the smallest batch that is split
-template <bool VEC, int MB>
+template <bool VEC, int MB, bool STREAM>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4)))
 void k_train_split(TrainArgs<float> a, SplitBatch sp) {
   using R = Real<float>;
@@ -824,7 +829,7 @@ void k_train_split(TrainArgs<float> a, SplitBatch sp) {
     for (int r = 0; r < 2; r++)
 #pragma unroll
       for (int v = 0; v < 4; v++) {
-        cwin.load_vec(cpre[r][v], at(r, v), 0);
+        cwin.template load_vec<STREAM ? kNonTemporal : 0>(cpre[r][v], at(r, v), 0);
 #pragma unroll
         for (int e = 0; e < MB; e++) mb[r][v][e] = mwin.load((r0 + 16 * r + v) * (unsigned)a.H + hc[e], 0);
       }

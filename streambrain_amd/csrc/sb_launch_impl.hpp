@@ -514,9 +514,19 @@ int launch_train_fused(hipStream_t st, const T *x, const T *y, T *Cij, T *W, con
       a.by_panel = FastDiv::of(a.tiles_i * a.panel_cols);
       launch(k_trace_sums<T, true>, sums, true, false, sp);
       const dim3 tiles((unsigned)(a.tiles_i * a.tiles_j) + a.prefetch_groups);
-      if (vec && one_byte) launch(k_train_split<true, 1>, tiles, false, true, sp);
-      else if (vec) launch(k_train_split<true, VW>, tiles, false, true, sp);
-      else launch(k_train_split<false, VW>, tiles, false, true, sp);  // (one_byte implies vec)
+      // Non-temporal loads of Cij from 320 MiB of it (time without over with them: rows of whole lines, 4000 to 20000
+      // columns, 100 to 256 batch rows, 244 MiB 0.99, 343 MiB 1.06 to 1.08, 600 MiB to 4.2 GiB 1.05 to 1.23; 32 batch rows
+      // 1.0; 6000 columns, 1.1 GiB 1.07), where rows are whole half lines or many batch rows pass by (3000 to 13400
+      // columns, 256 and 300 rows 1.05 to 1.12; up to 128 rows, 450 MiB to 1.1 GiB, 0.77 to 0.89).
+      const bool stream = N * M * (long)sizeof(T) > (320L << 20) && (M % 16 == 0 || B >= 192);
+      auto launch_tiles = [&](auto streamed) {
+        constexpr bool S = decltype(streamed)::value;
+        if (vec && one_byte) launch(k_train_split<true, 1, S>, tiles, false, true, sp);
+        else if (vec) launch(k_train_split<true, VW, S>, tiles, false, true, sp);
+        else launch(k_train_split<false, VW, S>, tiles, false, true, sp);  // (one_byte implies vec)
+      };
+      if (stream) launch_tiles(std::true_type{});
+      else launch_tiles(std::false_type{});
       SB_LAUNCH_CHECK();
       return 0;
     }
