@@ -637,6 +637,10 @@ void k_train_fused(TrainArgs<T> a) {
 
   // ---- epilogue: decay + clamp and the Cij stores first (they need nothing from the other wavefronts),
   // then, once the reciprocals are published, weight, mask and the W stores
+  // In doubles an epilogue is some hundred vector instructions (the logarithms), which beside wavefronts that stream MFMAs
+  // advance by one per MFMA slot; ahead of them they advance at nearly their own rate, and the matrix cores lose little
+  // (1568 x 10000, batch 512, all weights written: 310 -> 295 us; floats: no difference).
+  if constexpr (sizeof(T) == 8) __builtin_amdgcn_s_setprio(3);
   const T scale = a.invB * a.tau;
   T cn[4][NG][VW];
 #pragma unroll
@@ -666,21 +670,25 @@ void k_train_fused(TrainArgs<T> a) {
   if (VEC && MB == 1 && !slow) {
     // short form: no row or column is dead, no argument is tiny; a vector lies in one hypercolumn.
     // Where the mask is 0 the weight is 0, and when the caller vouches that W holds 0 there already,
-    // such vectors are not stored, and a wavefront without a connected vector computes nothing.
+    // such vectors are not stored.  A wavefront without a connected vector computes nothing then, and in doubles, where
+    // that is worth the branch, when all of W is written too (density 0.1: 318 -> 310 us).
 #pragma unroll
     for (int v = 0; v < 4; v++)
 #pragma unroll
       for (int g = 0; g < NG; g++) {
         const bool connected = !masked || mb[v][g][0] != 0;
-        if (a.w_masked && __builtin_amdgcn_ballot_w64(connected) == 0) continue;
+        const bool none = __builtin_amdgcn_ballot_w64(connected) == 0;  // (uniform)
+        if (a.w_masked && none) continue;
         T wv[VW];
 #pragma unroll
-        // (max(max(cn, 0), cthr^4) = max(cn, cthr^4), cthr^4 as well when cn is NaN)
-        for (int e = 0; e < VW; e++)
-          wv[e] = R::wlog_normal(R::max_floor(cn[v][g][e], a.cthr4) * rci[v] * rcj[g][e]);
-        if (!a.w_masked) {  // uniform
+        for (int e = 0; e < VW; e++) wv[e] = T(0);
+        if (sizeof(T) == 4 || !none) {
 #pragma unroll
-          for (int e = 0; e < VW; e++) wv[e] = connected ? wv[e] : T(0);
+          // (max(max(cn, 0), cthr^4) = max(cn, cthr^4), cthr^4 as well when cn is NaN)
+          for (int e = 0; e < VW; e++) {
+            wv[e] = R::wlog_normal(R::max_floor(cn[v][g][e], a.cthr4) * rci[v] * rcj[g][e]);
+            if (!a.w_masked) wv[e] = connected ? wv[e] : T(0);  // (uniform)
+          }
         }
         wwin.template store_vec<AUX>(wv, (a.w_masked && !connected) ? kOutside : tat[g], v * vstep);
       }
@@ -698,12 +706,25 @@ void k_train_fused(TrainArgs<T> a) {
 #pragma unroll
       for (int e = 0; e < MB; e++) connected = connected || mb[v][g][e] != 0;
       if (a.w_masked && __builtin_amdgcn_ballot_w64(connected) == 0) continue;
-      T wv[VW];
+      bool keep[VW], any = false;
 #pragma unroll
       for (int e = 0; e < VW; e++) {
-        const T wgt = R::wlog(R::max_floor(cn[v][g][e], a.cthr4) * rci[v] * rcj[g][e]);
-        const bool keep = row_live && !(rcj[g][e] < T(0)) && (MB == 1 || !masked || mb[v][g][e] != 0);
-        wv[e] = keep ? wgt : T(0);
+        keep[e] = row_live && !(rcj[g][e] < T(0)) && (MB == 1 || !masked || mb[v][g][e] != 0);
+        any = any || keep[e];
+      }
+      T wv[VW];
+#pragma unroll
+      for (int e = 0; e < VW; e++) wv[e] = T(0);
+      if (sizeof(T) == 4 || __builtin_amdgcn_ballot_w64(any) != 0) {  // (uniform)
+        // (an argument that is positive and normal where the weight is dropped: in doubles the negative reciprocal of a dead
+        // row would send the whole wavefront through the library's logarithm as well.  Images of which some pixels are never
+        // on have dead rows in most tiles: 1568 x 10000, batch 512: 307 -> 286 us)
+#pragma unroll
+        for (int e = 0; e < VW; e++) {
+          const T arg = R::max_floor(cn[v][g][e], a.cthr4) * rci[v] * rcj[g][e];
+          const T wgt = R::wlog(sizeof(T) == 4 || keep[e] ? arg : T(1));
+          wv[e] = keep[e] ? wgt : T(0);
+        }
       }
       wwin.template store<VEC, AUX>(wv, tat[g], v * vstep, ecol[g], a.M);
     }
