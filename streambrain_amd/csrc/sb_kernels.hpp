@@ -560,6 +560,26 @@ __global__ __launch_bounds__(256) void k_copy_pair(T *dst1, const T *src1, size_
   }
 }
 
+// dst[0 .. n) = src[0 .. n) into pinned host memory, then *flag = ticket there: a host thread that waits for the flag has the
+// data 4 us earlier than one that waits for an event behind the kernel.  The stores go past the caches as they happen
+// (system scope); a workgroup counts itself once all of its own have been acknowledged, and the last to do so sets the flag
+// and clears the counter for the next launch.
+template <int UNUSED>
+__global__ __launch_bounds__(256) void k_copy_out(uint32_t *dst, const uint32_t *src, size_t n, unsigned *counter,
+                                                  unsigned *flag, unsigned ticket) {
+  const size_t stride = (size_t)gridDim.x * 256;
+  for (size_t e = (size_t)blockIdx.x * 256 + threadIdx.x; e < n; e += stride)
+    __hip_atomic_store(dst + e, src[e], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+  const unsigned before = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (before + 1 != gridDim.x) return;
+  __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __hip_atomic_store(flag, ticket, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 }  // namespace sb
 
 #include "sb_k_forward.hpp"

@@ -14,6 +14,17 @@ int launch_fill_bytes(hipStream_t st, void *dst, int value, size_t bytes) {
   return 0;
 }
 
+int launch_copy_out(hipStream_t st, void *dst, const void *src, size_t words, unsigned *counter, unsigned *flag,
+                    unsigned ticket) {
+  SB_REQUIRE(dst && src && counter && flag && words > 0, "null pointer");
+  const size_t blocks = (words + 255) / 256 < 256 ? (words + 255) / 256 : 256;
+  ProfScope prof_(st, K_FILL);
+  hipLaunchKernelGGL((k_copy_out<0>), dim3((unsigned)blocks), dim3(256), 0, st, (uint32_t *)dst, (const uint32_t *)src,
+                     words, counter, flag, ticket);
+  SB_LAUNCH_CHECK();
+  return 0;
+}
+
 int launch_mask_rows(hipStream_t st, int *rows, int *row_cnt, const uint8_t *wmask, long N, long H,
                      long cap, long h0, long count) {
   SB_REQUIRE(rows && row_cnt && wmask, "null pointer");

@@ -183,5 +183,9 @@ int launch_fill(hipStream_t st, T *dst, T value, size_t n);
 template <typename T>
 int launch_copy_pair(hipStream_t st, T *dst1, const T *src1, size_t n1, T *dst2, const T *src2, size_t n2);
 int launch_fill_bytes(hipStream_t st, void *dst, int value, size_t bytes);
+// `words` 32-bit words into pinned host memory, then *flag = ticket (pinned too).  counter: device memory that is zero ahead
+// of the launch and behind it.
+int launch_copy_out(hipStream_t st, void *dst, const void *src, size_t words, unsigned *counter, unsigned *flag,
+                    unsigned ticket);
 
 }  // namespace sb

@@ -695,6 +695,35 @@ def test_state_round_trip_around_the_sizes_that_change_the_way_of_the_copy(units
         _capi.check(lib.sb_net_destroy(net))
 
 
+@pytest.mark.parametrize("N,M,B", [(7, 40, 5), (100, 48, 32), (784, 60, 33), (2000, 50, 128), (3000, 64, 77)])
+def test_calls_with_small_copies_reuse_the_ring(hb, N, M, B):
+    """Training steps one after the other, which read nothing back (the ring of pinned chunks goes round), and with
+    activations and state read in between: the same bits, and what is read is what the steps so far have left."""
+    rng = np.random.default_rng(N)
+    data = [(rng.random((B, N)).astype(np.float32), rng.random((B, M)).astype(np.float32)) for _ in range(11)]
+
+    def network():
+        np.random.seed(N)
+        net = hb.Network(np.float32)
+        layer = hb.DenseLayer(N, M // 2, 2, 0.05, (0.3, 0.5, 0.15), np.float32)
+        net.add_layer(layer)
+        return net, layer
+
+    quiet, talking = network(), network()
+    for x, y in data:
+        quiet[1].train_step(x, y)
+    before = None
+    for x, y in data:
+        talking[1].train_step(x, y)
+        act = talking[1].compute_activation(x)
+        ci = talking[1].Ci
+        assert np.all(np.isfinite(act)) and (before is None or not np.array_equal(ci, before))
+        assert np.allclose(act.reshape(B, -1, 2).sum(2), 1, atol=1e-6)
+        before = ci
+    for name in ("Ci", "Cj", "Cij", "weights"):
+        assert np.array_equal(getattr(quiet[1], name), getattr(talking[1], name)), name
+
+
 def test_state_of_two_networks_from_two_threads():
     """The pinned ring that state goes through is one for all networks: small arrays (moved by a kernel) and big ones (by
     the copy engine, in pieces) of two networks, written and read back by a thread each, keep apart."""
