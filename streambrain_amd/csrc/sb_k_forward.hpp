@@ -236,10 +236,11 @@ __device__ __forceinline__ void forward_finish(const typename Real<T>::acc_t (&a
 // One workgroup per CU is all the tiling provides at small batch sizes, so the register allocator is told
 // to aim for NWAVES/4 wavefronts per SIMD and spend the registers on loads in flight instead.
 //
-// LW: column blocks of the LAST group (1..VW).  A hypercolumn of 100 columns needs 7 blocks of 16, not
-// 8: with LW = 3 the last group's lanes load LW consecutive columns (12 bytes) instead of VW, and a
-// quarter of that group's MFMAs disappears.  The launcher picks LW < VW only when no vector of the last
-// group straddles the end of the tile.
+// LW: column blocks of the LAST group (1..VW).  A hypercolumn of 67 columns needs 5 blocks of 16, not
+// 8: with LW = 1 the last group's lanes load LW consecutive columns (4 bytes) instead of VW, and three quarters
+// of that group's MFMAs disappear (1003 -> 13 x 67, batch 100: 13.7 -> 10.9 us; 2000 -> 60 x 67, batch 256: 76.8 -> 56.3 us,
+// doubles, which had whole powers of two of groups, 147 -> 100 us; 1003 -> 13 x 10 8.1 -> 6.6 us).  A vector of the last
+// group that straddles the end of the tile fetches a few of its neighbour's columns, as above.
 //
 // RB: row blocks per workgroup.  The tile is 16*RB batch rows, every W vector a lane loads feeds RB MFMAs
 // instead of one, and W crosses the L2 -> L1 path 1/RB as often: for batches of many rows, where that path

@@ -33,7 +33,7 @@ static inline int device_cu_count() {
 }
 
 // ------------------------------------------------------------------------------------------- forward
-template <typename T, int NG, bool FUSE>
+template <typename T, int NG, bool FUSE, int LW = Real<T>::VW>
 static int forward_variant(hipStream_t st, ForwardArgs<T> a, bool vec) {
   ProfScope prof_(st, K_FORWARD);
   a.by_batch_tiles = FastDiv::of(a.batch_tiles);
@@ -45,9 +45,9 @@ static int forward_variant(hipStream_t st, ForwardArgs<T> a, bool vec) {
     return -1;
   }
   if (vec)
-    hipLaunchKernelGGL((k_forward<T, NG, FUSE, true, 8>), dim3((unsigned)grid), dim3(512), 0, st, a);
+    hipLaunchKernelGGL((k_forward<T, NG, FUSE, true, 8, LW>), dim3((unsigned)grid), dim3(512), 0, st, a);
   else
-    hipLaunchKernelGGL((k_forward<T, NG, FUSE, false, 8>), dim3((unsigned)grid), dim3(512), 0, st, a);
+    hipLaunchKernelGGL((k_forward<T, NG, FUSE, false, 8, LW>), dim3((unsigned)grid), dim3(512), 0, st, a);
   SB_LAUNCH_CHECK();
   return 0;
 }
@@ -170,8 +170,21 @@ int launch_forward_classify(hipStream_t st, T *act, const T *x, const T *W, cons
         return 0;
       }
     }
-    if (need <= 1) return forward_variant<T, 1, true>(st, a, vec);
-    if (need <= 2) return forward_variant<T, 2, true>(st, a, vec);
+    // As many blocks of 16 columns as the hypercolumn has, up to 8; wider ones in whole groups.
+    auto blocks = [&](auto count) {
+      constexpr int NB = decltype(count)::value, NG = (NB + VW - 1) / VW;
+      return forward_variant<T, NG, true, NB - (NG - 1) * VW>(st, a, vec);
+    };
+    switch (nblocks) {
+      case 1: return blocks(std::integral_constant<int, 1>{});
+      case 2: return blocks(std::integral_constant<int, 2>{});
+      case 3: return blocks(std::integral_constant<int, 3>{});
+      case 4: return blocks(std::integral_constant<int, 4>{});
+      case 5: return blocks(std::integral_constant<int, 5>{});
+      case 6: return blocks(std::integral_constant<int, 6>{});
+      case 7: return blocks(std::integral_constant<int, 7>{});
+      case 8: return blocks(std::integral_constant<int, 8>{});
+    }
     if (need <= 4) return forward_variant<T, 4, true>(st, a, vec);
     if constexpr (sizeof(T) == 8) return forward_variant<T, 7, true>(st, a, vec);
   }
@@ -355,6 +368,7 @@ int launch_forward_rows(hipStream_t st, T *act, const T *x, const T *W, const T 
   const RowsGroups groups = forward_rows_groups<T>(Mc);
   if (groups.last > 0 && cdiv(Mc, 16) == 7) return forward_rows_variant<T, NGL, LWL>(st, a, like);
   if (groups.last > 0) return forward_rows_variant<T, NGM, 1>(st, a, like);
+  if (Mc <= 16) return forward_rows_variant<T, 1, 1>(st, a, like);  // (one block of columns)
   if (groups.n == 1) return forward_rows_variant<T, 1>(st, a, like);
   if (groups.n == 2) return forward_rows_variant<T, 2>(st, a, like);
   if (groups.n == 4) return forward_rows_variant<T, 4>(st, a, like);

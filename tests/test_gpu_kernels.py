@@ -748,6 +748,32 @@ def test_forward_with_few_tiles(k, dtype, B, N, H, Mc):
 
 
 @pytest.mark.parametrize("dtype", DT)
+@pytest.mark.parametrize("Mc", [5, 10, 16, 17, 31, 33, 47, 49, 64, 66, 67, 80, 81, 95, 97, 101, 111, 113, 127, 128])
+@pytest.mark.parametrize("B,N", [(17, 203), (33, 1024)])
+def test_forward_in_blocks_of_columns(k, dtype, Mc, B, N):
+    """Hypercolumns of one to eight blocks of 16 columns, full ones and ones that end inside a lane's vector, the last of them
+    at the end of W, dense and (where the row lists take the shape) over connected rows."""
+    rng = np.random.default_rng(Mc)
+    H = 9
+    M = H * Mc
+    wmask = (rng.random((N, H)) < 0.4).astype(np.uint8)
+    x = rng.random((B, N)).astype(dtype)
+    W = (rng.standard_normal((N, M)) * 4 / np.sqrt(N)).astype(dtype)
+    bias = rng.standard_normal(M).astype(dtype)
+
+    def want(w):
+        z = (x.astype(np.float64) @ w.astype(np.float64) + bias).reshape(B, H, Mc)
+        e = np.exp(z - z.max(2, keepdims=True))
+        return (e / e.sum(2, keepdims=True)).reshape(B, M)
+
+    assert_close(k.compute_activation(W, bias, x, H, Mc), want(W), dtype, "dense", scale=10)
+    if Mc % (4 if dtype is np.float32 else 2) == 0:
+        W = W * np.repeat(wmask, Mc, axis=1).astype(dtype)
+        for blocked in (False, True):
+            assert_close(k.compute_activation_rows(W, bias, x, wmask, H, Mc, blocked), want(W), dtype, "rows", scale=10)
+
+
+@pytest.mark.parametrize("dtype", DT)
 @pytest.mark.parametrize("B,N,H,Mc,more", [(100, 34000, 4, 12, 1552), (33, 3000, 5, 100, 448), (128, 2500, 9, 200, 272),
                                            (7, 9000, 3, 64, 704), (16, 2100, 2, 36, 1040), (80, 2600, 3, 128, 704)])
 def test_chains_of_the_row_lists(k, dtype, B, N, H, Mc, more):
