@@ -105,7 +105,8 @@ int launch_mask_rows(hipStream_t st, int *rows, int *row_cnt, const uint8_t *wma
 template <typename T>
 int launch_softmax(hipStream_t st, T *act, long B, long H, long Mc);
 // Fused Ci/Cj/Cij + weights (+ regularised bias when bias_mode == 1, + mask when wmask != nullptr).
-// Reads the old traces from Ci/Cj and writes the new ones to Ci_next/Cj_next (distinct buffers).
+// Reads the old traces from Ci/Cj and writes the new ones to Ci_next/Cj_next: distinct buffers, or both the same where
+// train_in_place_supported (a launch of its own then forms the traces).
 // W == nullptr: the traces only.
 // w_masked: the caller vouches that W is zero wherever wmask is 0; such entries may then be left alone.
 // prefetch / prefetch_bytes: memory the next launches read first (the next batch), pulled into the
@@ -120,6 +121,8 @@ int launch_train_fused(hipStream_t st, const T *x, const T *y, T *Cij, T *W, con
 // sizes; 0: none.  Without it (nullptr) the launch does without the kernel that needs it.
 template <typename T>
 size_t train_split_bytes(long B, long N, long H, long Mc);
+template <typename T>
+bool train_in_place_supported(const void *split, long B, long N, long H, long Mc, T taupdt);
 // launch_train_fused for `rows` rows in batches of B, one after the other, of a layer without mask and regularised bias of a
 // few units (train_skinny_epoch_supported).  Batch row b is x[order[b]] (order: device memory) and y[b].
 template <typename T>

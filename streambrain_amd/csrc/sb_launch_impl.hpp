@@ -423,6 +423,34 @@ size_t train_split_bytes(long B, long N, long H, long Mc) {
   return (size_t)(xw + yw) * 6 * (size_t)(cdiv(B, kSumRows) * kSumRows) + (size_t)(xw + yw) / 64 * sizeof(int);
 }
 
+// x^T y through the pieces: the scratch is there, the layer is one for it, and the factor of the sums stays normal with the
+// pieces' scale in it.
+template <typename T>
+static bool train_splits(const void *split, long B, long N, long H, long Mc, T tau) {
+  return sizeof(T) == 4 && split && train_split_bytes<T>(B, N, H, Mc) > 0 &&
+         (float)((T)1 / (T)B * tau) * kSplitUnscale >= 0x1p-126f;
+}
+
+// Every tile adds up the batch's x and y columns for its own rows and columns, which with many tile
+// rows and columns is most of the kernel's vector arithmetic (43 % at 65536 x 100000, batch 1024).
+// From one and a half rounds of workgroups on (floats with more than 32 rows; doubles: two and a half), a small launch
+// computes the new traces once and the tiles read them (floats: where k_train_split does not run).  Timed, 4096
+// inputs, batch 128, floats, with / without that launch: 23.7 / 22.5 us at 1.05 rounds, 29.3 / 29.9 at 1.5, 34.6 /
+// 35.6 at 2, 45.5 / 48.5 at 3, 67.1 / 69.2 at 5; doubles: 48.1 / 47.3 at 1.6 rounds, 55.8 / 54.3 at 2, 110.3 /
+// 113.7 at 2.5.  (Whole vectors only.)
+template <typename T>
+static bool train_sums_apart(long B, long N, long H, long Mc) {
+  const long pre_from = sizeof(T) == 8 ? 5 * 4 : 3 * 5;  // in half workgroups per CU
+  return H * Mc > 32 && Mc % Real<T>::VW == 0 &&
+         2 * cdiv(N, 64) * cdiv(H * Mc, 64) >= pre_from * device_cu_count() && (sizeof(T) == 8 || B > 32);
+}
+// A launch of its own that forms the traces reads and writes each once, in one thread, and nobody else reads the old ones.
+template <typename T>
+bool train_in_place_supported(const void *split, long B, long N, long H, long Mc, T taupdt) {
+  if (B <= 0 || N <= 0 || H <= 0 || Mc <= 0) return false;
+  return train_splits<T>(split, B, N, H, Mc, TraceScalars<T>::from(taupdt, T(0)).tau) || train_sums_apart<T>(B, N, H, Mc);
+}
+
 template <typename T>
 int launch_train_fused(hipStream_t st, const T *x, const T *y, T *Cij, T *W, const T *Ci, const T *Cj,
                        T *Ci_next, T *Cj_next, const uint8_t *wmask, int bias_mode, T *bias, T *kbi,
@@ -430,8 +458,9 @@ int launch_train_fused(hipStream_t st, const T *x, const T *y, T *Cij, T *W, con
                        bool w_masked, const void *prefetch, size_t prefetch_bytes, void *split) {
   constexpr int VW = Real<T>::VW;
   SB_REQUIRE(x && y && Cij && Ci && Cj && Ci_next && Cj_next, "null pointer");  // W may be null: traces only
-  SB_REQUIRE(Ci != Ci_next && Cj != Cj_next, "old and new traces must be distinct buffers");
   SB_REQUIRE(bias_mode == 0 || (bias && kbi), "bias update needs bias and kbi");
+  const bool in_place = Ci == Ci_next && Cj == Cj_next;
+  SB_REQUIRE(in_place || (Ci != Ci_next && Cj != Cj_next), "old and new traces: the same buffers or distinct ones");
   SB_REQUIRE(B > 0 && N > 0 && H > 0 && Mc > 0, "sizes must be positive");
   const long M = H * Mc;
   SB_REQUIRE(M < (1L << 31) && N < (1L << 31) && B < (1L << 31), "dimension too large");
@@ -467,6 +496,7 @@ int launch_train_fused(hipStream_t st, const T *x, const T *y, T *Cij, T *W, con
   // (a multiple of 8: they come first in the grid, and the tiles behind them keep their XCDs)
   a.prefetch_groups = a.prefetch_lines ? (unsigned)std::min<long>(512, 8 * cdiv(a.prefetch_lines, 8 * 256)) : 0u;
   if (M <= 32) {  // a handful of output units: plain vector arithmetic
+    SB_REQUIRE(!in_place, "traces of this layer cannot be updated in place");
     const long rows = skinny_train_rows(M);
     SB_REQUIRE(cdiv(N, rows) < (1L << 31), "too many rows for one launch");
     ProfScope prof_(st, K_TRAIN_FUSED, true);
@@ -510,8 +540,7 @@ int launch_train_fused(hipStream_t st, const T *x, const T *y, T *Cij, T *W, con
   };
   const dim3 sums((unsigned)(cdiv(N, 64) + cdiv(M, 64)));
   if constexpr (sizeof(T) == 4) {
-    // (the factor of the sums stays normal with the pieces' scale in it)
-    if (split && train_split_bytes<T>(B, N, H, Mc) > 0 && a.invB * a.tau * kSplitUnscale >= 0x1p-126f) {
+    if (train_splits<T>(split, B, N, H, Mc, a.tau)) {
       SplitBatch sp;
       sp.x_width = (unsigned)(cdiv(N, kSplitTileI) * kSplitTileI);
       sp.y_width = (unsigned)(cdiv(M, kSplitTileJ) * kSplitTileJ);
@@ -545,16 +574,10 @@ int launch_train_fused(hipStream_t st, const T *x, const T *y, T *Cij, T *W, con
       return 0;
     }
   }
-  // Every tile adds up the batch's x and y columns for its own rows and columns, which with many tile
-  // rows and columns is most of the kernel's vector arithmetic (43 % at 65536 x 100000, batch 1024).
-  // From one and a half rounds of workgroups on (floats with more than 32 rows; doubles: two and a half), a small launch
-  // computes the new traces once and the tiles read them (floats: where k_train_split does not run).  Timed, 4096
-  // inputs, batch 128, floats, with / without that launch: 23.7 / 22.5 us at 1.05 rounds, 29.3 / 29.9 at 1.5, 34.6 /
-  // 35.6 at 2, 45.5 / 48.5 at 3, 67.1 / 69.2 at 5; doubles: 48.1 / 47.3 at 1.6 rounds, 55.8 / 54.3 at 2, 110.3 /
-  // 113.7 at 2.5.
   const long ntiles = a.tiles_i * a.tiles_j;
   const bool one_round = ntiles <= train_tiles_of_one_round<T>();
-  const long pre_from = sizeof(T) == 8 ? 5 * 4 : 3 * 5;  // in half workgroups per CU
+  const bool apart = train_sums_apart<T>(B, N, H, Mc);
+  SB_REQUIRE(!in_place || apart, "traces of this layer cannot be updated in place");
   if constexpr (sizeof(T) == 8) {
     // Cij and W together beyond what the memory-side cache keeps: non-temporal stores (whole steps, batch 128, written
     // through / non-temporal: 7208 x 3000, 330 MiB, 190 / 141 us, 9174 x 3000, 420 MiB, 238 / 180, 20000 rows
@@ -572,7 +595,7 @@ int launch_train_fused(hipStream_t st, const T *x, const T *y, T *Cij, T *W, con
       return 0;
     }
   }
-  if (vec && one_byte && 2 * ntiles >= pre_from * device_cu_count() && (sizeof(T) == 8 || B > 32)) {
+  if (apart) {
     launch(k_trace_sums<T>, sums, true, false, SplitBatch{});
     launch(k_train_fused<T, KCH, true, 1, true>, grid, false, true);
   } else if (vec && one_byte && one_round)
@@ -897,6 +920,7 @@ int launch_copy_pair(hipStream_t st, T *dst1, const T *src1, size_t n1, T *dst2,
                                      T *, T *, const uint8_t *, int, T *, T *, long, long, long, long, \
                                      T, T, T, T, T, bool, const void *, size_t, void *);              \
   template size_t train_split_bytes<T>(long, long, long, long);                                       \
+  template bool train_in_place_supported<T>(const void *, long, long, long, long, T);                 \
   template bool train_skinny_epoch_supported<T>(long);                                                \
   template int launch_train_skinny_epoch<T>(hipStream_t, const T *, const int64_t *, const T *, T *,  \
                                             T *, const T *, const T *, T *, T *, long, long, long,    \

@@ -465,15 +465,16 @@ static int train_in_place(const T *x, const T *y, T *Cij, T *W, T *Ci, T *Cj, co
   const long M = H * Mc;
   SB_REQUIRE(N > 0 && M > 0, "sizes must be positive");
   std::lock_guard<std::mutex> lock(g_work_mutex);
-  int rc = fixed_scratch ? 0 : ensure_trace_scratch(N + M);
-  if (rc) return rc;
-  T *ci_next = fixed_scratch ? fixed_scratch : (T *)g_ctx.trace_next, *cj_next = ci_next + N;
   const bool as_noalloc = !wmask && N + M <= (long)SB_NOALLOC_MAX_UNITS;
-  const size_t split = train_split_bytes<T>(B, N, H, Mc);
-  rc = launch_train_fused<T>(st, x, y, Cij, W, Ci, Cj, ci_next, cj_next, wmask, bias_mode, bias, kbi, B,
-                             N, H, Mc, taupdt, cthr, khalf, pmin, taubdt, false, nullptr, 0,
-                             as_noalloc || split > kWorkLimit ? nullptr : optional_scratch(g_work, split));
+  const size_t split_bytes = train_split_bytes<T>(B, N, H, Mc);
+  void *const split = as_noalloc || split_bytes > kWorkLimit ? nullptr : optional_scratch(g_work, split_bytes);
+  const bool in_place = train_in_place_supported<T>(split, B, N, H, Mc, taupdt);
+  int rc = fixed_scratch || in_place ? 0 : ensure_trace_scratch(N + M);
   if (rc) return rc;
+  T *ci_next = in_place ? Ci : fixed_scratch ? fixed_scratch : (T *)g_ctx.trace_next, *cj_next = in_place ? Cj : ci_next + N;
+  rc = launch_train_fused<T>(st, x, y, Cij, W, Ci, Cj, ci_next, cj_next, wmask, bias_mode, bias, kbi, B,
+                             N, H, Mc, taupdt, cthr, khalf, pmin, taubdt, false, nullptr, 0, split);
+  if (rc || in_place) return rc;
   return launch_copy_pair<T>(st, Ci, ci_next, (size_t)N, Cj, cj_next, (size_t)M);
 }
 
