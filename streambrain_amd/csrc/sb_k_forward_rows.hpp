@@ -33,10 +33,14 @@ constexpr int forward_rows_regs(int NG, int rb) {  // registers of the three, in
   return (2 * VW * NG * VW + rb * NG * VW * 4 + 2 * rb * VW) * D;
 }
 constexpr int kRowsRegsTwoWaves = 150, kRowsRegsThreeWaves = 104;  // measured: no spills up to these
-template <typename T, int NG, int RB>
+// By the column blocks there are: 13 of them in floats (200 columns) still go twice into a SIMD's registers (203 and 234 of
+// 256; 5000 rows of 784 -> 15 x 200, density 0.1: 104 us with one wavefront, 76 with two; 300 rows of 4000 -> 60 x 200
+// 56.8 / 50.0).
+template <typename T, int NG, int RB, int LW>
 constexpr int forward_rows_waves_per_simd() {
-  constexpr int regs = forward_rows_regs<T>(NG, RB);
-  return regs <= kRowsRegsThreeWaves ? 3 : regs <= kRowsRegsTwoWaves ? 2 : 1;
+  constexpr int VW = Real<T>::VW, blocks = (NG - 1) * VW + LW;
+  constexpr int regs = (2 * VW * blocks + RB * blocks * 4 + 2 * RB * VW) * ((int)sizeof(T) / 4);
+  return regs <= kRowsRegsThreeWaves ? 3 : regs <= (RB == 1 && sizeof(T) == 4 ? 170 : kRowsRegsTwoWaves) ? 2 : 1;
 }
 
 // A workgroup owns 16 batch rows x one hypercolumn (as k_forward with FUSE).  The hypercolumn's row list
@@ -68,8 +72,8 @@ constexpr int forward_rows_waves_per_simd() {
 template <typename T, int NG, int NWAVES, int RB = 1, bool XT = false, int LW = Real<T>::VW, int SEG = 2048,
           bool WIDE = false>
 __global__ __launch_bounds__(64 * NWAVES)
-__attribute__((amdgpu_waves_per_eu(forward_rows_waves_per_simd<T, NG, RB>(),
-                                   forward_rows_waves_per_simd<T, NG, RB>())))
+__attribute__((amdgpu_waves_per_eu(forward_rows_waves_per_simd<T, NG, RB, LW>(),
+                                   forward_rows_waves_per_simd<T, NG, RB, LW>())))
 void k_forward_rows(ForwardRowsArgs<T> ar) {
   const ForwardArgs<T> &a = ar.f;
   constexpr int VW = Real<T>::VW;
