@@ -469,7 +469,10 @@ static int train_in_place(const T *x, const T *y, T *Cij, T *W, T *Ci, T *Cj, co
   const size_t split_bytes = train_split_bytes<T>(B, N, H, Mc);
   void *const split = as_noalloc || split_bytes > kWorkLimit ? nullptr : optional_scratch(g_work, split_bytes);
   const bool in_place = train_in_place_supported<T>(split, B, N, H, Mc, taupdt);
-  int rc = fixed_scratch || in_place ? 0 : ensure_trace_scratch(N + M);
+  // Traces that are formed in place only thanks to the optional scratch have theirs kept ready as well: the same call, once
+  // it is captured, does without that scratch and has to find room for the new traces without allocating.
+  const bool never_needed = train_in_place_supported<T>(nullptr, B, N, H, Mc, taupdt);
+  int rc = fixed_scratch || never_needed ? 0 : ensure_trace_scratch(N + M);
   if (rc) return rc;
   T *ci_next = in_place ? Ci : fixed_scratch ? fixed_scratch : (T *)g_ctx.trace_next, *cj_next = in_place ? Cj : ci_next + N;
   rc = launch_train_fused<T>(st, x, y, Cij, W, Ci, Cj, ci_next, cj_next, wmask, bias_mode, bias, kbi, B,

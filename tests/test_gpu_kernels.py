@@ -667,9 +667,11 @@ def test_train_pass_of_big_double_layers_with_odd_rows(k, B, N, H, Mc):
     assert_close(got["weights"], w * np.repeat(st["wmask"], Mc, axis=1), np.float64, "W")
 
 
-def test_captured_train_step_does_without_the_scratch_that_later_calls_replace(k):
+@pytest.mark.parametrize("B,N,H,Mc", [(128, 4353, 30, 100), (128, 4353, 60, 50), (32, 12288, 30, 100)])
+def test_captured_train_step_does_without_the_scratch_that_later_calls_replace(k, B, N, H, Mc):
     """A big float step recorded into a graph takes the kernels that need no optional scratch: it allocates nothing, and
-    its replays give the eager result, also after an eager call has grown, and so moved, the scratch."""
+    its replays give the eager result, also after an eager call has grown, and so moved, the scratch.  Traces updated in
+    place with and without that scratch, and with it only (hypercolumns of no whole vectors, 32 batch rows)."""
     from streambrain_amd import _capi
     from streambrain_amd._capi import DeviceArray, check
     lib, f = _capi.lib(), np.float32
@@ -679,7 +681,9 @@ def test_captured_train_step_does_without_the_scratch_that_later_calls_replace(k
                        ("hipGraphInstantiate", [ctypes.POINTER(P), P, P, P, ctypes.c_size_t]), ("hipGraphLaunch", [P, P]),
                        ("hipGraphExecDestroy", [P]), ("hipGraphDestroy", [P])):
         getattr(hip, name).argtypes, getattr(hip, name).restype = args, I
-    N, H, Mc, big = 4353, 30, 100, 256
+    check(lib.sb_shutdown())  # (scratch that earlier calls have grown is given back)
+    check(lib.sb_init(0))
+    big = 2 * B
     M, rng = H * Mc, np.random.default_rng(3)
     names = ("weights", "bias", "Ci", "Cj", "Cij", "kbi", "wmask")
     st = {"weights": np.zeros((N, M), f), "bias": np.zeros(M, f), "kbi": np.ones(M, f), "Ci": rng.random(N).astype(f),
@@ -688,22 +692,22 @@ def test_captured_train_step_does_without_the_scratch_that_later_calls_replace(k
     dev = {n: DeviceArray.from_numpy(st[n]) for n in names}
     x, y = (DeviceArray.from_numpy(rng.random((big, n)).astype(f)) for n in (N, M))
 
-    def step(B):
-        check(lib.sb_plastic_train_step_f32(*(dev[n].ptr for n in names), x.ptr, y.ptr, B, N, H, Mc, 0.1, -139.0, 0.062,
+    def step(rows):
+        check(lib.sb_plastic_train_step_f32(*(dev[n].ptr for n in names), x.ptr, y.ptr, rows, N, H, Mc, 0.1, -139.0, 0.062,
                                             0.022, -1))
 
     def reset():
         for n in names:
             check(lib.sb_memcpy_h2d(dev[n].ptr, st[n].ctypes.data, st[n].nbytes))
 
-    step(128)
+    step(B)
     check(lib.sb_sync())
     eager = {n: dev[n].numpy() for n in names}
     stream, graph, run = lib.sb_stream(), P(), P()
     reset()
     before = lib.sb_allocation_calls()
     assert hip.hipStreamBeginCapture(stream, 1) == 0  # (thread-local mode)
-    step(128)
+    step(B)
     assert hip.hipStreamEndCapture(stream, ctypes.byref(graph)) == 0
     assert lib.sb_allocation_calls() == before
     assert hip.hipGraphInstantiate(ctypes.byref(run), graph, None, None, 0) == 0
@@ -716,7 +720,7 @@ def test_captured_train_step_does_without_the_scratch_that_later_calls_replace(k
         for n in names:
             assert_close(replays[-1][n], eager[n], f, n)
             assert np.array_equal(replays[-1][n], replays[0][n]), n
-        step(128 if k_ else big)  # the scratch grows to twice its size
+        step(B if k_ else big)  # the scratch grows to twice its size
         check(lib.sb_sync())
     assert hip.hipGraphExecDestroy(run) == 0 and hip.hipGraphDestroy(graph) == 0
 
