@@ -67,8 +67,8 @@ constexpr int forward_rows_waves_per_simd() {
 // of the time (54000 -> 190 x 100, density 0.05, batch 256: 315 -> 263 us; 3000 -> 100 x 64, density 0.1: 21.4 -> 19.1;
 // doubles 256 rows of 3000 -> 30 x 64, density 0.3: 25.5 -> 23.1).
 // WIDE: W beyond the 4 GiB that such an offset reaches.  Offsets then count from the segment's first row; a segment that
-// spans more than 4 GiB is walked with 64-bit addresses (55296 -> 200 x 100, density 0.05, batch 256: 362 -> 314 us, all
-// addresses in 64 bits 420).
+// spans more than 4 GiB (in some layers of few inputs a single row does) is walked with 64-bit addresses (55296 -> 200 x
+// 100, density 0.05, batch 256: 362 -> 314 us, all addresses in 64 bits 420).
 template <typename T, int NG, int NWAVES, int RB = 1, bool XT = false, int LW = Real<T>::VW, int SEG = 2048,
           bool WIDE = false>
 __global__ __launch_bounds__(64 * NWAVES)
@@ -104,7 +104,9 @@ void k_forward_rows(ForwardRowsArgs<T> ar) {
   const int *list = ar.rows + ct * ar.cap;
 
   constexpr unsigned XSTEP = (XT ? 16u : 1u) * (unsigned)sizeof(T);  // bytes between input columns
-  const unsigned wrow = (unsigned)(a.M * sizeof(T));  // bytes of a row of W (launcher: 16 rows are below 2 GiB)
+  // Bytes of a row of W: below 4 GiB, except with WIDE, where rows of more take the 64-bit path (see publish_segment).
+  typedef std::conditional_t<WIDE, unsigned long, unsigned> row_bytes_t;
+  const row_bytes_t wrow = (row_bytes_t)(a.M * sizeof(T));
 
   // first segment of the list on its way before anything else
   constexpr int PT = SEG / (64 * NWAVES);  // entries per thread and segment
@@ -131,7 +133,7 @@ void k_forward_rows(ForwardRowsArgs<T> ar) {
       const int r = k < ar.cap ? mine[t] : -1, e = tid + t * (64 * NWAVES);
       const long rel = r < 0 ? 0 : r - wbase;
       if constexpr (WIDE) reach = reach && rel >= 0 && (rel + 1) * (long)wrow <= (1L << 32);
-      woff[e] = (unsigned)rel * wrow;
+      woff[e] = (unsigned)rel * (unsigned)wrow;
       xoff[e] = r < 0 ? BufferWindow<T>::kOutside : (unsigned)r * XSTEP;
     }
     return reach;
@@ -162,9 +164,10 @@ void k_forward_rows(ForwardRowsArgs<T> ar) {
                 : (unsigned)((long)(16 * r + p) * a.N * sizeof(T));
   // W: this lane's columns of group g, or the tile's first columns where the group hangs over the end
   // of the hypercolumn (those accumulator columns are never stored)
+  auto first_col = [&](int g) { return j0 + (TC::gcol(g, p) < ncol ? TC::gcol(g, p) : 0); };
   unsigned wcol[NG];  // bytes
 #pragma unroll
-  for (int g = 0; g < NG; g++) wcol[g] = (unsigned)((j0 + (TC::gcol(g, p) < ncol ? TC::gcol(g, p) : 0)) * sizeof(T));
+  for (int g = 0; g < NG; g++) wcol[g] = (unsigned)(first_col(g) * sizeof(T));
 
   T xr[2][RB][VW];
   T wr[2][VW][NG][VW];
@@ -187,7 +190,7 @@ void k_forward_rows(ForwardRowsArgs<T> ar) {
       for (int g = 0; g < NG; g++) {
         const char *from = wfrom + (wcol[g] + wv[s]);
         if constexpr (FAR)
-          from = wfrom + (wcol[g] + (unsigned long)(xv[s] == BufferWindow<T>::kOutside ? 0u : xv[s] / XSTEP) * wrow);
+          from = wfrom + first_col(g) * sizeof(T) + (xv[s] == BufferWindow<T>::kOutside ? 0u : xv[s] / XSTEP) * wrow;
         if (TC::gwidth(g) == VW) {
           const vec_t v = *reinterpret_cast<const vec_t *>(from);
 #pragma unroll

@@ -203,3 +203,44 @@ def test_row_lists_whose_rows_lie_more_than_4_gib_apart_f32(B, entries):
                                                        cols, H, Mc, None))
         acts.append(d_act.numpy())
     assert np.array_equal(acts[0], acts[1])
+
+
+@pytest.mark.parametrize("dtype,Mc", [(np.float32, 256), (np.float64, 224)])
+def test_row_lists_of_a_layer_whose_rows_are_longer_than_4_gib(dtype, Mc):
+    """Three inputs and so many hypercolumns that one row of W is longer than 4 GiB: the activations of the first, the
+    last and a few hypercolumns around the 4 GiB have the bits of a layer of just those."""
+    from streambrain_amd import _capi
+    from streambrain_amd._capi import DeviceArray
+    _capi.init(0)
+    lib, es = _capi.lib(), np.dtype(dtype).itemsize
+    f = getattr(lib, "sb_compute_activation_rows" + ("_f32" if dtype == np.float32 else "_f64"))
+    N, B, cap = 3, 2, 16
+    edge = (1 << 32) // (Mc * es)  # the hypercolumn at byte 4 GiB of a row
+    H = edge + 3
+    M, rng = H * Mc, np.random.default_rng(5)
+    some = np.array([0, 1, edge - 1, edge, edge + 1, H - 1])
+    w = rng.standard_normal((N, len(some), Mc)).astype(dtype)
+    x = rng.random((B, N)).astype(dtype)
+    lists = np.full((H, cap), -1, np.int32)
+    lists[:, :2] = [0, 2]
+    lists[some[::2], :3] = [0, 1, 2]
+    cnt = (lists >= 0).sum(1).astype(np.int32)
+    d_w, d_bias, d_act = DeviceArray((N, M), dtype), DeviceArray((M,), dtype), DeviceArray((B, M), dtype)
+    for d in (d_w, d_bias):
+        _capi.check(lib.sb_fill_bytes(d.ptr, 0, d.nbytes))
+    for i in range(N):
+        for k, h in enumerate(some):
+            _capi.check(lib.sb_memcpy_h2d(ctypes.c_void_p(int(d_w.ptr) + (i * M + int(h) * Mc) * es), w[i, k].ctypes.data,
+                                          Mc * es))
+    d_x, d_rows, d_cnt = DeviceArray.from_numpy(x), DeviceArray.from_numpy(lists), DeviceArray.from_numpy(cnt)
+    _capi.check(f(d_act.ptr, d_x.ptr, d_w.ptr, d_bias.ptr, d_rows.ptr, d_cnt.ptr, cap, B, N, H, Mc, None))
+    d_small = DeviceArray((B, len(some) * Mc), dtype)
+    s_w, s_rows, s_cnt = (DeviceArray.from_numpy(a) for a in (w, lists[some], cnt[some]))
+    _capi.check(f(d_small.ptr, d_x.ptr, s_w.ptr, d_bias.ptr, s_rows.ptr, s_cnt.ptr, cap, B, N, len(some), Mc, None))
+    small = d_small.numpy().reshape(B, len(some), Mc)
+    assert small.std() > 1e-4
+    for k, h in enumerate(some):
+        got = _rows_to_host(_capi, lib, d_act, range(B), M, int(h) * Mc, Mc, dtype)
+        assert np.array_equal(got, small[:, k]), h
+    free = _rows_to_host(_capi, lib, d_act, range(B), M, 2 * Mc, Mc, dtype)  # (no weights)
+    assert np.all(free == dtype(1) / dtype(Mc))
