@@ -821,34 +821,36 @@ static int net_train_batches(sb_net *net, int layer, long maxB, const int64_t *h
   // images[idx, :]  (_cpu_base_backend.py:258-260)
   auto lay_out_images = [&]() -> int {
     if (!net->Xp) SB_HIP(dev_malloc(&net->Xp, (size_t)Ns * net->NF * net->esize));
-    net->images_laid = true;
     // A first layer that walks row lists reads its input column by column: it gets the shuffled images a
     // second time, in blocks of 16 rows (batches must then start on block boundaries); one kernel writes
     // both copies from one read.
-    if (net->layers[0].rows && maxB % 16 == 0) {
-      if (!net->XpB) SB_HIP(dev_malloc(&net->XpB, (size_t)cdiv_l(Ns, 16) * 16 * net->NF * net->esize));
-      net->XpB_batch = maxB;
-      return launch_gather_rows_blocked<T>(st, (T *)net->XpB, (T *)net->Xp, (const T *)net->X, net->d_perm, Ns, net->NF);
-    }
-    net->XpB_batch = 0;
-    return launch_gather_rows<T>(st, (T *)net->Xp, (const T *)net->X, net->d_perm, Ns, net->NF);
+    const bool blocked = net->layers[0].rows && maxB % 16 == 0;
+    if (blocked && !net->XpB) SB_HIP(dev_malloc(&net->XpB, (size_t)cdiv_l(Ns, 16) * 16 * net->NF * net->esize));
+    const int failed = blocked ? launch_gather_rows_blocked<T>(st, (T *)net->XpB, (T *)net->Xp, (const T *)net->X, net->d_perm,
+                                                               Ns, net->NF)
+                               : launch_gather_rows<T>(st, (T *)net->Xp, (const T *)net->X, net->d_perm, Ns, net->NF);
+    if (failed) return failed;
+    net->XpB_batch = blocked ? maxB : 0;
+    net->images_laid = true;
+    return 0;
   };
   if (permute) {
     SB_REQUIRE(h_sample_perm, "sample order missing");
     for (long r = 0; r < Ns; r++)
       SB_REQUIRE(h_sample_perm[r] >= 0 && h_sample_perm[r] < Ns, "sample index out of range");
 
+    // (nothing of an epoch that could not be laid out is left for its later ranges to go on with)
+    net->epoch_begun = net->images_laid = false;
     if (last && !net->Yp) SB_HIP(dev_malloc(&net->Yp, (size_t)Ns * net->NC * net->esize));
     SB_HIP(hipEventSynchronize(net->perm_copied));  // staging buffer free again
     std::memcpy(net->h_perm, h_sample_perm, (size_t)Ns * sizeof(int64_t));
     SB_HIP(hipMemcpyAsync(net->d_perm, net->h_perm, (size_t)Ns * sizeof(int64_t), hipMemcpyHostToDevice,
                           st));
     SB_HIP(hipEventRecord(net->perm_copied, st));
-    net->epoch_begun = true;
-    net->images_laid = false;
     if (last)  // labels[idx, :]
       if ((rc = launch_gather_rows<T>(st, (T *)net->Yp, (const T *)net->Y, net->d_perm, Ns, net->NC)))
         return rc;
+    net->epoch_begun = true;
     if (cache_fits) {
       if (net->Hc_layer != layer - 1 && (rc = build_frozen_cache<T>(net, layer - 1, maxB, like))) return rc;
       if (net->Hc_layer == layer - 1 && !in_one) {

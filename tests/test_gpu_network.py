@@ -242,6 +242,100 @@ def test_classifier_epochs_without_the_activation_cache_are_bit_identical(hb, dt
             assert np.array_equal(value, other[name]), name
 
 
+@pytest.mark.parametrize("n_out", [5, 40])
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+def test_classifier_epoch_that_loses_the_activation_cache_between_its_ranges(hb, dtype, n_out):
+    """The first batches of an epoch on cached activations, the rest without the cache: the images are laid out in the
+    epoch's order then, and the bits are those of the epoch without a cache.  Output layers whose batches run in one
+    launch and in launches of their own."""
+    rng = np.random.default_rng(79)
+    n_pix, H, Mc, Ns, B = 40, 4, 12, 200, 16
+    X, Y = synthetic_images(rng, Ns, n_pix).astype(dtype), one_hot_labels(rng, Ns, n_out).astype(dtype)
+    orders, none = [rng.permutation(Ns) for _ in range(2)], np.arange(1)
+    states = []
+    for limits in ((None, 1000), (0, 0)):
+        net = build_two_layer(hb, 2 * n_pix, H, Mc, n_out, dict(MNIST_HP, l1_density=0.4), dtype, seed=5)
+        if limits[0] is not None:
+            net.net.set_frozen_cache_limit(limits[0])
+        net.net.initiate_training(X, Y)
+        net.net.train_epoch(0, B, orders[0], np.arange(H), 0)  # (leaves images in another order)
+        net.net.train_batches(1, B, orders[1], none, 0, 0, 6, False)
+        net.net.set_frozen_cache_limit(limits[1])
+        net.net.train_batches(1, B, orders[1], none, 0, 6, 7, True)
+        net.net.training_done()
+        states.append({name: np.array(getattr(net._layers[1], name)) for name in ("Ci", "Cj", "Cij", "weights", "bias")})
+    for name, value in states[0].items():
+        assert np.array_equal(value, states[1][name]), name
+
+
+def test_epoch_whose_images_could_not_be_laid_out_goes_on_when_they_can():
+    """The second copy of the images, for a first layer that has become sparse, does not fit the device: the first range of
+    the epoch fails, a later one fails too instead of training on images of another order, and once there is
+    room it gives what it gives in an epoch that never failed."""
+    import ctypes
+    from streambrain_amd import _capi
+    _capi.init()
+    lib, rng, P = _capi.lib(), np.random.default_rng(4), ctypes.c_void_p
+    info = ctypes.CDLL(_capi.LIB_PATH).hipMemGetInfo  # (of the runtime that the library is linked with)
+    info.argtypes = [ctypes.POINTER(ctypes.c_size_t)] * 2
+    N, Mc, classes, Ns, B = 1 << 22, 36, 3, 17, 16  # the second copy: 512 MiB
+    X = (rng.random((Ns, N), dtype=np.float32) < 0.3).astype(np.float32)
+    Y = np.eye(classes, dtype=np.float32)[rng.integers(0, classes, Ns)]
+    W = np.zeros((N, Mc), np.float32)
+    W[:4096:2] = rng.standard_normal((2048, Mc), dtype=np.float32) * np.float32(0.05)
+    orders = [np.arange(Ns, dtype=np.int64), rng.permutation(Ns).astype(np.int64)]
+    mask = np.zeros((N, 1), np.uint8)
+    mask[:4096:2] = 1
+
+    def free_bytes():
+        left, total = ctypes.c_size_t(), ctypes.c_size_t()
+        assert info(ctypes.byref(left), ctypes.byref(total)) == 0
+        return left.value
+
+    def train(net, order, first, count):
+        return lib.sb_net_train_batches(net, 1, B, order.ctypes.data, None, 0, first, count, 0)
+
+    results = []
+    for fails in (False, True):
+        net, held = P(), []
+        _capi.check(lib.sb_net_create(ctypes.byref(net), 0))
+        try:
+            assert lib.sb_net_add_plastic_layer(net, N, 1, Mc, 0.01, 0.1, -100.0, 0.1, 1.0, 1.0, 1.0) == 0
+            assert lib.sb_net_add_dense_layer(net, Mc, 1, classes, 0.01, 1.0 / Mc, 1.0 / classes, 0.01) == 1
+            _capi.check(lib.sb_net_set_frozen_cache_limit(net, 0))
+            _capi.check(lib.sb_net_set_training_data(net, X.ctypes.data, Y.ctypes.data, Ns, N, classes))
+            _capi.check(train(net, orders[0], 0, 2))  # (every connection present: one copy of the images)
+            for name, a in ((b"weights", W), (b"wmask", mask)):
+                _capi.check(lib.sb_net_set_layer_state(net, 0, name, a.ctypes.data, a.nbytes))
+            if fails:
+                piece = 1 << 40
+                while piece >= 1 << 24:
+                    if free_bytes() < 300 << 20:
+                        break
+                    p = P()
+                    piece = min(piece, free_bytes() - (200 << 20))
+                    if piece > 0 and lib.sb_malloc(ctypes.byref(p), piece) == 0:
+                        held.append(p)
+                    else:
+                        piece //= 2
+                assert free_bytes() < 400 << 20
+                assert train(net, orders[1], 0, 1) == -2, "SB_ERR_HIP"
+                assert train(net, orders[1], 1, 1) == -2, "SB_ERR_HIP"
+                while held:
+                    _capi.check(lib.sb_free(held.pop()))
+            else:
+                _capi.check(train(net, orders[1], 0, 0))
+            _capi.check(train(net, orders[1], 1, 1))
+            state = np.zeros((Mc, classes), np.float32)
+            _capi.check(lib.sb_net_get_layer_state(net, 1, b"Cij", state.ctypes.data, state.nbytes))
+            results.append(state)
+        finally:
+            while held:
+                _capi.check(lib.sb_free(held.pop()))
+            _capi.check(lib.sb_net_destroy(net))
+    assert np.array_equal(*results) and results[0].std() > 0
+
+
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
 @pytest.mark.parametrize("n_pix,H,Mc,density,Ns,B", [(784, 30, 100, 0.1, 6000, 128), (100, 15, 200, 1.0, 6100, 256),
                                                    (300, 70, 60, 0.3, 4500, 64)])
