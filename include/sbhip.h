@@ -249,13 +249,14 @@ int sb_net_training_done(sb_net *net);
  * the last layer trains on the labels, any other on its own activation; ends with train_finalize.
  * When n_batches / (H + 1) is zero the reference divides by zero; here no rewiring happens.
  * While the last layer trains, the layers below it do not change: their activations of the training set
- * are computed in its first epoch and kept (two copies of [n_samples, its input width], as long as
- * they stay below 16 GiB and half of the free device memory) until a lower layer trains, state is written or the training set is replaced.
+ * are computed in its first epoch and kept (two copies of [n_samples, its input width], one for
+ * a dense last layer of up to 32 units, as long as they stay below 16 GiB and half of the free device
+ * memory) until a lower layer trains, state is written or the training set is replaced.
  * Asynchronous: returns once the epoch is enqueued. */
 int sb_net_train_epoch(sb_net *net, int layer, long maximal_batch_size,
                        const int64_t *h_sample_perm, const int64_t *h_hc_perm, long epoch_index);
 
-/* Upper bound, in bytes (both copies together), of the cache of frozen layers' activations that
+/* Upper bound, in bytes (all copies together), of the cache of frozen layers' activations that
  * sb_net_train_epoch keeps while the last layer trains; 16 GiB unless set.  0 switches the cache off: every
  * step then runs the forward passes of the layers below, as the reference does
  * (_cpu_base_backend.py:279-295), with identical results.  A cache already held that exceeds the new bound

@@ -524,7 +524,7 @@ struct sb_net {
   // read it in the epoch's order by themselves.
   void *Hc = nullptr, *Hcp = nullptr;
   int Hc_layer = -1;  // Hc holds the activations of this layer for the current training set (-1: none)
-  size_t frozen_cache_limit = (size_t)16 << 30;  // bytes, both copies together (sb_net_set_frozen_cache_limit)
+  size_t frozen_cache_limit = (size_t)16 << 30;  // bytes, all copies together (sb_net_set_frozen_cache_limit)
   unsigned long long *d_correct = nullptr;   // evaluate's counter
   unsigned long long *d_unmasked = nullptr;  // layer_check_masked's counter
   // evaluate / predict / forward: the device buffers of one chunk of the set (images, the same in blocks of 16
@@ -739,7 +739,7 @@ static int layer_mask_replaced(Layer &L, const uint8_t *mask) {
   return launch_mask_rows(g_ctx.stream, L.rows, L.row_cnt, L.wmask, L.N, L.H, L.rows_cap, 0, L.H);
 }
 
-// Largest cache of frozen activations kept (bytes, both copies together): at most 16 GiB, and at most half of
+// Largest cache of frozen activations kept (bytes, all copies together): at most 16 GiB, and at most half of
 // the device memory that is free when the cache is built; beyond it the activations are recomputed.
 static bool frozen_cache_affordable(const sb_net *net, size_t bytes) {
   if (bytes > net->frozen_cache_limit) return false;
@@ -764,14 +764,16 @@ static int drop_frozen_cache(sb_net *net) {
 
 // Activations of layer `upto` for all training samples in data-set order, as many samples per pass as pass_rows says
 // (157 batches of 128 through 784 -> 15x200: 1.25 ms of launches of 8 us and a copy each, in passes of 5504 0.45 ms).
-// like: the batch size whose bits they get, as the steps that do without the cache ask for it.
+// like: the batch size whose bits they get, as the steps that do without the cache ask for it.  copies: 1, or 2 with room for
+// the shuffled ones.
 template <typename T>
-static int build_frozen_cache(sb_net *net, int upto, long maxB, long like) {
+static int build_frozen_cache(sb_net *net, int upto, long maxB, long like, int copies) {
   const long Ns = net->Ns, Mo = net->layers[upto].M;
   int rc = drop_frozen_cache(net);
   if (rc) return rc;
   // without the memory the caller goes on uncached (Hc_layer stays -1): not an error
   if (dev_malloc(&net->Hc, (size_t)Ns * Mo * sizeof(T)) != hipSuccess) return 0;
+  if (copies > 1 && dev_malloc(&net->Hcp, (size_t)Ns * Mo * sizeof(T)) != hipSuccess) return drop_frozen_cache(net);
   long pass = std::min(Ns, pass_rows(net, maxB));
   if (upto > 0 && (rc = ensure_pass_act(net, pass, std::min(Ns, maxB), &pass))) return rc;
   for (long lo = 0; lo < Ns; lo += pass) {
@@ -813,11 +815,14 @@ static int net_train_batches(sb_net *net, int layer, long maxB, const int64_t *h
   // a training step of a layer below the last changes what the cache was computed from
   if (!last && (rc = drop_frozen_cache(net))) return rc;
   const long Mprev = layer > 0 ? net->layers[layer - 1].M : 0;
-  const bool cache_fits = last && layer > 0 &&
-                          (net->Hc_layer == layer - 1 || frozen_cache_affordable(net, 2 * (size_t)Ns * Mprev * sizeof(T)));
   // A dense output layer of a few units takes all of the call's batches in one launch, reading what it trains on in the
   // epoch's order by itself: the data set, or the cached activations of the layers below.
   const bool in_one = last && !target.plastic && train_skinny_epoch_supported<T>(target.M) && Ns < (1L << 31);
+  // (then one copy of those will do: there is no shuffled one)
+  const int copies = in_one ? 1 : 2;
+  const bool cache_fits =
+      last && layer > 0 &&
+      (net->Hc_layer == layer - 1 || frozen_cache_affordable(net, copies * (size_t)Ns * Mprev * sizeof(T)));
   // images[idx, :]  (_cpu_base_backend.py:258-260)
   auto lay_out_images = [&]() -> int {
     if (!net->Xp) SB_HIP(dev_malloc(&net->Xp, (size_t)Ns * net->NF * net->esize));
@@ -852,14 +857,10 @@ static int net_train_batches(sb_net *net, int layer, long maxB, const int64_t *h
         return rc;
     net->epoch_begun = true;
     if (cache_fits) {
-      if (net->Hc_layer != layer - 1 && (rc = build_frozen_cache<T>(net, layer - 1, maxB, like))) return rc;
-      if (net->Hc_layer == layer - 1 && !in_one) {
-        if (!net->Hcp && dev_malloc(&net->Hcp, (size_t)Ns * Mprev * sizeof(T)) != hipSuccess) {
-          if ((rc = drop_frozen_cache(net))) return rc;
-        } else if ((rc = launch_gather_rows<T>(st, (T *)net->Hcp, (const T *)net->Hc, net->d_perm, Ns, Mprev))) {
-          return rc;
-        }
-      }
+      if (net->Hc_layer != layer - 1 && (rc = build_frozen_cache<T>(net, layer - 1, maxB, like, copies))) return rc;
+      if (net->Hc_layer == layer - 1 && !in_one &&
+          (rc = launch_gather_rows<T>(st, (T *)net->Hcp, (const T *)net->Hc, net->d_perm, Ns, Mprev)))
+        return rc;
     } else if (last && (rc = drop_frozen_cache(net))) {
       return rc;
     }
@@ -1505,8 +1506,9 @@ int sb_net_set_frozen_cache_limit(sb_net *net, size_t bytes) {
   SB_READY();
   SB_REQUIRE(net, "null pointer");
   net->frozen_cache_limit = bytes;
-  if (net->Hc && 2 * (size_t)net->Ns * (size_t)net->layers[net->Hc_layer].M * net->esize > bytes)
-    return drop_frozen_cache(net);
+  if (net->Hc_layer < 0) return drop_frozen_cache(net);  // (what a cache that could not be built has left)
+  const size_t copy = (size_t)net->Ns * (size_t)net->layers[net->Hc_layer].M * net->esize;
+  if ((net->Hcp ? 2 : 1) * copy > bytes) return drop_frozen_cache(net);
   return 0;
 }
 

@@ -268,6 +268,32 @@ def test_classifier_epoch_that_loses_the_activation_cache_between_its_ranges(hb,
         assert np.array_equal(value, states[1][name]), name
 
 
+@pytest.mark.parametrize("n_out,copies,B", [(5, 1, 16), (40, 2, 20)])
+def test_activation_cache_is_kept_where_the_copies_it_takes_fit_its_limit(hb, n_out, copies, B):
+    """Output layers whose batches run in one launch read the cached activations in the epoch's order by themselves: one
+    copy of them has to fit.  The others take a shuffled copy as well.  (Without the cache the images are laid out, twice
+    where batches are whole blocks of 16 rows.)"""
+    from streambrain_amd import _capi
+    rng = np.random.default_rng(80)
+    n_pix, H, Mc, Ns = 40, 4, 12, 200
+    X, Y = synthetic_images(rng, Ns, n_pix).astype(np.float32), one_hot_labels(rng, Ns, n_out).astype(np.float32)
+    one_copy, allocated = Ns * H * Mc * 4, []
+    for limit in (None, copies * one_copy, copies * one_copy - 1, 0):
+        net = build_two_layer(hb, 2 * n_pix, H, Mc, n_out, dict(MNIST_HP, l1_density=0.4), np.float32, seed=5)
+        if limit is not None:
+            net.net.set_frozen_cache_limit(limit)
+        net.net.initiate_training(X, Y)
+        for l, rows in ((0, X), (1, net._layers[0].compute_activation(X))):  # (what the passes need is there)
+            net._layers[l].compute_activation(rows)
+        before = _capi.lib().sb_allocation_calls()
+        net.net.train_epoch(1, B, rng.permutation(Ns), np.arange(1), 0)
+        allocated.append(_capi.lib().sb_allocation_calls() - before)
+        net.net.set_frozen_cache_limit(0)
+        net.net.training_done()
+    images = 2 if B % 16 == 0 else 1
+    assert allocated == [1 + copies, 1 + copies, 1 + images, 1 + images], allocated  # (labels, and copies)
+
+
 def test_epoch_whose_images_could_not_be_laid_out_goes_on_when_they_can():
     """The second copy of the images, for a first layer that has become sparse, does not fit the device: the first range of
     the epoch fails, a later one fails too instead of training on images of another order, and once there is
