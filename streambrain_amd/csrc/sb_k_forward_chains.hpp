@@ -77,23 +77,23 @@ void k_forward_chains(ForwardChainsArgs<T> ac) {
   const int chunks = (cnt + KC - 1) / KC;
   const int mine = chunks > (int)ch ? (chunks - 1 - (int)ch) / kChains + 1 : 1;
 
-  auto run = [&](auto nblocks) {
-    constexpr int NB = decltype(nblocks)::value, NG = (NB + VW - 1) / VW, LW = NB - (NG - 1) * VW, GW = 16 * VW;
+  // sums of the piece's blocks of 16 columns: those of NB = 4 (a piece of fewer leaves the last ones alone)
+  acc_t acc[4];
+#pragma unroll
+  for (int k = 0; k < 4; k++) acc[k] = acc_t{0, 0, 0, 0};
+  // the lane's first column of group g; a vector that would run over the piece's end starts earlier (its columns are
+  // computed twice, with the same result)
+  auto first_col = [&](int g, int width) {
+    const int c = g * 16 * VW + width * p, last = ncol - width;
+    return c < last ? c : (last > 0 ? last : 0);
+  };
+  // adds up the n chunks of the staged segment (per wavefront: no barriers in here)
+  auto walk = [&](auto nblocks, int n) {
+    constexpr int NB = decltype(nblocks)::value, NG = (NB + VW - 1) / VW, LW = NB - (NG - 1) * VW;
     auto width = [](int g) { return g == NG - 1 ? LW : VW; };
-    // the lane's first column of group g; a vector that would run over the piece's end starts earlier (its columns are
-    // computed twice, with the same result)
-    auto col = [&](int g) {
-      const int c = g * GW + (g == NG - 1 ? LW : VW) * p, last = ncol - (g == NG - 1 ? LW : VW);
-      return c < last ? c : (last > 0 ? last : 0);
-    };
-    acc_t acc[NG][VW];
-#pragma unroll
-    for (int g = 0; g < NG; g++)
-#pragma unroll
-      for (int c = 0; c < VW; c++) acc[g][c] = acc_t{0, 0, 0, 0};
     unsigned wcol[NG];
 #pragma unroll
-    for (int g = 0; g < NG; g++) wcol[g] = (unsigned)((j0 + col(g)) * sizeof(T));
+    for (int g = 0; g < NG; g++) wcol[g] = (unsigned)((j0 + first_col(g, width(g))) * sizeof(T));
     T xr[D][VW], wt[D][VW][NG][VW];
     auto request = [&](int c, T(&xo)[VW], T(&wo)[VW][NG][VW]) {
       const int at = (c < SEGC ? c : SEGC - 1) * KC + VW * q;
@@ -125,54 +125,28 @@ void k_forward_chains(ForwardChainsArgs<T> ac) {
         for (int g = 0; g < NG; g++)
 #pragma unroll
           for (int c = 0; c < VW; c++)
-            if (c < width(g)) acc[g][c] = Real<T>::mfma(xi[s], wi[s][g][c], acc[g][c]);
+            if (c < width(g)) acc[g * VW + c] = Real<T>::mfma(xi[s], wi[s][g][c], acc[g * VW + c]);
     };
-    int left = mine;
-    for (int c0 = 0; left > 0; c0 += SEGC, left -= SEGC) {
-      const int n = left < SEGC ? left : SEGC;
-      if (c0 > 0) __syncthreads();  // everyone is done with the staged segment
-      // (D - 1 chunks beyond the last one are requested and not used: padding)
-      const int stage = (n + D - 1 < SEGC ? n + D - 1 : SEGC) * KC;
-      constexpr int U = 4;
-      for (int e0 = tid; e0 < stage; e0 += threads * U) {
-        int r[U];
 #pragma unroll
-        for (int u = 0; u < U; u++) {
-          const int e = e0 + threads * u;
-          const long k = ((long)(c0 + e / KC) * kChains + ch) * KC + e % KC;
-          const bool on = e < n * KC && k < ar.cap;
-          r[u] = list[on ? k : 0];
-          r[u] = on ? r[u] : -1;
-        }
+    for (int u = 0; u < D - 1; u++) request(u, xr[u], wt[u]);
+    __builtin_amdgcn_sched_barrier(0);
+    int i = 0;
+    for (; i + D <= n; i += D) {
 #pragma unroll
-        for (int u = 0; u < U; u++) {
-          const int e = e0 + threads * u;
-          if (e < stage) {
-            woff[e] = r[u] < 0 ? 0u : (unsigned)r[u] * (unsigned)(a.M * sizeof(T));
-            xoff[e] = r[u] < 0 ? BufferWindow<T>::kOutside : (unsigned)r[u] * XSTEP;
-          }
-        }
+      for (int u = 0; u < D; u++) {
+        request(i + u + D - 1, xr[(u + D - 1) % D], wt[(u + D - 1) % D]);
+        __builtin_amdgcn_sched_barrier(0);
+        compute(xr[u], wt[u]);
+        __builtin_amdgcn_sched_barrier(0);
       }
-      __syncthreads();
-      if (!active) continue;  // uniform per wavefront
-#pragma unroll
-      for (int u = 0; u < D - 1; u++) request(u, xr[u], wt[u]);
-      __builtin_amdgcn_sched_barrier(0);
-      int i = 0;
-      for (; i + D <= n; i += D) {
-#pragma unroll
-        for (int u = 0; u < D; u++) {
-          request(i + u + D - 1, xr[(u + D - 1) % D], wt[(u + D - 1) % D]);
-          __builtin_amdgcn_sched_barrier(0);
-          compute(xr[u], wt[u]);
-          __builtin_amdgcn_sched_barrier(0);
-        }
-      }
-#pragma unroll
-      for (int u = 0; u < D - 1; u++)
-        if (i + u < n) compute(xr[u], wt[u]);
     }
-    if (!active) return;
+#pragma unroll
+    for (int u = 0; u < D - 1; u++)
+      if (i + u < n) compute(xr[u], wt[u]);
+  };
+  auto store = [&](auto nblocks) {
+    constexpr int NB = decltype(nblocks)::value, NG = (NB + VW - 1) / VW, LW = NB - (NG - 1) * VW;
+    auto width = [](int g) { return g == NG - 1 ? LW : VW; };
     T *const out = ac.part + (long)ch * a.B * a.M + j0;
 #pragma unroll
     for (int v = 0; v < 4; v++) {
@@ -180,17 +154,51 @@ void k_forward_chains(ForwardChainsArgs<T> ac) {
       if (row >= a.B) continue;
 #pragma unroll
       for (int g = 0; g < NG; g++) {
-        const int c0 = col(g);
+        const int c0 = first_col(g, width(g));
 #pragma unroll
         for (int e = 0; e < VW; e++)
-          if (e < width(g) && c0 + e < ncol) out[row * a.M + c0 + e] = acc[g][e][v];
+          if (e < width(g) && c0 + e < ncol) out[row * a.M + c0 + e] = acc[g * VW + e][v];
       }
     }
   };
-  if (nb == 4) run(std::integral_constant<int, 4>{});
-  else if (nb == 3) run(std::integral_constant<int, 3>{});
-  else if (nb == 2) run(std::integral_constant<int, 2>{});
-  else run(std::integral_constant<int, 1>{});
+  auto with_blocks = [&](auto what) {  // (uniform per wavefront)
+    if (nb == 4) what(std::integral_constant<int, 4>{});
+    else if (nb == 3) what(std::integral_constant<int, 3>{});
+    else if (nb == 2) what(std::integral_constant<int, 2>{});
+    else what(std::integral_constant<int, 1>{});
+  };
+
+  // All wavefronts of the workgroup, whatever their pieces, stage the list and meet at the barriers here.
+  int left = mine;
+  for (int c0 = 0; left > 0; c0 += SEGC, left -= SEGC) {
+    const int n = left < SEGC ? left : SEGC;
+    if (c0 > 0) __syncthreads();  // everyone is done with the staged segment
+    // (D - 1 chunks beyond the last one are requested and not used: padding)
+    const int stage = (n + D - 1 < SEGC ? n + D - 1 : SEGC) * KC;
+    constexpr int U = 4;
+    for (int e0 = tid; e0 < stage; e0 += threads * U) {
+      int r[U];
+#pragma unroll
+      for (int u = 0; u < U; u++) {
+        const int e = e0 + threads * u;
+        const long k = ((long)(c0 + e / KC) * kChains + ch) * KC + e % KC;
+        const bool on = e < n * KC && k < ar.cap;
+        r[u] = list[on ? k : 0];
+        r[u] = on ? r[u] : -1;
+      }
+#pragma unroll
+      for (int u = 0; u < U; u++) {
+        const int e = e0 + threads * u;
+        if (e < stage) {
+          woff[e] = r[u] < 0 ? 0u : (unsigned)r[u] * (unsigned)(a.M * sizeof(T));
+          xoff[e] = r[u] < 0 ? BufferWindow<T>::kOutside : (unsigned)r[u] * XSTEP;
+        }
+      }
+    }
+    __syncthreads();
+    if (active) with_blocks([&](auto nblocks) { walk(nblocks, n); });
+  }
+  if (active) with_blocks(store);
 }
 
 // act = softmax_per_hypercolumn(the four chains added up as forward_finish does + bias), with forward_finish's arithmetic

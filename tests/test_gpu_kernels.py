@@ -779,11 +779,12 @@ def test_forward_in_blocks_of_columns(k, dtype, Mc, B, N):
 
 @pytest.mark.parametrize("dtype", DT)
 @pytest.mark.parametrize("B,N,H,Mc,more", [(100, 34000, 4, 12, 1552), (33, 3000, 5, 100, 448), (128, 2500, 9, 200, 272),
-                                           (7, 9000, 3, 64, 704), (16, 2100, 2, 36, 1040), (80, 2600, 3, 128, 704)])
+                                           (7, 9000, 3, 64, 704), (16, 2100, 2, 36, 1040), (80, 2600, 3, 128, 704),
+                                           (40, 33500, 10, 100, 224)])
 def test_chains_of_the_row_lists(k, dtype, B, N, H, Mc, more):
     """The four sums of a tile on four CUs (few tiles, long lists): the bits that a larger batch, whose tiles form them
     on one, gives the same rows.  Lists of more than one staged segment, of a few entries and of none; workgroups of four
-    and of eight wavefronts, some of them without batch rows or columns."""
+    and of eight wavefronts, some of them without batch rows or columns, or with pieces of different widths."""
     rng = np.random.default_rng(N + B)
     M = H * Mc
     wmask = (rng.random((N, H)) < 0.51).astype(np.uint8)
