@@ -124,9 +124,10 @@ size_t train_split_bytes(long B, long N, long H, long Mc);
 template <typename T>
 bool train_in_place_supported(const void *split, long B, long N, long H, long Mc, T taupdt);
 // launch_train_fused for `rows` rows in batches of B, one after the other, of a layer without mask and regularised bias of a
-// few units (train_skinny_epoch_supported).  Batch row b is x[order[b]] (order: device memory) and y[b].
+// few units (at most 32; train_skinny_epoch_pays: where that is the faster way).  Batch row b is x[order[b]] (order: device
+// memory) and y[b].
 template <typename T>
-bool train_skinny_epoch_supported(long M);
+bool train_skinny_epoch_pays(long B, long N, long M);
 template <typename T>
 int launch_train_skinny_epoch(hipStream_t st, const T *x, const int64_t *order, const T *y, T *Cij, T *W, const T *Ci,
                               const T *Cj, T *Ci_next, T *Cj_next, long B, long rows, long N, long H, long Mc, T taupdt,

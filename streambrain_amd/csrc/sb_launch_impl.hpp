@@ -614,6 +614,23 @@ int launch_train_fused(hipStream_t st, const T *x, const T *y, T *Cij, T *W, con
 
 template <typename T>
 bool train_skinny_epoch_supported(long M) { return M <= 32; }
+// Floats and up to 16 units: always (whole epochs of 4096 to 8192 rows, time of a launch per batch, shuffled inputs included,
+// over time of one launch, at batches of 16 / 128 / 512 / 2048 rows: 784 x 10 7.0 / 4.2 / 2.8 / 2.3, 3000 x 10 6.9 / 4.4 / 3.0
+// / 2.4, 20000 x 32 2.0 / 1.6 / 1.2 / 1.1, 50000 x 32 - / 1.5 / 1.2 / 1.1; doubles 3000 x 10 7.8 / 4.3 / 3.0 / 2.5, 50000 x
+// 16 - / 2.7 / 2.0 / 1.9).  Doubles of 17 to 32 units are bound by what the fullest CU has to do either way, and a workgroup
+// here has three quarters of the rows that one of k_train_skinny has: batches of 768 rows and more, which share the cost of
+// their launch among many rows, only where that leaves the fullest CU at most 4/3 as many workgroups (time as above,
+// at 512 / 768 / 1024 / 4096 rows: 3000 x 32, 2 and 2 of them, 1.29 / 1.28 / 1.23 / 1.15; 6000 x 28, 4 and 3, 1.20 / 1.16
+// / 1.12 / 1.02; 50000 x 32, 33 and 25, 1.10 / - / 1.03 / 0.99; 20000 x 32, 14 and 10, 1.05 / - / 0.99 / 0.94; 8000 x 28, 6
+// and 4, 0.98 / 0.94 / 0.91 / 0.82; 4000 x 25, 3 and 2, 0.99 / 0.93 / 0.90 / 0.81).
+template <typename T>
+bool train_skinny_epoch_pays(long B, long N, long M) {
+  if (!train_skinny_epoch_supported<T>(M)) return false;
+  if (sizeof(T) == 4 || M <= 16 || B < 768) return true;
+  const long cus = device_cu_count();
+  const long here = cdiv(cdiv(N, skinny_epoch_rows(M)), cus), there = cdiv(cdiv(N, skinny_train_rows(M)), cus);
+  return 3 * here <= 4 * there;
+}
 
 template <typename T>
 int launch_train_skinny_epoch(hipStream_t st, const T *x, const int64_t *order, const T *y, T *Cij, T *W, const T *Ci,
@@ -921,7 +938,7 @@ int launch_copy_pair(hipStream_t st, T *dst1, const T *src1, size_t n1, T *dst2,
                                      T, T, T, T, T, bool, const void *, size_t, void *);              \
   template size_t train_split_bytes<T>(long, long, long, long);                                       \
   template bool train_in_place_supported<T>(const void *, long, long, long, long, T);                 \
-  template bool train_skinny_epoch_supported<T>(long);                                                \
+  template bool train_skinny_epoch_pays<T>(long, long, long);                                         \
   template int launch_train_skinny_epoch<T>(hipStream_t, const T *, const int64_t *, const T *, T *,  \
                                             T *, const T *, const T *, T *, T *, long, long, long,    \
                                             long, long, T, T);                                        \

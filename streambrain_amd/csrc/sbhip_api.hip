@@ -513,6 +513,7 @@ struct sb_net {
   void *X = nullptr, *Y = nullptr, *Xp = nullptr, *Yp = nullptr;
   bool epoch_begun = false;  // d_perm holds the order of an epoch
   bool images_laid = false;  // ... and Xp (XpB) its images
+  bool cache_laid = false;   // ... and Hcp its cached activations
   long XpB_batch = 0;   // batch size XpB is valid for in the current epoch (0: not valid)
   void *XpB = nullptr;  // Xp in blocks of 16 rows (k_gather_rows_blocked), for the first layer's forward over row lists
   long Ns = 0, NF = 0, NC = 0;
@@ -752,6 +753,7 @@ static bool frozen_cache_affordable(const sb_net *net, size_t bytes) {
 }
 
 static int drop_frozen_cache(sb_net *net) {
+  net->cache_laid = false;
   if (!net->Hc && !net->Hcp) {
     net->Hc_layer = -1;
     return 0;
@@ -817,7 +819,7 @@ static int net_train_batches(sb_net *net, int layer, long maxB, const int64_t *h
   const long Mprev = layer > 0 ? net->layers[layer - 1].M : 0;
   // A dense output layer of a few units takes all of the call's batches in one launch, reading what it trains on in the
   // epoch's order by itself: the data set, or the cached activations of the layers below.
-  const bool in_one = last && !target.plastic && train_skinny_epoch_supported<T>(target.M) && Ns < (1L << 31);
+  const bool in_one = last && !target.plastic && train_skinny_epoch_pays<T>(std::min(maxB, Ns), target.N, target.M) && Ns < (1L << 31);
   // (then one copy of those will do: there is no shuffled one)
   const int copies = in_one ? 1 : 2;
   const bool cache_fits =
@@ -845,7 +847,7 @@ static int net_train_batches(sb_net *net, int layer, long maxB, const int64_t *h
       SB_REQUIRE(h_sample_perm[r] >= 0 && h_sample_perm[r] < Ns, "sample index out of range");
 
     // (nothing of an epoch that could not be laid out is left for its later ranges to go on with)
-    net->epoch_begun = net->images_laid = false;
+    net->epoch_begun = net->images_laid = net->cache_laid = false;
     if (last && !net->Yp) SB_HIP(dev_malloc(&net->Yp, (size_t)Ns * net->NC * net->esize));
     SB_HIP(hipEventSynchronize(net->perm_copied));  // staging buffer free again
     std::memcpy(net->h_perm, h_sample_perm, (size_t)Ns * sizeof(int64_t));
@@ -858,14 +860,11 @@ static int net_train_batches(sb_net *net, int layer, long maxB, const int64_t *h
     net->epoch_begun = true;
     if (cache_fits) {
       if (net->Hc_layer != layer - 1 && (rc = build_frozen_cache<T>(net, layer - 1, maxB, like, copies))) return rc;
-      if (net->Hc_layer == layer - 1 && !in_one &&
-          (rc = launch_gather_rows<T>(st, (T *)net->Hcp, (const T *)net->Hc, net->d_perm, Ns, Mprev)))
-        return rc;
     } else if (last && (rc = drop_frozen_cache(net))) {
       return rc;
     }
   }
-  const bool cached = cache_fits && net->Hc_layer == layer - 1;
+  bool cached = cache_fits && net->Hc_layer == layer - 1;
   if (in_one && (layer == 0 || cached)) {
     const long lo = first_batch * maxB, rows = std::min(n_batches * maxB, Ns - lo);
     if (rows > 0) {
@@ -878,6 +877,17 @@ static int net_train_batches(sb_net *net, int layer, long maxB, const int64_t *h
       std::swap(target.Cj, target.Cj_alt);
     }
     return finalize ? launch_update_bias<T>(st, (T *)target.bias, (const T *)target.Cj, (T)(target.taupdt / 2), target.M) : 0;
+  }
+  if (cached && !net->Hcp) {  // (a cache that calls of another batch size have built)
+    const size_t bytes = (size_t)Ns * Mprev * sizeof(T);
+    if (2 * bytes > net->frozen_cache_limit || dev_malloc(&net->Hcp, bytes) != hipSuccess) {
+      if ((rc = drop_frozen_cache(net))) return rc;
+      cached = false;
+    }
+  }
+  if (cached && !net->cache_laid) {
+    if ((rc = launch_gather_rows<T>(st, (T *)net->Hcp, (const T *)net->Hc, net->d_perm, Ns, Mprev))) return rc;
+    net->cache_laid = true;
   }
   if (!cached && !net->images_laid && (rc = lay_out_images())) return rc;
 
@@ -1397,7 +1407,7 @@ int sb_net_training_done(sb_net *net) {
   rc |= free_dev(net->X); rc |= free_dev(net->Y); rc |= free_dev(net->Xp); rc |= free_dev(net->Yp);
   rc |= free_dev(net->XpB);
   net->XpB_batch = 0;
-  net->epoch_begun = net->images_laid = false;
+  net->epoch_begun = net->images_laid = net->cache_laid = false;
   rc |= free_dev(net->Hc); rc |= free_dev(net->Hcp);
   net->Hc_layer = -1;
   rc |= free_dev(p);

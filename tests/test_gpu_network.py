@@ -175,10 +175,12 @@ def test_classifier_epochs_follow_changes_below_them_f64(hb):
 
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
 @pytest.mark.parametrize("N,H,Mc,Ns,B", [(3000, 1, 10, 700, 128), (1003, 1, 10, 350, 100), (37, 1, 2, 300, 32), (513, 4, 8, 300, 77),
-                                         (17, 1, 1, 5, 64), (16, 1, 17, 129, 64), (50, 1, 31, 200, 65), (200, 3, 4, 999, 500)])
+                                         (17, 1, 1, 5, 64), (16, 1, 17, 129, 64), (50, 1, 31, 200, 65), (200, 3, 4, 999, 500),
+                                         (3000, 1, 25, 1700, 800), (4000, 1, 25, 1700, 800)])
 def test_classifier_epoch_in_one_launch_is_bit_identical(hb, dtype, N, H, Mc, Ns, B):
     """All batches of a call in one launch: the bits of a launch per batch, batches that end inside and on the bounds of a
-    chunk, a short last one, columns and units that do not fill a workgroup, an epoch in two ranges."""
+    chunk, a short last one, columns and units that do not fill a workgroup, an epoch in two ranges; batches on both sides
+    of the line from which doubles take a launch each."""
     rng = np.random.default_rng(N + Mc)
     X = (rng.random((Ns, N)) * (rng.random((Ns, N)) < 0.5)).astype(dtype)
     Y = np.eye(H * Mc)[rng.integers(0, H * Mc, Ns)].astype(dtype)
@@ -292,6 +294,29 @@ def test_activation_cache_is_kept_where_the_copies_it_takes_fit_its_limit(hb, n_
         net.net.training_done()
     images = 2 if B % 16 == 0 else 1
     assert allocated == [1 + copies, 1 + copies, 1 + images, 1 + images], allocated  # (labels, and copies)
+
+
+def test_classifier_epoch_in_ranges_of_different_batches_f64(hb):
+    """Small batches read the cached activations in the epoch's order by themselves, big ones of many units and inputs want
+    them shuffled: an epoch of both, also where only one copy fits, has the bits of the epoch without a cache."""
+    rng = np.random.default_rng(81)
+    n_pix, H, Mc, n_out, Ns = 30, 125, 32, 25, 1700
+    X, Y = synthetic_images(rng, Ns, n_pix), one_hot_labels(rng, Ns, n_out)
+    orders, none = [rng.permutation(Ns) for _ in range(3)], np.arange(1)
+    states = []
+    for limit in (1 << 30, Ns * H * Mc * 8, 0):
+        net = build_two_layer(hb, 2 * n_pix, H, Mc, n_out, MNIST_HP, np.float64, seed=5, density=1.0)
+        net.net.set_frozen_cache_limit(limit)
+        net.net.initiate_training(X, Y)
+        net.net.train_batches(1, 800, orders[0], none, 0, 0, 3, True)
+        for order in orders[1:]:  # 800 rows in batches of 100, the other 900 in two
+            net.net.train_batches(1, 100, order, none, 0, 0, 8, False)
+            net.net.train_batches(1, 800, order, none, 0, 1, 2, True)
+        net.net.training_done()
+        states.append({name: np.array(getattr(net._layers[1], name)) for name in ("Ci", "Cj", "Cij", "weights", "bias")})
+    for other in states[:2]:
+        for name, value in states[2].items():
+            assert np.array_equal(value, other[name]), name
 
 
 def test_epoch_whose_images_could_not_be_laid_out_goes_on_when_they_can():
