@@ -869,6 +869,64 @@ def test_calls_with_small_copies_reuse_the_ring(hb, N, M, B):
         assert np.array_equal(getattr(quiet[1], name), getattr(talking[1], name)), name
 
 
+@pytest.mark.parametrize("N,M,B", [(7, 40, 5), (100, 48, 32), (784, 60, 33), (2000, 50, 128), (3000, 64, 77)])
+def test_small_copies_bring_what_belongs_to_their_call(hb, N, M, B):
+    """More calls in a row than the ring has chunks, other inputs each time: activations alone, steps alone, and steps,
+    weights written, activations and state read in turn.  Every result is compared with what numpy makes of that call's
+    own inputs (float64), from which those of the call before are further away than the tolerance."""
+    tau, tol = 0.05, 1e-5
+    rng = np.random.default_rng(N + 1)
+    net = hb.Network(np.float32)
+    layer = hb.DenseLayer(N, M // 2, 2, tau, (0.3, 0.5, 0.15), np.float32)
+    net.add_layer(layer)
+    bias = np.float64(layer.bias)
+    traces = [np.full(N, 0.3), np.full(M, 0.5), np.full((N, M), 0.15)]
+    seen = {}
+
+    def check(name, got, want):
+        assert np.max(np.abs(got - want)) <= tol, name
+        assert name not in seen or np.max(np.abs(got - seen[name])) > 10 * tol, name
+        seen[name] = got
+
+    def batch():
+        return rng.random((B, N)).astype(np.float32), rng.random((B, M)).astype(np.float32)
+
+    def activation(W):
+        x, _ = batch()
+        logits = (np.float64(x) @ np.float64(W) + bias).reshape(B, M // 2, 2)
+        e = np.exp(logits - logits.max(2, keepdims=True))
+        check("activation", layer.compute_activation(x), (e / e.sum(2, keepdims=True)).reshape(B, M))
+
+    def step():
+        x, y = batch()
+        layer.train_step(x, y)
+        for t, mean in zip(traces, (np.float64(x).mean(0), np.float64(y).mean(0), np.float64(x).T @ np.float64(y) / B)):
+            t *= 1 - tau
+            t += tau * mean
+
+    def state():
+        for name, t in zip(("Ci", "Cj", "Cij"), traces):
+            check(name, getattr(layer, name), t)
+
+    def weights():
+        # (sum |x w| of a logit is about 1: its float32 error stays far below the tolerance)
+        return (rng.standard_normal((N, M)) / N).astype(np.float32) * np.float32(2 * np.sqrt(N))
+
+    W = weights()
+    layer.weights = W
+    for _ in range(9):
+        activation(W)
+    for _ in range(9):
+        step()
+    state()
+    for _ in range(9):
+        step()
+        W = weights()
+        layer.weights = W
+        activation(W)
+        state()
+
+
 def test_state_of_two_networks_from_two_threads():
     """The pinned ring that state goes through is one for all networks: small arrays (moved by a kernel) and big ones (by
     the copy engine, in pieces) of two networks, written and read back by a thread each, keep apart."""
