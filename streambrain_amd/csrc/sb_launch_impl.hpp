@@ -52,13 +52,13 @@ static int forward_variant(hipStream_t st, ForwardArgs<T> a, bool vec) {
   return 0;
 }
 
-// The softmax behind a pass whose hypercolumns are spread over workgroups (TPR: as of the fused kernel it stands in for).
-template <typename T, int TPR>
+// The softmax behind a pass whose hypercolumns are spread over workgroups.
+template <typename T>
 static int launch_softmax_as_fused(hipStream_t st, T *act, long B, long H, long Mc) {
-  SB_REQUIRE(Mc <= 16 * TPR, "hypercolumn too wide");
-  const long groups = B * H, blocks = cdiv(groups, 256 / TPR);
+  SB_REQUIRE(Mc <= 16 * 32, "hypercolumn too wide");
+  const long groups = B * H, blocks = cdiv(groups, 256 / 32);
   SB_REQUIRE(blocks < (1L << 31), "too many groups");
-  hipLaunchKernelGGL((k_softmax_as_fused<T, TPR>), dim3((unsigned)blocks), dim3(256), 0, st, act, groups, Mc);
+  hipLaunchKernelGGL((k_softmax_as_fused<T>), dim3((unsigned)blocks), dim3(256), 0, st, act, groups, Mc);
   SB_LAUNCH_CHECK();
   return 0;
 }
@@ -126,7 +126,7 @@ int launch_forward_classify(hipStream_t st, T *act, const T *x, const T *W, cons
       a.col_tiles = cdiv(M, GW);
       int rc = forward_variant<T, 1, false>(st, a, base_vec);
       if (rc) return rc;
-      return launch_softmax_as_fused<T, 32>(st, act, B, H, Mc);
+      return launch_softmax_as_fused<T>(st, act, B, H, Mc);
     }
     a.col_tiles = H;
     // Hypercolumns that need 7 column blocks of 16 (97..112 columns, e.g. 100): the last group runs
@@ -185,8 +185,8 @@ int launch_forward_classify(hipStream_t st, T *act, const T *x, const T *W, cons
       case 7: return blocks(std::integral_constant<int, 7>{});
       case 8: return blocks(std::integral_constant<int, 8>{});
     }
-    if (need <= 4) return forward_variant<T, 4, true>(st, a, vec);
-    if constexpr (sizeof(T) == 8) return forward_variant<T, 7, true>(st, a, vec);
+    if constexpr (sizeof(T) == 4) return forward_variant<T, 4, true>(st, a, vec);
+    else return forward_variant<T, 7, true>(st, a, vec);
   }
   // Tiles of two column groups, of one where the former leave half the CUs idle (time of two over time of one, 5 to 128
   // tiles: 64 inputs 1.0 to 1.1, 200 1.3, 300 1.4, 1000 1.55; doubles 1.0, 1.25, 1.3, 1.5; at 192 tiles 0.75 to 0.9 for all)
