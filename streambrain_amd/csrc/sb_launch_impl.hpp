@@ -129,46 +129,44 @@ int launch_forward_classify(hipStream_t st, T *act, const T *x, const T *W, cons
       return launch_softmax_as_fused<T>(st, act, B, H, Mc);
     }
     a.col_tiles = H;
-    // Hypercolumns that need 7 column blocks of 16 (97..112 columns, e.g. 100): the last group runs
-    // with 3 (float) or 1 (double) blocks instead of VW, provided none of its vectors straddles the
-    // end of the hypercolumn.
+    // Hypercolumns that need 7 column blocks of 16 (97..112 columns, e.g. 100).
     const long nblocks = cdiv(Mc, 16);
     if (vec && nblocks == 7) {
       constexpr int NGL = 8 / VW, LWL = 7 - (NGL - 1) * VW;  // float: 2 groups, 3 blocks; double: 4, 1
-      if ((Mc - (NGL - 1) * GW) % LWL == 0) {
-        // Large batches: 64 or 32 rows per workgroup instead of 16 while there still are enough tiles for
-        // eight rounds / one round of workgroups, so that W crosses the L2 -> L1 path a quarter / half as
-        // often (64 rows with fewer rounds lose more to the last, partly filled round than they gain).
-        const long cus = device_cu_count();
-        // (double: at most 32 rows, 64 do not fit the register file)
-        long rb = sizeof(T) == 4 && H * cdiv(B, 64) >= 8 * cus ? 4 : (H * cdiv(B, 32) >= cus ? 2 : 1);
-        // (32-bit byte offsets inside the tile's rows)
-        while (rb > 1 && 16 * rb * N * (long)sizeof(T) >= (1L << 31)) rb /= 2;
-        a.batch_tiles = cdiv(B, 16 * rb);
-        a.by_batch_tiles = FastDiv::of(a.batch_tiles);
-        ProfScope prof_(st, K_FORWARD);
-        const long grid = 8 * cdiv(a.col_tiles * a.batch_tiles, 8);
-        SB_REQUIRE(grid < (1L << 31), "too many tiles for one launch");
-        const dim3 g((unsigned)grid);
-        if constexpr (sizeof(T) == 4) {
-          // 100 columns = 6 blocks of 16 + 4: the last four as 4x4 products instead of a seventh block
-          if (Mc == 6 * 16 + 4) {
-            if (rb == 4) hipLaunchKernelGGL((k_forward<T, 2, true, true, 8, 2, 4, true>), g, dim3(512), 0, st, a);
-            else if (rb == 2) hipLaunchKernelGGL((k_forward<T, 2, true, true, 8, 2, 2, true>), g, dim3(512), 0, st, a);
-            else hipLaunchKernelGGL((k_forward<T, 2, true, true, 8, 2, 1, true>), g, dim3(512), 0, st, a);
-            SB_LAUNCH_CHECK();
-            return 0;
-          }
-          if (rb == 4) hipLaunchKernelGGL((k_forward<T, NGL, true, true, 8, LWL, 4>), g, dim3(512), 0, st, a);
+      // Large batches: 64 or 32 rows per workgroup instead of 16 while there still are enough tiles for
+      // eight rounds / one round of workgroups, so that W crosses the L2 -> L1 path a quarter / half as
+      // often (64 rows with fewer rounds lose more to the last, partly filled round than they gain).  A vector of
+      // the last group may straddle the hypercolumn's end here (1568 -> 30 x 104, 16 rows a workgroup / as many as
+      // this says: batch 512 62 / 56 us, 4096 414 / 373; 60 x 104, batch 256 62 / 56).
+      const long cus = device_cu_count();
+      // (double: at most 32 rows, 64 do not fit the register file)
+      long rb = sizeof(T) == 4 && H * cdiv(B, 64) >= 8 * cus ? 4 : (H * cdiv(B, 32) >= cus ? 2 : 1);
+      // (32-bit byte offsets inside the tile's rows)
+      while (rb > 1 && 16 * rb * N * (long)sizeof(T) >= (1L << 31)) rb /= 2;
+      a.batch_tiles = cdiv(B, 16 * rb);
+      a.by_batch_tiles = FastDiv::of(a.batch_tiles);
+      ProfScope prof_(st, K_FORWARD);
+      const long grid = 8 * cdiv(a.col_tiles * a.batch_tiles, 8);
+      SB_REQUIRE(grid < (1L << 31), "too many tiles for one launch");
+      const dim3 g((unsigned)grid);
+      if constexpr (sizeof(T) == 4) {
+        // 100 columns = 6 blocks of 16 + 4: the last four as 4x4 products instead of a seventh block
+        if (Mc == 6 * 16 + 4) {
+          if (rb == 4) hipLaunchKernelGGL((k_forward<T, 2, true, true, 8, 2, 4, true>), g, dim3(512), 0, st, a);
+          else if (rb == 2) hipLaunchKernelGGL((k_forward<T, 2, true, true, 8, 2, 2, true>), g, dim3(512), 0, st, a);
+          else hipLaunchKernelGGL((k_forward<T, 2, true, true, 8, 2, 1, true>), g, dim3(512), 0, st, a);
+          SB_LAUNCH_CHECK();
+          return 0;
         }
-        if (rb == 4) {
-        } else if (rb == 2)
-          hipLaunchKernelGGL((k_forward<T, NGL, true, true, 8, LWL, 2>), g, dim3(512), 0, st, a);
-        else
-          hipLaunchKernelGGL((k_forward<T, NGL, true, true, 8, LWL>), g, dim3(512), 0, st, a);
-        SB_LAUNCH_CHECK();
-        return 0;
+        if (rb == 4) hipLaunchKernelGGL((k_forward<T, NGL, true, true, 8, LWL, 4>), g, dim3(512), 0, st, a);
       }
+      if (rb == 4) {
+      } else if (rb == 2)
+        hipLaunchKernelGGL((k_forward<T, NGL, true, true, 8, LWL, 2>), g, dim3(512), 0, st, a);
+      else
+        hipLaunchKernelGGL((k_forward<T, NGL, true, true, 8, LWL>), g, dim3(512), 0, st, a);
+      SB_LAUNCH_CHECK();
+      return 0;
     }
     // As many blocks of 16 columns as the hypercolumn has, up to 8; wider ones in whole groups.
     auto blocks = [&](auto count) {
@@ -215,7 +213,8 @@ template <typename T>
 static RowsGroups forward_rows_groups(long Mc) {
   constexpr int VW = Real<T>::VW, GW = 16 * VW, NGL = 8 / VW, LWL = 7 - (NGL - 1) * VW;
   // hypercolumns of 7 column blocks of 16 (97..112 columns): the last group runs with 3 (float) or 1
-  // (double) blocks, provided none of its vectors straddles the end of the hypercolumn (as in launch_forward)
+  // (double) blocks, provided none of its vectors straddles the end of the hypercolumn (this kernel's loads of W
+  // know no bounds)
   if (cdiv(Mc, 16) == 7 && (Mc - (NGL - 1) * GW) % LWL == 0) return {NGL, LWL};
   // and of 13 column blocks (193..208 columns, 200 among them): one block in the last group
   // (float: 4 groups, 12 + 1 blocks; double: 7, 12 + 1)

@@ -752,7 +752,7 @@ def test_forward_with_few_tiles(k, dtype, B, N, H, Mc):
 
 
 @pytest.mark.parametrize("dtype", DT)
-@pytest.mark.parametrize("Mc", [5, 10, 16, 17, 31, 33, 47, 49, 64, 66, 67, 80, 81, 95, 97, 101, 111, 113, 127, 128])
+@pytest.mark.parametrize("Mc", [5, 10, 16, 17, 31, 33, 40, 44, 47, 49, 64, 66, 67, 80, 81, 95, 97, 101, 104, 108, 111, 113, 127, 128])
 @pytest.mark.parametrize("B,N", [(17, 203), (33, 1024)])
 def test_forward_in_blocks_of_columns(k, dtype, Mc, B, N):
     """Hypercolumns of one to eight blocks of 16 columns, full ones and ones that end inside a lane's vector, the last of them
@@ -775,6 +775,27 @@ def test_forward_in_blocks_of_columns(k, dtype, Mc, B, N):
         W = W * np.repeat(wmask, Mc, axis=1).astype(dtype)
         for blocked in (False, True):
             assert_close(k.compute_activation_rows(W, bias, x, wmask, H, Mc, blocked), want(W), dtype, "rows", scale=10)
+
+
+@pytest.mark.parametrize("dtype", DT)
+@pytest.mark.parametrize("Mc", [100, 104, 108, 112])
+@pytest.mark.parametrize("B", [1000, 14700])
+def test_forward_of_seven_blocks_of_columns_in_batches_of_many_rows(k, dtype, Mc, B):
+    """Hypercolumns of 97 to 112 columns in tiles of 32 and of 64 batch rows, ragged ones among them: numpy's values, and in
+    floats the bits that a batch of a few rows gives the same rows (doubles, four column groups, have a softmax of its own
+    behind the pass where the tiles fill the chip badly)."""
+    rng, N, H = np.random.default_rng(Mc), 68, 9
+    x = rng.random((B, N)).astype(dtype)
+    W = (rng.standard_normal((N, H * Mc)) * 4 / np.sqrt(N)).astype(dtype)
+    bias = rng.standard_normal(H * Mc).astype(dtype)
+    act = k.compute_activation(W, bias, x, H, Mc)
+    for lo in (0, B // 2, B - 17):
+        rows = x[lo:lo + 17]
+        if dtype is np.float32:
+            assert np.array_equal(act[lo:lo + 17], k.compute_activation(W, bias, rows, H, Mc)), lo
+        z = (rows.astype(np.float64) @ W.astype(np.float64) + bias).reshape(17, H, Mc)
+        e = np.exp(z - z.max(2, keepdims=True))
+        assert_close(act[lo:lo + 17], (e / e.sum(2, keepdims=True)).reshape(17, -1), dtype, "dense", scale=10)
 
 
 @pytest.mark.parametrize("dtype", DT)
