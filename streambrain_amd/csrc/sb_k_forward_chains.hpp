@@ -32,8 +32,12 @@ constexpr int kChains = 4;
 constexpr int kChainSeg = 4096;  // list entries of a chain staged at a time
 
 // XT: as in k_forward_rows.  W stays below 4 GiB.
-template <typename T, bool XT>
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(3)))
+// MIXED: wavefronts of a workgroup may have pieces of different widths, each walked in code of its own, between barriers
+// that all of them meet at.  Otherwise a workgroup is in one such code from start to end, with fewer registers
+// (27648 -> 15 x 100, lists of 15800, batch 128, whose pieces are of four and of three blocks: 94 us this way, 88.5
+// otherwise).
+template <typename T, bool XT, bool MIXED>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(MIXED ? 2 : 3)))
 void k_forward_chains(ForwardChainsArgs<T> ac) {
   const ForwardRowsArgs<T> &ar = ac.r;
   const ForwardArgs<T> &a = ar.f;
@@ -77,18 +81,14 @@ void k_forward_chains(ForwardChainsArgs<T> ac) {
   const int chunks = (cnt + KC - 1) / KC;
   const int mine = chunks > (int)ch ? (chunks - 1 - (int)ch) / kChains + 1 : 1;
 
-  // sums of the piece's blocks of 16 columns: those of NB = 4 (a piece of fewer leaves the last ones alone)
-  acc_t acc[4];
-#pragma unroll
-  for (int k = 0; k < 4; k++) acc[k] = acc_t{0, 0, 0, 0};
   // the lane's first column of group g; a vector that would run over the piece's end starts earlier (its columns are
   // computed twice, with the same result)
   auto first_col = [&](int g, int width) {
     const int c = g * 16 * VW + width * p, last = ncol - width;
     return c < last ? c : (last > 0 ? last : 0);
   };
-  // adds up the n chunks of the staged segment (per wavefront: no barriers in here)
-  auto walk = [&](auto nblocks, int n) {
+  // adds up the n chunks of the staged segment (per wavefront: no barriers in here); acc: a sum per block of 16 columns
+  auto walk = [&](auto nblocks, int n, auto &acc) {
     constexpr int NB = decltype(nblocks)::value, NG = (NB + VW - 1) / VW, LW = NB - (NG - 1) * VW;
     auto width = [](int g) { return g == NG - 1 ? LW : VW; };
     unsigned wcol[NG];
@@ -144,7 +144,7 @@ void k_forward_chains(ForwardChainsArgs<T> ac) {
     for (int u = 0; u < D - 1; u++)
       if (i + u < n) compute(xr[u], wt[u]);
   };
-  auto store = [&](auto nblocks) {
+  auto store = [&](auto nblocks, const auto &acc) {
     constexpr int NB = decltype(nblocks)::value, NG = (NB + VW - 1) / VW, LW = NB - (NG - 1) * VW;
     auto width = [](int g) { return g == NG - 1 ? LW : VW; };
     T *const out = ac.part + (long)ch * a.B * a.M + j0;
@@ -161,44 +161,58 @@ void k_forward_chains(ForwardChainsArgs<T> ac) {
       }
     }
   };
-  auto with_blocks = [&](auto what) {  // (uniform per wavefront)
-    if (nb == 4) what(std::integral_constant<int, 4>{});
-    else if (nb == 3) what(std::integral_constant<int, 3>{});
-    else if (nb == 2) what(std::integral_constant<int, 2>{});
+  auto with_blocks = [&](int count, auto what) {
+    if (count == 4) what(std::integral_constant<int, 4>{});
+    else if (count == 3) what(std::integral_constant<int, 3>{});
+    else if (count == 2) what(std::integral_constant<int, 2>{});
     else what(std::integral_constant<int, 1>{});
   };
-
-  // All wavefronts of the workgroup, whatever their pieces, stage the list and meet at the barriers here.
-  int left = mine;
-  for (int c0 = 0; left > 0; c0 += SEGC, left -= SEGC) {
-    const int n = left < SEGC ? left : SEGC;
-    if (c0 > 0) __syncthreads();  // everyone is done with the staged segment
-    // (D - 1 chunks beyond the last one are requested and not used: padding)
-    const int stage = (n + D - 1 < SEGC ? n + D - 1 : SEGC) * KC;
-    constexpr int U = 4;
-    for (int e0 = tid; e0 < stage; e0 += threads * U) {
-      int r[U];
+  // Stages the list segment by segment, all wavefronts together; `on_segment` of the active ones in between.
+  auto segments = [&](auto on_segment) {
+    int left = mine;
+    for (int c0 = 0; left > 0; c0 += SEGC, left -= SEGC) {
+      const int n = left < SEGC ? left : SEGC;
+      if (c0 > 0) __syncthreads();  // everyone is done with the staged segment
+      // (D - 1 chunks beyond the last one are requested and not used: padding)
+      const int stage = (n + D - 1 < SEGC ? n + D - 1 : SEGC) * KC;
+      constexpr int U = 4;
+      for (int e0 = tid; e0 < stage; e0 += threads * U) {
+        int r[U];
 #pragma unroll
-      for (int u = 0; u < U; u++) {
-        const int e = e0 + threads * u;
-        const long k = ((long)(c0 + e / KC) * kChains + ch) * KC + e % KC;
-        const bool on = e < n * KC && k < ar.cap;
-        r[u] = list[on ? k : 0];
-        r[u] = on ? r[u] : -1;
-      }
+        for (int u = 0; u < U; u++) {
+          const int e = e0 + threads * u;
+          const long k = ((long)(c0 + e / KC) * kChains + ch) * KC + e % KC;
+          const bool on = e < n * KC && k < ar.cap;
+          r[u] = list[on ? k : 0];
+          r[u] = on ? r[u] : -1;
+        }
 #pragma unroll
-      for (int u = 0; u < U; u++) {
-        const int e = e0 + threads * u;
-        if (e < stage) {
-          woff[e] = r[u] < 0 ? 0u : (unsigned)r[u] * (unsigned)(a.M * sizeof(T));
-          xoff[e] = r[u] < 0 ? BufferWindow<T>::kOutside : (unsigned)r[u] * XSTEP;
+        for (int u = 0; u < U; u++) {
+          const int e = e0 + threads * u;
+          if (e < stage) {
+            woff[e] = r[u] < 0 ? 0u : (unsigned)r[u] * (unsigned)(a.M * sizeof(T));
+            xoff[e] = r[u] < 0 ? BufferWindow<T>::kOutside : (unsigned)r[u] * XSTEP;
+          }
         }
       }
+      __syncthreads();
+      if (active) on_segment(n);
     }
-    __syncthreads();
-    if (active) with_blocks([&](auto nblocks) { walk(nblocks, n); });
+  };
+  if constexpr (MIXED) {
+    acc_t acc[4] = {acc_t{0, 0, 0, 0}, acc_t{0, 0, 0, 0}, acc_t{0, 0, 0, 0}, acc_t{0, 0, 0, 0}};
+    segments([&](int n) { with_blocks(nb, [&](auto nblocks) { walk(nblocks, n, acc); }); });
+    if (active) with_blocks(nb, [&](auto nblocks) { store(nblocks, acc); });
+  } else {
+    const int first = cg * ac.waves_cols;  // (its width is that of all of the workgroup's pieces)
+    with_blocks(each + (first < more ? 1 : 0), [&](auto nblocks) {
+      acc_t acc[decltype(nblocks)::value];
+#pragma unroll
+      for (auto &sum : acc) sum = acc_t{0, 0, 0, 0};
+      segments([&](int n) { walk(nblocks, n, acc); });
+      if (active) store(nblocks, acc);
+    });
   }
-  if (active) with_blocks(store);
 }
 
 // act = softmax_per_hypercolumn(the four chains added up as forward_finish does + bias), with forward_finish's arithmetic

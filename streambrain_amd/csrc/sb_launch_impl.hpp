@@ -353,8 +353,11 @@ int launch_forward_rows(hipStream_t st, T *act, const T *x, const T *W, const T 
       plan.args.r = a;
       plan.args.part = (T *)scratch;
       const dim3 g((unsigned)(8 * cdiv(plan.workgroups, 8))), blk(64 * plan.waves);
-      if (x_blocked) hipLaunchKernelGGL((k_forward_chains<T, true>), g, blk, 0, st, plan.args);
-      else hipLaunchKernelGGL((k_forward_chains<T, false>), g, blk, 0, st, plan.args);
+      const bool mixed = plan.args.waves_cols > 1 && cdiv(Mc, 16) % plan.args.pieces != 0;
+      if (x_blocked && mixed) hipLaunchKernelGGL((k_forward_chains<T, true, true>), g, blk, 0, st, plan.args);
+      else if (x_blocked) hipLaunchKernelGGL((k_forward_chains<T, true, false>), g, blk, 0, st, plan.args);
+      else if (mixed) hipLaunchKernelGGL((k_forward_chains<T, false, true>), g, blk, 0, st, plan.args);
+      else hipLaunchKernelGGL((k_forward_chains<T, false, false>), g, blk, 0, st, plan.args);
       SB_LAUNCH_CHECK();
       hipLaunchKernelGGL((k_softmax_of_chains<T>), dim3((unsigned)cdiv(B * H, 8)), dim3(128), 0, st, act,
                          (const T *)plan.args.part, bias, B, H, Mc);
