@@ -435,10 +435,11 @@ void k_forward(ForwardArgs<T> a) {
 
 // The softmax of forward_finish on stored logits (kernels_numpy.py:13-25), in place, with the same arithmetic in the same
 // order, so that a pass whose hypercolumns are computed by several workgroups gives the bits of one that is
-// fused: 32 threads per (row, hypercolumn), thread lr has units lr + 32 t, at most 16 of them.
-template <typename T>
+// fused: TPR threads per (row, hypercolumn), thread lr has units lr + TPR t, at most 16 of them.
+template <typename T, int TPR>
 __global__ __launch_bounds__(256) void k_softmax_as_fused(T *act, long groups, long Mc) {
-  constexpr int TPR = 32, PT = 16;
+  constexpr int PT = 16;
+  static_assert(TPR == 16 || TPR == 32, "rows of 16 lanes");
   const long g = (long)blockIdx.x * (256 / TPR) + threadIdx.x / TPR;
   const int lr = threadIdx.x % TPR;
   T *const v = act + (g < groups ? g : groups - 1) * Mc;  // (lanes past the end take part in the exchanges)
@@ -450,8 +451,10 @@ __global__ __launch_bounds__(256) void k_softmax_as_fused(T *act, long groups, l
     mx = (col < Mc && vals[t] > mx) ? vals[t] : mx;
   }
   mx = row16_reduce(mx, [](T x, T y) { return y > x ? y : x; });
-  const T other = __shfl_xor(mx, 16);
-  mx = other > mx ? other : mx;
+  if constexpr (TPR == 32) {
+    const T other = __shfl_xor(mx, 16);
+    mx = other > mx ? other : mx;
+  }
   T sum = T(0);
 #pragma unroll
   for (int t = 0; t < PT; t++)
@@ -460,7 +463,7 @@ __global__ __launch_bounds__(256) void k_softmax_as_fused(T *act, long groups, l
       sum += vals[t];
     }
   sum = row16_reduce(sum, [](T x, T y) { return x + y; });
-  sum += __shfl_xor(sum, 16);
+  if constexpr (TPR == 32) sum += __shfl_xor(sum, 16);
   const T r = T(1) / sum;
   if (g >= groups) return;
 #pragma unroll

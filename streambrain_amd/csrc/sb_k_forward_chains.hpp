@@ -17,7 +17,8 @@ namespace sb {
 // blocks of 16 columns (200 columns: 4 + 3 + 3 + 3 blocks, not 64 + 64 + 64 + 8 columns), two to a SIMD where the chip
 // is filled twice.  W is read once per 64 or 128 batch rows, by wavefronts side by side on a CU.
 // 27648 -> 15 x 200, lists of 15800, batch 128, floats: 151 us with the softmax where W is found in the memory-side cache,
-// 202 where it has just been written past it (a workgroup of k_forward_rows per column group: 223 and 252).  Then the
+// 202 where it has just been written past it (passes one after the other 134, a workgroup of k_forward_rows per column
+// group 162).  Then the
 // lines that a CU's L1 holds for what is on its way are the bound, a half line of x per entry and 16 batch rows among
 // them: four or twelve chunks ahead, the same time.  32 rows (30 tiles, narrower pieces): 113 -> 64 us.
 template <typename T>

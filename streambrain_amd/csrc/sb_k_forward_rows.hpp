@@ -69,8 +69,10 @@ constexpr int forward_rows_waves_per_simd() {
 // WIDE: W beyond the 4 GiB that such an offset reaches.  Offsets then count from the segment's first row; a segment that
 // spans more than 4 GiB (in some layers of few inputs a single row does) is walked with 64-bit addresses (55296 -> 200 x
 // 100, density 0.05, batch 256: 362 -> 314 us, all addresses in 64 bits 420).
+// SPLIT: a workgroup computes column group blockIdx.y (NG groups wide) of its hypercolumn only and stores the logits;
+// every sum is formed as without (same wavefronts, same chunks), k_softmax_as_fused does the rest.
 template <typename T, int NG, int NWAVES, int RB = 1, bool XT = false, int LW = Real<T>::VW, int SEG = 2048,
-          bool WIDE = false>
+          bool WIDE = false, bool SPLIT = false>
 __global__ __launch_bounds__(64 * NWAVES)
 __attribute__((amdgpu_waves_per_eu(forward_rows_waves_per_simd<T, NG, RB, LW>(),
                                    forward_rows_waves_per_simd<T, NG, RB, LW>())))
@@ -100,7 +102,9 @@ void k_forward_rows(ForwardRowsArgs<T> ar) {
   const int tid = threadIdx.x, lane = tid & 63, p = lane & 15, q = lane >> 4;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const long b0 = bt * (16 * RB);
-  const long j0 = ct * a.Mc, ncol = a.Mc;
+  const long jg = SPLIT ? (long)blockIdx.y * (NG * 16 * VW) : 0;  // first column inside the hypercolumn
+  const long j0 = ct * a.Mc + jg;
+  const long ncol = SPLIT && a.Mc - jg > NG * 16 * VW ? NG * 16 * VW : a.Mc - jg;
   const int *list = ar.rows + ct * ar.cap;
 
   constexpr unsigned XSTEP = (XT ? 16u : 1u) * (unsigned)sizeof(T);  // bytes between input columns
@@ -258,7 +262,7 @@ void k_forward_rows(ForwardRowsArgs<T> ar) {
 #pragma unroll
   for (int r = 0; r < RB; r++) {
     if (r > 0) __syncthreads();  // the previous row block's sums have been read
-    forward_finish<T, NG, true, NWAVES, LW, false, NT>(acc[r], bv, red, a.act, a.B, a.M, b0 + 16 * r, j0, ncol);
+    forward_finish<T, NG, !SPLIT, NWAVES, LW, false, NT>(acc[r], bv, red, a.act, a.B, a.M, b0 + 16 * r, j0, ncol);
   }
 }
 

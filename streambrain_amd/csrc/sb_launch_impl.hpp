@@ -52,13 +52,13 @@ static int forward_variant(hipStream_t st, ForwardArgs<T> a, bool vec) {
   return 0;
 }
 
-// The softmax behind a pass whose hypercolumns are spread over workgroups.
-template <typename T>
+// The softmax behind a pass whose hypercolumns are spread over workgroups (TPR: as of the fused kernel it stands in for).
+template <typename T, int TPR>
 static int launch_softmax_as_fused(hipStream_t st, T *act, long B, long H, long Mc) {
-  SB_REQUIRE(Mc <= 16 * 32, "hypercolumn too wide");
-  const long groups = B * H, blocks = cdiv(groups, 256 / 32);
+  SB_REQUIRE(Mc <= 16 * TPR, "hypercolumn too wide");
+  const long groups = B * H, blocks = cdiv(groups, 256 / TPR);
   SB_REQUIRE(blocks < (1L << 31), "too many groups");
-  hipLaunchKernelGGL((k_softmax_as_fused<T>), dim3((unsigned)blocks), dim3(256), 0, st, act, groups, Mc);
+  hipLaunchKernelGGL((k_softmax_as_fused<T, TPR>), dim3((unsigned)blocks), dim3(256), 0, st, act, groups, Mc);
   SB_LAUNCH_CHECK();
   return 0;
 }
@@ -126,7 +126,7 @@ int launch_forward_classify(hipStream_t st, T *act, const T *x, const T *W, cons
       a.col_tiles = cdiv(M, GW);
       int rc = forward_variant<T, 1, false>(st, a, base_vec);
       if (rc) return rc;
-      return launch_softmax_as_fused<T>(st, act, B, H, Mc);
+      return launch_softmax_as_fused<T, 32>(st, act, B, H, Mc);
     }
     a.col_tiles = H;
     // Hypercolumns that need 7 column blocks of 16 (97..112 columns, e.g. 100).
@@ -287,6 +287,21 @@ static int forward_rows_variant(hipStream_t st, ForwardRowsArgs<T> a, long like)
   return 0;
 }
 
+// Few tiles: a workgroup of k_forward_rows per column group of a hypercolumn, then the softmax, every sum as in the fused
+// kernel.  The second launch costs about a microsecond.  Time this way over time fused, at 8 / 40 / 80 / 128 / 152 tiles:
+// 100 columns, lists of 300 1.09 / 1.11 / 1.12 / 1.13 / -, of 600 0.95 / 0.95 / 0.96 / 0.97 / 1.19, of 6000 0.68 / 0.67 / 0.69 /
+// 0.71 / 1.07; 200 columns, lists of 300 0.81 / 0.82 / 0.94 / 0.99 / -, of 6000 0.41 / 0.42 / 0.66 / 0.72 / 0.94; doubles, 64
+// columns, lists of 300 1.12 / 1.13 / 1.13 / 1.14 / -, of 600 0.98 / 0.98 / 1.00 / 1.01 / 1.19, of 6000 0.84 / 0.85 / 0.86 / 0.87
+// / 1.06; 128 columns, lists of 300 0.82 / 0.85 / 0.97 / 0.99 / -, of 1200 0.54 / 0.62 / 0.76 / 0.77 / 0.93, of 6000 0.50 / 0.51 /
+// 0.63 / 0.65 / 0.83.
+template <typename T>
+static bool forward_rows_splits(long B, long H, long Mc, long cap) {
+  const long tiles = H * cdiv(B, 16), cus = device_cu_count(), blocks = cdiv(Mc, 16);
+  if (blocks <= Real<T>::VW || cap <= 256) return false;  // (one column group; lists that may be summed in another order)
+  if (2 * tiles <= cus) return cap >= 608 || blocks >= (sizeof(T) == 4 ? 10 : 8);
+  return sizeof(T) == 8 && blocks >= 7 && 5 * tiles <= 3 * cus && cap >= 1280;
+}
+
 // How k_forward_chains covers a pass; no workgroups: it does not run.
 template <typename T>
 struct ChainsPlan {
@@ -302,16 +317,20 @@ static ChainsPlan<T> forward_chains_plan(long B, long N, long H, long Mc, long c
   const long M = H * Mc, cus = device_cu_count(), rbs = cdiv(B, 16), tiles = H * rbs;
   if (forward_rows_short<T>(like > 0 ? like : B, N, H, Mc, cap)) return plan;  // (another order of the four sums)
   if (N * M * (long)sizeof(T) > (1L << 32)) return plan;
-  // Few tiles and lists that pay for the second launch.  Time of k_forward_rows over time this way, at 40 / 80 / 120 / 152
-  // tiles: 100 columns, lists of 600 1.00 / 0.90 / 0.81 / 0.64, of 1200 1.26 / 1.13 / 1.01 / 0.76, of 6000 2.0 / 1.65 /
-  // 1.42 / 1.00; 200 columns 1.15 / 0.87 / 0.83 / 0.60, 1.52 / 1.06 / 1.03 / 0.71, 2.6 / 1.6 / 1.6 / 0.91; 64 columns,
-  // lists of 1200 1.02 / 0.92 / 0.89 / 0.71, of 2400 1.34 / 1.15 / 1.13 / 0.87; 12 columns 1.1, 1.47 whatever the tiles (at
-  // 320 1.30, 1.47); doubles, 64 columns, lists of 600 0.96 / 0.86 / 0.82 / 0.64, of 1200 1.24 / 1.05 / 1.01 / 0.77; 200
-  // columns 1.29 / 0.96 / 0.94 / 0.71, 1.71 / 1.21 / 1.18 / 0.78; 12 columns 0.97, 1.3.
   const long blocks = cdiv(Mc, 16), fewest = cdiv(blocks, 4);
-  const bool heavy = blocks * (long)sizeof(T) >= 28, few = 6 * tiles <= cus;
+  const bool few = 6 * tiles <= cus;
   if (2 * tiles > (blocks == 1 ? 3 * cus : cus)) return plan;
-  if (cap < (heavy ? (few ? 640 : 1152) : (few || blocks == 1 ? 1280 : 2048))) return plan;
+  // One and two blocks of columns: where the lists pay for the second launch (time of k_forward_rows over time this way:
+  // 12 columns, lists of 2400 0.84, of 3600 0.88 at 36 tiles, 1.1 from 112, of 6000 0.95 at 16, 1.25 from 40; 32 columns, of 900
+  // 0.9 to 0.98, of 1800 1.2; doubles, 12 columns, of 1800 0.82 up to 48 tiles, 1.08 from 112, of 3600 1.35; 32 columns, of 900
+  // 0.88, of 1800 1.08 to 1.19).
+  if (blocks <= 2) {
+    const long from = blocks == 2 ? (sizeof(T) == 4 ? 1152 : 1408)
+                                  : sizeof(T) == 4 ? (few ? 6016 : 3600) : (few ? 3072 : 1792);
+    if (cap < from) return plan;
+  } else if (cap < 640) {
+    return plan;
+  }
   ForwardChainsArgs<T> &c = plan.args;
   c.waves_rows = rbs >= 4 ? 4 : rbs >= 2 ? 2 : 1;
   c.row_groups = (int)cdiv(rbs, c.waves_rows);
@@ -327,7 +346,33 @@ static ChainsPlan<T> forward_chains_plan(long B, long N, long H, long Mc, long c
     else c.waves_rows *= 2, c.row_groups = (int)cdiv(rbs, c.waves_rows);
   }
   c.col_groups = (int)cdiv(c.pieces, c.waves_cols);
-  plan.workgroups = H * kChains * c.row_groups * c.col_groups;
+  const long workgroups = H * kChains * c.row_groups * c.col_groups;
+  if (blocks > 2) {
+    // Wider hypercolumns: which way the fullest CU is done first, by what 1300 shapes took (3 to 14 blocks, 8 to 128
+    // tiles, lists of 600 to 15800): microseconds per list entry, and per entry and block that a SIMD has in all (this way:
+    // wavefronts of a SIMD times blocks of a piece; k_forward_rows: workgroups on a CU, three at a time), and per million
+    // logits that pass through memory.  Estimates are within a tenth of the measured times in nine of ten; the way they choose
+    // is on average 0.7 % slower than the better one, k_forward_rows alone 13 % (doubles, 80 tiles of 200 columns, lists of
+    // 1200: 25.5 us there, 33.8 this way; 14 blocks of 16 batch rows, which fill neither, 9 x 160 columns, lists of 3600:
+    // 59 and 93; 27648 -> 15 x 200, lists of 15800, batch 128: 162 and 134).
+    const double L = (double)(cap - 24), logits = 1e-6 * (double)(B * M);  // (a list and its padding)
+    const long on_cu = cdiv(workgroups, cus) * (plan.waves / 4);
+    const double load = (double)(on_cu * cdiv(blocks, pieces));
+    const bool f = sizeof(T) == 4;
+    const double here = f ? 7.1 + L * (0.0014 + 0.00087 * load - (on_cu > 1 ? 0.0008 : 0)) + 19 * logits
+                          : 8.1 + L * (0.0025 + 0.0016 * load - (on_cu > 1 ? 0.0006 : 0)) + 27 * logits;
+    double there;
+    if (blocks <= Real<T>::VW) {
+      there = 3.9 + L * (0.0023 + 0.00083 * (double)blocks);
+    } else {
+      const long all = tiles * cdiv(blocks, Real<T>::VW), rounds = cdiv(all, 3 * cus);
+      const double load_there = (double)(3 * (rounds - 1) + cdiv(all - 3 * cus * (rounds - 1), cus));
+      there = f ? 6.2 + L * (0.0016 * (double)rounds + 0.0039 * load_there) + 4.3 * logits
+                : 4.9 + L * (0.0053 * (double)rounds + 0.0028 * load_there) + 15 * logits;
+    }
+    if (here >= there) return plan;
+  }
+  plan.workgroups = workgroups;
   return plan;
 }
 template <typename T>
@@ -365,8 +410,24 @@ int launch_forward_rows(hipStream_t st, T *act, const T *x, const T *W, const T 
       return 0;
     }
   }
+  constexpr int VW = Real<T>::VW, GW = 16 * VW;
+  if (forward_rows_splits<T>(B, H, Mc, cap)) {
+    ProfScope prof_(st, K_FORWARD);
+    a.f.by_batch_tiles = FastDiv::of(a.f.batch_tiles);
+    const dim3 g((unsigned)(8 * cdiv(H * a.f.batch_tiles, 8)), (unsigned)cdiv(Mc, GW)), blk(256);
+    const bool wide = N * H * Mc * (long)sizeof(T) > (1L << 32);
+    auto launch = [&](auto blocked) {
+      constexpr bool XT = decltype(blocked)::value;
+      if (wide) hipLaunchKernelGGL((k_forward_rows<T, 1, 4, 1, XT, VW, 2048, true, true>), g, blk, 0, st, a);
+      else hipLaunchKernelGGL((k_forward_rows<T, 1, 4, 1, XT, VW, 2048, false, true>), g, blk, 0, st, a);
+    };
+    if (x_blocked) launch(std::true_type{});
+    else launch(std::false_type{});
+    SB_LAUNCH_CHECK();
+    return launch_softmax_as_fused<T, 16>(st, act, B, H, Mc);
+  }
   if (like <= 0) like = B;
-  constexpr int VW = Real<T>::VW, NGL = 8 / VW, LWL = 7 - (NGL - 1) * VW, NGM = VW == 2 ? 7 : 4;
+  constexpr int NGL = 8 / VW, LWL = 7 - (NGL - 1) * VW, NGM = VW == 2 ? 7 : 4;
   const RowsGroups groups = forward_rows_groups<T>(Mc);
   if (groups.last > 0 && cdiv(Mc, 16) == 7) return forward_rows_variant<T, NGL, LWL>(st, a, like);
   if (groups.last > 0) return forward_rows_variant<T, NGM, 1>(st, a, like);

@@ -819,6 +819,76 @@ def test_chains_of_the_row_lists(k, dtype, B, N, H, Mc, more):
         assert np.array_equal(few, k.compute_activation_rows(W, bias, x, wmask, H, Mc, blocked)[:B])
 
 
+@pytest.mark.parametrize("dtype", DT)
+@pytest.mark.parametrize("B,N,H,Mc,more", [(40, 1500, 5, 100, 464), (128, 1300, 9, 200, 272), (7, 1400, 3, 68, 720),
+                                           (100, 620, 4, 256, 600), (16, 620, 7, 224, 320), (120, 2700, 16, 128, 160)])
+def test_row_lists_with_a_workgroup_per_column_group(k, dtype, B, N, H, Mc, more):
+    """Few tiles, lists that do not pay for four CUs a tile: a workgroup per group of columns gives the bits that a
+    larger batch gives the same rows.  Last groups of a few columns and whole ones; lists of a few entries and of none."""
+    if dtype is np.float64 and Mc > 224:
+        pytest.skip("wider than the row-list kernels of doubles take")
+    rng = np.random.default_rng(N + Mc)
+    M = H * Mc
+    wmask = (rng.random((N, H)) < 0.6).astype(np.uint8)
+    wmask[:, 1] = 0
+    wmask[:37, 2] = rng.random(37) < 0.8
+    x = rng.random((more, N), dtype=dtype)
+    W = rng.standard_normal((N, M), dtype=dtype) * np.repeat(wmask, Mc, axis=1).astype(dtype) * dtype(4 / np.sqrt(N))
+    bias = rng.standard_normal(M).astype(dtype)
+    z = (x[:B].astype(np.float64) @ W.astype(np.float64) + bias).reshape(B, H, Mc)
+    e = np.exp(z - z.max(2, keepdims=True))
+    for blocked in (False, True):
+        few = k.compute_activation_rows(W, bias, x[:B], wmask, H, Mc, blocked)
+        assert_close(few, (e / e.sum(2, keepdims=True)).reshape(B, M), dtype, "rows", scale=10)
+        assert np.array_equal(few, k.compute_activation_rows(W, bias, x, wmask, H, Mc, blocked)[:B])
+
+
+@pytest.mark.parametrize("dtype", DT)
+@pytest.mark.parametrize("B,N,H,Mc", [(33, 9000, 5, 100), (128, 6000, 9, 200), (16, 9000, 3, 48), (40, 12000, 4, 12)])
+def test_captured_row_list_pass_has_the_bits_of_the_eager_one(k, dtype, B, N, H, Mc):
+    """A captured pass does without the scratch in which an eager one spreads its tiles over more CUs: nothing is
+    allocated, and every replay gives the eager call's bits."""
+    from streambrain_amd import _capi
+    from streambrain_amd._capi import DeviceArray, check
+    lib, P, I = _capi.lib(), ctypes.c_void_p, ctypes.c_int
+    hip = ctypes.CDLL(_capi.LIB_PATH)
+    for name, args in (("hipStreamBeginCapture", [P, I]), ("hipStreamEndCapture", [P, ctypes.POINTER(P)]),
+                       ("hipGraphInstantiate", [ctypes.POINTER(P), P, P, P, ctypes.c_size_t]), ("hipGraphLaunch", [P, P]),
+                       ("hipGraphExecDestroy", [P]), ("hipGraphDestroy", [P])):
+        getattr(hip, name).argtypes, getattr(hip, name).restype = args, I
+    rng, M = np.random.default_rng(N + B), H * Mc
+    wmask = (rng.random((N, H)) < 0.6).astype(np.uint8)
+    cap = (int(wmask.sum(0, dtype=np.int64).max()) + 15) // 16 * 16 + 16
+    W = rng.standard_normal((N, M), dtype=dtype) * np.repeat(wmask, Mc, axis=1).astype(dtype) * dtype(4 / np.sqrt(N))
+    x, W, bias, wmask = (DeviceArray.from_numpy(a) for a in (rng.random((B, N), dtype=dtype), W,
+                                                            rng.standard_normal(M).astype(dtype), wmask))
+    act, rows, cnt = DeviceArray((B, M), dtype), DeviceArray((H, cap), np.int32), DeviceArray((H,), np.int32)
+    check(lib.sb_mask_rows(rows.ptr, cnt.ptr, wmask.ptr, N, H, cap))
+    forward = getattr(lib, "sb_compute_activation_rows" + ("_f32" if dtype is np.float32 else "_f64"))
+
+    def run():
+        check(forward(act.ptr, x.ptr, W.ptr, bias.ptr, rows.ptr, cnt.ptr, cap, B, N, H, Mc, None))
+
+    run()
+    check(lib.sb_sync())
+    eager = act.numpy()
+    stream, graph, replay = lib.sb_stream(), P(), P()
+    before = lib.sb_allocation_calls()
+    assert hip.hipStreamBeginCapture(stream, 1) == 0  # (thread-local mode)
+    run()
+    assert hip.hipStreamEndCapture(stream, ctypes.byref(graph)) == 0
+    assert lib.sb_allocation_calls() == before
+    assert hip.hipGraphInstantiate(ctypes.byref(replay), graph, None, None, 0) == 0
+    for k_ in range(4):
+        check(lib.sb_fill_bytes(act.ptr, 0, act.nbytes))
+        assert hip.hipGraphLaunch(replay, stream) == 0
+        check(lib.sb_sync())
+        assert np.array_equal(act.numpy(), eager), k_
+        run()
+        check(lib.sb_sync())
+    assert hip.hipGraphExecDestroy(replay) == 0 and hip.hipGraphDestroy(graph) == 0
+
+
 def _random_shapes(seed, count):
     """Shapes off every tiling's grid: mostly odd widths, batches around the 16- and 32-row boundaries."""
     rng = np.random.default_rng(seed)
