@@ -68,7 +68,8 @@ constexpr int forward_rows_waves_per_simd() {
 // doubles 256 rows of 3000 -> 30 x 64, density 0.3: 25.5 -> 23.1).
 // WIDE: W beyond the 4 GiB that such an offset reaches.  Offsets then count from the segment's first row; a segment that
 // spans more than 4 GiB (in some layers of few inputs a single row does) is walked with 64-bit addresses (55296 -> 200 x
-// 100, density 0.05, batch 256: 362 -> 314 us, all addresses in 64 bits 420).
+// 100, density 0.05, batch 256: 362 -> 314 us in passes one after the other, all addresses in 64 bits 420; in training steps,
+// behind the writing of W, 403 -> 364).
 // SPLIT: a workgroup computes column group blockIdx.y (NG groups wide) of its hypercolumn only and stores the logits;
 // every sum is formed as without (same wavefronts, same chunks), k_softmax_as_fused does the rest.
 template <typename T, int NG, int NWAVES, int RB = 1, bool XT = false, int LW = Real<T>::VW, int SEG = 2048,
